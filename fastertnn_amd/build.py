@@ -6,7 +6,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libftnn_hip.so")
-SOURCES = ["ftnn_api.hip", "pack_kernels.hip", "mm_kernels.hip", "mfma_kernels.hip", "stem_kernels.hip", "ftnn_net.hip",
+SOURCES = ["ftnn_api.hip", "pack_kernels.hip", "mm_kernels.hip", "mfma_kernels.hip", "rows_kernels.hip", "stem_kernels.hip", "ftnn_net.hip",
            "host_hash.cpp"]   # the last one is plain host C++
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
@@ -19,7 +19,8 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hi
 # refuses scratch use in them (the library checks the same at run time before the first launch).  The layer kernels
 # use ordinary loads that the compiler counts; scratch there would only be slow, and is refused as a performance guard.
 # Source -> name fragments.
-NO_SCRATCH = {"mfma_kernels.hip": ("k_conv_f4", "k_mfma")}   # "k_mfma" covers k_mfma_p4 as well
+NO_SCRATCH = {"mfma_kernels.hip": ("k_conv_f4", "k_mfma"),   # "k_mfma" covers k_mfma_p4 as well
+              "rows_kernels.hip": ("k_rows",)}
 
 
 def check_no_scratch(src, remarks):

@@ -260,11 +260,18 @@ int64_t mfma_packed4_bytes(int64_t rows, int Kw);
 hipError_t launch_mfma_pack4(bool ternary, const int64_t* d_rows, int rows, int Kw, void* d_out, hipStream_t st);
 hipError_t launch_mfma_gemm_packed4(int type, const void* d_ac, const void* d_bc, int64_t M, int OHW, int KN, int Kw, int K_unpack,
                                     float alpha, float* d_y, hipStream_t st);
-// scratch of launch_mm_mfma on the fp4 engine (it picks the operand form by shape)
+// whether launch_mm_mfma runs an fp4 product straight from the packed rows (launch_mm_rows): by shape
+bool mm_from_rows(int64_t M, int KN);
+// scratch of launch_mm_mfma on the fp4 engine
 int64_t mfma_f4_mm_scratch_bytes(int64_t M, int KN, int Kw);
 hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW,
                           int KN, int Kw, int K_unpack, float alpha, float* d_y, void* d_scratch,
                           hipStream_t st);
+
+// ---- rows_kernels.hip: the fp4 matrix-core product of packed rows as they are, one launch, no scratch ----
+bool mm_rows_within_limits(int Kw);   // fp32 sums of +-1 products stay exact
+hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
+                          float alpha, float* d_y, hipStream_t st);
 
 // conv layer on the fp4 matrix cores: activations from launch_quantize_f4, weights as the fp4 fragments
 // launch_mfma_expand(true, ...) makes of the packed weight rows (Kw = round4(cg.K) words per row)

@@ -1222,13 +1222,14 @@ hipError_t launch_gemm(const uint4* Pf, const uint4* Qf, float* Y, int M, int KN
     bool small = big < mfma_small_tile_below();
     // two fragments per step and a ring of four: four fragments per step with a ring of two (the same LDS, half
     // the barriers) measured 0.87 against 0.76 ms on 8192 x 8192 x 32768 -- the ring then no longer covers the loads
-    // Fewer than 112 tiles of 128 x 128 leave most compute units idle: tiles of 64 x 64 then, four K words per step
-    // (1024 x 1024 x 8192 as a whole call: 25.7 -> 19.0 us, 768: 21.2 -> 15.7, 1280 (100 tiles): 29.6 -> 27.2; from 144
-    // tiles on the larger tile is faster, 33.6 against 39.6 us at 1536; tiles of 128 x 64 lose everywhere).
-    // FTNN_MFMA_TINY_BELOW = n moves the threshold (tuning aid).
-    static const int tiny_below = getenv("FTNN_MFMA_TINY_BELOW") ? atoi(getenv("FTNN_MFMA_TINY_BELOW")) : 112;
-    const int64_t mid = (((int64_t)M + 127) / 128) * ((KN + 127) / 128);
-    if (small && mid < tiny_below) return launch_gemm_tile<F4, SWAP, 1, 1, 4, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st);
+    if constexpr (!F4) {
+        // Fewer than 112 tiles of 128 x 128 leave most compute units idle: tiles of 64 x 64 then, four K words per step
+        // (from 144 tiles on the larger tile is faster; tiles of 128 x 64 lose everywhere).  fp4 comes here from the layers'
+        // GEMM route only, which starts at 256 tiles.  FTNN_MFMA_TINY_BELOW = n moves the threshold (tuning aid).
+        static const int tiny_below = getenv("FTNN_MFMA_TINY_BELOW") ? atoi(getenv("FTNN_MFMA_TINY_BELOW")) : 112;
+        const int64_t mid = (((int64_t)M + 127) / 128) * ((KN + 127) / 128);
+        if (small && mid < tiny_below) return launch_gemm_tile<F4, SWAP, 1, 1, 4, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st);
+    }
     return small ? launch_gemm_tile<F4, SWAP, 2, 2, 2, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st)
                  : launch_gemm_tile<F4, SWAP, 4, 4, 2, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st);
 }
@@ -1505,24 +1506,27 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
     return by_mode(std::true_type{}, std::false_type{});   // BTN, BNN
 }
 
-// A whole call from packed rows expands both operands itself, so it may pick the operand form by shape: problems on
-// 128 x 128 tiles (few tiles; one workgroup per compute unit, nothing to hide the read -> unpack -> multiply chain of the
-// packed4 kernel's short steps) run faster on plain fp4 fragments (2048 x 2048 x 16384: 54 against 62 us, 1024 x 1024 x
-// 8192: 30 against 36), the large ones on packed4 in offset codes.
-static bool f4_whole_call_plain(int64_t M, int KN) {
-    return ((M + 255) / 256) * ((KN + 255) / 256) < mfma_small_tile_below();
+// A whole call from packed rows below 160 tiles of 256 x 256 multiplies the rows as they are (k_rows): packing both operands
+// first costs such a product more than the packed4 kernel gains.  Device time of the two, us (rows / packed4 or, before
+// k_rows, fragments): 2048 x 2048 x 16384 (64 tiles) 31.5 / 44, 3072 x 3072 x 24576 (144) 107 / 136; from 256 tiles on packed4
+// is ahead at any K (4096 x 4096 x 32768 218 / 190, x 2048 35 / 32, x 512 27 / 24).  Products narrower than 128 would leave more
+// than half of such a tile empty.
+bool mm_from_rows(int64_t M, int KN) {
+    return ((M + 255) / 256) * ((KN + 255) / 256) < mfma_small_tile_below() || KN < 128 || M < 128;
 }
 
+// (a product that runs from the rows uses none of it; callers size one buffer for whatever shapes they run)
 int64_t mfma_f4_mm_scratch_bytes(int64_t M, int KN, int Kw) {
-    return f4_whole_call_plain(M, KN) ? mfma_fragment_bytes(true, M, Kw) + mfma_fragment_bytes(true, KN, Kw)
-                                      : mfma_packed4_bytes(M, Kw) + mfma_packed4_bytes(KN, Kw);
+    return mm_from_rows(M, KN) ? mfma_fragment_bytes(true, M, Kw) + mfma_fragment_bytes(true, KN, Kw)
+                               : mfma_packed4_bytes(M, Kw) + mfma_packed4_bytes(KN, Kw);
 }
 
 hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW,
                           int KN, int Kw, int K_unpack, float alpha, float* d_y, void* d_scratch,
                           hipStream_t st) {
     const bool a_tern = (type == kTNN || type == kTBN), b_tern = (type == kTNN || type == kBTN);
-    if (f4 && !f4_whole_call_plain(M, KN)) {   // the fp4 GEMM takes its operands at two bits per lane
+    if (f4 && mm_from_rows(M, KN)) return launch_mm_rows(type, d_a, d_b, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
+    if (f4) {   // the fp4 GEMM takes its operands at two bits per lane
         void* Ac = d_scratch;
         void* Bc = static_cast<char*>(d_scratch) + mfma_packed4_bytes(M, Kw);
         const int64_t na64 = (M + 31) / 32 * 32, nb64 = ((int64_t)KN + 31) / 32 * 32;
@@ -1547,25 +1551,22 @@ hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* 
         return launch_mfma_gemm_packed4(type, Ac, Bc, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
     }
     void* Af = d_scratch;
-    void* Bf = static_cast<char*>(d_scratch) + mfma_fragment_bytes(f4, M, Kw);
+    void* Bf = static_cast<char*>(d_scratch) + mfma_fragment_bytes(false, M, Kw);
     {   // both operands expanded by one launch
         const dim3 grid((unsigned)((M + 31) / 32 + (KN + 31) / 32), (unsigned)((Kw / 4 + 3) / 4));
         if (grid.y > 65535) return hipErrorInvalidValue;
         const uint32_t *Ra = reinterpret_cast<const uint32_t*>(d_a), *Rb = reinterpret_cast<const uint32_t*>(d_b);
         uint4 *Oa = static_cast<uint4*>(Af), *Ob = static_cast<uint4*>(Bf);
-#define FTNN_EXP2(F4_, TA_, TB_) hipLaunchKernelGGL((k_expand2<F4_, TA_, TB_>), grid, dim3(256), 0, st, Ra, (int)M, Oa, Rb, KN, Ob, Kw / 4)
-#define FTNN_EXP2T(F4_)                          \
-    if (a_tern && b_tern) FTNN_EXP2(F4_, true, true);  \
-    else if (a_tern) FTNN_EXP2(F4_, true, false);      \
-    else if (b_tern) FTNN_EXP2(F4_, false, true);      \
-    else FTNN_EXP2(F4_, false, false)
-        if (f4) { FTNN_EXP2T(true); } else { FTNN_EXP2T(false); }
-#undef FTNN_EXP2T
+#define FTNN_EXP2(TA_, TB_) hipLaunchKernelGGL((k_expand2<false, TA_, TB_>), grid, dim3(256), 0, st, Ra, (int)M, Oa, Rb, KN, Ob, Kw / 4)
+        if (a_tern && b_tern) FTNN_EXP2(true, true);
+        else if (a_tern) FTNN_EXP2(true, false);
+        else if (b_tern) FTNN_EXP2(false, true);
+        else FTNN_EXP2(false, false);
 #undef FTNN_EXP2
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    return launch_mfma_gemm(f4, type, Af, Bf, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
+    return launch_mfma_gemm(false, type, Af, Bf, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
 }
 
 }  // namespace ftnn

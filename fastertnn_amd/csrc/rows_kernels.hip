@@ -1,0 +1,438 @@
+// The fp4 matrix-core GEMM straight from packed rows: one launch, no expansion pass, no scratch.
+//
+// k_mfma and k_mfma_p4 (mfma_kernels.hip) read operands that a launch of their own has brought into matrix-core form.  For
+// products below a few hundred 256 x 256 tiles that launch and its round trip through memory cost as much as the product
+// itself.  Here a wavefront fetches the bit planes as they lie, 16 bytes of signs and zeros per lane, and makes the
+// E2M1 nibbles in registers beside the multiplies: 10 vector instructions per 32 rows x 64 lanes, so that a wavefront
+// tile of 4 x 4 blocks of 32 x 32 spends 6 issue slots per multiply of 8 slots.
+//
+//   * The wavefronts of a workgroup work on ONE output tile and split K: wavefront w takes the groups of four words
+//     w, w + KS, ...  Nothing is shared in the K loop, so it has no barrier; the partial tiles meet in LDS at the end.
+//   * A group travels global -> LDS by LDS-direct loads into a ring of the wavefront's own, four lanes on the 64 contiguous
+//     bytes of a ternary row (two on the 32 of a binary one), and from there to registers in the operand's order.
+//     Loaded straight into that order, 64 lanes touch 64 pieces of cache lines per instruction and the L1 delivers
+//     16 bytes per cycle; in row order it delivers 64 (both measured on operands that lie in the L2).  The pieces of a row
+//     are permuted by its number on the way, so that the 16-byte LDS reads spread over all banks.
+//   * Neighbouring wavefronts take neighbouring groups: two groups of a row share a 128-byte line.
+//   * Signed nibbles (0x2, 0x0, 0xA): a lane flagged zero becomes +-0 whatever its sign bit, which adds nothing, and no
+//     row sums are needed; sums are exact while 64 Kw < 2^24.
+//
+// What bounds it: a lone wavefront per SIMD issues about 2550 cycles of instructions per group on 4 x 4 blocks for 2048
+// cycles of matrix pipe (the LDS-direct loads and LDS reads of a group add 14 cycles each to a slot's multiply), at the
+// clock that sustained multiplies of mixed signs allow (1.9 GHz on all compute units).  Device time of a whole call from
+// packed rows, before (expansion launch + k_mfma, or the vector ALU) and now: 256 x 256 x 4096 4.8 -> 3.6 us,
+// 512 x 512 x 4096 10.2 -> 3.8, 1024 x 1024 x 8192 17.8 -> 7.8, 1500 x 1500 x 12032 32.6 -> 18.1, 2048 x 2048 x 16384 44.1 ->
+// 31.5, 8 x 16384 x 16384 57.8 -> 12.3.
+#include <algorithm>
+#include <type_traits>
+#include <utility>
+
+#include "ftnn_internal.h"
+
+namespace ftnn {
+
+namespace {
+
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+
+// fn(0), ..., fn(N - 1) with compile-time indices
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& fn, std::integer_sequence<int, I...>) {
+    (fn(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& fn) {
+    static_for_impl(fn, std::make_integer_sequence<int, N>{});
+}
+
+// a lane's share of one group of a row: the 128 lanes of its half, as planes
+template <bool TERN>
+struct RawRow {
+    v4u s, z;
+};
+template <>
+struct RawRow<false> {
+    v4u s;
+};
+
+__device__ __forceinline__ void mfma_f4(v16f& c, const v4u& a, const v4u& b) {
+    const v8i va = {(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0};
+    const v8i vb = {(int)b.x, (int)b.y, (int)b.z, (int)b.w, 0, 0, 0, 0};
+    // cbsz = blgp = 4: both operands E2M1, unscaled
+    c = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(va, vb, c, 4, 4, 0, 0, 0, 0);
+}
+
+// Half of a lane's operand for one K word from 32 lanes of its row: HALF 0 the nibble dwords 0 and 1, HALF 1 the dwords 2
+// and 3.  Nibble j of dword k is lane 4 j + k: both operands take their lanes in the same order, so any order serves.
+template <bool TERN, int HALF>
+__device__ __forceinline__ void unpack_half(const RawRow<TERN>& r, int i, v4u& e) {
+    if constexpr (TERN) {
+        const uint32_t s = r.s[i], z = r.z[i];
+        // nibble bits 0, 1: nonzero, bits 2, 3: sign, of two lanes: (~z & 0x3) | (s & 0xC) as one three-input operation
+        // (f = (~a & c) | (b & ~c): table 0x4E; written with operators, the compiler folds the masks below into it twice)
+        const uint32_t w = HALF == 0 ? __builtin_amdgcn_bitop3_b32(z, s << 2, 0x33333333u, 0x4E)
+                                     : __builtin_amdgcn_bitop3_b32(z >> 2, s, 0x33333333u, 0x4E);
+        e[2 * HALF] = (w << 1) & 0xAAAAAAAAu;
+        e[2 * HALF + 1] = w & 0xAAAAAAAAu;
+    } else {
+        const uint32_t s = r.s[i];
+        e[2 * HALF] = ((HALF == 0 ? s << 3 : s << 1) & 0x88888888u) | 0x22222222u;
+        e[2 * HALF + 1] = ((HALF == 0 ? s << 2 : s) & 0x88888888u) | 0x22222222u;
+    }
+}
+
+// LDS-direct loads: 16 bytes per lane from base + voff (base uniform); the 64 lanes land contiguously.  M0 holds the LDS
+// address (one wait state after writing it); the instruction's immediate offset moves the source and the LDS address
+// alike, so a run of up to four loads into adjacent KiB shares one M0 (base + voff is then the source less OFF).  Inline
+// asm, so that the compiler does not order its own LDS reads against the loads; the kernel counts them by hand.
+__device__ __forceinline__ void set_m0(uint32_t lds_byte_addr) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(lds_byte_addr) : "memory"); }
+template <int OFF>
+__device__ __forceinline__ void dma16_at(const char* base, uint32_t voff) {
+    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(base), "n"(OFF) : "memory");
+}
+
+// Which tile a workgroup works on.  Workgroups go to the eight XCDs round-robin by number; XCD x takes the x-th eighth of the
+// tiles, in bands of four P tiles walked along Q, so that the 32 tiles an XCD works on at a time are about 4 x 8 and its
+// L2 fetches 12 panels of rows for them instead of up to 33 (3072 x 3072 x 24576 on 4 x 4 blocks: 119 -> 115 us).
+struct RowsOrder {
+    uint32_t tiles, per_xcd, px;   // tiles in all, per XCD (rounded up), along P
+    FastDiv band, last;            // tiles of a whole band; P tiles of the last band (px % 4, or 4)
+    __device__ __forceinline__ bool tile(uint32_t wg, int* tx, int* ty) const {
+        const uint32_t t = (wg & 7u) * per_xcd + (wg >> 3);
+        if (t >= tiles) return false;
+        const uint32_t b = fastdiv(t, band), r = t - b * band.d;
+        uint32_t y = r >> 2, x = r & 3u;
+        if (b * 4u + 4u > px) {   // the last, narrower band
+            y = fastdiv(r, last);
+            x = r - y * last.d;
+        }
+        *tx = (int)(b * 4u + x);
+        *ty = (int)y;
+        return true;
+    }
+};
+
+// where a result goes: element q_img * img_stride + q_pix + p * p_stride for P row p and Q row q = (q_img, q_pix).  A row-major
+// result (P = activation rows, Q = weight rows: lanes along the columns) has one image; an NCHW result (P = weights, Q =
+// activations: lanes along the pixels) splits q by OH * OW.
+struct RowsOut {
+    float* y;
+    int64_t img_stride;
+    uint32_t p_stride;
+    FastDiv img;
+    float bias, lim, alpha;   // r = sum - bias; PReLU scales r < lim by alpha
+};
+
+// A wavefront's tile is WTP x WTQ blocks of 32 x 32, a workgroup's the same tile: its KS wavefronts split K.
+template <bool TP, bool TQ, int WTP, int WTQ, int KS>
+struct RowsTile {
+    static constexpr int NS = 2;                             // ring slots: deeper rings (where they fit) measured no faster
+    static constexpr int NM = WTP * WTQ, NB = WTP + WTQ;
+    static constexpr int LP = TP ? 2 : 1, LQ = TQ ? 2 : 1;   // KiB (and loads) per row block and group
+    static constexpr int LPG = WTP * LP + WTQ * LQ;          // per wavefront and group
+    static constexpr int R = NM * KS * 4 > 144 ? NM / 2 : NM;   // blocks that meet in LDS at a time
+    static constexpr size_t ring = (size_t)KS * NS * LPG * 1024, red = (size_t)R * KS * 4096;
+    static constexpr size_t lds = ring > red ? ring : red;
+    static_assert(lds <= (160u << 10), "LDS of a compute unit");
+};
+
+template <bool TP, bool TQ, int WTP, int WTQ, int KS>
+__global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, const char* __restrict__ Q, int prow, int qrow, int G,
+                                                  RowsOrder od, RowsOut ro) {
+    extern __shared__ float4 lds[];
+    typedef RowsTile<TP, TQ, WTP, WTQ, KS> TL;
+    constexpr int NM = TL::NM, NB = TL::NB, NS = TL::NS, LP = TL::LP, LQ = TL::LQ, LPG = TL::LPG;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, h = lane >> 5;
+    const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int tx, ty;
+    if (!od.tile(blockIdx.x, &tx, &ty)) return;   // past the last tile (the whole workgroup)
+    const int prb0 = tx * WTP, qrb0 = ty * WTQ;   // first row blocks: within the operands
+    constexpr uint32_t GP = TP ? 64u : 32u, GQ = TQ ? 64u : 32u;   // bytes of a group of 4 words
+    const uint32_t rbp = (uint32_t)G * GP, rbq = (uint32_t)G * GQ;  // bytes of a row
+
+    // Sources of the LDS-direct loads: a ternary row block and group is two loads of 16 rows x 64 bytes, four lanes per
+    // row, a binary one a single load of 32 rows x 32 bytes, two lanes per row; rows past the operand are clamped (their
+    // results are never stored).  One base per side, advanced by GP or GQ per group; row block, row, piece and the
+    // immediate offset a load carries are in its 32-bit lane offset.
+    constexpr uint32_t SPAN = 3072;   // the largest immediate offset
+    const char* const pbase = P + (size_t)prb0 * 32 * rbp - SPAN;
+    const char* const qbase = Q + (size_t)qrb0 * 32 * rbq - SPAN;
+    auto src_row = [&](int j, bool tern) { return tern ? j * 16 + (lane >> 2) : lane >> 1; };
+    auto src_piece = [&](bool tern) { return (uint32_t)(tern ? (lane & 3) ^ ((lane >> 4) & 3) : (lane & 1) ^ ((lane >> 4) & 1)) * 16u; };
+    uint32_t pv[WTP][LP], qv[WTQ][LQ];
+#pragma unroll
+    for (int a = 0; a < WTP; a++)
+#pragma unroll
+        for (int j = 0; j < LP; j++)
+            pv[a][j] = (uint32_t)min(a * 32 + src_row(j, TP), prow - 1 - prb0 * 32) * rbp + src_piece(TP) + SPAN -
+                       (uint32_t)((a * LP + j) & 3) * 1024u;
+#pragma unroll
+    for (int b = 0; b < WTQ; b++)
+#pragma unroll
+        for (int j = 0; j < LQ; j++)
+            qv[b][j] = (uint32_t)min(b * 32 + src_row(j, TQ), qrow - 1 - qrb0 * 32) * rbq + src_piece(TQ) + SPAN -
+                       (uint32_t)((WTP * LP + b * LQ + j) & 3) * 1024u;
+    // this lane's pieces of a row block in LDS: the signs and the zeros of its half
+    auto piece_at = [&](bool tern, int piece) {
+        return (uint32_t)(tern ? lr * 64 + (piece ^ ((lr >> 2) & 3)) * 16 : lr * 32 + (piece ^ ((lr >> 3) & 1)) * 16);
+    };
+    const uint32_t rd_ts = piece_at(true, h), rd_tz = piece_at(true, 2 + h), rd_b = piece_at(false, h);
+    const uint32_t ring0 = (uint32_t)ks * (NS * LPG * 1024);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
+    const char* const ring = reinterpret_cast<const char*>(lds) + ring0;
+
+    // load number i of group gg, into KiB i of the ring slot (M0: KiB i & ~3 of the slot)
+    auto m0_for = [&](int i, int slot) { set_m0(lds0 + ring0 + (uint32_t)(slot * LPG + (i & ~3)) * 1024u); };
+    auto issue = [&](auto itag, int gg) {
+        constexpr int i = decltype(itag)::value, OFF = (i & 3) * 1024;
+        if constexpr (i < WTP * LP) dma16_at<OFF>(pbase + (size_t)gg * GP, pv[i / LP][i % LP]);
+        else dma16_at<OFF>(qbase + (size_t)gg * GQ, qv[(i - WTP * LP) / LQ][(i - WTP * LP) % LQ]);
+    };
+    // planes of operand f (P blocks, then Q blocks) of the group in registers; its nibbles for two K words
+    RawRow<TP> rp[WTP];
+    RawRow<TQ> rq[WTQ];
+    v4u ep[2][WTP], eq[2][WTQ];
+    auto read_plane = [&](int slot, int f, bool zeros) {
+        const char* L = ring + (size_t)slot * LPG * 1024 + (f < WTP ? f * LP : WTP * LP + (f - WTP) * LQ) * 1024;
+        if (f < WTP) {
+            if (!zeros) rp[f].s = *reinterpret_cast<const v4u*>(L + (TP ? rd_ts : rd_b));
+            if constexpr (TP) {
+                if (zeros) rp[f].z = *reinterpret_cast<const v4u*>(L + rd_tz);
+            }
+        } else {
+            if (!zeros) rq[f - WTP].s = *reinterpret_cast<const v4u*>(L + (TQ ? rd_ts : rd_b));
+            if constexpr (TQ) {
+                if (zeros) rq[f - WTP].z = *reinterpret_cast<const v4u*>(L + rd_tz);
+            }
+        }
+    };
+    auto unpack = [&](auto half, int i, int set, int f) {
+        constexpr int H = decltype(half)::value;
+        if (f < WTP) unpack_half<TP, H>(rp[f], i, ep[set][f]);
+        else unpack_half<TQ, H>(rq[f - WTP], i, eq[set][f - WTP]);
+    };
+    v16f acc[WTP][WTQ];
+    // One K word of the group in `slot`: multiply operand set I & 1 and unpack the next word's operands, half an operand at a
+    // time between the multiplies.  Words 0 and 1 also issue the loads of group gl into this slot (whose contents are in
+    // registers), word 2 reads the next group, each operand's planes right behind its last unpacking.
+    constexpr int NW = 2 * NB;
+    auto step = [&](auto itag, int slot, int next_slot, int gl) {
+        constexpr int I = decltype(itag)::value;
+        if constexpr (I == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPG * (NS - 1)) : "memory");   // the next group has landed
+        static_for<NM>([&](auto mtag) {
+            constexpr int m = decltype(mtag)::value;
+            mfma_f4(acc[m / WTQ][m % WTQ], ep[I & 1][m / WTQ], eq[I & 1][m % WTQ]);
+            static_for<(m + 1) * NW / NM - m * NW / NM>([&](auto ktag) {
+                constexpr int j = m * NW / NM + decltype(ktag)::value, i = (I + 1) & 3;
+                if constexpr (I == 2 && (j & 1) == 0 && j > 0) read_plane(next_slot, (j >> 1) - 1, true);
+                unpack(std::integral_constant<int, j & 1>{}, i, (I + 1) & 1, j >> 1);
+                if constexpr (I == 2 && (j & 1) == 1) read_plane(next_slot, j >> 1, false);
+                if constexpr (I == 2 && j == NW - 1) read_plane(next_slot, j >> 1, true);
+            });
+            if constexpr (I < 2) {
+                constexpr int lo = I == 0 ? 0 : LPG / 2, n = I == 0 ? LPG / 2 : LPG - LPG / 2;
+                static_for<(m + 1) * n / NM - m * n / NM>([&](auto ktag) {
+                    constexpr int i = lo + m * n / NM + decltype(ktag)::value;
+                    if constexpr ((i & 3) == 0 || i == lo) m0_for(i, slot);
+                    issue(std::integral_constant<int, i>{}, gl);
+                });
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    int g = ks, gl = ks;   // this wavefront's groups are ks, ks + KS, ...; gl: the next one to be loaded (past the end: the last one again)
+    if (g < G) {
+#pragma unroll
+        for (int t = 0; t < NS; t++) {
+            static_for<LPG>([&](auto itag) {
+                constexpr int i = decltype(itag)::value;
+                if constexpr ((i & 3) == 0) m0_for(i, t);
+                issue(itag, min(gl, G - 1));
+            });
+            gl += KS;
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int a = 0; a < WTP; a++)
+#pragma unroll
+        for (int b = 0; b < WTQ; b++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[a][b][e] = 0.0f;
+    if (g < G) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPG * (NS - 1)) : "memory");
+#pragma unroll
+        for (int f = 0; f < NB; f++) {
+            read_plane(0, f, false);
+            read_plane(0, f, true);
+        }
+#pragma unroll
+        for (int f = 0; f < NB; f++) {
+            unpack(std::integral_constant<int, 0>{}, 0, 0, f);
+            unpack(std::integral_constant<int, 1>{}, 0, 0, f);
+        }
+        int slot = 0;
+        while (g < G) {
+            const int next_slot = slot + 1 == NS ? 0 : slot + 1;
+            const int gc = min(gl, G - 1);
+            step(std::integral_constant<int, 0>{}, slot, next_slot, gc);
+            step(std::integral_constant<int, 1>{}, slot, next_slot, gc);
+            step(std::integral_constant<int, 2>{}, slot, next_slot, gc);
+            step(std::integral_constant<int, 3>{}, slot, next_slot, gc);
+            slot = next_slot;
+            g += KS;
+            gl += KS;
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in the LDS that the partial tiles take now
+
+    // Accumulator e of block (a, b): P row 32 (prb0 + a) + 8 (e / 4) + 4 h + e % 4, Q row 32 (qrb0 + b) + lr.  Four of them
+    // (a quad) are one 16-byte piece per lane in LDS; wavefront ks sums the quads ks, ks + KS, ... over all wavefronts.
+    // PReLU in the reference's two forms, "f <= 0 -> f *= alpha" (mm_p2_final_tnn_avx2.c:204-208) and "r >= 0 ? r : alpha * r"
+    // (mm_p2_final_tbn_avx2.c:73): results are integers below 2^24, so both are one compare, against 0.5 or 0.
+    auto result = [&](float v) {
+        const float r = v - ro.bias;
+        return r < ro.lim ? r * ro.alpha : r;
+    };
+    const size_t stride = ro.p_stride;
+    const bool inside = (prb0 + WTP) * 32 <= prow && (qrb0 + WTQ) * 32 <= qrow;   // uniform
+    auto put4 = [&](const float4& t, int p0, int b, auto whole) {   // P rows p0 + 4 h .. + 3 (p0 uniform) of Q block b
+        const uint32_t q = (uint32_t)((qrb0 + b) * 32 + lr), img = fastdiv(q, ro.img);
+        float* const d = ro.y + (size_t)p0 * stride;
+        const size_t lo = (size_t)img * (size_t)ro.img_stride + (q - img * ro.img.d) + (size_t)(4 * h) * stride;
+        if constexpr (decltype(whole)::value) {
+            __builtin_nontemporal_store(result(t.x), d + lo);
+            __builtin_nontemporal_store(result(t.y), d + stride + lo);
+            __builtin_nontemporal_store(result(t.z), d + 2 * stride + lo);
+            __builtin_nontemporal_store(result(t.w), d + 3 * stride + lo);
+        } else if (q < (uint32_t)qrow) {
+            const int p = p0 + 4 * h;
+            if (p < prow) __builtin_nontemporal_store(result(t.x), d + lo);
+            if (p + 1 < prow) __builtin_nontemporal_store(result(t.y), d + stride + lo);
+            if (p + 2 < prow) __builtin_nontemporal_store(result(t.z), d + 2 * stride + lo);
+            if (p + 3 < prow) __builtin_nontemporal_store(result(t.w), d + 3 * stride + lo);
+        }
+    };
+    constexpr int R = TL::R, QUADS = R * 4 / KS;
+    static_assert(R * 4 % KS == 0 && NM % R == 0, "whole quads per wavefront");
+#pragma unroll
+    for (int r0 = 0; r0 < NM; r0 += R) {
+        __syncthreads();   // every wavefront is done with its ring, or with the round before
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+            const v16f& c = acc[(r0 + j) / WTQ][(r0 + j) % WTQ];
+#pragma unroll
+            for (int e4 = 0; e4 < 4; e4++)
+                lds[((ks * R + j) * 4 + e4) * 64 + lane] = make_float4(c[4 * e4], c[4 * e4 + 1], c[4 * e4 + 2], c[4 * e4 + 3]);
+        }
+        __syncthreads();
+        float4 t[QUADS];   // all sums before the first store: the branch around the stores would hold the reads back
+#pragma unroll
+        for (int i = 0; i < QUADS; i++) {
+            const int quad = i * KS + ks;
+            t[i] = lds[quad * 64 + lane];
+#pragma unroll
+            for (int v = 1; v < KS; v++) {
+                const float4 u = lds[(v * R * 4 + quad) * 64 + lane];
+                t[i].x += u.x;
+                t[i].y += u.y;
+                t[i].z += u.z;
+                t[i].w += u.w;
+            }
+        }
+        auto put_all = [&](auto whole) {
+#pragma unroll
+            for (int i = 0; i < QUADS; i++) {
+                const int quad = i * KS + ks, blk = r0 + (quad >> 2);
+                put4(t[i], (prb0 + blk / WTQ) * 32 + 8 * (quad & 3), blk % WTQ, whole);
+            }
+        };
+        if (inside) put_all(std::true_type{});
+        else put_all(std::false_type{});
+    }
+}
+
+template <bool TP, bool TQ, int WT>
+hipError_t launch_rows_tile(const char* P, const char* Q, int64_t prow, int64_t qrow, int G, const RowsOut& ro, hipStream_t st) {
+    constexpr int KS = 4;   // 8 wavefronts measured no faster on any tile
+    typedef RowsTile<TP, TQ, WT, WT, KS> TL;
+    auto kern = k_rows<TP, TQ, WT, WT, KS>;
+    // the loads are counted by hand (s_waitcnt vmcnt(N)): a build with scratch accesses is refused; the opt-in to more than
+    // 64 KiB of dynamic LDS is per kernel
+    static const hipError_t configured = []() {
+        const void* k = reinterpret_cast<const void*>(&k_rows<TP, TQ, WT, WT, KS>);
+        hipFuncAttributes attr;
+        hipError_t e = hipFuncGetAttributes(&attr, k);
+        if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
+        if (e != hipSuccess) return e;
+        return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)TL::lds);
+    }();
+    if (configured != hipSuccess) return configured;
+    const int64_t px = (prow + 32 * WT - 1) / (32 * WT), qy = (qrow + 32 * WT - 1) / (32 * WT);
+    if (px * qy > 0x3fffffffLL) return hipErrorInvalidValue;
+    RowsOrder od;
+    od.tiles = (uint32_t)(px * qy);
+    od.per_xcd = (od.tiles + 7) / 8;
+    od.px = (uint32_t)px;
+    od.band = make_fastdiv((uint32_t)(4 * qy));
+    od.last = make_fastdiv((uint32_t)(px % 4 ? px % 4 : 4));
+    hipLaunchKernelGGL(kern, dim3(8 * od.per_xcd), dim3(64 * KS), TL::lds, st, P, Q, (int)prow, (int)qrow, G, od, ro);
+    return hipGetLastError();
+}
+
+// Wavefront tile of a product: blocks of 32 x 32 per side.  Small tiles fill the chip with little work and pay less for the
+// meeting of the partial tiles, large ones spend fewer instructions and bytes per multiply.  The estimates (us) are
+// fits to sweeps from 32 x 32 x 256 to 4096 x 4096 x 32768 on MI355X (n rounds of 256 tiles, w words per wavefront); where
+// two tiles are within 15 % of each other either may be picked.
+int rows_tile_of(int64_t prow, int64_t qrow, int Kw) {
+    auto rounds = [&](int edge) { return (double)((((prow + edge - 1) / edge) * ((qrow + edge - 1) / edge) + 255) / 256); };
+    const double w = Kw / 4.0;
+    const double n1 = rounds(32), n2 = rounds(64), n3 = rounds(96), n4 = rounds(128);
+    const double t1 = 2.65 + 0.42 * (n1 - 1) + w * (0.06 + 0.039 * (n1 - 1));
+    const double t2 = 3.55 + 1.33 * (n2 - 1) + w * (0.118 + 0.145 * (n2 - 1));
+    const double t3 = 5.0 + 4.0 * (n3 - 1) + 0.25 * n3 * w;
+    const double t4 = 8.0 + 5.5 * (n4 - 1) + 0.35 * n4 * w;
+    const double best = std::min(std::min(t1, t2), std::min(t3, t4));
+    return best == t1 ? 1 : best == t2 ? 2 : best == t3 ? 3 : 4;
+}
+
+template <bool TP, bool TQ>
+hipError_t launch_rows_types(const char* P, const char* Q, int64_t prow, int64_t qrow, int Kw, const RowsOut& ro, hipStream_t st) {
+    switch (rows_tile_of(prow, qrow, Kw)) {
+        case 1: return launch_rows_tile<TP, TQ, 1>(P, Q, prow, qrow, Kw / 4, ro, st);
+        case 2: return launch_rows_tile<TP, TQ, 2>(P, Q, prow, qrow, Kw / 4, ro, st);
+        case 3: return launch_rows_tile<TP, TQ, 3>(P, Q, prow, qrow, Kw / 4, ro, st);
+        default: return launch_rows_tile<TP, TQ, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
+    }
+}
+
+}  // namespace
+
+bool mm_rows_within_limits(int Kw) { return 64LL * Kw < (1LL << 24); }
+
+hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
+                          float alpha, float* d_y, hipStream_t st) {
+    const bool at = type == kTNN || type == kTBN, wt = type == kTNN || type == kBTN;
+    const bool nchw = OHW > 1;
+    RowsOut ro;
+    ro.y = d_y;
+    ro.img_stride = (int64_t)KN * OHW;
+    ro.p_stride = (uint32_t)(nchw ? OHW : KN);
+    ro.img = make_fastdiv(nchw ? (uint32_t)OHW : 0xffffffffu);
+    // BNN: the lanes past K_unpack are +1 in both operands and add 64 Kw - K_unpack (mm_p2_final_bnn_avx2.c:55-58)
+    ro.bias = type == kBNN ? (float)(64 * Kw - K_unpack) : 0.0f;
+    ro.lim = type == kTNN ? 0.5f : 0.0f;
+    ro.alpha = alpha;
+    const char* P = reinterpret_cast<const char*>(nchw ? d_b : d_a);
+    const char* Q = reinterpret_cast<const char*>(nchw ? d_a : d_b);
+    const int64_t prow = nchw ? KN : M, qrow = nchw ? M : KN;
+    const bool tp = nchw ? wt : at, tq = nchw ? at : wt;
+    if (tp && tq) return launch_rows_types<true, true>(P, Q, prow, qrow, Kw, ro, st);
+    if (tp) return launch_rows_types<true, false>(P, Q, prow, qrow, Kw, ro, st);
+    if (tq) return launch_rows_types<false, true>(P, Q, prow, qrow, Kw, ro, st);
+    return launch_rows_types<false, false>(P, Q, prow, qrow, Kw, ro, st);
+}
+
+}  // namespace ftnn

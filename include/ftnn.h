@@ -194,7 +194,9 @@ FTNN_API int ftnn_mm(int type, const int64_t *d_a, const int64_t *d_b, int N, in
 #define FTNN_ENGINE_MFMA_I8 2 /* v_mfma_i32_32x32x32_i8 on expanded operands         */
 #define FTNN_ENGINE_MFMA_F4 3 /* v_mfma_f32_32x32x64_f8f6f4 (fp4); GEMM rows of at most 65536 words */
 
-/* the engine FTNN_ENGINE_AUTO resolves to for this shape (never AUTO) */
+/* the engine FTNN_ENGINE_AUTO resolves to for this shape (never AUTO).  Under AUTO a product below 160 tiles of
+ * 256 x 256 runs on the fp4 matrix cores straight from its packed rows, without scratch, where this says VALU or
+ * MFMA_F4 alike. */
 FTNN_API int ftnn_select_engine(int type, int N, int OH, int OW, int KN, int K);
 
 /* device scratch, in bytes, that ftnn_mm_engine needs for `engine` (0 for the VALU engine;
