@@ -116,32 +116,59 @@ def pack_scratch_bytes(n, c, h, w, ternary):
 
 # ------------------------------------------------------------ device entry points
 
-def _stream():
+# A call queues 2.5 us of launch work per kernel; what the binding adds must stay below that.  torch is imported once, on
+# the first device call (importing it inside every wrapper costs 0.3 us), and the stream is asked for as the bare handle
+# (0.1 us; the Stream object of torch.cuda.current_stream() costs 2.7).
+torch = None
+
+
+def _torch():
+    global torch
     import torch
-    return torch.cuda.current_stream().cuda_stream
+    return torch
+
+
+def _stream():
+    t = torch or _torch()
+    return t._C._cuda_getCurrentRawStream(t._C._cuda_getDevice())
 
 
 def _dev(t, dtype=None):
-    import torch
     assert t.is_cuda and t.is_contiguous(), "expected a contiguous CUDA tensor"
     if dtype is not None:
         assert t.dtype == dtype, "expected %s, got %s" % (dtype, t.dtype)
     return t.data_ptr()
 
 
+def _f32(t):
+    return _dev(t, (torch or _torch()).float32)
+
+
+def _empty(shape, dtype, device):
+    t = torch or _torch()
+    return t.empty(shape, dtype=getattr(t, dtype), device=device)
+
+
+def _layer_out(x, kn, kh, kw, pad, stride):
+    n, _, h, w = x.shape
+    oh, ow = out_dim(h, pad, kh, stride), out_dim(w, pad, kw, stride)
+    if oh <= 0 or ow <= 0:
+        raise FtnnError("kernel larger than padded input")
+    return _empty((n, kn, oh, ow), "float32", x.device)
+
+
 def quantize_im2row(x, thr, kh, kw, pad, stride, ternary, out=None, scratch=None):
     """t2r_p2_opt (ternary) / b2r (binary) on device tensors; returns int64 rows."""
-    import torch
     n, c, h, w = x.shape
     oh, ow = out_dim(h, pad, kh, stride), out_dim(w, pad, kw, stride)
     if oh <= 0 or ow <= 0:
         raise FtnnError("kernel larger than padded input")
     words = row_words(c, kh, kw, ternary)
     if out is None:
-        out = torch.empty(n * oh * ow * words, dtype=torch.int64, device=x.device)
+        out = _empty(n * oh * ow * words, "int64", x.device)
     if scratch is None:
-        scratch = torch.empty(pack_scratch_bytes(n, c, h, w, ternary), dtype=torch.uint8, device=x.device)
-    _check(_L.ftnn_quantize_im2row(int(ternary), _dev(x, torch.float32), _dev(thr, torch.float32),
+        scratch = _empty(pack_scratch_bytes(n, c, h, w, ternary), "uint8", x.device)
+    _check(_L.ftnn_quantize_im2row(int(ternary), _f32(x), _f32(thr),
                                    n, c, h, w, pad, pad, kh, kw, stride, stride, _dev(out), _dev(scratch),
                                    _stream()))
     return out
@@ -149,10 +176,9 @@ def quantize_im2row(x, thr, kh, kw, pad, stride, ternary, out=None, scratch=None
 
 def mm(typ, a, b, n, oh, ow, kn, k, alpha, k_unpack=0, out=None):
     """mm_tnn / mm_tbn / mm_btn / mm_bnn on device tensors; returns fp32 (n, kn, oh, ow)."""
-    import torch
     if out is None:
-        out = torch.empty((n, kn, oh, ow), dtype=torch.float32, device=a.device)
-    _check(_L.ftnn_mm(typ, _dev(a), _dev(b), n, oh, ow, kn, k, k_unpack, alpha, _dev(out, torch.float32),
+        out = _empty((n, kn, oh, ow), "float32", a.device)
+    _check(_L.ftnn_mm(typ, _dev(a), _dev(b), n, oh, ow, kn, k, k_unpack, alpha, _f32(out),
                       _stream()))
     return out
 
@@ -171,35 +197,33 @@ def mm_scratch_bytes(engine, typ, n, oh, ow, kn, k):
 
 def mm_engine(engine, typ, a, b, n, oh, ow, kn, k, alpha, k_unpack=0, out=None, scratch=None):
     """ftnn_mm_engine: the GEMM on an explicit engine (or AUTO); scratch is allocated if not given."""
-    import torch
     if out is None:
-        out = torch.empty((n, kn, oh, ow), dtype=torch.float32, device=a.device)
-    need = mm_scratch_bytes(engine, typ, n, oh, ow, kn, k)
-    if scratch is None and need > 0:
-        scratch = torch.empty(need, dtype=torch.uint8, device=a.device)
+        out = _empty((n, kn, oh, ow), "float32", a.device)
+    if scratch is None:
+        need = mm_scratch_bytes(engine, typ, n, oh, ow, kn, k)
+        if need > 0:
+            scratch = _empty(need, "uint8", a.device)
     sp = _dev(scratch) if scratch is not None else None
     sb = scratch.numel() * scratch.element_size() if scratch is not None else 0
     _check(_L.ftnn_mm_engine(engine, typ, _dev(a), _dev(b), n, oh, ow, kn, k, k_unpack, alpha,
-                             _dev(out, torch.float32), sp, sb, _stream()))
+                             _f32(out), sp, sb, _stream()))
     return out
 
 
 def expand_rows(engine, rows_t, n_rows, k, ternary, out=None):
     """ftnn_expand_rows: packed rows -> the operand format of a matrix-core engine."""
-    import torch
     if out is None:
-        out = torch.empty(int(_L.ftnn_expand_bytes(engine, n_rows, k)), dtype=torch.uint8, device=rows_t.device)
+        out = _empty(int(_L.ftnn_expand_bytes(engine, n_rows, k)), "uint8", rows_t.device)
     _check(_L.ftnn_expand_rows(engine, int(ternary), _dev(rows_t), n_rows, k, _dev(out), _stream()))
     return out
 
 
 def mm_expanded(engine, typ, a_exp, b_exp, n, oh, ow, kn, k, alpha, k_unpack=0, out=None):
     """ftnn_mm_expanded: the matrix-core GEMM on two expanded operands."""
-    import torch
     if out is None:
-        out = torch.empty((n, kn, oh, ow), dtype=torch.float32, device=a_exp.device)
+        out = _empty((n, kn, oh, ow), "float32", a_exp.device)
     _check(_L.ftnn_mm_expanded(engine, typ, _dev(a_exp), _dev(b_exp), n, oh, ow, kn, k, k_unpack, alpha,
-                               _dev(out, torch.float32), _stream()))
+                               _f32(out), _stream()))
     return out
 
 
@@ -209,19 +233,13 @@ def select_conv_engine(typ, n, c, h, w, kn, kh, kw, pad, stride):
 
 def conv(typ, x, thr, qw, kn, kh, kw, pad, stride, alpha, scratch=None, out=None, engine=ENGINE_AUTO):
     """One conv layer (tnn_conv_p2 & co.) on device tensors; engine: AUTO, VALU or MFMA_F4."""
-    import torch
     n, c, h, w = x.shape
-    oh, ow = out_dim(h, pad, kh, stride), out_dim(w, pad, kw, stride)
-    if oh <= 0 or ow <= 0:
-        raise FtnnError("kernel larger than padded input")
-    tern = act_is_ternary(typ)
     if scratch is None:
-        scratch = torch.empty(conv_scratch_bytes(typ, n, c, h, w, kn, kh, kw, pad, stride), dtype=torch.uint8,
-                              device=x.device)
+        scratch = _empty(conv_scratch_bytes(typ, n, c, h, w, kn, kh, kw, pad, stride), "uint8", x.device)
     if out is None:
-        out = torch.empty((n, kn, oh, ow), dtype=torch.float32, device=x.device)
-    args = (typ, _dev(x, torch.float32), _dev(thr, torch.float32), _dev(qw), n, c, h, w, kn, kh, kw, pad, pad,
-            stride, stride, alpha, _dev(scratch), _dev(out, torch.float32), _stream())
+        out = _layer_out(x, kn, kh, kw, pad, stride)
+    args = (typ, _f32(x), _f32(thr), _dev(qw), n, c, h, w, kn, kh, kw, pad, pad,
+            stride, stride, alpha, _dev(scratch), _f32(out), _stream())
     _check(_L.ftnn_conv(*args) if engine == ENGINE_AUTO else _L.ftnn_conv_engine(engine, *args))
     return out
 
@@ -231,55 +249,46 @@ STATIC_SCRATCH_BYTES = int(_L.ftnn_static_scratch_bytes())   # FTNN_STATIC_SCRAT
 
 def conv_static(typ, x, thr, qw, kn, kh, kw, pad, stride, alpha, out):
     """ftnn_conv_static: the layer on the library's own fixed work space; allocates nothing (out is required)."""
-    import torch
     n, c, h, w = x.shape
-    _check(_L.ftnn_conv_static(typ, _dev(x, torch.float32), _dev(thr, torch.float32), _dev(qw), n, c, h, w, kn, kh,
-                               kw, pad, pad, stride, stride, alpha, _dev(out, torch.float32), _stream()))
+    _check(_L.ftnn_conv_static(typ, _f32(x), _f32(thr), _dev(qw), n, c, h, w, kn, kh,
+                               kw, pad, pad, stride, stride, alpha, _f32(out), _stream()))
     return out
 
 
 def prepare_conv_weights(typ, qw, c, kn, kh, kw):
     """ftnn_conv_prepare_weights: the packed rows in the form the layer's engine reads (once per layer)."""
-    import torch
-    out = torch.empty(int(_L.ftnn_conv_weights_bytes(typ, c, kn, kh, kw)), dtype=torch.uint8, device=qw.device)
+    out = _empty(int(_L.ftnn_conv_weights_bytes(typ, c, kn, kh, kw)), "uint8", qw.device)
     _check(_L.ftnn_conv_prepare_weights(typ, _dev(qw), c, kn, kh, kw, _dev(out), _stream()))
     return out
 
 
 def conv_prepared(typ, x, thr, prepared, kn, kh, kw, pad, stride, alpha, scratch=None, out=None):
     """ftnn_conv_prepared: one conv layer with weights from prepare_conv_weights."""
-    import torch
     n, c, h, w = x.shape
-    oh, ow = out_dim(h, pad, kh, stride), out_dim(w, pad, kw, stride)
-    if oh <= 0 or ow <= 0:
-        raise FtnnError("kernel larger than padded input")
     if scratch is None:
-        scratch = torch.empty(conv_scratch_bytes(typ, n, c, h, w, kn, kh, kw, pad, stride), dtype=torch.uint8,
-                              device=x.device)
+        scratch = _empty(conv_scratch_bytes(typ, n, c, h, w, kn, kh, kw, pad, stride), "uint8", x.device)
     if out is None:
-        out = torch.empty((n, kn, oh, ow), dtype=torch.float32, device=x.device)
-    _check(_L.ftnn_conv_prepared(typ, _dev(x, torch.float32), _dev(thr, torch.float32), _dev(prepared), n, c, h, w,
+        out = _layer_out(x, kn, kh, kw, pad, stride)
+    _check(_L.ftnn_conv_prepared(typ, _f32(x), _f32(thr), _dev(prepared), n, c, h, w,
                                  kn, kh, kw, pad, pad, stride, stride, alpha, _dev(scratch),
-                                 _dev(out, torch.float32), _stream()))
+                                 _f32(out), _stream()))
     return out
 
 
 def pack_weights(w, thr, ternary):
     """ternarize_opt_avx2 / binarize_opt_avx2 on device tensors."""
-    import torch
     kn, c, kh, kw = w.shape
-    out = torch.empty(kn * row_words(c, kh, kw, ternary), dtype=torch.int64, device=w.device)
-    _check(_L.ftnn_pack_weights(int(ternary), _dev(w, torch.float32), _dev(thr, torch.float32), kn, c, kh, kw,
+    out = _empty(kn * row_words(c, kh, kw, ternary), "int64", w.device)
+    _check(_L.ftnn_pack_weights(int(ternary), _f32(w), _f32(thr), kn, c, kh, kw,
                                 _dev(out), _stream()))
     return out
 
 
 def pack_gemm_operand(x):
     """bitpacking2 on a device tensor [I][J] of {-1,0,+1} floats."""
-    import torch
     i, j = x.shape
-    out = torch.empty(max(i * j // 32, 1), dtype=torch.int64, device=x.device)
-    _check(_L.ftnn_pack_gemm_operand(_dev(x, torch.float32), i, j, _dev(out), _stream()))
+    out = _empty(max(i * j // 32, 1), "int64", x.device)
+    _check(_L.ftnn_pack_gemm_operand(_f32(x), i, j, _dev(out), _stream()))
     return out
 
 
@@ -323,10 +332,9 @@ class Net:
         assert int(_L.ftnn_net_output_elems(self._h)) == int(np.prod(self.out_shape))
 
     def run(self, x, out=None, graph=False):
-        import torch
         if out is None:
-            out = torch.empty(self.out_shape, dtype=torch.float32, device=x.device)
-        _check(_L.ftnn_net_run(self._h, _dev(x, torch.float32), _dev(out, torch.float32), int(graph), _stream()))
+            out = _empty(self.out_shape, "float32", x.device)
+        _check(_L.ftnn_net_run(self._h, _f32(x), _f32(out), int(graph), _stream()))
         return out
 
     def close(self):
