@@ -23,7 +23,11 @@
 struct NetPart {
     int first = 0, batch = 0;               // images [first, first + batch)
     float* d_act[2] = {nullptr, nullptr};   // fp32 activations between layers that need them
-    void* d_p4[2] = {nullptr, nullptr};     // quantised input of the fp4 layers, by layer parity
+    // Quantised inputs of the fp4 layers: two buffers, by layer parity, for every size of a quantised image in the chain,
+    // so that an image lies at the same place of its buffer in all layers of that size.  The XCD that works on it
+    // (XcdOrder) then writes lines that no other XCD's L2 holds; with two buffers for all sizes the layer behind the
+    // stride-2 one of the ResNet-18-like chain took 9.7 instead of 7.6 us at batch 32.
+    std::vector<void*> d_p4;
     void* d_scratch = nullptr;              // work space of the vector-ALU layers
 };
 
@@ -33,6 +37,7 @@ struct ftnn_net {
     std::vector<int> OH, OW;
     std::vector<float*> d_thr;       // per layer: batch copies of its threshold
     std::vector<void*> d_wf;         // per layer on the fp4 engine: its weights as matrix-core fragments
+    std::vector<int> p4_buf;         // per layer: which of a part's d_p4 its quantised input lies in (-1: none)
     std::vector<char> rereads;       // per layer: its input is the leading part of the previous layer's fp32 output
     std::vector<NetPart> parts;      // one, or two that run concurrently
     hipStream_t side = nullptr;      // stream of the second part
@@ -61,7 +66,7 @@ int enqueue_layer(ftnn_net* net, const NetPart& part, int i, const float*& in, b
     QuantOut qo;
     if (next_f4) {
         const int nt = net->layers[i + 1].type;
-        qo.p4 = part.d_p4[(i + 1) & 1];
+        qo.p4 = part.d_p4[(size_t)net->p4_buf[i + 1]];
         qo.thr = net->d_thr[i + 1];   // every entry holds the layer's threshold: any run of `batch` entries serves
         qo.mode = (nt == kTNN || nt == kTBN) ? 1 : 2;
     }
@@ -69,8 +74,8 @@ int enqueue_layer(ftnn_net* net, const NetPart& part, int i, const float*& in, b
     int rc;
     if (net->d_wf[i])
         rc = conv_f4_expanded(L.type, p4_ready ? nullptr : in, net->d_thr[i], net->d_wf[i], part.batch, L.C, L.H, L.W,
-                              L.KN, L.KH, L.KW, L.pad, L.pad, L.stride, L.stride, L.prelu_alpha, part.d_p4[i & 1], out,
-                              st, qo);
+                              L.KN, L.KH, L.KW, L.pad, L.pad, L.stride, L.stride, L.prelu_alpha,
+                              part.d_p4[(size_t)net->p4_buf[i]], out, st, qo);
     else
         rc = conv_valu(L.type, in, net->d_thr[i], L.d_qw, part.batch, L.C, L.H, L.W, L.KN, L.KH, L.KW, L.pad, L.pad,
                        L.stride, L.stride, L.prelu_alpha, part.d_scratch, out, st, qo, false);
@@ -196,7 +201,14 @@ ftnn_net_t* ftnn_net_create_ex(int batch, int n_layers, const ftnn_layer_t* laye
     // engine of every layer (by the larger part: both parts must agree), then the buffers each part needs
     const int pb = net->parts[0].batch;
     std::vector<char> f4((size_t)n_layers, 0);
-    int64_t max_act = 0, max_scratch = 256, max_p4 = 0;
+    int64_t max_act = 0, max_scratch = 256;
+    struct P4Size {
+        int64_t image;       // bytes of one quantised image
+        int64_t bytes[2];    // largest operand region among its layers, by layer parity (0: no such layer)
+        int slot[2];
+    };
+    std::vector<P4Size> sizes;
+    std::vector<int> size_of((size_t)n_layers, -1);
     for (int i = 0; i < n_layers; i++) {
         const ftnn_layer_t& L = layers[i];
         f4[i] = ftnn_select_conv_engine(L.type, pb, L.C, L.H, L.W, L.KN, L.KH, L.KW, L.pad, L.pad, L.stride,
@@ -206,11 +218,21 @@ ftnn_net_t* ftnn_net_create_ex(int batch, int n_layers, const ftnn_layer_t* laye
             f4[i] = 0;   // beyond the 32-bit pixel indices of the fp4 layer kernel: the vector-ALU layer takes it
         // sized for the larger part; a very large layer's operand region depends on the batch in steps (the
         // im2row + GEMM form), so the smaller part is asked too
+        if (f4[i]) {
+            const int64_t image = (int64_t)cpack_of(L.C) * L.H * L.W * 32;
+            for (size_t k = 0; k < sizes.size() && size_of[i] < 0; k++)
+                if (sizes[k].image == image) size_of[i] = (int)k;
+            if (size_of[i] < 0) {
+                size_of[i] = (int)sizes.size();
+                sizes.push_back(P4Size{image, {0, 0}, {-1, -1}});
+            }
+        }
         for (const NetPart& part : net->parts) {
-            if (f4[i])
-                max_p4 = std::max(max_p4, conv_f4_operand_bytes(part.batch, L.C, L.H, L.W, L.KH, L.KW, net->OH[i],
-                                                                net->OW[i], L.KN, L.stride));
-            else
+            if (f4[i]) {
+                int64_t& bytes = sizes[(size_t)size_of[i]].bytes[i & 1];
+                bytes = std::max(bytes, conv_f4_operand_bytes(part.batch, L.C, L.H, L.W, L.KH, L.KW, net->OH[i], net->OW[i],
+                                                              L.KN, L.stride));
+            } else
                 max_scratch = std::max(max_scratch, ftnn_conv_scratch_bytes(L.type, part.batch, L.C, L.H, L.W, L.KN, L.KH,
                                                                             L.KW, L.pad, L.pad, L.stride, L.stride));
         }
@@ -221,12 +243,19 @@ ftnn_net_t* ftnn_net_create_ex(int batch, int n_layers, const ftnn_layer_t* laye
             max_act = std::max(max_act, (int64_t)pb * layers[i - 1].KN * net->OH[i - 1] * net->OW[i - 1]);
     }
     bool good = true;
+    int n_p4 = 0;
+    for (P4Size& z : sizes)
+        for (int b = 0; b < 2; b++)
+            if (z.bytes[b] > 0) z.slot[b] = n_p4++;
+    for (int i = 0; i < n_layers; i++) net->p4_buf.push_back(f4[i] ? sizes[(size_t)size_of[i]].slot[i & 1] : -1);
     for (NetPart& part : net->parts) {
+        part.d_p4.assign((size_t)n_p4, nullptr);
         good = good && hipMalloc(&part.d_scratch, (size_t)max_scratch) == hipSuccess;
         for (int b = 0; b < 2 && good && max_act > 0; b++)
             good = hipMalloc((void**)&part.d_act[b], (size_t)max_act * sizeof(float)) == hipSuccess;
-        for (int b = 0; b < 2 && good && max_p4 > 0; b++)
-            good = hipMalloc(&part.d_p4[b], (size_t)max_p4) == hipSuccess;
+        for (const P4Size& z : sizes)
+            for (int b = 0; b < 2 && good; b++)
+                if (z.slot[b] >= 0) good = hipMalloc(&part.d_p4[(size_t)z.slot[b]], (size_t)z.bytes[b]) == hipSuccess;
     }
     if (good && nparts > 1)
         good = hipStreamCreateWithFlags(&net->side, hipStreamNonBlocking) == hipSuccess &&
@@ -277,10 +306,10 @@ void ftnn_net_destroy(ftnn_net_t* net) {
     for (void* p : net->d_wf)
         if (p) (void)hipFree(p);
     for (NetPart& part : net->parts) {
-        for (int b = 0; b < 2; b++) {
+        for (int b = 0; b < 2; b++)
             if (part.d_act[b]) (void)hipFree(part.d_act[b]);
-            if (part.d_p4[b]) (void)hipFree(part.d_p4[b]);
-        }
+        for (void* p : part.d_p4)
+            if (p) (void)hipFree(p);
         if (part.d_scratch) (void)hipFree(part.d_scratch);
     }
     if (net->fork) (void)hipEventDestroy(net->fork);

@@ -809,7 +809,9 @@ template <bool ABIN, bool FORM0, int QMODE, int S, int NB, bool BUF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && QMODE != 0) ? 3 : 1, 8))) void k_conv_f4(const uint4* __restrict__ P4, const uint4* __restrict__ Wf,
                                                  float* __restrict__ Y, int M, int KN, int OHW, int KB,
                                                  int bias, float alpha, FastDiv dOHW, ConvGeom cg, QuantOut qo,
-                                                 uint32_t p4_bytes, uint32_t wf_bytes) {
+                                                 uint32_t p4_bytes, uint32_t wf_bytes, XcdOrder xo) {
+    uint32_t bx, by;   // pixel tiles, kernel tile
+    xo.tile(blockIdx.x + gridDim.x * blockIdx.y, bx, by);
     // NB register sets of fragments: NB - 1 steps of loads in flight
     constexpr int WPB = 4;                // wavefronts per workgroup (single-wavefront workgroups for S = 1
                                           // measured slower: neighbours no longer share weight fragments in L1)
@@ -819,7 +821,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ks = wave % S, pt = wave / S;   // K share and pixel tile of this wavefront
     const int h = lane >> 5, lr = lane & 31;
-    const int px0 = (blockIdx.x * (WPB / S) + pt) * 64, kn0 = blockIdx.y * 64;
+    const int px0 = (bx * (WPB / S) + pt) * 64, kn0 = by * 64;
 
     int ih0[2], iw0[2];
     uint32_t pb[2];
@@ -1026,7 +1028,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
                 // block: half of nibble dword g of the pixel, the other half sits in lane ^ 32.  Lane half h ends up
                 // with bytes 16a + 8h .. + 8 of the pixel's 64-channel word.
                 const uint2 out = hand_over_block<FORM0, QMODE>(r, alpha, qthr[b], direct_q[b], kn0 + 32 * a, h, KN);
-                const size_t word = ((size_t)img * gridDim.y + blockIdx.y) * OHW + pix;
+                const size_t word = ((size_t)img * gridDim.y + by) * OHW + pix;
                 if (q < M) *reinterpret_cast<uint2*>(static_cast<unsigned char*>(qo.p4) + word * 32 + 16 * a + 8 * h) = out;
             }
         }
@@ -1045,13 +1047,15 @@ template <bool ABIN, bool FORM0, int QMODE, bool BUF>
 __global__ __launch_bounds__(256) void k_conv_f4_small(const uint4* __restrict__ P4, const uint4* __restrict__ Wf,
                                                        float* __restrict__ Y, int M, int KN, int OHW, int KB, int bias,
                                                        float alpha, FastDiv dOHW, ConvGeom cg, QuantOut qo,
-                                                       uint32_t p4_bytes, uint32_t wf_bytes) {
+                                                       uint32_t p4_bytes, uint32_t wf_bytes, XcdOrder xo) {
+    uint32_t bx, by;   // pixel tiles, kernel tile
+    xo.tile(blockIdx.x + gridDim.x * blockIdx.y, bx, by);
     constexpr int S = 4, NB = 3;
     __shared__ float4 red[3 * 4 * 64];   // [wavefront - 1][e / 4][lane]
     const int tid = threadIdx.x, lane = tid & 63;
     const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, lr = lane & 31;
-    const int px0 = blockIdx.x * 32, kn0 = blockIdx.y * 32;
+    const int px0 = bx * 32, kn0 = by * 32;
 
     const int q = px0 + lr;
     const uint32_t qc = (uint32_t)min(q, M - 1);
@@ -1173,9 +1177,9 @@ __global__ __launch_bounds__(256) void k_conv_f4_small(const uint4* __restrict__
     } else {
         const uint2 out = hand_over_block<FORM0, QMODE>(r, alpha, qthr, direct_quant<QMODE>(alpha, qthr), kn0, h, KN);
         // this tile is half a 64-channel word: bytes 16 * (tile parity) of the pixel's 32
-        const size_t word = ((size_t)img * (gridDim.y >> 1) + (blockIdx.y >> 1)) * OHW + pix;
+        const size_t word = ((size_t)img * (gridDim.y >> 1) + (by >> 1)) * OHW + pix;
         if (q < M)
-            *reinterpret_cast<uint2*>(static_cast<unsigned char*>(qo.p4) + word * 32 + 16 * (blockIdx.y & 1) + 8 * h) = out;
+            *reinterpret_cast<uint2*>(static_cast<unsigned char*>(qo.p4) + word * 32 + 16 * (by & 1) + 8 * h) = out;
     }
 }
 
@@ -1469,10 +1473,13 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
     const int64_t p4_bytes = (int64_t)N * cg.CP * cg.H * cg.W * 32, wf_bytes = (int64_t)((KN + 31) / 32) * KB * 1024;
     static const bool no_buf = getenv("FTNN_CONV_NO_BUFFER_LOADS") != nullptr;   // tuning aid
     const bool buf = !no_buf && p4_bytes <= 0xf0000000LL && wf_bytes <= 0xf0000000LL;
+    const uint64_t wgs = (uint64_t)grid.x * grid.y;
+    if (wgs > 0xffffffffull) return hipErrorInvalidValue;   // (no such result fits in memory)
+    const XcdOrder xo = make_xcd_order(grid.x, grid.y);
     auto launch64 = [&](auto variant) -> hipError_t {
         constexpr auto kern = decltype(variant)::value;
         hipLaunchKernelGGL(kern, grid, dim3(64 * wpb), 0, st, P4, Wf, d_y, (int)M, KN, OHW, KB, bias, alpha, dOHW, cg, qo,
-                           (uint32_t)std::min<int64_t>(p4_bytes, 0xffffffffLL), (uint32_t)std::min<int64_t>(wf_bytes, 0xffffffffLL));
+                           (uint32_t)std::min<int64_t>(p4_bytes, 0xffffffffLL), (uint32_t)std::min<int64_t>(wf_bytes, 0xffffffffLL), xo);
         return hipGetLastError();
     };
     auto by_buf = [&](auto abin, auto form0, auto qmode, auto sp) -> hipError_t {

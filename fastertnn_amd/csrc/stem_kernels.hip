@@ -34,7 +34,9 @@ struct StemGeom {
     int H_pad, W_pad, H_stride, W_stride;
     int PH, PW;          // input patch of a tile: ((kTile - 1) * stride + K) per direction
     int tiles_x;
-    FastDiv dPW, dKW, dTX;
+    FastDiv dPW, dKW, dTX, dTiles;
+    uint32_t kn_tiles;
+    XcdOrder xo;
 };
 
 // ABIN / FORM0 / QMODE as in k_conv_f4; C is compile-time so that every shift below is a constant.
@@ -62,8 +64,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, lr = lane & 31;
-    const int n = blockIdx.z, kn0 = blockIdx.y * 64;
-    const int ty = (int)fastdiv(blockIdx.x, g.dTX), tx = (int)blockIdx.x - ty * g.tiles_x;
+    uint32_t img, bi;   // image, tile within it (kernel tile, pixel tile)
+    g.xo.tile(blockIdx.x, img, bi);
+    const uint32_t kt = fastdiv(bi, g.dTiles), bx = bi - kt * g.dTiles.d;
+    const int n = (int)img, kn0 = (int)kt * 64;
+    const int ty = (int)fastdiv(bx, g.dTX), tx = (int)bx - ty * g.tiles_x;
     const int NT = blockDim.x;   // 64 per wavefront: a tile is 4 rows of kTile pixels per wavefront
     const int oh0 = ty * (int)(blockDim.x >> 4), ow0 = tx * kTile;
     const int HW = g.H * g.W;
@@ -235,7 +240,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
             } else {
                 // as in k_conv_f4: lane half h ends up with bytes 16 a + 8 h .. + 8 of the pixel's 64-channel word
                 const uint2 out = hand_over_block<FORM0, QMODE>(r, alpha, qthr, dq, kn0 + 32 * a, h, KN);
-                const size_t word = ((size_t)n * gridDim.y + blockIdx.y) * OHW + pix;
+                const size_t word = ((size_t)n * g.kn_tiles + kt) * OHW + pix;
                 if (live)
                     *reinterpret_cast<uint2*>(static_cast<unsigned char*>(qo.p4) + word * 32 + 16 * a + 8 * h) = out;
             }
@@ -287,7 +292,11 @@ hipError_t launch_stem_f4(int type, const float* d_x, const float* d_thr, const 
     const int64_t tiles = (int64_t)g.tiles_x * tiles_y;
     const int kn_tiles = (KN + 63) / 64;
     if (tiles > 0x7fffffffLL || kn_tiles > 65535 || N > 65535) return hipErrorInvalidValue;
-    dim3 grid((unsigned)tiles, (unsigned)kn_tiles, (unsigned)N);
+    if ((uint64_t)tiles * kn_tiles * N > 0x7fffffffull) return hipErrorInvalidValue;   // (no such result fits in memory)
+    g.kn_tiles = (uint32_t)kn_tiles;
+    g.dTiles = make_fastdiv((uint32_t)tiles);
+    g.xo = make_xcd_order((uint64_t)N, (uint32_t)(tiles * kn_tiles));
+    const dim3 grid((unsigned)(tiles * kn_tiles * N));
     const uint4* Wf = static_cast<const uint4*>(d_wf);
     const int KB = round4(Kd);
     // BNN: every lane of the Kd words that is not a real (tap, channel) is +1 in both operands
