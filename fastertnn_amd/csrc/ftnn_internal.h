@@ -7,6 +7,8 @@ namespace ftnn {
 
 constexpr int kTNN = 0, kTBN = 1, kBTN = 2, kBNN = 3;
 
+typedef float v16f __attribute__((ext_vector_type(16)));
+
 inline int cpack_of(int C) { return (int)(((int64_t)C + 63) / 64); }
 inline int round4(int k) { return 4 * ((k + 3) / 4); }
 inline int out_dim(int in, int pad, int k, int stride) { return (in + 2 * pad - k) / stride + 1; }
@@ -61,13 +63,27 @@ struct ConvGeom {
 
 // Fused hand-over to a following fp4 layer: instead of the fp32 result, a GEMM kernel writes the
 // next layer's quantised input, P4[n][ceil(KN/64)][pixel][32 bytes] (see launch_quantize_f4), from
-// the same fp32 values: mode 1 = ternary with thr[n] (strict compares), 2 = binary, 0 = off.
+// the same fp32 values: mode 1 = ternary with threshold t (strict compares), 2 = binary, 0 = off.
 // Kernels past KN in the last 64-channel word get the padding nibble.
+//
+// cut = true: the thresholds as cuts on the integer r in front of PReLU, found on the host (make_quant_out).  PReLU does
+// not fall for a slope >= 0, so r -> sign is a staircase:
+//   ternary  -1 for r < lo, +1 for r > lo + width, 0 between
+//   binary   -1 (bit set) for r < lo, else +1
+// An accumulator that starts at `init` ends at a = r - lo (binary: r - lo + 1/2), and a value takes two vector
+// instructions, clamp(a - width, 0, 1) = p and med3(a, -1, p) (binary: one, med3(a, -1/2, 1/2)), before two of them
+// become two nibbles in one conversion (v_cvt_scalef32_pk_fp4_f32).  Other slopes and thresholds run PReLU and compare.
 struct QuantOut {
     void* p4 = nullptr;
-    const float* thr = nullptr;   // one threshold per batch item of the next layer
+    float t = 0.0f;       // the next layer's threshold
     int mode = 0;
+    bool cut = false;
+    float lo = 0.0f, width = 0.0f;
 };
+constexpr int kMaxCutSum = 1 << 22;   // largest |r| the cuts are made for: r - lo and its half steps stay exact in fp32
+
+// alpha, form0: the producing layer's PReLU; max_sum: bound of |r|
+QuantOut make_quant_out(void* p4, int mode, float t, float alpha, int64_t max_sum);
 
 // the E2M1 nibble of one value under QuantOut mode 1 / 2 (src/tnns/ternarize2row_avx2.c:443-449,
 // src/tnns/binarize2row_avx2.c:19-21); `live` = false gives the padding lane of that mode
@@ -85,78 +101,35 @@ __device__ __forceinline__ uint32_t quant_nibble(float v, float t, bool ternary,
     return r;
 }
 
-// The ternary hand-over without compares, for the slopes and thresholds layers use (anything else takes
-// quant_nibble on the PReLU result).  Both PReLU forms leave r > 0 as it is and turn r <= 0 into r * alpha <= 0, so
-// for alpha >= 0 and t >= 0: PReLU(r) > t <=> r > t, and PReLU(r) < -t <=> r * alpha < -t (r * alpha is the very
-// product PReLU forms; for r > 0 it is >= 0 >= -t).  r is an integer: with 2^-20 <= alpha <= 2^20 (or alpha = 0) and
-// t <= 2^40, a difference r - t or -(r * alpha) - t that is positive is at least 2^-44, so 2^60 times it clamps to
-// exactly 1, and one that is not positive clamps to +0.  The result is +1, -1 or +0 as a float, which
-// v_cvt_scalef32_pk_fp4_f32 turns into the E2M1 nibbles 0x2, 0xA, 0x0, two values per instruction.
-__device__ __forceinline__ bool tern_direct_applies(float alpha, float t) {
-    return (alpha == 0.0f || (alpha >= 0x1p-20f && alpha <= 0x1p20f)) && t >= 0.0f && t <= 0x1p40f;
-}
-__device__ __forceinline__ float tern_value_direct(float r, float alpha, float t_big /* t * 2^60 */) {
-    const float pos = __builtin_amdgcn_fmed3f(__builtin_fmaf(r, 0x1p60f, -t_big), 0.0f, 1.0f);
-    const float neg = __builtin_amdgcn_fmed3f(__builtin_fmaf(r * alpha, -0x1p60f, -t_big), 0.0f, 1.0f);
-    return pos - neg;
-}
-// The binary hand-over the same way: the bit is PReLU(r) < t.  For t > 0 that is r < t (r <= 0 gives PReLU <= 0 < t),
-// for t <= 0 it is r * alpha < t (r >= 0 gives PReLU >= 0 >= t).  With alpha = 0 or 2^-20 <= alpha <= 2^20 and t = 0
-// or 2^-20 <= |t| <= 2^40 a positive difference t - v is at least 2^-44; the result is -1 (bit set) or +1 as a float.
-// `t_pos` must be the same for all lanes of the wavefront.
-__device__ __forceinline__ bool bin_direct_applies(float alpha, float t) {
-    const float at = __builtin_fabsf(t);
-    return (alpha == 0.0f || (alpha >= 0x1p-20f && alpha <= 0x1p20f)) && (t == 0.0f || (at >= 0x1p-20f && at <= 0x1p40f));
-}
-__device__ __forceinline__ float bin_value_direct(float r, float alpha, float t_big /* t * 2^60 */, bool t_pos) {
-    const float v = t_pos ? r : r * alpha;
-    const float below = __builtin_amdgcn_fmed3f(__builtin_fmaf(v, -0x1p60f, t_big), 0.0f, 1.0f);
-    return __builtin_fmaf(below, -2.0f, 1.0f);
-}
-// Both hand-overs behind one face: whether the wavefront may take the compare-free form for its thresholds
-// (mode 1 ternary, 2 binary; for binary all thresholds must lie on the same side of zero), and the value.
-struct DirectQuant {
-    bool ok, t_pos;
-};
+// eight values -> one dword of E2M1 nibbles, value k in nibble k: ternary out of {+1, -1, 0}, binary out of {+1/2, -1/2}
+// (the conversion divides by its scale)
 template <int QMODE>
-__device__ __forceinline__ DirectQuant direct_quant(float alpha, float t) {
-    DirectQuant d = {false, false};
-    if constexpr (QMODE == 1) {
-        d.ok = __all(tern_direct_applies(alpha, t)) != 0;
-    } else if constexpr (QMODE == 2) {
-        const bool fits = bin_direct_applies(alpha, t);
-        d.t_pos = __all(fits && t > 0.0f) != 0;
-        d.ok = d.t_pos || __all(fits && !(t > 0.0f)) != 0;
-    }
-    return d;
-}
-template <int QMODE>
-__device__ __forceinline__ float direct_value(float r, float alpha, float t_big, bool t_pos, bool live) {
-    if constexpr (QMODE == 1) return live ? tern_value_direct(r, alpha, t_big) : 0.0f;
-    else return live ? bin_value_direct(r, alpha, t_big, t_pos) : 1.0f;   // padding lanes: 0 / +1
-}
-// eight values out of {+1, -1, +0} -> one dword of E2M1 nibbles, value k in nibble k
-__device__ __forceinline__ uint32_t pack_fp4x8(float z0, float z1, float z2, float z3, float z4, float z5, float z6,
-                                               float z7) {
+__device__ __forceinline__ uint32_t pack_fp4x8(const float* z) {
+    constexpr float scale = QMODE == 1 ? 1.0f : 0.5f;
     uint32_t d = 0u;
-    d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, z0, z1, 1.0f, 0);
-    d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, z2, z3, 1.0f, 1);
-    d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, z4, z5, 1.0f, 2);
-    d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, z6, z7, 1.0f, 3);
+    d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, z[0], z[1], scale, 0);
+    d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, z[2], z[3], scale, 1);
+    d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, z[4], z[5], scale, 2);
+    d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, z[6], z[7], scale, 3);
     return d;
 }
 
-// Hand-over store of one 32-kernel block: lanes l and l ^ 32 hold the nibbles of one pixel, lane half h those of
-// kernels 8 q + 4 h + {0..3}, as d0 (q = 0, 1) and d1 (q = 2, 3), 16 bits per q.  Returns the 8 bytes lane h
-// stores at byte 8 h of the block's 16: kernels in order.  v_permlane32_swap exchanges the upper half of d0 with the
-// lower half of d1, after which both lane halves combine their pair the same way.
-__device__ __forceinline__ uint2 exchange_halves(uint32_t d0, uint32_t d1) {
-    const auto r = __builtin_amdgcn_permlane32_swap(d0, d1, false, false);
-    // lanes 0..31: r[0] = own d0, r[1] = d0 of lane + 32; lanes 32..63: r[0] = d1 of lane - 32, r[1] = own d1
-    uint2 out;
-    out.x = (r[0] & 0xffffu) | (r[1] << 16);
-    out.y = (r[0] >> 16) | (r[1] & 0xffff0000u);
-    return out;
+// Lanes l and l ^ 32 hold the nibbles of one pixel for a 32-kernel block, lane half h those of kernels 8 q + 4 h + {0..3},
+// as d.x (q = 0, 1) and d.y (q = 2, 3), 16 bits per q; the block's dword q is the pair's 16 bits side by side.
+// v_permlane32_swap exchanges the upper half of its first operand with the lower half of its second.
+//
+// one block: lane half h returns dwords 2 h and 2 h + 1
+__device__ __forceinline__ uint2 exchange_halves(const uint2& d) {
+    const auto r = __builtin_amdgcn_permlane32_swap(d.x, d.y, false, false);
+    // lanes 0..31: r[0] = own d.x, r[1] = d.x of lane + 32; lanes 32..63: r[0] = d.y of lane - 32, r[1] = own d.y
+    return make_uint2((r[0] & 0xffffu) | (r[1] << 16), (r[0] >> 16) | (r[1] & 0xffff0000u));
+}
+// two blocks (the pixel's 64 kernels): lane half h returns the 16 bytes of block h
+__device__ __forceinline__ uint4 exchange_blocks(const uint2& b0, const uint2& b1) {
+    const auto r = __builtin_amdgcn_permlane32_swap(b0.x, b1.x, false, false);
+    const auto s = __builtin_amdgcn_permlane32_swap(b0.y, b1.y, false, false);
+    return make_uint4((r[0] & 0xffffu) | (r[1] << 16), (r[0] >> 16) | (r[1] & 0xffff0000u),
+                      (s[0] & 0xffffu) | (s[1] << 16), (s[0] >> 16) | (s[1] & 0xffff0000u));
 }
 
 // PReLU in the reference's two forms: "f <= 0 -> f *= alpha" (TNN, src/tnns/mm_p2_final_tnn_avx2.c:204-208; a zero
@@ -167,54 +140,41 @@ __device__ __forceinline__ float prelu_ref(float r, float alpha) {
     return scale ? r * alpha : r;
 }
 
-// One 32-kernel block of a pixel under the hand-over.  r[e] = this lane's 16 results before PReLU, kernel
-// kbase + 8 (e / 4) + 4 h + e % 4 (h = lane half); t = the next layer's threshold for the pixel's image; dq from
-// direct_quant.  Returns the 8 bytes this lane stores at byte 8 h of the block's 16.  Every lane of the wavefront
-// must call it (exchange_halves crosses lanes).
+// what an accumulator starts at: r = sum - bias with the hand-over's cut taken off, see QuantOut (wave-uniform)
+template <int QMODE>
+__device__ __forceinline__ float acc_init(const QuantOut& qo, float bias) {
+    if (QMODE == 0 || !qo.cut) return 0.0f - bias;
+    return 0.0f - qo.lo - bias + (QMODE == 2 ? 0.5f : 0.0f);
+}
+
+// One 32-kernel block of a pixel under the hand-over.  v[e] = this lane's 16 accumulators (started at acc_init), kernel
+// kbase + 8 (e / 4) + 4 h + e % 4 (h = lane half).  Returns the nibbles as exchange_halves / exchange_blocks take them.
 template <bool FORM0, int QMODE>
-__device__ __forceinline__ uint2 hand_over_block(const float (&r)[16], float alpha, float t, const DirectQuant& dq,
-                                                 int kbase, int h, int KN) {
+__device__ __forceinline__ uint2 hand_over_block(const v16f& v, float alpha, const QuantOut& qo, int kbase, int h, int KN) {
     const bool whole = kbase + 32 <= KN;   // wave-uniform: the block holds real kernels only
-    uint32_t d0, d1;
-    if (dq.ok) {
-        // no compares, two nibbles per conversion (see tern_value_direct)
-        const float t_big = t * 0x1p60f;
+    if (qo.cut) {
         float z[16];
-        if (whole) {
 #pragma unroll
-            for (int e = 0; e < 16; e++) z[e] = direct_value<QMODE>(r[e], alpha, t_big, dq.t_pos, true);
-        } else {   // kernels past KN hold the padding lane
+        for (int e = 0; e < 16; e++) {
+            if (QMODE == 1) z[e] = __builtin_amdgcn_fmed3f(v[e], -1.0f, __builtin_amdgcn_fmed3f(v[e] - qo.width, 0.0f, 1.0f));
+            else z[e] = __builtin_amdgcn_fmed3f(v[e], -0.5f, 0.5f);
+        }
+        if (!whole) {   // kernels past KN hold the padding lane
 #pragma unroll
             for (int e = 0; e < 16; e++)
-                z[e] = direct_value<QMODE>(r[e], alpha, t_big, dq.t_pos, kbase + 8 * (e >> 2) + 4 * h + (e & 3) < KN);
+                z[e] = kbase + 8 * (e >> 2) + 4 * h + (e & 3) < KN ? z[e] : (QMODE == 1 ? 0.0f : 0.5f);
         }
-        d0 = pack_fp4x8(z[0], z[1], z[2], z[3], z[4], z[5], z[6], z[7]);
-        d1 = pack_fp4x8(z[8], z[9], z[10], z[11], z[12], z[13], z[14], z[15]);
-    } else {
-        constexpr bool tern = QMODE == 1;
-        uint32_t half[4];
-        if (whole) {
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                half[g] = 0u;
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    half[g] |= quant_nibble(prelu_ref<FORM0>(r[4 * g + i], alpha), t, tern, true) << (4 * i);
-            }
-        } else {
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                half[g] = 0u;
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    half[g] |= quant_nibble(prelu_ref<FORM0>(r[4 * g + i], alpha), t, tern, kbase + 8 * g + 4 * h + i < KN)
-                               << (4 * i);
-            }
-        }
-        d0 = half[0] | (half[1] << 16);
-        d1 = half[2] | (half[3] << 16);
+        return make_uint2(pack_fp4x8<QMODE>(z), pack_fp4x8<QMODE>(z + 8));
     }
-    return exchange_halves(d0, d1);
+    uint32_t half[4];
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        half[g] = 0u;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            half[g] |= quant_nibble(prelu_ref<FORM0>(v[4 * g + i], alpha), qo.t, QMODE == 1, kbase + 8 * g + 4 * h + i < KN) << (4 * i);
+    }
+    return make_uint2(half[0] | (half[1] << 16), half[2] | (half[3] << 16));
 }
 
 // record a failure text for ftnn_last_error(); returns `code`

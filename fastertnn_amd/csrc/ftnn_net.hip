@@ -10,6 +10,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <cmath>
 #include <new>
 #include <vector>
 
@@ -51,6 +52,36 @@ struct ftnn_net {
     hipStream_t g_stream = nullptr;
 };
 
+namespace ftnn {
+
+// The cuts are found with the very fp32 products and compares the kernels would make (r * alpha rounds the same on both
+// sides), by bisection over the integers r: PReLU(r) does not fall with r for a slope >= 0.
+QuantOut make_quant_out(void* p4, int mode, float t, float alpha, int64_t max_sum) {
+    QuantOut q;
+    q.p4 = p4;
+    q.mode = mode;
+    q.t = t;
+    const bool finite = alpha >= 0.0f && alpha <= 3.0e38f && t >= -3.0e38f && t <= 3.0e38f;
+    if (!finite || max_sum > kMaxCutSum || (mode == 1 && t < 0.0f)) return q;
+    auto first_at_least = [&](float bound) {   // smallest r in [-max, max + 1] with PReLU(r) >= bound (max + 1: none)
+        int lo = -kMaxCutSum, hi = kMaxCutSum + 1;
+        while (lo < hi) {
+            const int mid = lo + (hi - lo) / 2;
+            const float r = (float)mid, v = mid > 0 ? r : r * alpha;
+            if (v >= bound) hi = mid;
+            else lo = mid + 1;
+        }
+        return lo;
+    };
+    q.cut = true;
+    q.lo = (float)first_at_least(mode == 1 ? -t : t);
+    // +1 from r > t on: r is positive there and PReLU leaves it as it is
+    if (mode == 1) q.width = (t >= (float)kMaxCutSum ? (float)kMaxCutSum : std::floor(t)) - q.lo;
+    return q;
+}
+
+}  // namespace ftnn
+
 namespace {
 
 using namespace ftnn;
@@ -66,9 +97,8 @@ int enqueue_layer(ftnn_net* net, const NetPart& part, int i, const float*& in, b
     QuantOut qo;
     if (next_f4) {
         const int nt = net->layers[i + 1].type;
-        qo.p4 = part.d_p4[(size_t)net->p4_buf[i + 1]];
-        qo.thr = net->d_thr[i + 1];   // every entry holds the layer's threshold: any run of `batch` entries serves
-        qo.mode = (nt == kTNN || nt == kTBN) ? 1 : 2;
+        qo = make_quant_out(part.d_p4[(size_t)net->p4_buf[i + 1]], (nt == kTNN || nt == kTBN) ? 1 : 2, net->layers[i + 1].threshold,
+                            L.prelu_alpha, (int64_t)64 * cpack_of(L.C) * L.KH * L.KW);
     }
     float* out = next_f4 ? nullptr : ((i == n - 1) ? d_y : part.d_act[i & 1]);
     int rc;

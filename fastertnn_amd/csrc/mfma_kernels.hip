@@ -34,7 +34,6 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
 // Ring of NS LDS buffers, each holding KF fragments (K words for fp4) per row-block: one barrier per KF fragments.
@@ -790,202 +789,205 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
 //     reference's fill, src/tnns/ternarize2row_avx2.c:748-755, src/tnns/binarize2row_avx2.c:151);
 //   * the padding words that round K up to a multiple of 4 are skipped: their products are zero
 //     except for BNN, whose epilogue constant counts the real words only.
-struct ConvFrag {
-    v4i w[2], x[2];
-    bool in[2];   // x[b] holds a real input pixel (else the padding value replaces it)
-};
-
 // ABIN: binary activations (padding value +1).  FORM0: the TNN form of PReLU, "f <= 0 -> f *= alpha"
 // (mm_p2_final_tnn_avx2.c:204-208), else "r >= 0 ? r : alpha * r" (mm_p2_final_tbn_avx2.c:73).
 // QMODE: 0 = fp32 NCHW result, 1 / 2 = ternary / binary hand-over to the next layer (QuantOut).
 // All three are compile-time so that the per-element epilogue carries no selects for them.
+// TA x TB: blocks of 32 kernels x 32 pixels per wavefront.  2 x 2, or 1 x 1 with S = 4 for layers with few tiles: a
+// wavefront moves a bounded number of bytes per cycle from a cold L2 whatever its prefetch depth (600-700 cycles per K word
+// of a 64 x 64 tile, measured), so a small layer gets faster only with more wavefronts, on more compute units.  Kernel
+// tiles of 32 come in pairs under the hand-over (a pixel's 64-channel word is written by two workgroups, 16 bytes each; a
+// tile past KN writes padding lanes).
 // The unsplit hand-over variants are the ones launched with several thousand wavefronts (stems,
 // first stages): they are asked to fit three wavefronts per SIMD, which they do without scratch.
-// BUF: fragments arrive through buffer loads.  Their offsets are 32-bit, the weight fragment of a word is addressed
-// by a scalar offset alone, and for ternary activations an offset beyond the buffer returns zeros, which is what a
-// tap outside the image must contribute: no select on the loaded data, a third of the K loop's vector instructions
-// gone (binary activations pad with +1 and keep the select).  Needs both operands below 4 GiB (p4_bytes, wf_bytes: the sizes the descriptors announce).
-template <bool ABIN, bool FORM0, int QMODE, int S, int NB, bool BUF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && QMODE != 0) ? 3 : 1, 8))) void k_conv_f4(const uint4* __restrict__ P4, const uint4* __restrict__ Wf,
-                                                 float* __restrict__ Y, int M, int KN, int OHW, int KB,
-                                                 int bias, float alpha, FastDiv dOHW, ConvGeom cg, QuantOut qo,
-                                                 uint32_t p4_bytes, uint32_t wf_bytes, XcdOrder xo) {
-    uint32_t bx, by;   // pixel tiles, kernel tile
-    xo.tile(blockIdx.x + gridDim.x * blockIdx.y, bx, by);
-    // NB register sets of fragments: NB - 1 steps of loads in flight
+// BUF: fragments arrive through buffer loads.  Their offsets are 32-bit, the place of a word within the operand is a
+// scalar offset, and for ternary activations an offset beyond the buffer returns zeros, which is what a
+// tap outside the image must contribute: no select on the loaded data (binary activations pad with +1 and keep the select).
+// Needs both operands and an fp32 result below 4 GiB (p4_bytes, wf_bytes, y_bytes: the sizes the descriptors announce).
+template <bool ABIN, bool FORM0, int QMODE, int TA, int TB, int S, bool BUF>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && QMODE != 0) ? 3 : 1, 8))) void k_conv_f4(
+    const uint4* __restrict__ P4, const uint4* __restrict__ Wf, float* __restrict__ Y, int M, int KN, int OHW, int KB, int bias,
+    float alpha, FastDiv dOHW, ConvGeom cg, QuantOut qo, uint32_t p4_bytes, uint32_t wf_bytes, uint32_t y_bytes, XcdOrder xo) {
     constexpr int WPB = 4;                // wavefronts per workgroup (single-wavefront workgroups for S = 1
                                           // measured slower: neighbours no longer share weight fragments in L1)
-    constexpr int PUB = 4 - 4 / S;        // blocks a wavefront hands to the others of its tile
+    constexpr int NB = 3;                 // register sets of fragments: NB - 1 words of loads in flight; more measured no faster
+    constexpr int NBLK = TA * TB;
+    constexpr int PUB = NBLK == 1 ? 1 : 4 - 4 / S;   // blocks a wavefront hands to the others of its tile
     __shared__ float4 red[S > 1 ? 4 * PUB * 4 * 64 : 1];   // [wavefront][slot][e / 4][lane]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ks = wave % S, pt = wave / S;   // K share and pixel tile of this wavefront
     const int h = lane >> 5, lr = lane & 31;
-    const int px0 = (bx * (WPB / S) + pt) * 64, kn0 = by * 64;
+    uint32_t bx, by;   // pixel tiles, kernel tile
+    xo.tile(blockIdx.x + gridDim.x * blockIdx.y, bx, by);
+    const int px0 = ((int)bx * (WPB / S) + pt) * 32 * TB, kn0 = (int)by * 32 * TA;
 
-    int ih0[2], iw0[2];
-    uint32_t pb[2];
+    int ih0[TB], iw0[TB];
+    uint32_t img[TB], pix[TB], xrec[TB];   // xrec: record of (image, plane 0, pixel (ih0, iw0)) in P4[n][C_pack][pixel]
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
+    for (int b = 0; b < TB; b++) {
         const uint32_t q = (uint32_t)min(px0 + 32 * b + lr, M - 1);
-        const uint32_t n = fastdiv(q, dOHW);
-        const uint32_t pix = q - n * (uint32_t)OHW;
-        const int oh = (int)fastdiv(pix, cg.dOW), ow = (int)pix - oh * cg.OW;
+        img[b] = fastdiv(q, dOHW);
+        pix[b] = q - img[b] * (uint32_t)OHW;
+        const int oh = (int)fastdiv(pix[b], cg.dOW), ow = (int)pix[b] - oh * cg.OW;
         ih0[b] = oh * cg.H_stride - cg.H_pad;
         iw0[b] = ow * cg.W_stride - cg.W_pad;
-        pb[b] = n * (uint32_t)(cg.CP * cg.H * cg.W);   // image n of P4[n][C_pack][pixel]
-    }
-    // threshold of each pixel block's image for the hand-over, fetched now, in front of the K loop's loads
-    float qthr[2] = {0.0f, 0.0f};
-    if constexpr (QMODE != 0) {
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-            qthr[b] = qo.thr[fastdiv((uint32_t)min(px0 + 32 * b + lr, M - 1), dOHW)];
+        xrec[b] = img[b] * (uint32_t)(cg.CP * cg.H * cg.W) + (uint32_t)(ih0[b] * cg.W + iw0[b]);
     }
     const int HWin = cg.H * cg.W;
     const int rbmax = (KN + 31) / 32 - 1;
-    const uint4* wb[2];
-#pragma unroll
-    for (int a = 0; a < 2; a++) wb[a] = Wf + (size_t)min(kn0 / 32 + a, rbmax) * KB * 64 + lane;
 
-    v16f acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[a][b][e] = 0.0f;
-
-    const uint32_t fillv = ABIN ? 0x22222222u : 0u;
-    // All four loads of a step are unconditional (a tap outside the image reads pixel 0 of its image and is replaced
-    // by the padding value before use) and are issued two steps ahead of the step being multiplied.  They are ordinary
-    // loads (plain, or buffer-load builtins), so the compiler owns the dependency between a load and the use of its
-    // registers and places every s_waitcnt vmcnt itself; what keeps a load where the code issues it -- and not next to
-    // its use, where the scheduler would sink it -- is the scheduling fence after each step's loads (fence_loads).
-    auto ld16 = [](v4i& dst, const uint4* src) { dst = *reinterpret_cast<const v4i*>(src); };
-    // buffer descriptors (base; stride 0; bytes; raw 32-bit data format) and this lane's fixed offsets
-    __amdgpu_buffer_rsrc_t brs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(P4), 0, (int)p4_bytes, 0x00020000);
-    __amdgpu_buffer_rsrc_t brs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(Wf), 0, (int)wf_bytes, 0x00020000);
-    uint32_t wofs[2] = {0u, 0u}, xofs[2] = {0u, 0u};
-    if constexpr (BUF) {
-#pragma unroll
-        for (int a = 0; a < 2; a++) wofs[a] = ((uint32_t)min(kn0 / 32 + a, rbmax) * (uint32_t)KB * 64u + (uint32_t)lane) * 16u;
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-            xofs[b] = ((pb[b] + (uint32_t)(ih0[b] * cg.W + iw0[b])) * 2u + (uint32_t)h) * 16u;
+    // The words of this wavefront, [w, w1) of the reference's K order (kh * KW + kw) * C_pack + ic: a word is a step of
+    // one plane within a tap, so the lanes compute addresses and borders once per tap and everything else is scalar.
+    int w = S == 1 ? 0 : (int)((uint32_t)(cg.K * ks) / S);
+    const int w1 = S == 1 ? cg.K : (int)((uint32_t)(cg.K * (ks + 1)) / S);
+    const int words = w1 - w;
+    int kh = 0, kw = 0, ic = 0;
+    if constexpr (S > 1) {
+        const int tap = (int)fastdiv((uint32_t)w, cg.dCP);
+        ic = w - tap * cg.CP;
+        kh = (int)fastdiv((uint32_t)tap, cg.dKW);
+        kw = tap - kh * cg.KW;
     }
-    auto ldbuf = [&](v4i& dst, uint32_t voff, uint32_t soff, bool weights) {
-        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(weights ? brs_w : brs_x, (int)voff, (int)soff, 0);
-        dst = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+    struct Frag {
+        v4i w[TA], x[TB];
+        bool in[TB];   // x[b] holds a real input pixel (else the padding value replaces it)
     };
-    auto load = [&](int w, ConvFrag& f) {   // w is wave-uniform
-        const int tap = (int)fastdiv((uint32_t)w, cg.dCP), ic = w - tap * cg.CP;
-        const int kh = (int)fastdiv((uint32_t)tap, cg.dKW), kw = tap - kh * cg.KW;
-        if constexpr (BUF) {
-            const uint32_t wsoff = (uint32_t)__builtin_amdgcn_readfirstlane(w) * 1024u;
+    uint32_t vx[TB];   // the tap's record (BUF: byte offset) for this lane's pixels
+    bool in[TB];
+    auto tap = [&]() {
 #pragma unroll
-            for (int a = 0; a < 2; a++) ldbuf(f.w[a], wofs[a], wsoff, true);
-            // byte offset of the record = this lane's part (xofs, fixed) + the word's part (scalar); the sum wraps
-            // to the right value whenever the tap lies inside the image
-            const uint32_t tapoff = (uint32_t)__builtin_amdgcn_readfirstlane((ic * HWin + kh * cg.W + kw) * 32);
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                const int ih = ih0[b] + kh, iw = iw0[b] + kw;
-                const bool in = (unsigned)ih < (unsigned)cg.H && (unsigned)iw < (unsigned)cg.W;
-                // ternary activations: an offset beyond p4_bytes returns the zeros that padding is; binary ones pad
-                // with +1, read record 0 instead and take the select in compute()
-                ldbuf(f.x[b], in ? xofs[b] + tapoff : (ABIN ? 0u : 0xffffff00u), 0u, false);
-                f.in[b] = ABIN ? in : true;
-            }
-        } else {
-#pragma unroll
-            for (int a = 0; a < 2; a++) ld16(f.w[a], wb[a] + (size_t)w * 64);
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                const int ih = ih0[b] + kh, iw = iw0[b] + kw;
-                const bool in = (unsigned)ih < (unsigned)cg.H && (unsigned)iw < (unsigned)cg.W;
-                const size_t o = (size_t)(pb[b] + (uint32_t)(ic * HWin + (in ? ih * cg.W + iw : 0))) * 2 + h;
-                ld16(f.x[b], P4 + o);
-                f.in[b] = in;
-            }
+        for (int b = 0; b < TB; b++) {
+            in[b] = (unsigned)(ih0[b] + kh) < (unsigned)cg.H && (unsigned)(iw0[b] + kw) < (unsigned)cg.W;
+            const uint32_t rec = xrec[b] + (uint32_t)(kh * cg.W + kw);   // wraps to the right value whenever the tap is inside
+            // a tap outside the image: an offset beyond the buffer returns zeros, the padding of ternary activations;
+            // binary ones read record 0 and take the padding value in compute()
+            if (BUF) vx[b] = in[b] ? rec * 32u + 16u * (uint32_t)h : (ABIN ? 0u : 0xffffff00u);
+            else vx[b] = in[b] ? rec : 0u;
         }
     };
-    auto fence_loads = []() { __builtin_amdgcn_sched_barrier(0); };   // the loads issued so far stay in front of this point
-    auto compute = [&](const ConvFrag& f) {
-        v8i x[2], wv[2];
+    tap();
+    // buffer descriptors (base; stride 0; bytes; raw 32-bit data format)
+    const __amdgpu_buffer_rsrc_t brs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(P4), 0, (int)p4_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t brs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(Wf), 0, (int)wf_bytes, 0x00020000);
+    // All loads of a word are unconditional and are issued two words ahead of the one being multiplied.  They are ordinary
+    // loads (plain, or buffer-load builtins), so the compiler owns the dependency between a load and the use of its
+    // registers and places every s_waitcnt vmcnt itself; what keeps a load where the code issues it -- and not next to
+    // its use, where the scheduler would sink it -- is the scheduling fence after each word's loads.
+    uint32_t vw = (uint32_t)lane * 16u;
+    auto load = [&](Frag& f) {   // word w, then on to the next one
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
+        for (int a = 0; a < TA; a++) {
+            const uint32_t block = (uint32_t)min(kn0 / 32 + a, rbmax) * (uint32_t)KB + (uint32_t)w;
+            if constexpr (BUF) {
+                const v4u v = __builtin_amdgcn_raw_buffer_load_b128(brs_w, (int)vw, (int)(block * 1024u), 0);
+                f.w[a] = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+            } else {
+                f.w[a] = *reinterpret_cast<const v4i*>(Wf + (size_t)block * 64 + lane);
+            }
+        }
 #pragma unroll
-            for (int i = 0; i < 4; i++) x[b][i] = ((BUF && !ABIN) || f.in[b]) ? f.x[b][i] : (int)fillv;
+        for (int b = 0; b < TB; b++) {
+            if constexpr (BUF) {
+                const v4u v = __builtin_amdgcn_raw_buffer_load_b128(brs_x, (int)vx[b], ic * HWin * 32, 0);
+                f.x[b] = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+            } else {
+                f.x[b] = *reinterpret_cast<const v4i*>(P4 + (size_t)(vx[b] + (uint32_t)(in[b] ? ic * HWin : 0)) * 2 + h);
+            }
+            f.in[b] = in[b];
+        }
+        if (w + 1 < w1) {
+            w++;
+            if (++ic == cg.CP) {
+                ic = 0;
+                if (++kw == cg.KW) {
+                    kw = 0;
+                    kh++;
+                }
+                tap();
+            }
+        } else if (BUF) {   // past the end: offsets beyond the buffers, which move no data (else the last word is read again)
+            vw = 0xffffff00u;
+#pragma unroll
+            for (int b = 0; b < TB; b++) vx[b] = 0xffffff00u;
+        }
+        __builtin_amdgcn_sched_barrier(0);   // these loads stay in front of the multiplies that follow
+    };
+    v16f acc[TA][TB];
+    auto compute = [&](const Frag& f) {
+        v8i x[TB], wv[TA];
+#pragma unroll
+        for (int b = 0; b < TB; b++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[b][i] = ((BUF && !ABIN) || f.in[b]) ? f.x[b][i] : (ABIN ? 0x22222222 : 0);
 #pragma unroll
             for (int i = 4; i < 8; i++) x[b][i] = 0;
         }
 #pragma unroll
-        for (int a = 0; a < 2; a++) wv[a] = v8i{f.w[a][0], f.w[a][1], f.w[a][2], f.w[a][3], 0, 0, 0, 0};
+        for (int a = 0; a < TA; a++) wv[a] = v8i{f.w[a][0], f.w[a][1], f.w[a][2], f.w[a][3], 0, 0, 0, 0};
         // cbsz = blgp = 4: both operands E2M1, unscaled (see mfma<true>)
 #pragma unroll
-        for (int a = 0; a < 2; a++)
+        for (int a = 0; a < TA; a++)
 #pragma unroll
-            for (int b = 0; b < 2; b++)
+            for (int b = 0; b < TB; b++)
                 acc[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wv[a], x[b], acc[a][b], 4, 4, 0, 0, 0, 0);
     };
 
-    // The register sets rotate by name (the loop is unrolled by NB); loads past the last word
-    // re-read it and are not multiplied (whole rounds of NB steps).
-    const int K = cg.K;
-    ConvFrag f[NB];
-    int w = ks;
+    // The register sets rotate by name (the loop is unrolled by NB); loads past the last word are not multiplied.
+    Frag f[NB];
 #pragma unroll
-    for (int j = 0; j < NB - 1; j++) load(min(w + S * j, K - 1), f[j]);
-    for (; w < K; w += S * NB) {
+    for (int j = 0; j < NB - 1; j++) load(f[j]);
+    {   // the accumulators are cleared while the first loads are on their way
+        const float init = ks == 0 ? acc_init<QMODE>(qo, FORM0 ? 0.0f : (float)bias) : 0.0f;   // only BNN has a bias
+#pragma unroll
+        for (int a = 0; a < TA; a++)
+#pragma unroll
+            for (int b = 0; b < TB; b++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[a][b][e] = init;
+    }
+    for (int i = 0; i < words; i += NB) {   // (a share of K is empty where K < S)
 #pragma unroll
         for (int j = 0; j < NB; j++) {
-            load(min(w + S * (j + NB - 1), K - 1), f[(j + NB - 1) % NB]);
-            fence_loads();
-            if (j == 0 || w + S * j < K) compute(f[j]);
+            load(f[(j + NB - 1) % NB]);
+            if (j == 0 || i + j < words) compute(f[j]);
         }
     }
 
-    // hand-over: whether every lane of a pixel block may take the compare-free form
-    DirectQuant direct_q[2] = {{false, false}, {false, false}};
-    if constexpr (QMODE != 0) {
-#pragma unroll
-        for (int b = 0; b < 2; b++) direct_q[b] = direct_quant<QMODE>(alpha, qthr[b]);
-    }
-    // Block id = 2*a + b; wavefront ks of a tile finishes the blocks with id % S == ks and hands
+    // Block id = TB * a + b; wavefront ks of a tile finishes the blocks with id % S == ks and hands
     // the others over through LDS.  Every copy below names its accumulator registers statically,
     // under a wave-uniform branch, so that no register array is indexed at run time.
     auto for_blocks = [&](auto&& fn) {
         fn(std::integral_constant<int, 0>{});
-        fn(std::integral_constant<int, 1>{});
-        fn(std::integral_constant<int, 2>{});
-        fn(std::integral_constant<int, 3>{});
+        if constexpr (NBLK == 4) {
+            fn(std::integral_constant<int, 1>{});
+            fn(std::integral_constant<int, 2>{});
+            fn(std::integral_constant<int, 3>{});
+        }
+    };
+    auto slot_of = [](int blk, int v) {   // slot of blk among the blocks that wavefront v does not own
+        return NBLK == 1 ? 0 : (S == 4 ? (blk < v ? blk : blk - 1) : blk / 2);
     };
     if constexpr (S > 1) {
         for_blocks([&](auto blk_tag) {
             constexpr int BLK = decltype(blk_tag)::value;
             if (BLK % S != ks) {
-                // slot of BLK among the blocks wavefront ks does not own
-                const int slot = S == 4 ? (BLK < ks ? BLK : BLK - 1) : BLK / 2;
-                float4* dst = red + (size_t)((wave * PUB + slot) * 4) * 64 + lane;
-                const v16f& c = acc[BLK >> 1][BLK & 1];
+                float4* dst = red + (size_t)((wave * PUB + slot_of(BLK, ks)) * 4) * 64 + lane;
+                const v16f& c = acc[BLK / TB][BLK % TB];
 #pragma unroll
                 for (int e4 = 0; e4 < 4; e4++)
                     dst[e4 * 64] = make_float4(c[4 * e4], c[4 * e4 + 1], c[4 * e4 + 2], c[4 * e4 + 3]);
             }
         });
         __syncthreads();
-    }
-    for_blocks([&](auto blk_tag) {
-        constexpr int BLK = decltype(blk_tag)::value;
-        if (BLK % S == ks) {
-            v16f mine = acc[BLK >> 1][BLK & 1];
-            if constexpr (S > 1) {
+        for_blocks([&](auto blk_tag) {
+            constexpr int BLK = decltype(blk_tag)::value;
+            if (BLK % S == ks) {
+                v16f& mine = acc[BLK / TB][BLK % TB];
 #pragma unroll
                 for (int v = 0; v < S; v++) {
-                    if (v != BLK % S) {   // source wavefront pt*S + v holds BLK in the slot computed as above
-                        const int slot = S == 4 ? (BLK < v ? BLK : BLK - 1) : BLK / 2;
-                        const float4* src = red + (size_t)(((pt * S + v) * PUB + slot) * 4) * 64 + lane;
+                    if (v != BLK % S) {   // source wavefront pt * S + v
+                        const float4* src = red + (size_t)(((pt * S + v) * PUB + slot_of(BLK, v)) * 4) * 64 + lane;
 #pragma unroll
                         for (int e4 = 0; e4 < 4; e4++) {
                             const float4 t = src[e4 * 64];
@@ -997,189 +999,71 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
                     }
                 }
             }
-            // accumulator e: kernel = 32*a + 8*(e/4) + 4*(lane/32) + e%4, pixel = 32*b + lane%32
-            constexpr int a = BLK >> 1, b = BLK & 1;
-            const int q = px0 + 32 * b + lr;
-            const uint32_t qc = (uint32_t)min(q, M - 1);
-            const uint32_t img = fastdiv(qc, dOHW);
-            const uint32_t pix = qc - img * (uint32_t)OHW;
-            // r = acc - bias: both are integers below 2^24 in fp32, and so is their difference (only BNN has a bias)
-            const float fbias = (float)bias;
-            float r[16];
+        });
+    }
+    // accumulator e of block (a, b): kernel = kn0 + 32 a + 8 (e / 4) + 4 h + e % 4, pixel = px0 + 32 b + lr
+    if constexpr (QMODE == 0) {
+        const __amdgpu_buffer_rsrc_t brs_y = __builtin_amdgcn_make_buffer_rsrc(Y, 0, (int)y_bytes, 0x00020000);
+        const bool as_max = alpha >= 0.0f && alpha <= 1.0f;   // PReLU is then max(r, r * alpha), bit for bit
+        for_blocks([&](auto blk_tag) {
+            constexpr int BLK = decltype(blk_tag)::value, a = BLK / TB, b = BLK % TB;
+            if (BLK % S == ks) {
+                const v16f& c = acc[a][b];
+                float r[16];
+                if (as_max) {
 #pragma unroll
-            for (int e = 0; e < 16; e++) r[e] = FORM0 ? mine[e] : mine[e] - fbias;
-            if constexpr (QMODE == 0) {
-                float* yq = Y + ((size_t)img * KN + kn0 + 32 * a + 4 * h) * OHW + pix;
-                if (q < M) {
-                    if (kn0 + 32 * a + 32 <= KN) {   // whole block inside: no per-kernel checks
+                    for (int e = 0; e < 16; e++) r[e] = __builtin_fmaxf(c[e], c[e] * alpha);
+                } else {
 #pragma unroll
-                        for (int e = 0; e < 16; e++)
-                            yq[(size_t)(8 * (e >> 2) + (e & 3)) * OHW] = prelu_ref<FORM0>(r[e], alpha);
-                    } else {
+                    for (int e = 0; e < 16; e++) r[e] = prelu_ref<FORM0>(c[e], alpha);
+                }
+                const bool live = px0 + 32 * b + lr < M;
+                const bool whole = kn0 + 32 * a + 32 <= KN;   // uniform: no per-kernel checks
+                const int p0 = kn0 + 32 * a + 4 * h;
+                if constexpr (BUF) {
+                    // a lane's part, and the kernel's row as a scalar; lanes past the pixels store beyond the buffer: nothing
+                    const uint32_t vy = live ? ((img[b] * (uint32_t)KN + (uint32_t)p0) * (uint32_t)OHW + pix[b]) * 4u : 0xffffff00u;
 #pragma unroll
-                        for (int e = 0; e < 16; e++) {
-                            const int p = kn0 + 32 * a + 8 * (e >> 2) + 4 * h + (e & 3);
-                            if (p < KN) yq[(size_t)(8 * (e >> 2) + (e & 3)) * OHW] = prelu_ref<FORM0>(r[e], alpha);
-                        }
+                    for (int e = 0; e < 16; e++) {
+                        const int row = 8 * (e >> 2) + (e & 3);
+                        if (whole || p0 + row < KN)
+                            __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_uint(r[e]), brs_y, (int)vy, row * OHW * 4, 0);
+                    }
+                } else if (live) {
+                    float* yq = Y + ((size_t)img[b] * KN + p0) * OHW + pix[b];
+#pragma unroll
+                    for (int e = 0; e < 16; e++) {
+                        const int row = 8 * (e >> 2) + (e & 3);
+                        if (whole || p0 + row < KN) yq[(size_t)row * OHW] = r[e];
                     }
                 }
-            } else {
-                // Hand-over to an fp4 layer.  Registers 4g .. 4g+3 of this lane are kernels 8g + 4h + {0..3} of the
-                // block: half of nibble dword g of the pixel, the other half sits in lane ^ 32.  Lane half h ends up
-                // with bytes 16a + 8h .. + 8 of the pixel's 64-channel word.
-                const uint2 out = hand_over_block<FORM0, QMODE>(r, alpha, qthr[b], direct_q[b], kn0 + 32 * a, h, KN);
-                const size_t word = ((size_t)img * gridDim.y + by) * OHW + pix;
-                if (q < M) *reinterpret_cast<uint2*>(static_cast<unsigned char*>(qo.p4) + word * 32 + 16 * a + 8 * h) = out;
             }
-        }
-    });
-}
-
-// The same layer on tiles of 32 kernels x 32 pixels, for layers with few tiles of 64 x 64: a wavefront moves a
-// bounded number of bytes per cycle from a cold L2 whatever its prefetch depth (600-700 cycles per K word of a
-// 64 x 64 tile, measured), so a small layer gets faster only with more wavefronts, on more compute units.  A
-// workgroup is one tile; its four wavefronts split the K loop four ways (word w to wavefront w % 4, one weight and
-// one activation fragment per word), wavefronts 1..3 hand their partial block over through LDS and wavefront 0
-// finishes it.  Kernel tiles come in pairs under the hand-over (a pixel's 64-channel word is written by two
-// workgroups, 16 bytes each; a tile past KN writes padding lanes).
-// BUF: fragments through buffer loads, as in k_conv_f4.
-template <bool ABIN, bool FORM0, int QMODE, bool BUF>
-__global__ __launch_bounds__(256) void k_conv_f4_small(const uint4* __restrict__ P4, const uint4* __restrict__ Wf,
-                                                       float* __restrict__ Y, int M, int KN, int OHW, int KB, int bias,
-                                                       float alpha, FastDiv dOHW, ConvGeom cg, QuantOut qo,
-                                                       uint32_t p4_bytes, uint32_t wf_bytes, XcdOrder xo) {
-    uint32_t bx, by;   // pixel tiles, kernel tile
-    xo.tile(blockIdx.x + gridDim.x * blockIdx.y, bx, by);
-    constexpr int S = 4, NB = 3;
-    __shared__ float4 red[3 * 4 * 64];   // [wavefront - 1][e / 4][lane]
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = lane >> 5, lr = lane & 31;
-    const int px0 = bx * 32, kn0 = by * 32;
-
-    const int q = px0 + lr;
-    const uint32_t qc = (uint32_t)min(q, M - 1);
-    const uint32_t img = fastdiv(qc, dOHW);
-    const uint32_t pix = qc - img * (uint32_t)OHW;
-    const int oh = (int)fastdiv(pix, cg.dOW), ow = (int)pix - oh * cg.OW;
-    const int ih0 = oh * cg.H_stride - cg.H_pad, iw0 = ow * cg.W_stride - cg.W_pad;
-    const uint32_t pb = img * (uint32_t)(cg.CP * cg.H * cg.W);   // image of P4[n][C_pack][pixel]
-    float qthr = 0.0f;
-    if constexpr (QMODE != 0) qthr = qo.thr[img];   // fetched in front of the K loop's loads (see k_conv_f4)
-    const int HWin = cg.H * cg.W;
-    const int rbmax = (KN + 31) / 32 - 1;
-    const uint4* wb = Wf + (size_t)min(kn0 / 32, rbmax) * KB * 64 + lane;
-
-    v16f acc;
-#pragma unroll
-    for (int e = 0; e < 16; e++) acc[e] = 0.0f;
-    const uint32_t fillv = ABIN ? 0x22222222u : 0u;
-
-    struct Frag {
-        v4i w, x;
-        bool in;
-    };
-    auto ld16 = [](v4i& dst, const uint4* src) { dst = *reinterpret_cast<const v4i*>(src); };   // loads as in k_conv_f4
-    __amdgpu_buffer_rsrc_t brs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(P4), 0, (int)p4_bytes, 0x00020000);
-    __amdgpu_buffer_rsrc_t brs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(Wf), 0, (int)wf_bytes, 0x00020000);
-    uint32_t wofs = 0u, xofs = 0u;
-    if constexpr (BUF) {
-        wofs = ((uint32_t)min(kn0 / 32, rbmax) * (uint32_t)KB * 64u + (uint32_t)lane) * 16u;
-        xofs = ((pb + (uint32_t)(ih0 * cg.W + iw0)) * 2u + (uint32_t)h) * 16u;
-    }
-    auto ldbuf = [&](v4i& dst, uint32_t voff, uint32_t soff, bool weights) {
-        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(weights ? brs_w : brs_x, (int)voff, (int)soff, 0);
-        dst = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
-    };
-    auto load = [&](int w, Frag& f) {   // w is wave-uniform
-        const int tap = (int)fastdiv((uint32_t)w, cg.dCP), ic = w - tap * cg.CP;
-        const int kh = (int)fastdiv((uint32_t)tap, cg.dKW), kw = tap - kh * cg.KW;
-        const int ih = ih0 + kh, iw = iw0 + kw;
-        if constexpr (BUF) {
-            ldbuf(f.w, wofs, (uint32_t)__builtin_amdgcn_readfirstlane(w) * 1024u, true);
-            const bool in = (unsigned)ih < (unsigned)cg.H && (unsigned)iw < (unsigned)cg.W;
-            const uint32_t tapoff = (uint32_t)__builtin_amdgcn_readfirstlane((ic * HWin + kh * cg.W + kw) * 32);
-            ldbuf(f.x, in ? xofs + tapoff : (ABIN ? 0u : 0xffffff00u), 0u, false);   // as in k_conv_f4
-            f.in = ABIN ? in : true;
-        } else {
-            ld16(f.w, wb + (size_t)w * 64);
-            f.in = (unsigned)ih < (unsigned)cg.H && (unsigned)iw < (unsigned)cg.W;
-            const size_t o = (size_t)(pb + (uint32_t)(ic * HWin + (f.in ? ih * cg.W + iw : 0))) * 2 + h;
-            ld16(f.x, P4 + o);
-        }
-    };
-    auto fence_loads = []() { __builtin_amdgcn_sched_barrier(0); };
-    auto compute = [&](const Frag& f) {
-        v8i x, wv;
-#pragma unroll
-        for (int i = 0; i < 4; i++) x[i] = ((BUF && !ABIN) || f.in) ? f.x[i] : (int)fillv;
-#pragma unroll
-        for (int i = 4; i < 8; i++) x[i] = 0;
-        wv = v8i{f.w[0], f.w[1], f.w[2], f.w[3], 0, 0, 0, 0};
-        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wv, x, acc, 4, 4, 0, 0, 0, 0);
-    };
-
-    // as in k_conv_f4: register sets rotate by name, loads past the last word re-read it and are not multiplied
-    const int K = cg.K;
-    Frag f[NB];
-    int w = ks;
-#pragma unroll
-    for (int j = 0; j < NB - 1; j++) load(min(w + S * j, K - 1), f[j]);
-    for (; w < K; w += S * NB) {
-#pragma unroll
-        for (int j = 0; j < NB; j++) {
-            load(min(w + S * (j + NB - 1), K - 1), f[(j + NB - 1) % NB]);
-            fence_loads();
-            if (j == 0 || w + S * j < K) compute(f[j]);
-        }
-    }
-
-    if (ks != 0) {
-        float4* dst = red + (size_t)((ks - 1) * 4) * 64 + lane;
-#pragma unroll
-        for (int e4 = 0; e4 < 4; e4++)
-            dst[e4 * 64] = make_float4(acc[4 * e4], acc[4 * e4 + 1], acc[4 * e4 + 2], acc[4 * e4 + 3]);
-    }
-    __syncthreads();
-    if (ks != 0) return;
-#pragma unroll
-    for (int v = 0; v < 3; v++) {
-        const float4* src = red + (size_t)(v * 4) * 64 + lane;
-#pragma unroll
-        for (int e4 = 0; e4 < 4; e4++) {
-            const float4 t = src[e4 * 64];
-            acc[4 * e4] += t.x;
-            acc[4 * e4 + 1] += t.y;
-            acc[4 * e4 + 2] += t.z;
-            acc[4 * e4 + 3] += t.w;
-        }
-    }
-
-    // accumulator e: kernel = kn0 + 8*(e/4) + 4*h + e%4, pixel = px0 + lr
-    const float fbias = (float)bias;
-    float r[16];
-#pragma unroll
-    for (int e = 0; e < 16; e++) r[e] = FORM0 ? acc[e] : acc[e] - fbias;   // only BNN has a bias
-    if constexpr (QMODE == 0) {
-        float* yq = Y + ((size_t)img * KN + kn0 + 4 * h) * OHW + pix;
-        if (q < M) {
-            if (kn0 + 32 <= KN) {   // uniform: whole block inside
-#pragma unroll
-                for (int e = 0; e < 16; e++) yq[(size_t)(8 * (e >> 2) + (e & 3)) * OHW] = prelu_ref<FORM0>(r[e], alpha);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const int p = kn0 + 8 * (e >> 2) + 4 * h + (e & 3);
-                    if (p < KN) yq[(size_t)(8 * (e >> 2) + (e & 3)) * OHW] = prelu_ref<FORM0>(r[e], alpha);
-                }
-            }
-        }
+        });
     } else {
-        const uint2 out = hand_over_block<FORM0, QMODE>(r, alpha, qthr, direct_quant<QMODE>(alpha, qthr), kn0, h, KN);
-        // this tile is half a 64-channel word: bytes 16 * (tile parity) of the pixel's 32
-        const size_t word = ((size_t)img * (gridDim.y >> 1) + (by >> 1)) * OHW + pix;
-        if (q < M)
-            *reinterpret_cast<uint2*>(static_cast<unsigned char*>(qo.p4) + word * 32 + 16 * (by & 1) + 8 * h) = out;
+        // Hand-over to an fp4 layer: a pixel's 64-channel word is 32 bytes, 16 per 32-kernel block
+        const uint32_t KT = TA == 2 ? gridDim.y : gridDim.y >> 1, kt = TA == 2 ? by : by >> 1;
+        auto out_word = [&](int b) {
+            return static_cast<unsigned char*>(qo.p4) + (((size_t)img[b] * KT + kt) * (uint32_t)OHW + pix[b]) * 32;
+        };
+        if constexpr (NBLK == 4 && S < 4) {   // the wavefront finishes both kernel blocks of a pixel block: lane half h stores block h
+#pragma unroll
+            for (int b = 0; b < TB; b++)
+                if (b % S == ks) {
+                    const uint2 d0 = hand_over_block<FORM0, QMODE>(acc[0][b], alpha, qo, kn0, h, KN);
+                    const uint2 d1 = hand_over_block<FORM0, QMODE>(acc[TA - 1][b], alpha, qo, kn0 + 32, h, KN);
+                    const uint4 out = exchange_blocks(d0, d1);
+                    if (px0 + 32 * b + lr < M) *reinterpret_cast<uint4*>(out_word(b) + 16 * h) = out;
+                }
+        } else {   // one block: lane half h stores 8 bytes
+            for_blocks([&](auto blk_tag) {
+                constexpr int BLK = decltype(blk_tag)::value, a = BLK / TB, b = BLK % TB;
+                if (BLK % S == ks) {
+                    const uint2 out = exchange_halves(hand_over_block<FORM0, QMODE>(acc[a][b], alpha, qo, kn0 + 32 * a, h, KN));
+                    const int part = TA == 2 ? a : (int)(by & 1u);
+                    if (px0 + 32 * b + lr < M) *reinterpret_cast<uint2*>(out_word(b) + 16 * part + 8 * h) = out;
+                }
+            });
+        }
     }
 }
 
@@ -1472,34 +1356,31 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
     // operand sizes: the buffer-load variants announce them in their descriptors
     const int64_t p4_bytes = (int64_t)N * cg.CP * cg.H * cg.W * 32, wf_bytes = (int64_t)((KN + 31) / 32) * KB * 1024;
     static const bool no_buf = getenv("FTNN_CONV_NO_BUFFER_LOADS") != nullptr;   // tuning aid
-    const bool buf = !no_buf && p4_bytes <= 0xf0000000LL && wf_bytes <= 0xf0000000LL;
+    const int64_t y_bytes = M * KN * 4;
+    const bool buf = !no_buf && p4_bytes <= 0xf0000000LL && wf_bytes <= 0xf0000000LL && (qo.mode != 0 || y_bytes <= 0xf0000000LL);
+    auto clip = [](int64_t v) { return (uint32_t)std::min<int64_t>(v, 0xffffffffLL); };
     const uint64_t wgs = (uint64_t)grid.x * grid.y;
     if (wgs > 0xffffffffull) return hipErrorInvalidValue;   // (no such result fits in memory)
     const XcdOrder xo = make_xcd_order(grid.x, grid.y);
-    auto launch64 = [&](auto variant) -> hipError_t {
-        constexpr auto kern = decltype(variant)::value;
-        hipLaunchKernelGGL(kern, grid, dim3(64 * wpb), 0, st, P4, Wf, d_y, (int)M, KN, OHW, KB, bias, alpha, dOHW, cg, qo,
-                           (uint32_t)std::min<int64_t>(p4_bytes, 0xffffffffLL), (uint32_t)std::min<int64_t>(wf_bytes, 0xffffffffLL), xo);
-        return hipGetLastError();
-    };
-    auto by_buf = [&](auto abin, auto form0, auto qmode, auto sp) -> hipError_t {
+    // kernel variant: activation kind and PReLU form follow the type, then hand-over mode, tile and split, loads
+    auto launch = [&](auto abin, auto form0, auto qmode, auto blocks, auto sp) -> hipError_t {
         constexpr bool A = decltype(abin)::value, F = decltype(form0)::value;
-        constexpr int Q = decltype(qmode)::value, SP = decltype(sp)::value;
-        if (buf) return launch64(std::integral_constant<decltype(&k_conv_f4<A, F, Q, SP, 3, true>), &k_conv_f4<A, F, Q, SP, 3, true>>{});
-        return launch64(std::integral_constant<decltype(&k_conv_f4<A, F, Q, SP, 3, false>), &k_conv_f4<A, F, Q, SP, 3, false>>{});
+        constexpr int Q = decltype(qmode)::value, T = decltype(blocks)::value, SP = decltype(sp)::value;
+        auto go = [&](auto kern) -> hipError_t {
+            hipLaunchKernelGGL(kern, grid, dim3(64 * wpb), 0, st, P4, Wf, d_y, (int)M, KN, OHW, KB, bias, alpha, dOHW, cg, qo,
+                               clip(p4_bytes), clip(wf_bytes), clip(y_bytes), xo);
+            return hipGetLastError();
+        };
+        return buf ? go(k_conv_f4<A, F, Q, T, T, SP, true>) : go(k_conv_f4<A, F, Q, T, T, SP, false>);
     };
-    // kernel variant: activation kind and PReLU form follow the type, then hand-over mode and split
     auto by_split = [&](auto abin, auto form0, auto qmode) -> hipError_t {
-        constexpr bool A = decltype(abin)::value, F = decltype(form0)::value;
-        constexpr int Q = decltype(qmode)::value;
-        if (small) {
-            if (buf) return launch64(std::integral_constant<decltype(&k_conv_f4_small<A, F, Q, true>), &k_conv_f4_small<A, F, Q, true>>{});
-            return launch64(std::integral_constant<decltype(&k_conv_f4_small<A, F, Q, false>), &k_conv_f4_small<A, F, Q, false>>{});
-        }
-        // three register sets: deeper prefetch measured no faster at any layer size
-        if (split == 1) return by_buf(abin, form0, qmode, std::integral_constant<int, 1>{});
-        if (split == 2) return by_buf(abin, form0, qmode, std::integral_constant<int, 2>{});
-        if (split == 4) return by_buf(abin, form0, qmode, std::integral_constant<int, 4>{});
+        typedef std::integral_constant<int, 1> one;
+        typedef std::integral_constant<int, 2> two;
+        typedef std::integral_constant<int, 4> four;
+        if (small) return launch(abin, form0, qmode, one{}, four{});
+        if (split == 1) return launch(abin, form0, qmode, two{}, one{});
+        if (split == 2) return launch(abin, form0, qmode, two{}, two{});
+        if (split == 4) return launch(abin, form0, qmode, two{}, four{});
         return hipErrorInvalidValue;
     };
     auto by_mode = [&](auto abin, auto form0) -> hipError_t {

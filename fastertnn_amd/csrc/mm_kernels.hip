@@ -391,7 +391,7 @@ __global__ __launch_bounds__(KS ? 64 * KS : 256) void k_mm(const uint32_t* __res
                 // hand-over to an fp4 layer: this lane's TN kernels are TN consecutive nibbles of one pixel
                 const uint32_t img = fastdiv((uint32_t)i, dOHW);
                 const uint32_t pix = (uint32_t)i - img * (uint32_t)OHW;
-                const float t = qo.thr[img];
+                const float t = qo.t;
                 uint32_t dw = 0u;
                 const bool tern = qo.mode == 1;
                 if (col0 + TN <= KN) {   // uniform: all of this wavefront's columns are real kernels

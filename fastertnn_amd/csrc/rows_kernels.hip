@@ -34,7 +34,6 @@ namespace ftnn {
 namespace {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
 // fn(0), ..., fn(N - 1) with compile-time indices

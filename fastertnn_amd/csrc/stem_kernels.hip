@@ -25,7 +25,6 @@ namespace ftnn {
 namespace {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kTile = 16;   // output pixels per workgroup: kTile wide, 4 rows per wavefront (16 rows with four wavefronts)
 
@@ -156,13 +155,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         ow[b] = ow0 + col;
         po[b] = (uint32_t)((row * g.H_stride) * g.PW + col * g.W_stride) * 4u;
     }
+    const float init = acc_init<QMODE>(qo, FORM0 ? 0.0f : (float)bias);   // only BNN has a bias
     v16f acc[2][2];
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
         for (int b = 0; b < 2; b++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[a][b][e] = 0.0f;
+            for (int e = 0; e < 16; e++) acc[a][b][e] = init;
 
     const unsigned char* patch_b = reinterpret_cast<const unsigned char*>(patch);
     const uint32_t* toff_h = toff + h * J1;   // the upper half starts at tap J1 of each word
@@ -209,42 +209,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
 
     // ---- epilogue: accumulator e of block (a, b): kernel = 32 a + 8 (e / 4) + 4 h + e % 4, pixel = lane's ----
     const int OHW = g.OH * g.OW;
-    const float fbias = (float)bias;
-    float qthr = 0.0f;
-    if constexpr (QMODE != 0) qthr = qo.thr[n];
-    const DirectQuant dq = direct_quant<QMODE>(alpha, qthr);   // whether the hand-over may take its compare-free form
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int b = 0; b < 2; b++) {
+        const bool live = oh[b] < g.OH && ow[b] < g.OW;
+        const int pix = live ? oh[b] * g.OW + ow[b] : 0;
+        if constexpr (QMODE == 0) {
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const bool live = oh[b] < g.OH && ow[b] < g.OW;
-            const int pix = live ? oh[b] * g.OW + ow[b] : 0;
-            float r[16];
-#pragma unroll
-            for (int e = 0; e < 16; e++) r[e] = FORM0 ? acc[a][b][e] : acc[a][b][e] - fbias;   // only BNN has a bias
-            if constexpr (QMODE == 0) {
+            for (int a = 0; a < 2; a++) {
                 float* yq = Y + ((size_t)n * KN + kn0 + 32 * a + 4 * h) * OHW + pix;
                 if (live) {
                     if (kn0 + 32 * a + 32 <= KN) {   // uniform: whole block inside
 #pragma unroll
                         for (int e = 0; e < 16; e++)
-                            yq[(size_t)(8 * (e >> 2) + (e & 3)) * OHW] = prelu_ref<FORM0>(r[e], alpha);
+                            yq[(size_t)(8 * (e >> 2) + (e & 3)) * OHW] = prelu_ref<FORM0>(acc[a][b][e], alpha);
                     } else {
 #pragma unroll
                         for (int e = 0; e < 16; e++) {
                             const int p = kn0 + 32 * a + 8 * (e >> 2) + 4 * h + (e & 3);
-                            if (p < KN) yq[(size_t)(8 * (e >> 2) + (e & 3)) * OHW] = prelu_ref<FORM0>(r[e], alpha);
+                            if (p < KN) yq[(size_t)(8 * (e >> 2) + (e & 3)) * OHW] = prelu_ref<FORM0>(acc[a][b][e], alpha);
                         }
                     }
                 }
-            } else {
-                // as in k_conv_f4: lane half h ends up with bytes 16 a + 8 h .. + 8 of the pixel's 64-channel word
-                const uint2 out = hand_over_block<FORM0, QMODE>(r, alpha, qthr, dq, kn0 + 32 * a, h, KN);
-                const size_t word = ((size_t)n * g.kn_tiles + kt) * OHW + pix;
-                if (live)
-                    *reinterpret_cast<uint2*>(static_cast<unsigned char*>(qo.p4) + word * 32 + 16 * a + 8 * h) = out;
             }
+        } else {
+            // as in k_conv_f4: lane half h ends up with bytes 16 h .. 16 h + 15 of the pixel's 64-channel word
+            const uint2 d0 = hand_over_block<FORM0, QMODE>(acc[0][b], alpha, qo, kn0, h, KN);
+            const uint2 d1 = hand_over_block<FORM0, QMODE>(acc[1][b], alpha, qo, kn0 + 32, h, KN);
+            const size_t word = ((size_t)n * g.kn_tiles + kt) * OHW + pix;
+            const uint4 out = exchange_blocks(d0, d1);
+            if (live) *reinterpret_cast<uint4*>(static_cast<unsigned char*>(qo.p4) + word * 32 + 16 * h) = out;
         }
+    }
 }
 
 }  // namespace
