@@ -766,6 +766,29 @@ static int64_t gemm_route_plane_bytes(int N, int C, int H, int W) {
 }
 static int64_t gemm_route_row_bytes(int64_t M, int Kw) { return (M * Kw * 16 + 255) / 256 * 256; }
 
+// Fully connected layers (1 x 1 kernels on one pixel per image) run as a product of packed rows (k_rows): the fragments of
+// the fp4 layer kernels take twice the bytes, and a layer over few images does little but read its weights; over many images
+// the layer kernels scatter their results, a column of them per image.  Whole call, weights prepared and read from beyond the
+// L2, fragments / rows on MI355X: 8 images of 16384 -> 16384 31.5 / 15.4 us (64 MiB of weights: 5.4 TB/s beside the quantiser's
+// launch), 64 57.9 / 21.9, 8 of 4096 -> 4096 8.0 / 6.1, 8 of 512 -> 1000 5.6 / 5.0, 1024 of 4096 -> 4096 120 / 23, 4096 of
+// 1000 -> 16000 1854 / 145: ahead from 1 to 4096 images on every size tried.  Up to 64 channels the rows, four words at least,
+// would be larger than the layer's operand region, and a row is mostly padding: those stay with the layer kernels.
+static bool fc_weights(int C, int KH, int KW) { return C > 64 && KH == 1 && KW == 1; }
+static bool fc_from_rows(int C, int H, int W, int KH, int KW, int H_pad, int W_pad) {
+    return fc_weights(C, KH, KW) && H == 1 && W == 1 && H_pad == 0 && W_pad == 0;
+}
+
+// quantise + product; d_qw: the weights' packed rows, d_scratch: N rows of at most 16 bytes per word (within the operand region:
+// 32 bytes per channel word, and round4(words) <= 2 words from two words on)
+static int conv_fc_rows(int type, const float* d_x, const float* d_thr, const int64_t* d_qw, int N, int C, int KN,
+                        float prelu_alpha, void* d_scratch, float* d_y, hipStream_t st) {
+    int64_t* d_a = static_cast<int64_t*>(d_scratch);
+    hipError_t e = launch_quantize_rows(type == kTNN || type == kTBN, d_x, d_thr, N, C, d_a, st);
+    if (e != hipSuccess) return hip_fail(e, "quantise launch");
+    e = launch_mm_rows(type, d_a, d_qw, N, 1, KN, round4(cpack_of(C)), C, prelu_alpha, d_y, st);
+    return e == hipSuccess ? FTNN_OK : hip_fail(e, "packed-row GEMM launch");
+}
+
 // operand region of the fp4 layer for this shape, whichever form it takes
 int64_t conv_f4_operand_bytes(int N, int C, int H, int W, int KH, int KW, int OH, int OW, int KN, int W_stride) {
     if (dense_f4_applies(C, KH, KW)) return conv_f4_dense_bytes(N, C, H, W, KH, KW, OH, OW);
@@ -1166,6 +1189,8 @@ int ftnn_conv_engine(int engine, int type, const float* d_x, const float* d_thr,
         if (64LL * Kw >= (1LL << 24))
             return fail(FTNN_EINVAL, "K too long for exact fp32 accumulation; use the vector-ALU engine");
         if (!fits_f4) return fail(FTNN_EINVAL, "more than 2^31-1 input pixel words: use the vector-ALU engine");
+        if (fc_from_rows(C, H, W, KH, KW, H_pad, W_pad))
+            return conv_fc_rows(type, d_x, d_thr, d_qw, N, C, KN, prelu_alpha, d_scratch, d_y, (hipStream_t)stream);
         char* d_wf = static_cast<char*>(d_scratch) + conv_f4_operand_bytes(N, C, H, W, KH, KW, OH, OW, KN, W_stride);
         const int64_t* rows = d_qw;
         hipError_t e;
@@ -1196,7 +1221,9 @@ static int64_t prepared_bytes(int type, int C, int KN, int KH, int KW, int64_t* 
         const int64_t frag = (mfma_fragment_bytes(true, KN, conv_f4_weight_words(C, KH, KW)) + 255) / 256 * 256;
         if (tmp_off) *tmp_off = frag;
         // the dense path expands the re-packed rows, which need a place of their own
-        return frag + (dense_f4_applies(C, KH, KW) ? (int64_t)KN * round4(Kd) * (wt ? 16 : 8) : 0);
+        if (dense_f4_applies(C, KH, KW)) return frag + (int64_t)KN * round4(Kd) * (wt ? 16 : 8);
+        // the packed rows as they are, behind the fragments: operand of conv_fc_rows
+        return frag + (fc_weights(C, KH, KW) ? (int64_t)KN * round4(cpack_of(C)) * (wt ? 16 : 8) : 0);
     }
     return (int64_t)KN * (dense ? round4(Kd) : round4(cpack_of(C) * KH * KW)) * (wt ? 16 : 8);
 }
@@ -1231,7 +1258,8 @@ int ftnn_conv_prepare_weights(int type, const int64_t* d_qw, int C, int KN, int 
             if (e != hipSuccess) return hip_fail(e, "dense weights launch");
             rows = d_wd;
         }
-        e = launch_mfma_expand(true, wt, rows, KN, conv_f4_weight_words(C, KH, KW), d_prepared, st);
+        int64_t* kept = fc_weights(C, KH, KW) ? reinterpret_cast<int64_t*>(static_cast<char*>(d_prepared) + tmp_off) : nullptr;
+        e = launch_mfma_expand(true, wt, rows, KN, conv_f4_weight_words(C, KH, KW), d_prepared, st, kept);
         return e == hipSuccess ? FTNN_OK : hip_fail(e, "weight expansion launch");
     }
     if (dense) {
@@ -1258,6 +1286,13 @@ int ftnn_conv_prepared(int type, const float* d_x, const float* d_thr, const voi
         if ((int64_t)N * H * W * cpack_of(C) > 0x7fffffffLL ||
             (int64_t)N * OH * OW * conv_f4_weight_words(C, KH, KW) > 0x7fffffffLL)
             return fail(FTNN_EINVAL, "more than 2^31-1 input pixel words");
+        if (fc_from_rows(C, H, W, KH, KW, H_pad, W_pad)) {
+            int64_t rows_off;
+            prepared_bytes(type, C, KN, KH, KW, &rows_off);
+            const char* rows = static_cast<const char*>(d_prepared) + rows_off;
+            return conv_fc_rows(type, d_x, d_thr, reinterpret_cast<const int64_t*>(rows), N, C, KN, prelu_alpha, d_scratch, d_y,
+                                (hipStream_t)stream);
+        }
         return conv_f4_expanded(type, d_x, d_thr, d_prepared, N, C, H, W, KN, KH, KW, H_pad, W_pad, H_stride,
                                 W_stride, prelu_alpha, d_scratch, d_y, (hipStream_t)stream, QuantOut());
     }

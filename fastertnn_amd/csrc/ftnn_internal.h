@@ -208,6 +208,8 @@ hipError_t launch_quantize(bool ternary, const float* d_x, const float* d_thr, i
 // quantise only, into fp4 nibbles: fp32 NCHW -> P4[n][C_pack][pixel][32 bytes] (operand of launch_conv_f4)
 hipError_t launch_quantize_f4(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
                               void* d_p4, hipStream_t st);
+// quantise only, into Packing-2 rows: fp32 [N][C] -> N rows (activations of a fully connected layer as launch_mm_rows reads them)
+hipError_t launch_quantize_rows(bool ternary, const float* d_x, const float* d_thr, int N, int C, int64_t* d_out, hipStream_t st);
 
 // dense re-packing of both operands for layers with C <= 32 (several taps per 64-lane word)
 bool dense_applies(int C, int KH, int KW, int* T_out, int* Kd_out);
@@ -234,7 +236,7 @@ hipError_t launch_dense_rows_f4(bool ternary, const float* d_x, const float* d_t
 // ---- mfma_kernels.hip: matrix-core formulation (int8 or fp4 operands expanded into d_scratch) ----
 int64_t mfma_fragment_bytes(bool f4, int64_t rows, int Kw);
 hipError_t launch_mfma_expand(bool f4, bool ternary, const int64_t* d_rows, int rows, int Kw, void* d_out,
-                              hipStream_t st);
+                              hipStream_t st, int64_t* d_kept = nullptr /* also copies the rows there */);
 hipError_t launch_mfma_gemm(bool f4, int type, const void* d_af, const void* d_bf, int64_t M, int OHW, int KN,
                             int Kw, int K_unpack, float alpha, float* d_y, hipStream_t st);
 // the fp4 GEMM's own operand form, two bits per lane ("packed4"): what ftnn_expand_rows / ftnn_mm_expanded /

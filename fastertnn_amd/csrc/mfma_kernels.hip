@@ -59,7 +59,7 @@ struct Tile {
 // rows, 8 dwords for binary rows.  Rows past `rows` expand to zeros.
 template <bool F4, bool TERN>
 __device__ __forceinline__ void expand_block(const uint32_t* __restrict__ P, int rows, int G, uint4* __restrict__ out, int rb,
-                                             int gy, uint32_t* stage) {
+                                             int gy, uint32_t* stage, uint32_t* __restrict__ kept = nullptr) {
     // A workgroup expands kGPB adjacent groups of its 32 rows: 256 contiguous bytes of each ternary row (128 of a
     // binary one).  They are fetched row-wise, 16 bytes per thread with neighbouring threads on neighbouring bytes,
     // and turned through LDS into the (row, dword) order the expansion works in: fetched in that order directly,
@@ -78,6 +78,7 @@ __device__ __forceinline__ void expand_block(const uint32_t* __restrict__ P, int
             const int srow = min(rb * 32 + rr, rows - 1);
             uint4 v = make_uint4(0u, 0u, 0u, 0u);
             if (pc < gmax) v = *reinterpret_cast<const uint4*>(P + ((size_t)srow * G + g0) * DPG + pc * 4);
+            if (kept && pc < gmax && rb * 32 + rr < rows) *reinterpret_cast<uint4*>(kept + ((size_t)srow * G + g0) * DPG + pc * 4) = v;
             uint32_t* d = stage + rr * RS + pc * 4;
             d[0] = v.x;
             d[1] = v.y;
@@ -136,10 +137,12 @@ __device__ __forceinline__ void expand_block(const uint32_t* __restrict__ P, int
     }
 }
 
+// kept: where the packed rows themselves are copied to on the way (a copy of its own costs the caller 20 us), or null
 template <bool F4, bool TERN>
-__global__ __launch_bounds__(256) void k_expand(const uint32_t* __restrict__ P, int rows, int G, uint4* __restrict__ out) {
+__global__ __launch_bounds__(256) void k_expand(const uint32_t* __restrict__ P, int rows, int G, uint4* __restrict__ out,
+                                                uint32_t* __restrict__ kept) {
     __shared__ uint32_t stage[32 * 65];
-    expand_block<F4, TERN>(P, rows, G, out, blockIdx.x, blockIdx.y, stage);
+    expand_block<F4, TERN>(P, rows, G, out, blockIdx.x, blockIdx.y, stage, kept);
 }
 
 // both operands of a GEMM in one launch (the same K): the first ceil(rows_a / 32) workgroup columns expand A, the others B
@@ -1123,11 +1126,11 @@ hipError_t launch_gemm(const uint4* Pf, const uint4* Qf, float* Y, int M, int KN
 }
 
 template <bool F4>
-hipError_t launch_expand(bool tern, const uint32_t* rows_ptr, int rows, int G, uint4* out, hipStream_t st) {
+hipError_t launch_expand(bool tern, const uint32_t* rows_ptr, int rows, int G, uint4* out, uint32_t* kept, hipStream_t st) {
     dim3 grid((rows + 31) / 32, (G + 3) / 4);   // 4 groups per workgroup (kGPB in the kernel)
     if (grid.y > 65535) return hipErrorInvalidValue;
-    if (tern) hipLaunchKernelGGL((k_expand<F4, true>), grid, dim3(256), 0, st, rows_ptr, rows, G, out);
-    else hipLaunchKernelGGL((k_expand<F4, false>), grid, dim3(256), 0, st, rows_ptr, rows, G, out);
+    if (tern) hipLaunchKernelGGL((k_expand<F4, true>), grid, dim3(256), 0, st, rows_ptr, rows, G, out, kept);
+    else hipLaunchKernelGGL((k_expand<F4, false>), grid, dim3(256), 0, st, rows_ptr, rows, G, out, kept);
     return hipGetLastError();
 }
 
@@ -1169,11 +1172,12 @@ int64_t mfma_fragment_bytes(bool f4, int64_t rows, int Kw) {
 }
 
 hipError_t launch_mfma_expand(bool f4, bool ternary, const int64_t* d_rows, int rows, int Kw, void* d_out,
-                              hipStream_t st) {
+                              hipStream_t st, int64_t* d_kept) {
     const uint32_t* R = reinterpret_cast<const uint32_t*>(d_rows);
     uint4* out = static_cast<uint4*>(d_out);
-    return f4 ? launch_expand<true>(ternary, R, rows, Kw / 4, out, st)
-              : launch_expand<false>(ternary, R, rows, Kw / 4, out, st);
+    uint32_t* kept = reinterpret_cast<uint32_t*>(d_kept);
+    return f4 ? launch_expand<true>(ternary, R, rows, Kw / 4, out, kept, st)
+              : launch_expand<false>(ternary, R, rows, Kw / 4, out, kept, st);
 }
 
 hipError_t launch_mfma_gemm(bool f4, int type, const void* d_af, const void* d_bf, int64_t M, int OHW, int KN,

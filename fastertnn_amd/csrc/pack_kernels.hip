@@ -645,6 +645,18 @@ hipError_t launch_quantize_f4(bool ternary, const float* d_x, const float* d_thr
     return hipGetLastError();
 }
 
+// fp32 rows -> Packing-2 rows of round4(ceil(C / 64)) words, the pad words filled as the im2row operand's: a row per image of a
+// fully connected layer, in one launch
+hipError_t launch_quantize_rows(bool ternary, const float* d_x, const float* d_thr, int N, int C, int64_t* d_out, hipStream_t st) {
+    const int Kw = round4(cpack_of(C));
+    const dim3 grid((unsigned)N, (unsigned)(Kw / 4));
+    if (grid.y > 65535) return hipErrorInvalidValue;
+    unsigned long long* out = reinterpret_cast<unsigned long long*>(d_out);
+    if (ternary) hipLaunchKernelGGL((k_quantize_ballot<0, true>), grid, dim3(256), 0, st, d_x, d_thr, C, Kw, out);
+    else hipLaunchKernelGGL((k_quantize_ballot<1, false>), grid, dim3(256), 0, st, d_x, d_thr, C, Kw, out);
+    return hipGetLastError();
+}
+
 // bytes of T4 (k_quantize_f4 with TILED) for this input and column stride
 int64_t quantize_f4_tiled_bytes(int N, int C, int H, int W, int W_stride) {
     return (int64_t)N * cpack_of(C) * 2 * H * W_stride * ((W + W_stride - 1) / W_stride) * 16 + 16;   // + the fill piece
