@@ -1348,7 +1348,7 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
     if (tune) split = tune;
     while (split > 1 && cg.K < split) split /= 2;   // no wavefront without K words of its own, forced or not
     const int wpb = 4, tpb = wpb / split;   // wavefronts and pixel tiles per workgroup (see the kernel)
-    // few 64 x 64 tiles: tiles of 32 x 32, four times the workgroups (k_conv_f4_small)
+    // few 64 x 64 tiles: tiles of 32 x 32, four times the workgroups
     static const int small_below = getenv("FTNN_CONV_SMALL_BELOW") ? atoi(getenv("FTNN_CONV_SMALL_BELOW")) : 150;
     const bool small = tiles < small_below;
     dim3 grid((unsigned)(((M + 63) / 64 + tpb - 1) / tpb), (unsigned)((KN + 63) / 64));
