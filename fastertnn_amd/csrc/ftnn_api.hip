@@ -1147,7 +1147,7 @@ int ftnn_mm_engine(int engine, int type, const int64_t* d_a, const int64_t* d_b,
         // 4.8, 100000 x 10 x 512 7.8 against 9.8) and needs no scratch; it also takes the larger ones that come without
         // scratch (4096 x 4096 x 32768 0.22 ms against 1.8).
         const bool scratch_ok = d_scratch && scratch_bytes >= ftnn_mm_scratch_bytes(engine, type, N, OH, OW, KN, K);
-        if (mm_rows_within_limits(Kw) && (engine == FTNN_ENGINE_VALU || mm_from_rows(M, KN) || !scratch_ok)) {
+        if (mm_rows_within_limits(M, KN, Kw) && (engine == FTNN_ENGINE_VALU || mm_from_rows(M, KN) || !scratch_ok)) {
             const hipError_t e = launch_mm_rows(type, d_a, d_b, M, OH * OW, KN, Kw, K_unpack, prelu_alpha, d_y, (hipStream_t)stream);
             return e == hipSuccess ? FTNN_OK : hip_fail(e, "mm launch");
         }

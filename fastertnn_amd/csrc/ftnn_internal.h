@@ -254,7 +254,8 @@ hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* 
                           hipStream_t st);
 
 // ---- rows_kernels.hip: the fp4 matrix-core product of packed rows as they are, one launch, no scratch ----
-bool mm_rows_within_limits(int Kw);   // fp32 sums of +-1 products stay exact
+// fp32 sums of +-1 products stay exact, and the grid holds the product
+bool mm_rows_within_limits(int64_t M, int KN, int Kw);
 hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
                           float alpha, float* d_y, hipStream_t st);
 

@@ -353,6 +353,11 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
     }
 }
 
+// A grid dimension holds fewer than 2^32 threads: tiles, rounded up to whole eighths, times the 256 of a workgroup.  It also
+// keeps row numbers below 2^31 in the last tile.
+constexpr int64_t kMaxRowsTiles = (1 << 24) - 8;
+int64_t rows_tiles(int64_t prow, int64_t qrow, int edge) { return ((prow + edge - 1) / edge) * ((qrow + edge - 1) / edge); }
+
 template <bool TP, bool TQ, int WT>
 hipError_t launch_rows_tile(const char* P, const char* Q, int64_t prow, int64_t qrow, int G, const RowsOut& ro, hipStream_t st) {
     constexpr int KS = 4;   // 8 wavefronts measured no faster on any tile
@@ -370,7 +375,7 @@ hipError_t launch_rows_tile(const char* P, const char* Q, int64_t prow, int64_t 
     }();
     if (configured != hipSuccess) return configured;
     const int64_t px = (prow + 32 * WT - 1) / (32 * WT), qy = (qrow + 32 * WT - 1) / (32 * WT);
-    if (px * qy > 0x3fffffffLL) return hipErrorInvalidValue;
+    if (px * qy > kMaxRowsTiles) return hipErrorInvalidValue;
     RowsOrder od;
     od.tiles = (uint32_t)(px * qy);
     od.per_xcd = (od.tiles + 7) / 8;
@@ -384,9 +389,12 @@ hipError_t launch_rows_tile(const char* P, const char* Q, int64_t prow, int64_t 
 // Wavefront tile of a product: blocks of 32 x 32 per side.  Small tiles fill the chip with little work and pay less for the
 // meeting of the partial tiles, large ones spend fewer instructions and bytes per multiply.  The estimates (us) are
 // fits to sweeps from 32 x 32 x 256 to 4096 x 4096 x 32768 on MI355X (n rounds of 256 tiles, w words per wavefront); where
-// two tiles are within 15 % of each other either may be picked.
+// two tiles are within 15 % of each other either may be picked.  A tile too small for the grid counts as endless.
 int rows_tile_of(int64_t prow, int64_t qrow, int Kw) {
-    auto rounds = [&](int edge) { return (double)((((prow + edge - 1) / edge) * ((qrow + edge - 1) / edge) + 255) / 256); };
+    auto rounds = [&](int edge) {
+        const int64_t n = rows_tiles(prow, qrow, edge);
+        return n > kMaxRowsTiles ? 1e30 : (double)((n + 255) / 256);
+    };
     const double w = Kw / 4.0;
     const double n1 = rounds(32), n2 = rounds(64), n3 = rounds(96), n4 = rounds(128);
     const double t1 = 2.65 + 0.42 * (n1 - 1) + w * (0.06 + 0.039 * (n1 - 1));
@@ -409,7 +417,9 @@ hipError_t launch_rows_types(const char* P, const char* Q, int64_t prow, int64_t
 
 }  // namespace
 
-bool mm_rows_within_limits(int Kw) { return 64LL * Kw < (1LL << 24); }
+bool mm_rows_within_limits(int64_t M, int KN, int Kw) {
+    return 64LL * Kw < (1LL << 24) && rows_tiles(M, KN, 128) <= kMaxRowsTiles;
+}
 
 hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
                           float alpha, float* d_y, hipStream_t st) {

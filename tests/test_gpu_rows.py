@@ -4,7 +4,7 @@ of words (fewer groups than wavefronts) to K tails, bit for bit against the orac
 import numpy as np
 import pytest
 
-from fastertnn_amd import TNN, TYPE_NAMES, act_is_ternary, weight_is_ternary
+from fastertnn_amd import BNN, TNN, TYPE_NAMES, act_is_ternary, weight_is_ternary
 from tests.cases import ALL_TYPES
 
 pytestmark = pytest.mark.gpu
@@ -70,3 +70,17 @@ def test_large_product_without_scratch(hip, oracle):
     rc = hip._L.ftnn_mm_engine(hip.ENGINE_AUTO, TNN, a_d.data_ptr(), b_d.data_ptr(), m, 1, 1, n, kw, 0, 0.5, y.data_ptr(), None, 0,
                                hip._stream())
     assert rc == 0 and y.cpu().numpy().tobytes() == want.tobytes()
+
+
+def test_more_rows_than_the_smallest_tile_has_workgroups_for(hip):
+    """one column under 2^29 + 33 rows: 2^24 + 2 tiles of 32 x 32 would be 2^32 threads and more, which no launch takes; the
+    next larger tile does it, against the vector ALU's integers"""
+    import torch
+    m, kw = (1 << 29) + 33, 4
+    print("case many rows", m, kw, flush=True)
+    torch.manual_seed(3)
+    a_d = torch.randint(-2 ** 62, 2 ** 62, (m * kw,), dtype=torch.int64, device="cuda")
+    b_d = torch.randint(-2 ** 62, 2 ** 62, (kw,), dtype=torch.int64, device="cuda")
+    want = hip.mm_engine(hip.ENGINE_VALU, BNN, a_d, b_d, m, 1, 1, 1, kw, 0.5, 64 * kw)
+    got = hip.mm_engine(hip.ENGINE_AUTO, BNN, a_d, b_d, m, 1, 1, 1, kw, 0.5, 64 * kw)
+    assert torch.equal(got, want)
