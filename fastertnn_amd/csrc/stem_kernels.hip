@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, lr = lane & 31;
     uint32_t img, bi;   // image, tile within it (kernel tile, pixel tile)
-    g.xo.tile(blockIdx.x, img, bi);
+    g.xo.tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), img, bi);
     const uint32_t kt = fastdiv(bi, g.dTiles), bx = bi - kt * g.dTiles.d;
     const int n = (int)img, kn0 = (int)kt * 64;
     const int ty = (int)fastdiv(bx, g.dTX), tx = (int)bx - ty * g.tiles_x;
@@ -291,7 +291,7 @@ hipError_t launch_stem_f4(int type, const float* d_x, const float* d_thr, const 
     g.kn_tiles = (uint32_t)kn_tiles;
     g.dTiles = make_fastdiv((uint32_t)tiles);
     g.xo = make_xcd_order((uint64_t)N, (uint32_t)(tiles * kn_tiles));
-    const dim3 grid((unsigned)(tiles * kn_tiles * N));
+    const dim3 grid((unsigned)tiles, (unsigned)kn_tiles, (unsigned)N);   // (in one dimension 2^32 threads would bound it)
     const uint4* Wf = static_cast<const uint4*>(d_wf);
     const int KB = round4(Kd);
     // BNN: every lane of the Kd words that is not a real (tap, channel) is +1 in both operands
