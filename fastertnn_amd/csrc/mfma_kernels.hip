@@ -1007,7 +1007,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
     // accumulator e of block (a, b): kernel = kn0 + 32 a + 8 (e / 4) + 4 h + e % 4, pixel = px0 + 32 b + lr
     if constexpr (QMODE == 0) {
         const __amdgpu_buffer_rsrc_t brs_y = __builtin_amdgcn_make_buffer_rsrc(Y, 0, (int)y_bytes, 0x00020000);
-        const bool as_max = alpha >= 0.0f && alpha <= 1.0f;   // PReLU is then max(r, r * alpha), bit for bit
+        // slopes from +0 to 1: PReLU is then max(r, r * alpha), bit for bit (with -0 a zero TNN sum becomes -0, which no maximum gives)
+        const bool as_max = __float_as_uint(alpha) <= __float_as_uint(1.0f);
         for_blocks([&](auto blk_tag) {
             constexpr int BLK = decltype(blk_tag)::value, a = BLK / TB, b = BLK % TB;
             if (BLK % S == ks) {
