@@ -806,11 +806,13 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
 // BUF: fragments arrive through buffer loads.  Their offsets are 32-bit, the place of a word within the operand is a
 // scalar offset, and for ternary activations an offset beyond the buffer returns zeros, which is what a
 // tap outside the image must contribute: no select on the loaded data (binary activations pad with +1 and keep the select).
-// Needs both operands and an fp32 result below 4 GiB (p4_bytes, wf_bytes, y_bytes: the sizes the descriptors announce).
+// Needs both operands below 4 GiB (p4_bytes, wf_bytes: the sizes the descriptors announce).  fp32 results leave through buffer
+// stores too, relative to the tile's first image and kernel: y_span bounds what a tile reaches from there, whatever the size
+// of the result.
 template <bool ABIN, bool FORM0, int QMODE, int TA, int TB, int S, bool BUF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && QMODE != 0) ? 3 : 1, 8))) void k_conv_f4(
     const uint4* __restrict__ P4, const uint4* __restrict__ Wf, float* __restrict__ Y, int M, int KN, int OHW, int KB, int bias,
-    float alpha, FastDiv dOHW, ConvGeom cg, QuantOut qo, uint32_t p4_bytes, uint32_t wf_bytes, uint32_t y_bytes, XcdOrder xo, uint32_t grid_x, uint32_t grid_y) {
+    float alpha, FastDiv dOHW, ConvGeom cg, QuantOut qo, uint32_t p4_bytes, uint32_t wf_bytes, uint32_t y_span, XcdOrder xo, uint32_t grid_x, uint32_t grid_y) {
     constexpr int WPB = 4;                // wavefronts per workgroup (single-wavefront workgroups for S = 1
                                           // measured slower: neighbours no longer share weight fragments in L1)
     constexpr int NB = 3;                 // register sets of fragments: NB - 1 words of loads in flight; more measured no faster
@@ -1006,7 +1008,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
     }
     // accumulator e of block (a, b): kernel = kn0 + 32 a + 8 (e / 4) + 4 h + e % 4, pixel = px0 + 32 b + lr
     if constexpr (QMODE == 0) {
-        const __amdgpu_buffer_rsrc_t brs_y = __builtin_amdgcn_make_buffer_rsrc(Y, 0, (int)y_bytes, 0x00020000);
+        const uint32_t img0 = __builtin_amdgcn_readfirstlane(img[0]);
+        const __amdgpu_buffer_rsrc_t brs_y =
+            __builtin_amdgcn_make_buffer_rsrc(Y + ((size_t)img0 * KN + kn0) * OHW, 0, (int)y_span, 0x00020000);
         // slopes from +0 to 1: PReLU is then max(r, r * alpha), bit for bit (with -0 a zero TNN sum becomes -0, which no maximum gives)
         const bool as_max = __float_as_uint(alpha) <= __float_as_uint(1.0f);
         for_blocks([&](auto blk_tag) {
@@ -1026,12 +1030,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
                 auto put = [&](auto whole) {
                     if constexpr (BUF) {
                         // a lane's part, and the kernel's row as a scalar; lanes past the pixels store beyond the buffer: nothing
-                        const uint32_t vy = live ? ((img[b] * (uint32_t)KN + (uint32_t)p0) * (uint32_t)OHW + pix[b]) * 4u : 0xffffff00u;
+                        const uint32_t vy =
+                            live ? (((img[b] - img0) * (uint32_t)KN + (uint32_t)(32 * a + 4 * h)) * (uint32_t)OHW + pix[b]) * 4u : 0xffffff00u;
 #pragma unroll
                         for (int e = 0; e < 16; e++) {
                             const int row = 8 * (e >> 2) + (e & 3);
                             if (decltype(whole)::value || p0 + row < KN)
-                                __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_uint(r[e]), brs_y, (int)vy, row * OHW * 4, 0);
+                                __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_uint(r[e]), brs_y, (int)vy, (int)((uint32_t)(row * 4) * (uint32_t)OHW), 0);
                         }
                     } else if (live) {
                         float* yq = Y + ((size_t)img[b] * KN + p0) * OHW + pix[b];
@@ -1367,8 +1372,9 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
     // operand sizes: the buffer-load variants announce them in their descriptors
     const int64_t p4_bytes = (int64_t)N * cg.CP * cg.H * cg.W * 32, wf_bytes = (int64_t)((KN + 31) / 32) * KB * 1024;
     static const bool no_buf = getenv("FTNN_CONV_NO_BUFFER_LOADS") != nullptr;   // tuning aid
-    const int64_t y_bytes = M * KN * 4;
-    const bool buf = !no_buf && p4_bytes <= 0xf0000000LL && wf_bytes <= 0xf0000000LL && (qo.mode != 0 || y_bytes <= 0xf0000000LL);
+    // an fp32 tile reaches over 64 kernels of its first image and as many more images as 64 pixels may touch
+    const int64_t y_span = ((int64_t)std::min(N - 1, 63 / OHW + 1) * KN + 64) * OHW * 4;
+    const bool buf = !no_buf && p4_bytes <= 0xf0000000LL && wf_bytes <= 0xf0000000LL && (qo.mode != 0 || y_span <= 0xf0000000LL);
     auto clip = [](int64_t v) { return (uint32_t)std::min<int64_t>(v, 0xffffffffLL); };
     const uint64_t wgs = (uint64_t)grid.x * grid.y;
     if (wgs > 0xffffffffull) return hipErrorInvalidValue;   // (no such result fits in memory)
@@ -1379,7 +1385,7 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
         constexpr int Q = decltype(qmode)::value, T = decltype(blocks)::value, SP = decltype(sp)::value;
         auto go = [&](auto kern) -> hipError_t {
             hipLaunchKernelGGL(kern, grid, dim3(64 * wpb), 0, st, P4, Wf, d_y, (int)M, KN, OHW, KB, bias, alpha, dOHW, cg, qo,
-                               clip(p4_bytes), clip(wf_bytes), clip(y_bytes), xo, grid.x, grid.y);
+                               clip(p4_bytes), clip(wf_bytes), clip(y_span), xo, grid.x, grid.y);
             return hipGetLastError();
         };
         return buf ? go(k_conv_f4<A, F, Q, T, T, SP, true>) : go(k_conv_f4<A, F, Q, T, T, SP, false>);

@@ -215,3 +215,35 @@ def test_large_layer_takes_the_gemm_route(hip, oracle, typ):
     prepared = hip.prepare_conv_weights(typ, qw, c, kn, 3, 3)
     got2 = hip.conv_prepared(typ, x, thr, prepared, kn, 3, 3, 1, 1, 0.5)
     assert torch.equal(got2, ref)
+
+
+@pytest.mark.parametrize("typ", [TNN, BNN], ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("h", [4096, 8192])
+def test_chain_result_beyond_32_bit_offsets(hip, oracle, typ, h):
+    """the last layer of a chain, whose quantised input the layer before hands over, with an fp32 result of more than 4 GiB:
+    two images of 130 x h x 1024, whose tiles stay within 32-bit offsets (h = 4096) or do not (8192: one image alone
+    is larger).  Every element against the same layers one by one on the vector-ALU engine"""
+    import torch
+    from fastertnn_amd import synth
+    n, w, mid, kn = 2, 1024, 64, 130
+    assert n * kn * h * w * 4 > 2 ** 32
+    print("case", TYPE_NAMES[typ], h, flush=True)
+    tern = typ == TNN
+    thr = 0.5 if tern else 0.0
+    rows = [(3, h, w, mid, 3, 3, 1, 1), (mid, h, w, kn, 1, 1, 0, 1)]
+    qws = []
+    for i, (c, _, _, k, ks, _, _, _) in enumerate(rows):
+        wt = (synth.ternary if tern else synth.binary)(60 + i, (k, c, ks, ks))
+        qws.append(torch.from_numpy(oracle.pack_weights(wt, np.full(k, 0.5 if tern else 0.0, np.float32), tern)).cuda())
+    g = torch.Generator(device="cuda")
+    g.manual_seed(6)
+    x = torch.randn((n, 3, h, w), generator=g, device="cuda")
+    thr_d = torch.full((n,), thr, device="cuda")
+    net = hip.Net(n, [dict(type=typ, shape=r, threshold=thr, alpha=0.5, qw=q) for r, q in zip(rows, qws)])
+    y = torch.full(net.out_shape, float("nan"), device="cuda")
+    net.run(x, out=y)
+    torch.cuda.synchronize()
+    net.close()
+    a = hip.conv(typ, x, thr_d, qws[0], mid, 3, 3, 1, 1, 0.5, engine=hip.ENGINE_VALU)
+    want = hip.conv(typ, a, thr_d, qws[1], kn, 1, 1, 0, 1, 0.5, engine=hip.ENGINE_VALU)
+    assert torch.equal(y, want)
