@@ -37,19 +37,30 @@ __device__ __forceinline__ uint32_t fastdiv(uint32_t n, const FastDiv& f) {
 // before, and the kernel tiles of a pixel tile and the halo of neighbouring ones are fetched once
 // (152-layer chain at batch 8: 1103 -> 980 us; in plain order every XCD fetches nearly all of the input from beyond its L2).
 // Weights as the outer index (an XCD then reads an eighth of them and all pixels): 1134 us.
+//
+// fp32 results beyond the 256 MiB of the Infinity Cache keep the plain order (`plain`): such a layer is bound by its
+// stores, and neighbouring workgroups then fill neighbouring pages of HBM instead of eight regions at a time.  First layers,
+// plain / XCD order: 32 x 3 x 224 x 224 -> 64, 3 x 3 (392 MiB) 120 / 131 us, 8 x 3 x 1024 x 1024 -> 130 (4 GiB) 1405 / 1495; last layers of
+// a chain: 40 x 256 x 112 x 112 -> 256, 1 x 1 (490 MiB) 147 / 155, 40 x 64 x 128 x 128 -> 2048 (5 GiB) 933 / 1078 (some sizes go the other
+// way by up to 6 %).  Up to 245 MiB the XCD order is ahead: 40 x 64 x 112 x 112 -> 128, 3 x 3 66 / 57.
+// The plain order is the same arithmetic on one share (mask 0), so that a launch takes no branch before its arguments.
 struct XcdOrder {
     uint32_t per, rem;   // tiles of an XCD; the first `rem` XCDs take one more
+    uint32_t mask;       // 7, or 0: plain
     FastDiv inner;
+    template <bool MAYBE_PLAIN>
     __device__ __forceinline__ void tile(uint32_t wg, uint32_t& o, uint32_t& i) const {
-        const uint32_t x = wg & 7u, t = x * per + min(x, rem) + (wg >> 3);
+        const uint32_t x = wg & (MAYBE_PLAIN ? mask : 7u), t = x * per + min(x, rem) + (wg >> (MAYBE_PLAIN ? mask & 3u : 3u));
         o = fastdiv(t, inner);
         i = t - o * inner.d;
     }
 };
-inline XcdOrder make_xcd_order(uint64_t outer, uint32_t inner) {   // outer * inner below 2^32
+constexpr int64_t kXcdOrderResultBytes = 256LL << 20;
+inline XcdOrder make_xcd_order(uint64_t outer, uint32_t inner, bool plain) {   // outer * inner below 2^32
     XcdOrder x;
     x.per = (uint32_t)(outer * inner / 8);
     x.rem = (uint32_t)(outer * inner % 8);
+    x.mask = plain ? 0u : 7u;
     x.inner = make_fastdiv(inner);
     return x;
 }

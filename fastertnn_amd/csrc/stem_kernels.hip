@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, lr = lane & 31;
     uint32_t img, bi;   // image, tile within it (kernel tile, pixel tile)
-    g.xo.tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), img, bi);
+    g.xo.tile<QMODE == 0>(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), img, bi);
     const uint32_t kt = fastdiv(bi, g.dTiles), bx = bi - kt * g.dTiles.d;
     const int n = (int)img, kn0 = (int)kt * 64;
     const int ty = (int)fastdiv(bx, g.dTX), tx = (int)bx - ty * g.tiles_x;
@@ -290,7 +290,7 @@ hipError_t launch_stem_f4(int type, const float* d_x, const float* d_thr, const 
     if ((uint64_t)tiles * kn_tiles * N > 0x7fffffffull) return hipErrorInvalidValue;   // (no such result fits in memory)
     g.kn_tiles = (uint32_t)kn_tiles;
     g.dTiles = make_fastdiv((uint32_t)tiles);
-    g.xo = make_xcd_order((uint64_t)N, (uint32_t)(tiles * kn_tiles));
+    g.xo = make_xcd_order((uint64_t)N, (uint32_t)(tiles * kn_tiles), qo.mode == 0 && (int64_t)N * KN * OH * OW * 4 > kXcdOrderResultBytes);
     const dim3 grid((unsigned)tiles, (unsigned)kn_tiles, (unsigned)N);   // (in one dimension 2^32 threads would bound it)
     const uint4* Wf = static_cast<const uint4*>(d_wf);
     const int KB = round4(Kd);

@@ -247,3 +247,24 @@ def test_chain_result_beyond_32_bit_offsets(hip, oracle, typ, h):
     a = hip.conv(typ, x, thr_d, qws[0], mid, 3, 3, 1, 1, 0.5, engine=hip.ENGINE_VALU)
     want = hip.conv(typ, a, thr_d, qws[1], kn, 1, 1, 0, 1, 0.5, engine=hip.ENGINE_VALU)
     assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("typ", [TNN, TBN, BTN, BNN], ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("c", [3, 64], ids=["first-layer", "layer"])
+def test_layers_with_results_beyond_256_mib(hip, oracle, typ, c):
+    """fp32 results beyond 256 MiB take their tiles in another order than smaller ones: ragged images and kernels, a first
+    layer and one of 64 channels (9 K words: the layer kernel), against the vector-ALU engine on every element"""
+    import torch
+    from fastertnn_amd import act_is_ternary, synth, weight_is_ternary
+    n, h, w, kn = 5, 411, 503, 70
+    assert n * kn * h * w * 4 > 256 << 20
+    print("case", TYPE_NAMES[typ], c, flush=True)
+    wt = weight_is_ternary(typ)
+    weights = (synth.ternary if wt else synth.binary)(70 + c, (kn, c, 3, 3))
+    qw = torch.from_numpy(oracle.pack_weights(weights, np.full(kn, 0.5 if wt else 0.0, np.float32), wt)).cuda()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(8)
+    x = torch.randn((n, c, h, w), generator=g, device="cuda")
+    thr = torch.full((n,), 0.5 if act_is_ternary(typ) else 0.0, device="cuda")
+    got, want = (hip.conv(typ, x, thr, qw, kn, 3, 3, 1, 1, -0.5, engine=e) for e in (hip.ENGINE_MFMA_F4, hip.ENGINE_VALU))
+    assert torch.equal(got, want)
