@@ -990,27 +990,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
             }
         });
         __syncthreads();
-        for_blocks([&](auto blk_tag) {
-            constexpr int BLK = decltype(blk_tag)::value;
-            if (BLK % S == ks) {
-                v16f& mine = acc[BLK / TB][BLK % TB];
+    }
+    // whole sum of a block that this wavefront finishes, in ordinary registers (accumulated in place it would go back into
+    // the accumulator registers and out again)
+    auto total = [&](auto blk_tag) {
+        constexpr int BLK = decltype(blk_tag)::value;
+        v16f c = acc[BLK / TB][BLK % TB];
+        if constexpr (S > 1) {
 #pragma unroll
-                for (int v = 0; v < S; v++) {
-                    if (v != BLK % S) {   // source wavefront pt * S + v
-                        const float4* src = red + (size_t)(((pt * S + v) * PUB + slot_of(BLK, v)) * 4) * 64 + lane;
+            for (int v = 0; v < S; v++) {
+                if (v != BLK % S) {   // source wavefront pt * S + v
+                    const float4* src = red + (size_t)(((pt * S + v) * PUB + slot_of(BLK, v)) * 4) * 64 + lane;
 #pragma unroll
-                        for (int e4 = 0; e4 < 4; e4++) {
-                            const float4 t = src[e4 * 64];
-                            mine[4 * e4] += t.x;
-                            mine[4 * e4 + 1] += t.y;
-                            mine[4 * e4 + 2] += t.z;
-                            mine[4 * e4 + 3] += t.w;
-                        }
+                    for (int e4 = 0; e4 < 4; e4++) {
+                        const float4 t = src[e4 * 64];
+                        c[4 * e4] += t.x;
+                        c[4 * e4 + 1] += t.y;
+                        c[4 * e4 + 2] += t.z;
+                        c[4 * e4 + 3] += t.w;
                     }
                 }
             }
-        });
-    }
+        }
+        return c;
+    };
     // accumulator e of block (a, b): kernel = kn0 + 32 a + 8 (e / 4) + 4 h + e % 4, pixel = px0 + 32 b + lr
     if constexpr (QMODE == 0) {
         const uint32_t img0 = __builtin_amdgcn_readfirstlane(img[0]);
@@ -1021,7 +1024,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
         for_blocks([&](auto blk_tag) {
             constexpr int BLK = decltype(blk_tag)::value, a = BLK / TB, b = BLK % TB;
             if (BLK % S == ks) {
-                const v16f& c = acc[a][b];
+                const v16f c = total(blk_tag);
                 float r[16];
                 if (as_max) {
 #pragma unroll
@@ -1066,19 +1069,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
             return static_cast<unsigned char*>(qo.p4) + (((size_t)img[b] * KT + kt) * (uint32_t)OHW + pix[b]) * 32;
         };
         if constexpr (NBLK == 4 && S < 4) {   // the wavefront finishes both kernel blocks of a pixel block: lane half h stores block h
-#pragma unroll
-            for (int b = 0; b < TB; b++)
+            auto pixel_block = [&](auto b_tag) {
+                constexpr int b = decltype(b_tag)::value;
                 if (b % S == ks) {
-                    const uint2 d0 = hand_over_block<FORM0, QMODE>(acc[0][b], alpha, qo, kn0, h, KN);
-                    const uint2 d1 = hand_over_block<FORM0, QMODE>(acc[TA - 1][b], alpha, qo, kn0 + 32, h, KN);
+                    const uint2 d0 = hand_over_block<FORM0, QMODE>(total(b_tag), alpha, qo, kn0, h, KN);
+                    const uint2 d1 = hand_over_block<FORM0, QMODE>(total(std::integral_constant<int, TB + b>{}), alpha, qo, kn0 + 32, h, KN);
                     const uint4 out = exchange_blocks(d0, d1);
                     if (px0 + 32 * b + lr < M) *reinterpret_cast<uint4*>(out_word(b) + 16 * h) = out;
                 }
+            };
+            pixel_block(std::integral_constant<int, 0>{});
+            pixel_block(std::integral_constant<int, 1>{});
         } else {   // one block: lane half h stores 8 bytes
             for_blocks([&](auto blk_tag) {
                 constexpr int BLK = decltype(blk_tag)::value, a = BLK / TB, b = BLK % TB;
                 if (BLK % S == ks) {
-                    const uint2 out = exchange_halves(hand_over_block<FORM0, QMODE>(acc[a][b], alpha, qo, kn0 + 32 * a, h, KN));
+                    const uint2 out = exchange_halves(hand_over_block<FORM0, QMODE>(total(blk_tag), alpha, qo, kn0 + 32 * a, h, KN));
                     const int part = TA == 2 ? a : (int)(by & 1u);
                     if (px0 + 32 * b + lr < M) *reinterpret_cast<uint2*>(out_word(b) + 16 * part + 8 * h) = out;
                 }
