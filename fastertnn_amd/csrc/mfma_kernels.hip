@@ -187,7 +187,7 @@ __device__ __forceinline__ void dma16(const uint4* gsrc, uint32_t lds_byte_addr)
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :
                  : "v"(gsrc), "s"(lds_byte_addr)
-                 : "memory");
+                 : "memory", "m0");
 }
 
 // Epilogue of the GEMM kernels: r = acc - bias, then PReLU in the reference's form for the type (form 0 "f = r; if

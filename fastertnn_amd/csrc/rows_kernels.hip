@@ -84,12 +84,21 @@ __device__ __forceinline__ void unpack_half(const RawRow<TERN>& r, int i, v4u& e
 
 // LDS-direct loads: 16 bytes per lane from base + voff (base uniform); the 64 lanes land contiguously.  M0 holds the LDS
 // address (one wait state after writing it); the instruction's immediate offset moves the source and the LDS address
-// alike, so a run of up to four loads into adjacent KiB shares one M0 (base + voff is then the source less OFF).  Inline
-// asm, so that the compiler does not order its own LDS reads against the loads; the kernel counts them by hand.
-__device__ __forceinline__ void set_m0(uint32_t lds_byte_addr) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(lds_byte_addr) : "memory"); }
-template <int OFF>
-__device__ __forceinline__ void dma16_at(const char* base, uint32_t voff) {
-    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(base), "n"(OFF) : "memory");
+// alike, so two loads into adjacent KiB share one M0 (v1 is then the source less 1024).  Inline asm, so that the compiler does
+// not order its own LDS reads against the loads; the kernel counts them by hand.  M0 is written and used within one statement and
+// declared: single loads, pairs and runs of four measured the same within 2 % from 256 x 256 to 3072 x 3072.
+template <bool TWO>
+__device__ __forceinline__ void dma16(uint32_t lds_byte_addr, const char* b0, uint32_t v0, const char* b1, uint32_t v1) {
+    if constexpr (TWO)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %3, %4 offset:1024"
+                     :
+                     : "s"(lds_byte_addr), "v"(v0), "s"(b0), "v"(v1), "s"(b1)
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :
+                     : "s"(lds_byte_addr), "v"(v0), "s"(b0)
+                     : "memory", "m0");
 }
 
 // Which tile a workgroup works on.  Workgroups go to the eight XCDs round-robin by number; XCD x takes the x-th eighth of the
@@ -155,7 +164,7 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
     // row, a binary one a single load of 32 rows x 32 bytes, two lanes per row; rows past the operand are clamped (their
     // results are never stored).  One base per side, advanced by GP or GQ per group; row block, row, piece and the
     // immediate offset a load carries are in its 32-bit lane offset.
-    constexpr uint32_t SPAN = 3072;   // the largest immediate offset
+    constexpr uint32_t SPAN = 1024;   // the largest immediate offset
     const char* const pbase = P + (size_t)prb0 * 32 * rbp - SPAN;
     const char* const qbase = Q + (size_t)qrb0 * 32 * rbq - SPAN;
     auto src_row = [&](int j, bool tern) { return tern ? j * 16 + (lane >> 2) : lane >> 1; };
@@ -166,13 +175,13 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
 #pragma unroll
         for (int j = 0; j < LP; j++)
             pv[a][j] = (uint32_t)min(a * 32 + src_row(j, TP), prow - 1 - prb0 * 32) * rbp + src_piece(TP) + SPAN -
-                       (uint32_t)((a * LP + j) & 3) * 1024u;
+                       (uint32_t)((a * LP + j) & 1) * 1024u;
 #pragma unroll
     for (int b = 0; b < WTQ; b++)
 #pragma unroll
         for (int j = 0; j < LQ; j++)
             qv[b][j] = (uint32_t)min(b * 32 + src_row(j, TQ), qrow - 1 - qrb0 * 32) * rbq + src_piece(TQ) + SPAN -
-                       (uint32_t)((WTP * LP + b * LQ + j) & 3) * 1024u;
+                       (uint32_t)((WTP * LP + b * LQ + j) & 1) * 1024u;
     // this lane's pieces of a row block in LDS: the signs and the zeros of its half
     auto piece_at = [&](bool tern, int piece) {
         return (uint32_t)(tern ? lr * 64 + (piece ^ ((lr >> 2) & 3)) * 16 : lr * 32 + (piece ^ ((lr >> 3) & 1)) * 16);
@@ -182,12 +191,16 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
     const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
     const char* const ring = reinterpret_cast<const char*>(lds) + ring0;
 
-    // load number i of group gg, into KiB i of the ring slot (M0: KiB i & ~3 of the slot)
-    auto m0_for = [&](int i, int slot) { set_m0(lds0 + ring0 + (uint32_t)(slot * LPG + (i & ~3)) * 1024u); };
-    auto issue = [&](auto itag, int gg) {
-        constexpr int i = decltype(itag)::value, OFF = (i & 3) * 1024;
-        if constexpr (i < WTP * LP) dma16_at<OFF>(pbase + (size_t)gg * GP, pv[i / LP][i % LP]);
-        else dma16_at<OFF>(qbase + (size_t)gg * GQ, qv[(i - WTP * LP) / LQ][(i - WTP * LP) % LQ]);
+    // load number i of group gg into KiB i of the ring slot and, if i is even and below `end`, load i + 1 with it
+    auto issue = [&](auto itag, auto end, int gg, int slot) {
+        constexpr int i = decltype(itag)::value;
+        constexpr bool two = (i & 1) == 0 && i + 1 < decltype(end)::value;
+        const char *pg = pbase + (size_t)gg * GP, *qg = qbase + (size_t)gg * GQ;
+        auto base = [&](int k) { return k < WTP * LP ? pg : qg; };
+        auto voff = [&](int k) { return k < WTP * LP ? pv[k / LP][k % LP] : qv[(k - WTP * LP) / LQ][(k - WTP * LP) % LQ]; };
+        // (an odd load by itself carries no immediate offset: its source is whole again)
+        const uint32_t kib = lds0 + ring0 + (uint32_t)(slot * LPG + i) * 1024u;
+        dma16<two>(kib, base(i), voff(i) + ((i & 1) ? 1024u : 0u), base(i + two), voff(i + two));
     };
     // planes of operand f (P blocks, then Q blocks) of the group in registers; its nibbles for two K words
     RawRow<TP> rp[WTP];
@@ -234,8 +247,7 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
                 constexpr int lo = I == 0 ? 0 : LPG / 2, n = I == 0 ? LPG / 2 : LPG - LPG / 2;
                 static_for<(m + 1) * n / NM - m * n / NM>([&](auto ktag) {
                     constexpr int i = lo + m * n / NM + decltype(ktag)::value;
-                    if constexpr ((i & 3) == 0 || i == lo) m0_for(i, slot);
-                    issue(std::integral_constant<int, i>{}, gl);
+                    if constexpr ((i & 1) == 0 || i == lo) issue(std::integral_constant<int, i>{}, std::integral_constant<int, lo + n>{}, gl, slot);
                 });
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -247,8 +259,7 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
         for (int t = 0; t < NS; t++) {
             static_for<LPG>([&](auto itag) {
                 constexpr int i = decltype(itag)::value;
-                if constexpr ((i & 3) == 0) m0_for(i, t);
-                issue(itag, min(gl, G - 1));
+                if constexpr ((i & 1) == 0) issue(itag, std::integral_constant<int, LPG>{}, min(gl, G - 1), t);
             });
             gl += KS;
         }

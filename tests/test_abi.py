@@ -231,3 +231,17 @@ def test_layer_chain_refuses_unknown_flags():
     d.threshold, d.prelu_alpha, d.d_qw = 0.5, 0.5, ctypes.c_void_p(256)
     assert not lib._L.ftnn_net_create_ex(1, 1, arr, 6)
     assert "flags" in lib._L.ftnn_last_error().decode()
+
+
+def test_lds_direct_loads_declare_m0():
+    """inline assembly that loads straight into LDS takes the address from M0: every such statement must set M0 itself and
+    declare that, or the compiler may use the register between a write in one statement and a load in another"""
+    import glob
+    statements = []
+    for path in sorted(glob.glob(os.path.join(ROOT, "fastertnn_amd", "csrc", "*.hip")) + glob.glob(os.path.join(ROOT, "bench_probe", "*.hip"))):
+        text = re.sub(r"//[^\n]*", "", open(path).read())
+        statements += [(os.path.basename(path), s) for s in re.findall(r"\basm\s+volatile\s*\((.*?)\)\s*;", text, re.S)
+                       if re.search(r"load_lds|load_dwordx?\d?\s[^;]*\blds\b", s)]
+    assert len(statements) >= 2
+    for path, s in statements:
+        assert s.index("s_mov_b32 m0") < s.index("load_lds") and re.search(r':[^:]*"m0"[^:]*$', s), (path, s)
