@@ -1053,16 +1053,23 @@ int ftnn_mm(int type, const int64_t* d_a, const int64_t* d_b, int N, int OH, int
     return e == hipSuccess ? FTNN_OK : hip_fail(e, "mm launch");
 }
 
-// Engine choice by shape, from measurements on MI355X (m x m x 8m, whole calls from packed rows, device time): the
-// matrix-core path pays one launch that expands both operands and works on tiles of 64 x 64, 128 x 128 or 256 x 256 by
-// tile count; the vector-ALU kernel is one launch near 0.3 PMAC/s.  m = 512 (1.1e9 lane-MACs): 12.0 us on the vector
-// ALU against 13.3 us on fp4; 576 (1.5e9): 13.9 against 13.0; 640 (2.1e9): 17.8 against 13.3; 768: 23.8 against 15.1;
-// other shapes with 1.6e9 - 1.9e9 lane-MACs are ties within 1 us either way, hence fp4 from 2e9 on.
+// The engine of a product by the amount of work: what runs it where packed rows are not multiplied as they are (auto_from_rows),
+// and what ftnn_select_engine answers.  Against the vector ALU the matrix cores with both operands expanded first pay from
+// about 2e9 lane-MACs on, by measurements on MI355X (m x m x 8m, whole calls from packed rows, device time): m = 512
+// (1.1e9 lane-MACs) 12.0 us on the vector ALU against 13.3 us on fp4, 576 (1.5e9) 13.9 / 13.0, 640 (2.1e9) 17.8 / 13.3, 768
+// 23.8 / 15.1; other shapes with 1.6e9 - 1.9e9 lane-MACs are ties within 1 us either way.
 static int select_engine(int type, int64_t M, int KN, int Kw) {
     (void)type;
     const double lane_macs = (double)M * KN * 64.0 * Kw;
     if (lane_macs >= 2e9 && KN >= 128 && Kw <= kMaxF4GemmWords) return FTNN_ENGINE_MFMA_F4;
     return FTNN_ENGINE_VALU;
+}
+
+// AUTO multiplies the packed rows as they are (k_rows) wherever the fp4 engine does and wherever select_engine would take the
+// vector ALU: that one launch is ahead of it down to the smallest product (32 x 32 x 256 a tie at 2.5 us, 256 x 256 x 4096 3.5
+// against 4.8, 100000 x 10 x 512 7.8 against 9.8).  Left to the engines are large products and those beyond the kernel's limits.
+static bool auto_from_rows(int engine, int64_t M, int KN, int Kw) {
+    return mm_rows_within_limits(M, KN, Kw) && (engine == FTNN_ENGINE_VALU || mm_from_rows(M, KN, Kw));
 }
 
 int ftnn_select_engine(int type, int N, int OH, int OW, int KN, int K) {
@@ -1074,7 +1081,10 @@ int64_t ftnn_mm_scratch_bytes(int engine, int type, int N, int OH, int OW, int K
     if (N <= 0 || OH <= 0 || OW <= 0 || KN <= 0 || K <= 0 || K > kMaxRowWords) return 0;
     const int64_t M = (int64_t)N * OH * OW;
     const int Kw = round4(K);
-    if (engine == FTNN_ENGINE_AUTO) engine = select_engine(type, M, KN, Kw);
+    if (engine == FTNN_ENGINE_AUTO) {
+        engine = select_engine(type, M, KN, Kw);
+        if (auto_from_rows(engine, M, KN, Kw)) return 0;
+    }
     if (engine != FTNN_ENGINE_MFMA_I8 && engine != FTNN_ENGINE_MFMA_F4) return 0;
     if (engine == FTNN_ENGINE_MFMA_F4) return mfma_f4_mm_scratch_bytes(M, KN, Kw);
     return mfma_fragment_bytes(false, M, Kw) + mfma_fragment_bytes(false, KN, Kw);
@@ -1142,12 +1152,10 @@ int ftnn_mm_engine(int engine, int type, const int64_t* d_a, const int64_t* d_b,
     if (M > 0x7fffffffLL) return fail(FTNN_EINVAL, "more than 2^31-1 output rows");
     if (engine == FTNN_ENGINE_AUTO) {
         engine = select_engine(type, M, KN, Kw);
-        // Products below 160 tiles of 256 x 256 (or narrower than 128) run straight from the packed rows, whatever their size: that one
-        // launch is ahead of the vector ALU down to the smallest (32 x 32 x 256 a tie at 2.5 us, 256 x 256 x 4096 3.5 against
-        // 4.8, 100000 x 10 x 512 7.8 against 9.8) and needs no scratch; it also takes the larger ones that come without
-        // scratch (4096 x 4096 x 32768 0.22 ms against 1.8).
         const bool scratch_ok = d_scratch && scratch_bytes >= ftnn_mm_scratch_bytes(engine, type, N, OH, OW, KN, K);
-        if (mm_rows_within_limits(M, KN, Kw) && (engine == FTNN_ENGINE_VALU || mm_from_rows(M, KN) || !scratch_ok)) {
+        // packed rows as they are, also for larger products that come without scratch (4096 x 4096 x 32768 0.22 ms against 1.8
+        // on the vector ALU)
+        if (auto_from_rows(engine, M, KN, Kw) || (!scratch_ok && mm_rows_within_limits(M, KN, Kw))) {
             const hipError_t e = launch_mm_rows(type, d_a, d_b, M, OH * OW, KN, Kw, K_unpack, prelu_alpha, d_y, (hipStream_t)stream);
             return e == hipSuccess ? FTNN_OK : hip_fail(e, "mm launch");
         }

@@ -257,8 +257,8 @@ hipError_t launch_mfma_pack4(bool ternary, const int64_t* d_rows, int rows, int 
 hipError_t launch_mfma_gemm_packed4(int type, const void* d_ac, const void* d_bc, int64_t M, int OHW, int KN, int Kw, int K_unpack,
                                     float alpha, float* d_y, hipStream_t st);
 // whether launch_mm_mfma runs an fp4 product straight from the packed rows (launch_mm_rows): by shape
-bool mm_from_rows(int64_t M, int KN);
-// scratch of launch_mm_mfma on the fp4 engine
+bool mm_from_rows(int64_t M, int KN, int Kw);
+// scratch that the explicit fp4 engine asks for
 int64_t mfma_f4_mm_scratch_bytes(int64_t M, int KN, int Kw);
 hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW,
                           int KN, int Kw, int K_unpack, float alpha, float* d_y, void* d_scratch,

@@ -1428,21 +1428,23 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
 // k_rows, fragments): 2048 x 2048 x 16384 (64 tiles) 31.5 / 44, 3072 x 3072 x 24576 (144) 107 / 136; from 256 tiles on packed4
 // is ahead at any K (4096 x 4096 x 32768 218 / 190, x 2048 35 / 32, x 512 27 / 24).  Products narrower than 128 would leave more
 // than half of such a tile empty.
-bool mm_from_rows(int64_t M, int KN) {
-    return ((M + 255) / 256) * ((KN + 255) / 256) < mfma_small_tile_below() || KN < 128 || M < 128;
+static bool few_big_tiles(int64_t M, int KN) { return ((M + 255) / 256) * ((KN + 255) / 256) < mfma_small_tile_below(); }
+bool mm_from_rows(int64_t M, int KN, int Kw) {
+    return mm_rows_within_limits(M, KN, Kw) && (few_big_tiles(M, KN) || KN < 128 || M < 128);
 }
 
-// (a product that runs from the rows uses none of it; callers size one buffer for whatever shapes they run)
+// What the explicit engine asks its callers for: both operands as fragments below 160 tiles, in packed4 form from there on.
+// A product from the rows touches none of it; AUTO asks for none there.
 int64_t mfma_f4_mm_scratch_bytes(int64_t M, int KN, int Kw) {
-    return mm_from_rows(M, KN) ? mfma_fragment_bytes(true, M, Kw) + mfma_fragment_bytes(true, KN, Kw)
-                               : mfma_packed4_bytes(M, Kw) + mfma_packed4_bytes(KN, Kw);
+    return few_big_tiles(M, KN) ? mfma_fragment_bytes(true, M, Kw) + mfma_fragment_bytes(true, KN, Kw)
+                                : mfma_packed4_bytes(M, Kw) + mfma_packed4_bytes(KN, Kw);
 }
 
 hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW,
                           int KN, int Kw, int K_unpack, float alpha, float* d_y, void* d_scratch,
                           hipStream_t st) {
     const bool a_tern = (type == kTNN || type == kTBN), b_tern = (type == kTNN || type == kBTN);
-    if (f4 && mm_from_rows(M, KN)) return launch_mm_rows(type, d_a, d_b, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
+    if (f4 && mm_from_rows(M, KN, Kw)) return launch_mm_rows(type, d_a, d_b, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
     if (f4) {   // the fp4 GEMM takes its operands at two bits per lane
         void* Ac = d_scratch;
         void* Bc = static_cast<char*>(d_scratch) + mfma_packed4_bytes(M, Kw);

@@ -39,8 +39,9 @@ int run(const char* version) {
         fill_values(static_cast<float*>(w.reserve(elems * sizeof(float))), elems, 12 + k, true, st);
         ftnn_check(ftnn_pack_gemm_operand(x.as<float>(), m, p, static_cast<int64_t*>(xp.reserve(elems / 4)), st), "ftnn_pack_gemm_operand");
         ftnn_check(ftnn_pack_gemm_operand(w.as<float>(), n, p, static_cast<int64_t*>(wp.reserve(elems / 4)), st), "ftnn_pack_gemm_operand");
-        const int engine = ftnn_select_engine(TNN, m, 1, 1, n, p_packed);
         const int64_t sb = ftnn_mm_scratch_bytes(FTNN_ENGINE_AUTO, TNN, m, 1, 1, n, p_packed);
+        // without scratch AUTO multiplies the packed rows as they are, on the fp4 matrix cores
+        const int engine = sb == 0 ? FTNN_ENGINE_MFMA_F4 : ftnn_select_engine(TNN, m, 1, 1, n, p_packed);
         void* d_scr = scratch.reserve((size_t)(sb > 0 ? sb : 16));
         float* out = static_cast<float*>(y.reserve((size_t)m * n * sizeof(float)));
         auto call = [&] {
@@ -64,7 +65,7 @@ int run(const char* version) {
         double wall = 0.0, dev_ms = 0.0;
         time_runs(call, 10, 30, st, &wall, &dev_ms);   // src/timing_gemm.c:25-30
         const double macs = (double)m * n * p;
-        fprintf(csv, "%d,%d,%d,%lf,%s,%.4f,%.1f,%s,%.4f\n", m, n, p, wall, version, dev_ms, macs / (dev_ms * 1e-3) / 1e9,
+        fprintf(csv, "%d,%d,%d,%lf,%s,%.4f,%.1f,%s,%.6f\n", m, n, p, wall, version, dev_ms, macs / (dev_ms * 1e-3) / 1e9,
                 engine_name(engine), roofline_fraction(engine, TNN, macs, macs, dev_ms * 1e-3));
         fflush(csv);
         printf("m = n = %d, p = %d: %.4f ms on %s\n", m, p, dev_ms, engine_name(engine));

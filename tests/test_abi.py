@@ -233,6 +233,25 @@ def test_layer_chain_refuses_unknown_flags():
     assert "flags" in lib._L.ftnn_last_error().decode()
 
 
+def test_products_from_packed_rows_ask_for_no_operand_scratch():
+    """AUTO asks for none where the packed rows are multiplied as they are; the explicit fp4 engine keeps its demand: both operands as
+    fragments below 160 tiles of 256 x 256, else in packed4 form, however narrow the product and beyond the other kernel's grid"""
+    import fastertnn_amd.lib as lib
+    packed4 = lambda m, n, k: int(lib._L.ftnn_expand_bytes(lib.ENGINE_MFMA_F4, m, k)) + int(lib._L.ftnn_expand_bytes(lib.ENGINE_MFMA_F4, n, k))
+    blocks = lambda m: (m + 31) // 32
+    for typ in range(4):
+        for m, n, k in ((1, 1, 4), (256, 256, 64), (1024, 1024, 128), (2048, 2048, 256), (33000, 100, 64)):
+            assert lib.mm_scratch_bytes(lib.ENGINE_AUTO, typ, m, 1, 1, n, k) == 0, (m, n, k)
+            assert lib.mm_scratch_bytes(lib.ENGINE_MFMA_F4, typ, m, 1, 1, n, k) == (blocks(m) + blocks(n)) * k * 1024, (m, n, k)
+        for m, n, k in ((50000, 100, 64), (100, 50000, 64), (40960, 127, 4), (2 ** 31 - 1, 100, 4)):
+            assert lib.mm_scratch_bytes(lib.ENGINE_MFMA_F4, typ, m, 1, 1, n, k) == packed4(m, n, k), (m, n, k)
+            if m < 2 ** 31 - 1:
+                assert lib.mm_scratch_bytes(lib.ENGINE_AUTO, typ, m, 1, 1, n, k) == 0, (m, n, k)
+        for m, n, k in ((4096, 4096, 512), (3333, 3100, 4), (40960, 256, 64)):
+            for engine in (lib.ENGINE_AUTO, lib.ENGINE_MFMA_F4):
+                assert lib.mm_scratch_bytes(engine, typ, m, 1, 1, n, k) == packed4(m, n, k), (m, n, k)
+
+
 def test_lds_direct_loads_declare_m0():
     """inline assembly that loads straight into LDS takes the address from M0: every such statement must set M0 itself and
     declare that, or the compiler may use the register between a write in one statement and a load in another"""

@@ -84,3 +84,25 @@ def test_more_rows_than_the_smallest_tile_has_workgroups_for(hip):
     want = hip.mm_engine(hip.ENGINE_VALU, BNN, a_d, b_d, m, 1, 1, 1, kw, 0.5, 64 * kw)
     got = hip.mm_engine(hip.ENGINE_AUTO, BNN, a_d, b_d, m, 1, 1, 1, kw, 0.5, 64 * kw)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("typ", ALL_TYPES, ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("shape", [(41000, 99, 8), (99, 41000, 8)], ids=["narrow", "low"])
+def test_explicit_fp4_engine_on_narrow_products(hip, oracle, typ, shape):
+    """products of 160 tiles of 256 x 256 and more that are narrower than 128 run from the packed rows on the explicit engine too,
+    with scratch for both operands in packed4 form, which stays as it was; less is refused"""
+    import torch
+    m, n, kw = shape
+    a, b = _operands(typ, m, n, kw, 7 + typ)
+    ku = 64 * kw - 9
+    print("case", TYPE_NAMES[typ], shape, flush=True)
+    want = oracle.mm(typ, a, b, m, 1, 1, n, kw, 0.5, ku)
+    a_d, b_d = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    packed4 = sum(int(hip._L.ftnn_expand_bytes(hip.ENGINE_MFMA_F4, r, kw)) for r in (m, n))
+    assert hip.mm_scratch_bytes(hip.ENGINE_MFMA_F4, typ, m, 1, 1, n, kw) == packed4
+    scratch = torch.full((packed4,), 0x5A, dtype=torch.uint8, device="cuda")
+    got = hip.mm_engine(hip.ENGINE_MFMA_F4, typ, a_d, b_d, m, 1, 1, n, kw, 0.5, ku, scratch=scratch).cpu().numpy()
+    assert got.tobytes() == want.tobytes()
+    assert bool((scratch == 0x5A).all())
+    with pytest.raises(hip.FtnnError):
+        hip.mm_engine(hip.ENGINE_MFMA_F4, typ, a_d, b_d, m, 1, 1, n, kw, 0.5, ku, scratch=scratch[:packed4 - 1].contiguous())
