@@ -580,10 +580,13 @@ static int area_of_slot(int slot) {
 // FTNN_HOST_WEIGHT_CACHE_MB = n sets it, FTNN_HOST_NO_WEIGHT_CACHE = 1 or a cap of 0 switches the cache off; a layer
 // whose prepared weights alone exceed the cap is uploaded and prepared on every call); ftnn_host_forget_weights()
 // drops them all.
+// The layer's geometry is known here, so an entry holds one form only: the packed rows of a fully connected layer (`rows`), else
+// what ftnn_conv_prepare_weights makes without the rows behind it (which are half as much again for 1 x 1 layers).
 struct PreparedWeights {
     size_t bytes;
     Hash128 hash;
     int type, C, KN, KH, KW;
+    bool rows;
     void* dev;
     size_t dev_bytes;
     uint64_t last_use;
@@ -622,25 +625,33 @@ static void drop_weight_entry(size_t i) {
     g_weights.erase(g_weights.begin() + (long)i);
 }
 
-// device pointer of the prepared weights of this layer (uploading and preparing them on a miss)
-static const void* prepared_weights(int type, const int64_t* host, size_t bytes, int C, int KN, int KH, int KW) {
-    const size_t dev_bytes = (size_t)ftnn_conv_weights_bytes(type, C, KN, KH, KW);
+static int64_t prepared_bytes(int type, int C, int KN, int KH, int KW, bool keep_rows, int64_t* tmp_off);
+static int prepare_weights(int type, const int64_t* d_qw, int C, int KN, int KH, int KW, bool keep_rows, void* d_prepared, hipStream_t st);
+
+// device pointer of the weights of this layer: its packed rows, or prepared (uploading and preparing them on a miss)
+static const void* prepared_weights(int type, const int64_t* host, size_t bytes, int C, int KN, int KH, int KW, bool rows) {
+    auto prepare = [&](void* dev) {
+        int64_t* d_rows = (int64_t*)upload(SLOT_W, host, bytes);
+        if (rows) hip_or_die(hipMemcpyAsync(dev, d_rows, bytes, hipMemcpyDeviceToDevice, host_stream()), "hipMemcpyAsync");
+        else if (prepare_weights(type, d_rows, C, KN, KH, KW, false, dev, host_stream()) != FTNN_OK) die("tnns_conv");
+    };
+    const size_t dev_bytes = rows ? bytes : (size_t)prepared_bytes(type, C, KN, KH, KW, false, nullptr);
     const size_t cap = weight_cache_cap();
     if (cap == 0 || dev_bytes > cap) {
-        // not kept: uploaded and prepared into a work buffer on every call
+        // not kept: uploaded (and prepared into a work buffer) on every call
+        if (rows) return upload(SLOT_W, host, bytes);
         void* d_prep = dev_buf(SLOT_PREP, dev_bytes);
-        int64_t* d_rows = (int64_t*)upload(SLOT_W, host, bytes);
-        if (ftnn_conv_prepare_weights(type, d_rows, C, KN, KH, KW, d_prep, host_stream()) != FTNN_OK) die("tnns_conv");
+        prepare(d_prep);
         return d_prep;
     }
     const Hash128 hash = content_hash(host, bytes);
     g_weights_clock++;
     for (PreparedWeights& e : g_weights)
-        if (e.bytes == bytes && e.hash == hash && e.type == type && e.C == C && e.KN == KN && e.KH == KH && e.KW == KW) {
+        if (e.bytes == bytes && e.hash == hash && e.type == type && e.C == C && e.KN == KN && e.KH == KH && e.KW == KW && e.rows == rows) {
             e.last_use = g_weights_clock;
             return e.dev;
         }
-    PreparedWeights e = {bytes, hash, type, C, KN, KH, KW, nullptr, dev_bytes, g_weights_clock};
+    PreparedWeights e = {bytes, hash, type, C, KN, KH, KW, rows, nullptr, dev_bytes, g_weights_clock};
     while (!g_weights.empty() && (g_weights.size() >= kWeightCacheEntries || g_weights_bytes + e.dev_bytes > cap)) {
         size_t oldest = 0;
         for (size_t i = 1; i < g_weights.size(); i++)
@@ -648,8 +659,7 @@ static const void* prepared_weights(int type, const int64_t* host, size_t bytes,
         drop_weight_entry(oldest);
     }
     hip_or_die(hipMalloc(&e.dev, e.dev_bytes ? e.dev_bytes : 16), "hipMalloc");
-    int64_t* d_rows = (int64_t*)upload(SLOT_W, host, bytes);
-    if (ftnn_conv_prepare_weights(type, d_rows, C, KN, KH, KW, e.dev, host_stream()) != FTNN_OK) die("tnns_conv");
+    prepare(e.dev);
     g_weights_bytes += e.dev_bytes;
     g_weights.push_back(e);
     return e.dev;
@@ -787,6 +797,65 @@ static int conv_fc_rows(int type, const float* d_x, const float* d_thr, const in
     if (e != hipSuccess) return hip_fail(e, "quantise launch");
     e = launch_mm_rows(type, d_a, d_qw, N, 1, KN, round4(cpack_of(C)), C, prelu_alpha, d_y, st);
     return e == hipSuccess ? FTNN_OK : hip_fail(e, "packed-row GEMM launch");
+}
+
+// Layer engine by shape, from measurements on MI355X: the fp4 matrix-core kernel wins wherever it
+// applies.
+static int select_conv_engine(int type, int N, int C, int H, int W, int KN, int KH, int KW, int OH, int OW) {
+    (void)type; (void)N; (void)H; (void)W; (void)KN; (void)OH; (void)OW;
+    int T, Kd;
+    // few channels: the dense re-packing feeds the matrix cores for C <= 8, the vector ALU beyond
+    if (dense_applies(C, KH, KW, &T, &Kd)) return C <= 8 ? FTNN_ENGINE_MFMA_F4 : FTNN_ENGINE_VALU;
+    if (64LL * cpack_of(C) * KH * KW >= (1LL << 24)) return FTNN_ENGINE_VALU;   // fp32 accumulation must stay exact
+    return FTNN_ENGINE_MFMA_F4;
+}
+
+// Weights in the form the layer's engine reads them, made once per layer instead of once per call.  keep_rows: for layers that
+// may be fully connected, the packed rows behind the fragments (ftnn_conv_prepare_weights does not know the image size; the
+// 1 x 1 layers on larger images leave them unread).  tmp_off: where what lies behind the fragments starts.
+static int64_t prepared_bytes(int type, int C, int KN, int KH, int KW, bool keep_rows, int64_t* tmp_off) {
+    const bool wt = (type == kTNN || type == kBTN);
+    const int engine = select_conv_engine(type, 1, C, KH, KW, KN, KH, KW, 1, 1);
+    int T, Kd;
+    const bool dense = dense_applies(C, KH, KW, &T, &Kd);
+    if (tmp_off) *tmp_off = 0;
+    if (engine == FTNN_ENGINE_MFMA_F4) {
+        const int64_t frag = (mfma_fragment_bytes(true, KN, conv_f4_weight_words(C, KH, KW)) + 255) / 256 * 256;
+        if (tmp_off) *tmp_off = frag;
+        // the dense path expands the re-packed rows, which need a place of their own
+        if (dense_f4_applies(C, KH, KW)) return frag + (int64_t)KN * round4(Kd) * (wt ? 16 : 8);
+        // the packed rows as they are, behind the fragments: operand of conv_fc_rows
+        return frag + (keep_rows && fc_weights(C, KH, KW) ? (int64_t)KN * round4(cpack_of(C)) * (wt ? 16 : 8) : 0);
+    }
+    return (int64_t)KN * (dense ? round4(Kd) : round4(cpack_of(C) * KH * KW)) * (wt ? 16 : 8);
+}
+
+static int prepare_weights(int type, const int64_t* d_qw, int C, int KN, int KH, int KW, bool keep_rows, void* d_prepared, hipStream_t st) {
+    const bool wt = (type == kTNN || type == kBTN);
+    int64_t tmp_off;
+    const int64_t bytes = prepared_bytes(type, C, KN, KH, KW, keep_rows, &tmp_off);
+    const int engine = select_conv_engine(type, 1, C, KH, KW, KN, KH, KW, 1, 1);
+    int T, Kd;
+    const bool dense = dense_applies(C, KH, KW, &T, &Kd);
+    hipError_t e;
+    if (engine == FTNN_ENGINE_MFMA_F4) {
+        const int64_t* rows = d_qw;
+        if (dense_f4_applies(C, KH, KW)) {
+            int64_t* d_wd = reinterpret_cast<int64_t*>(static_cast<char*>(d_prepared) + tmp_off);
+            e = launch_dense_weights(wt, d_qw, KN, C, KH, KW, d_wd, st);
+            if (e != hipSuccess) return hip_fail(e, "dense weights launch");
+            rows = d_wd;
+        }
+        int64_t* kept = keep_rows && fc_weights(C, KH, KW) ? reinterpret_cast<int64_t*>(static_cast<char*>(d_prepared) + tmp_off) : nullptr;
+        e = launch_mfma_expand(true, wt, rows, KN, conv_f4_weight_words(C, KH, KW), d_prepared, st, kept);
+        return e == hipSuccess ? FTNN_OK : hip_fail(e, "weight expansion launch");
+    }
+    if (dense) {
+        e = launch_dense_weights(wt, d_qw, KN, C, KH, KW, static_cast<int64_t*>(d_prepared), st);
+        return e == hipSuccess ? FTNN_OK : hip_fail(e, "dense weights launch");
+    }
+    e = hipMemcpyAsync(d_prepared, d_qw, (size_t)bytes, hipMemcpyDeviceToDevice, st);
+    return e == hipSuccess ? FTNN_OK : hip_fail(e, "weight copy");
 }
 
 // operand region of the fp4 layer for this shape, whichever form it takes
@@ -979,17 +1048,6 @@ int64_t ftnn_pack_scratch_bytes(int N, int C, int H, int W, int ternary) {
         __builtin_mul_overflow(bytes, (int64_t)(ternary ? 16 : 8), &bytes))
         return 0;
     return bytes;
-}
-
-// Layer engine by shape, from measurements on MI355X: the fp4 matrix-core kernel wins wherever it
-// applies.
-static int select_conv_engine(int type, int N, int C, int H, int W, int KN, int KH, int KW, int OH, int OW) {
-    (void)type; (void)N; (void)H; (void)W; (void)KN; (void)OH; (void)OW;
-    int T, Kd;
-    // few channels: the dense re-packing feeds the matrix cores for C <= 8, the vector ALU beyond
-    if (dense_applies(C, KH, KW, &T, &Kd)) return C <= 8 ? FTNN_ENGINE_MFMA_F4 : FTNN_ENGINE_VALU;
-    if (64LL * cpack_of(C) * KH * KW >= (1LL << 24)) return FTNN_ENGINE_VALU;   // fp32 accumulation must stay exact
-    return FTNN_ENGINE_MFMA_F4;
 }
 
 int ftnn_select_conv_engine(int type, int N, int C, int H, int W, int KN, int KH, int KW, int H_pad, int W_pad,
@@ -1218,28 +1276,10 @@ int ftnn_conv_engine(int engine, int type, const float* d_x, const float* d_thr,
                      d_scratch, d_y, (hipStream_t)stream, QuantOut(), false);
 }
 
-// Weights in the form the layer's engine reads them, made once per layer instead of once per call.
-static int64_t prepared_bytes(int type, int C, int KN, int KH, int KW, int64_t* tmp_off) {
-    const bool wt = (type == kTNN || type == kBTN);
-    const int engine = select_conv_engine(type, 1, C, KH, KW, KN, KH, KW, 1, 1);
-    int T, Kd;
-    const bool dense = dense_applies(C, KH, KW, &T, &Kd);
-    if (tmp_off) *tmp_off = 0;
-    if (engine == FTNN_ENGINE_MFMA_F4) {
-        const int64_t frag = (mfma_fragment_bytes(true, KN, conv_f4_weight_words(C, KH, KW)) + 255) / 256 * 256;
-        if (tmp_off) *tmp_off = frag;
-        // the dense path expands the re-packed rows, which need a place of their own
-        if (dense_f4_applies(C, KH, KW)) return frag + (int64_t)KN * round4(Kd) * (wt ? 16 : 8);
-        // the packed rows as they are, behind the fragments: operand of conv_fc_rows
-        return frag + (fc_weights(C, KH, KW) ? (int64_t)KN * round4(cpack_of(C)) * (wt ? 16 : 8) : 0);
-    }
-    return (int64_t)KN * (dense ? round4(Kd) : round4(cpack_of(C) * KH * KW)) * (wt ? 16 : 8);
-}
-
 int64_t ftnn_conv_weights_bytes(int type, int C, int KN, int KH, int KW) {
     if (type < kTNN || type > kBNN || C <= 0 || KN <= 0 || KH <= 0 || KW <= 0) return 0;
     if (!row_fits(C, KH, KW)) return 0;
-    return prepared_bytes(type, C, KN, KH, KW, nullptr);
+    return prepared_bytes(type, C, KN, KH, KW, true, nullptr);
 }
 
 int ftnn_conv_prepare_weights(int type, const int64_t* d_qw, int C, int KN, int KH, int KW, void* d_prepared,
@@ -1250,32 +1290,7 @@ int ftnn_conv_prepare_weights(int type, const int64_t* d_qw, int C, int KN, int 
         return fail(FTNN_EINVAL, "more than %d words per weight row", kMaxRowWords);
     if (!d_qw || !d_prepared || !aligned16(d_qw) || !aligned16(d_prepared))
         return fail(FTNN_EINVAL, "null or misaligned device pointer");
-    const bool wt = (type == kTNN || type == kBTN);
-    hipStream_t st = (hipStream_t)stream;
-    int64_t tmp_off;
-    const int64_t bytes = prepared_bytes(type, C, KN, KH, KW, &tmp_off);
-    const int engine = select_conv_engine(type, 1, C, KH, KW, KN, KH, KW, 1, 1);
-    int T, Kd;
-    const bool dense = dense_applies(C, KH, KW, &T, &Kd);
-    hipError_t e;
-    if (engine == FTNN_ENGINE_MFMA_F4) {
-        const int64_t* rows = d_qw;
-        if (dense_f4_applies(C, KH, KW)) {
-            int64_t* d_wd = reinterpret_cast<int64_t*>(static_cast<char*>(d_prepared) + tmp_off);
-            e = launch_dense_weights(wt, d_qw, KN, C, KH, KW, d_wd, st);
-            if (e != hipSuccess) return hip_fail(e, "dense weights launch");
-            rows = d_wd;
-        }
-        int64_t* kept = fc_weights(C, KH, KW) ? reinterpret_cast<int64_t*>(static_cast<char*>(d_prepared) + tmp_off) : nullptr;
-        e = launch_mfma_expand(true, wt, rows, KN, conv_f4_weight_words(C, KH, KW), d_prepared, st, kept);
-        return e == hipSuccess ? FTNN_OK : hip_fail(e, "weight expansion launch");
-    }
-    if (dense) {
-        e = launch_dense_weights(wt, d_qw, KN, C, KH, KW, static_cast<int64_t*>(d_prepared), st);
-        return e == hipSuccess ? FTNN_OK : hip_fail(e, "dense weights launch");
-    }
-    e = hipMemcpyAsync(d_prepared, d_qw, (size_t)bytes, hipMemcpyDeviceToDevice, st);
-    return e == hipSuccess ? FTNN_OK : hip_fail(e, "weight copy");
+    return prepare_weights(type, d_qw, C, KN, KH, KW, true, d_prepared, (hipStream_t)stream);
 }
 
 int ftnn_conv_prepared(int type, const float* d_x, const float* d_thr, const void* d_prepared, int N, int C, int H,
@@ -1296,7 +1311,7 @@ int ftnn_conv_prepared(int type, const float* d_x, const float* d_thr, const voi
             return fail(FTNN_EINVAL, "more than 2^31-1 input pixel words");
         if (fc_from_rows(C, H, W, KH, KW, H_pad, W_pad)) {
             int64_t rows_off;
-            prepared_bytes(type, C, KN, KH, KW, &rows_off);
+            prepared_bytes(type, C, KN, KH, KW, true, &rows_off);
             const char* rows = static_cast<const char*>(d_prepared) + rows_off;
             return conv_fc_rows(type, d_x, d_thr, reinterpret_cast<const int64_t*>(rows), N, C, KN, prelu_alpha, d_scratch, d_y,
                                 (hipStream_t)stream);
@@ -1424,9 +1439,12 @@ void tnns_conv(testcase_t* t) {
         ((int64_t)N * H * W * cpack_of(C) <= 0x7fffffffLL && (int64_t)rows * conv_f4_weight_words(C, KH, KW) <= 0x7fffffffLL);
     int rc;
     if (prepared_ok) {
-        const void* d_prep = prepared_weights(type, t->quantized_kernel_packing2, w_bytes, C, KN, KH, KW);
-        rc = ftnn_conv_prepared(type, d_x, d_thr, d_prep, N, C, H, W, KN, KH, KW, t->paddingH, t->paddingW, t->strideH,
-                                t->strideW, t->preluAlpha, d_scr, d_y, host_stream());
+        const bool fc = fc_from_rows(C, H, W, KH, KW, t->paddingH, t->paddingW) &&
+                        select_conv_engine(type, N, C, H, W, KN, KH, KW, OH, OW) == FTNN_ENGINE_MFMA_F4;
+        const void* d_prep = prepared_weights(type, t->quantized_kernel_packing2, w_bytes, C, KN, KH, KW, fc);
+        rc = fc ? conv_fc_rows(type, d_x, d_thr, static_cast<const int64_t*>(d_prep), N, C, KN, t->preluAlpha, d_scr, d_y, host_stream())
+                : ftnn_conv_prepared(type, d_x, d_thr, d_prep, N, C, H, W, KN, KH, KW, t->paddingH, t->paddingW, t->strideH,
+                                     t->strideW, t->preluAlpha, d_scr, d_y, host_stream());
     } else {
         int64_t* d_w = (int64_t*)upload(SLOT_W, t->quantized_kernel_packing2, w_bytes);
         rc = ftnn_conv(type, d_x, d_thr, d_w, N, C, H, W, KN, KH, KW, t->paddingH, t->paddingW, t->strideH, t->strideW,

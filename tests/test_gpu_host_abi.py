@@ -273,6 +273,27 @@ def test_same_rows_at_another_address_are_found_again(hip, oracle):
     assert hip.host_cached_weight_bytes() == held
 
 
+@pytest.mark.parametrize("typ", [TNN, TBN], ids=lambda t: TYPE_NAMES[t])
+def test_kept_weights_of_1x1_layers_hold_one_form(hip, oracle, typ):
+    """the cache holds what the layer reads and no more: fragments for a 1 x 1 layer on images, the packed rows for the same
+    weights on one pixel per image, both at once under their own entries"""
+    wt = weight_is_ternary(typ)
+    c, kn = 200, 70
+    fragments, rows = (kn + 31) // 32 * 4 * 1024, kn * 4 * (16 if wt else 8)
+    hip.host_forget_weights()
+    held = 0
+    for rep in range(2):
+        for hw, size in ((5, fragments), (1, rows)):
+            L = make_layer(typ, (c, hw, hw, kn, 1, 1, 0, 1), 3, seed=7300)
+            q = oracle.pack_weights(L["w"], L["wthr"], wt)
+            want = oracle.conv(typ, L["x"], L["thr"], q, kn, 1, 1, 0, 1, 0.5)
+            print("case kept weights", TYPE_NAMES[typ], hw, rep, flush=True)
+            assert hip.host_conv(typ, L["x"], L["thr"], q, kn, 1, 1, 0, 1, 0.5).tobytes() == want.tobytes()
+            held += size if rep == 0 else 0
+            assert hip.host_cached_weight_bytes() == held
+    hip.host_forget_weights()
+
+
 def test_large_weight_rows_are_hashed_in_slices_and_kept(hip, oracle):
     """rows of 17 MiB: hashed in slices on the copy threads, kept like any other layer's, and a single flipped bit
     anywhere in them is seen"""
