@@ -106,9 +106,9 @@ def test_row_major_gemm_all_types(hip, oracle, typ, mnk):
 @pytest.mark.parametrize("typ", ALL_TYPES, ids=lambda t: TYPE_NAMES[t])
 @pytest.mark.parametrize("shape", [(3333, 1, 1, 3100, 4), (5, 29, 29, 2700, 12)], ids=["row_major", "nchw"])
 def test_matrix_core_engines_with_256x256_tiles(hip, oracle, typ, shape):
-    """the matrix-core kernel works on 128 x 128 tiles while a problem has few of them and on 256 x 256
-    tiles from 160 of those on; the cases above are all of the first kind, these are of the second
-    (ragged in both directions, row-major and NCHW stores)"""
+    """the tile kernels work on 256 x 256 tiles from 160 of those on; below, the int8 engine takes smaller tiles and the fp4 engine
+    multiplies the packed rows: the cases above are all of the first kind, these are of the second (ragged in both
+    directions, row-major and NCHW stores)"""
     n, oh, ow, kn, kw = shape
     m = n * oh * ow
     assert ((m + 255) // 256) * ((kn + 255) // 256) >= 160
@@ -127,9 +127,10 @@ def test_matrix_core_engines_with_256x256_tiles(hip, oracle, typ, shape):
 @pytest.mark.parametrize("typ", ALL_TYPES, ids=lambda t: TYPE_NAMES[t])
 @pytest.mark.parametrize("shape", [(1500, 1, 1, 1480, 4), (3, 23, 23, 1500, 8)], ids=["row_major", "nchw"])
 def test_matrix_core_engines_with_128x128_tiles(hip, oracle, typ, shape):
-    """on plain fragments (the int8 engine, fp4 whole calls with few 256 x 256 tiles) the tile kernel works on
-    64 x 64 tiles below 112 tiles of 128 x 128, as in the small cases above, and on 128 x 128 tiles from there
-    up to 160 tiles of 256 x 256: these cases are of that middle kind"""
+    """the int8 engine's tile kernel works on 64 x 64 tiles below 112 tiles of 128 x 128, as in the small cases above, and on
+    128 x 128 tiles from there up to 160 tiles of 256 x 256: these cases are of that middle kind.  The fp4 engine
+    multiplies their packed rows; its tile kernel on 128 x 128 tiles of fragments serves large layers
+    (test_large_layer_on_the_gemm_route_with_128x128_tiles)"""
     n, oh, ow, kn, kw = shape
     m = n * oh * ow
     assert ((m + 127) // 128) * ((kn + 127) // 128) >= 112 and ((m + 255) // 256) * ((kn + 255) // 256) < 160

@@ -191,9 +191,9 @@ def test_nchw_results_beyond_2_32_elements(hip, oracle):
 
 @pytest.mark.parametrize("typ", [TNN, TBN, BTN, BNN], ids=lambda t: TYPE_NAMES[t])
 def test_large_layer_takes_the_gemm_route(hip, oracle, typ):
-    """a 29.6 GMAC layer (batch 16, 512 -> 512 channels at 28 x 28, 392 tiles of 128 x 128): the fp4 engine runs it as quantise + im2row +
-    expansion + the tiled GEMM kernel.  Same bits as the vector-ALU engine on every element, and as the oracle on
-    one image"""
+    """a 29.6 GMAC layer (batch 16, 512 -> 512 channels at 28 x 28, 392 tiles of 128 x 128): large enough for the quantise + im2row +
+    expansion + tiled GEMM route, but within the limits of the tile kernel with implicit im2row, which takes it.  Same bits
+    as the vector-ALU engine on every element, and as the oracle on one image"""
     import torch
     from fastertnn_amd import synth
     n, c, hw, kn = 16, 512, 28, 512
@@ -215,6 +215,33 @@ def test_large_layer_takes_the_gemm_route(hip, oracle, typ):
     prepared = hip.prepare_conv_weights(typ, qw, c, kn, 3, 3)
     got2 = hip.conv_prepared(typ, x, thr, prepared, kn, 3, 3, 1, 1, 0.5)
     assert torch.equal(got2, ref)
+
+
+@pytest.mark.parametrize("typ", [TNN, TBN, BTN, BNN], ids=lambda t: TYPE_NAMES[t])
+def test_large_layer_on_the_gemm_route_with_128x128_tiles(hip, oracle, typ):
+    """8 images of 7 x 7, 512 -> 8192 channels, 3 x 3 (392 pixels, too few for the implicit im2row): quantise + im2row + expansion +
+    the tile GEMM on 256 tiles of 128 x 128, seen by the rows it leaves in the scratch.  Same bits as the vector-ALU engine on
+    every element, and as the oracle on two images"""
+    import torch
+    from fastertnn_amd import act_is_ternary, synth, weight_is_ternary
+    n, c, hw, kn = 8, 512, 7, 8192
+    m, kw = n * hw * hw, c // 64 * 9
+    assert m < 512 and ((m + 127) // 128) * ((kn + 127) // 128) >= 256 and m * kn * 64 * kw >= 1.2e10
+    assert ((m + 255) // 256) * ((kn + 255) // 256) < 160
+    print("case", TYPE_NAMES[typ], flush=True)
+    at, wt = act_is_ternary(typ), weight_is_ternary(typ)
+    x = synth.normal(50 + typ, (n, c, hw, hw))
+    thr = np.full(n, 0.5 if at else 0.0, np.float32)
+    qw_h = oracle.pack_weights((synth.ternary if wt else synth.binary)(54 + typ, (kn, c, 3, 3)), np.full(kn, 0.5 if wt else 0.0, np.float32), wt)
+    x_d, thr_d, qw = (torch.from_numpy(v).cuda() for v in (x, thr, qw_h))
+    scratch = torch.full((hip.conv_scratch_bytes(typ, n, c, hw, hw, kn, 3, 3, 1, 1),), 0x5A, dtype=torch.uint8, device="cuda")
+    got = hip.conv(typ, x_d, thr_d, qw, kn, 3, 3, 1, 1, -0.5, engine=hip.ENGINE_MFMA_F4, scratch=scratch)
+    planes = (hip.pack_scratch_bytes(n, c, hw, hw, 1) + 255) // 256 * 256
+    rows = hip.quantize_im2row(x_d, thr_d, 3, 3, 1, 1, at).view(torch.uint8)
+    assert torch.equal(scratch[planes:planes + rows.numel()], rows)   # the tile kernel's input would end far below
+    assert torch.equal(got, hip.conv(typ, x_d, thr_d, qw, kn, 3, 3, 1, 1, -0.5, engine=hip.ENGINE_VALU))
+    want = oracle.conv(typ, x[3:5], thr[3:5], qw_h, kn, 3, 3, 1, 1, -0.5)
+    assert got[3:5].cpu().numpy().tobytes() == np.ascontiguousarray(want).tobytes()
 
 
 @pytest.mark.parametrize("typ", [TNN, BNN], ids=lambda t: TYPE_NAMES[t])
