@@ -66,13 +66,6 @@ def roofline_for(engine_name, m, n, kw, ms, ops_per_pair=4):
     return roofline_mfma_f4(float(m) * n * kw * 64, ms) if engine_name == "mfma_f4" else roofline_valu(m, n, kw, ms, ops_per_pair)
 
 
-def auto_engine(lib, typ, m, n, kw):
-    """name of the engine whose units an AUTO product runs on: fp4 for the ones straight from packed rows (which need no scratch)"""
-    if lib.mm_scratch_bytes(lib.ENGINE_AUTO, typ, m, 1, 1, n, kw) == 0 and 64 * kw < 1 << 24:
-        return lib.ENGINE_NAMES[lib.ENGINE_MFMA_F4]
-    return lib.ENGINE_NAMES[lib.select_engine(typ, m, 1, 1, n, kw)]
-
-
 def parse():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -211,7 +204,7 @@ def small_gemm(torch, lib, m, n, k, reps=30):
         want = cpu.mm(TNN, a_h, b_h, m, 1, 1, n, kw, alpha)
         t_cpu.append(time.perf_counter() - t0)
     out = {"cpu_ms": round(min(t_cpu) * 1e3, 3), "cpu_gmacs": round(float(m) * n * k / min(t_cpu) / 1e9, 1),
-           "auto_engine": auto_engine(lib, TNN, m, n, kw)}
+           "auto_engine": lib.ENGINE_NAMES[lib.mm_auto_engine(TNN, m, 1, 1, n, kw)]}
     for eng, name in lib.ENGINE_NAMES.items():
         def run(eng=eng):
             lib.mm_engine(eng, TNN, a, b, m, 1, 1, n, kw, alpha, out=y, scratch=scratch)
@@ -624,7 +617,7 @@ def reference_gemm_sweep(torch, lib, reps=10):
         for _ in range(3):
             run()
         t = sorted(event_times(torch, run, reps))[reps // 2]
-        row = {"engine": auto_engine(lib, TNN, m, m, kw), "device_ms": round(t, 4),
+        row = {"engine": lib.ENGINE_NAMES[lib.mm_auto_engine(TNN, m, 1, 1, m, kw)], "device_ms": round(t, 4),
                "gmacs": round(float(m) * m * p / t / 1e6, 1)}
         tg, same = graph_times(torch, run, y, reps)
         row["device_ms_in_a_graph_of_10_calls"], row["graph_replays_same_bits_as_eager"] = round(tg, 4), same

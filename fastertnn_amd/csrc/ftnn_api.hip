@@ -1111,7 +1111,7 @@ int ftnn_mm(int type, const int64_t* d_a, const int64_t* d_b, int N, int OH, int
     return e == hipSuccess ? FTNN_OK : hip_fail(e, "mm launch");
 }
 
-// The engine of a product by the amount of work: what runs it where packed rows are not multiplied as they are (auto_from_rows),
+// The engine of a product by the amount of work: what runs it where packed rows are not multiplied as they are (auto_engine),
 // and what ftnn_select_engine answers.  Against the vector ALU the matrix cores with both operands expanded first pay from
 // about 2e9 lane-MACs on, by measurements on MI355X (m x m x 8m, whole calls from packed rows, device time): m = 512
 // (1.1e9 lane-MACs) 12.0 us on the vector ALU against 13.3 us on fp4, 576 (1.5e9) 13.9 / 13.0, 640 (2.1e9) 17.8 / 13.3, 768
@@ -1123,11 +1123,40 @@ static int select_engine(int type, int64_t M, int KN, int Kw) {
     return FTNN_ENGINE_VALU;
 }
 
-// AUTO multiplies the packed rows as they are (k_rows) wherever the fp4 engine does and wherever select_engine would take the
-// vector ALU: that one launch is ahead of it down to the smallest product (32 x 32 x 256 a tie at 2.5 us, 256 x 256 x 4096 3.5
-// against 4.8, 100000 x 10 x 512 7.8 against 9.8).  Left to the engines are large products and those beyond the kernel's limits.
-static bool auto_from_rows(int engine, int64_t M, int KN, int Kw) {
-    return mm_rows_within_limits(M, KN, Kw) && (engine == FTNN_ENGINE_VALU || mm_from_rows(M, KN, Kw));
+// Where the vector ALU stays ahead of the product from packed rows (k_rows) among the shapes that select_engine gives it.  A sweep
+// over 7036 products (1 x 1 x 256 to 10^6 x 64 x 4096, four types, row-major and NCHW), device time: rows are ahead on 3 of 4, by up
+// to a factor of 11; they lose where
+//   * a launch is nearly all there is: few results and short rows (49 x 24 x 256 BNN NCHW 3.2 us on the vector ALU / 4.1 from rows,
+//     196 x 96 x 1024 TNN NCHW 3.6 / 4.0); binary operands are cheap there, so BNN holds out longest (256 x 64 x 262144 63 / 69);
+//   * a product has a few columns, of which a tile's 32 are mostly empty (10000 x 1 x 4096 BNN 3.8 / 4.8);
+//   * a row is one group of words, which keeps three of a workgroup's four wavefronts idle, and the results are many (10^6 x 1 x
+//     256 TNN 37 / 54, 4000 x 1000 x 256 BTN 7.9 / 9.9, 802816 x 64 x 256 BNN NCHW 49 / 77).
+// With these lines 2 in 100 products of the sweep are more than 5 % slower than on the vector ALU (16 in 100 without them), and the
+// mean over all is 0.6 % from the better of the two (2.0).
+static bool valu_ahead_of_rows(int type, int64_t M, bool nchw, int KN, int Kw) {
+    const int64_t results = M * KN;
+    const int short_rows = type == kTNN ? 16 : type != kBNN ? 64 : M <= 256 && KN < 128 ? 4096 : 256;
+    if (KN <= 512 && M <= 20000 && results <= 32768 && Kw <= short_rows) return true;
+    if (nchw && KN <= 1000 && M <= 30000 && results <= 131072 && Kw <= 16) return true;
+    if (M >= 32 && M <= 30000 && M * Kw <= 640000 && ((KN <= 4 && Kw <= 64) || (KN <= 8 && Kw <= 16))) return true;
+    if (Kw > 4) return false;
+    if (nchw) return KN <= 1000 && (type != kBTN || M < 10000);
+    return type == kBTN ? KN > 96 : M >= 100000 && KN <= 64 && KN % 32 != 0;
+}
+
+// What AUTO runs: packed rows as they are (*rows, on the units of the fp4 engine) wherever the fp4 engine does and wherever they
+// are ahead of the vector ALU; else the engine by the amount of work.
+static int auto_engine(int type, int64_t M, bool nchw, int KN, int Kw, bool* rows) {
+    const int engine = select_engine(type, M, KN, Kw);
+    *rows = mm_rows_within_limits(M, KN, Kw) &&
+            (engine == FTNN_ENGINE_MFMA_F4 ? mm_from_rows(M, KN, Kw) : !valu_ahead_of_rows(type, M, nchw, KN, Kw));
+    return *rows ? FTNN_ENGINE_MFMA_F4 : engine;
+}
+
+int ftnn_mm_auto_engine(int type, int N, int OH, int OW, int KN, int K) {
+    if (N <= 0 || OH <= 0 || OW <= 0 || KN <= 0 || K <= 0 || K > kMaxRowWords) return FTNN_ENGINE_VALU;
+    bool rows;
+    return auto_engine(type, (int64_t)N * OH * OW, (int64_t)OH * OW > 1, KN, round4(K), &rows);
 }
 
 int ftnn_select_engine(int type, int N, int OH, int OW, int KN, int K) {
@@ -1140,8 +1169,9 @@ int64_t ftnn_mm_scratch_bytes(int engine, int type, int N, int OH, int OW, int K
     const int64_t M = (int64_t)N * OH * OW;
     const int Kw = round4(K);
     if (engine == FTNN_ENGINE_AUTO) {
-        engine = select_engine(type, M, KN, Kw);
-        if (auto_from_rows(engine, M, KN, Kw)) return 0;
+        bool rows;
+        engine = auto_engine(type, M, (int64_t)OH * OW > 1, KN, Kw, &rows);
+        if (rows) return 0;
     }
     if (engine != FTNN_ENGINE_MFMA_I8 && engine != FTNN_ENGINE_MFMA_F4) return 0;
     if (engine == FTNN_ENGINE_MFMA_F4) return mfma_f4_mm_scratch_bytes(M, KN, Kw);
@@ -1209,16 +1239,19 @@ int ftnn_mm_engine(int engine, int type, const int64_t* d_a, const int64_t* d_b,
     if (!aligned16(d_a) || !aligned16(d_b)) return fail(FTNN_EINVAL, "GEMM operands must be 16-byte aligned");
     if (M > 0x7fffffffLL) return fail(FTNN_EINVAL, "more than 2^31-1 output rows");
     if (engine == FTNN_ENGINE_AUTO) {
-        engine = select_engine(type, M, KN, Kw);
-        const bool scratch_ok = d_scratch && scratch_bytes >= ftnn_mm_scratch_bytes(engine, type, N, OH, OW, KN, K);
-        // packed rows as they are, also for larger products that come without scratch (4096 x 4096 x 32768 0.22 ms against 1.8
-        // on the vector ALU)
-        if (auto_from_rows(engine, M, KN, Kw) || (!scratch_ok && mm_rows_within_limits(M, KN, Kw))) {
+        bool rows;
+        engine = auto_engine(type, M, (int64_t)OH * OW > 1, KN, Kw, &rows);
+        // AUTO never fails for lack of scratch: a large product that comes without runs from the packed rows too
+        // (4096 x 4096 x 32768 0.22 ms against 1.8 on the vector ALU), beyond that kernel's limits on the engine that needs none
+        if (!rows && engine == FTNN_ENGINE_MFMA_F4 &&
+            !(d_scratch && scratch_bytes >= ftnn_mm_scratch_bytes(engine, type, N, OH, OW, KN, K))) {
+            rows = mm_rows_within_limits(M, KN, Kw);
+            engine = FTNN_ENGINE_VALU;
+        }
+        if (rows) {
             const hipError_t e = launch_mm_rows(type, d_a, d_b, M, OH * OW, KN, Kw, K_unpack, prelu_alpha, d_y, (hipStream_t)stream);
             return e == hipSuccess ? FTNN_OK : hip_fail(e, "mm launch");
         }
-        // AUTO never fails for lack of scratch: it falls back to the engine that needs none
-        if (engine != FTNN_ENGINE_VALU && !scratch_ok) engine = FTNN_ENGINE_VALU;
     }
     if (engine == FTNN_ENGINE_VALU)
         return ftnn_mm(type, d_a, d_b, N, OH, OW, KN, K, K_unpack, prelu_alpha, d_y, stream);

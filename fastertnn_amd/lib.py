@@ -34,6 +34,7 @@ _L.ftnn_mm.argtypes = [C.c_int, _vp, _vp] + [C.c_int] * 6 + [C.c_float, _vp, _vp
 _L.ftnn_mm_scratch_bytes.restype = C.c_int64
 _L.ftnn_mm_scratch_bytes.argtypes = [C.c_int] * 7
 _L.ftnn_select_engine.argtypes = [C.c_int] * 6
+_L.ftnn_mm_auto_engine.argtypes = [C.c_int] * 6
 _L.ftnn_mm_engine.argtypes = [C.c_int, C.c_int, _vp, _vp] + [C.c_int] * 6 + [C.c_float, _vp, _vp, C.c_int64, _vp]
 _L.ftnn_expand_bytes.restype = C.c_int64
 _L.ftnn_expand_bytes.argtypes = [C.c_int] * 3
@@ -79,7 +80,7 @@ EXPORTS = ("tnns_conv", "tnns_gemm", "t2r_p2_opt", "b2r", "mm_tnn", "mm_tbn", "m
            "ftnn_static_scratch_bytes",
            "ftnn_last_error", "ftnn_version", "ftnn_out_dim", "ftnn_row_words",
            "ftnn_pack_scratch_bytes", "ftnn_quantize_im2row", "ftnn_mm", "ftnn_conv",
-           "ftnn_pack_weights", "ftnn_pack_gemm_operand", "ftnn_select_engine", "ftnn_mm_scratch_bytes",
+           "ftnn_pack_weights", "ftnn_pack_gemm_operand", "ftnn_select_engine", "ftnn_mm_auto_engine", "ftnn_mm_scratch_bytes",
            "ftnn_mm_engine", "ftnn_expand_bytes", "ftnn_expand_rows", "ftnn_mm_expanded",
            "ftnn_conv_scratch_bytes", "ftnn_conv_engine", "ftnn_select_conv_engine",
            "ftnn_conv_static",
@@ -189,6 +190,10 @@ def conv_scratch_bytes(typ, n, c, h, w, kn, kh, kw, pad, stride):
 
 def select_engine(typ, n, oh, ow, kn, k):
     return int(_L.ftnn_select_engine(typ, n, oh, ow, kn, k))
+
+
+def mm_auto_engine(typ, n, oh, ow, kn, k):
+    return int(_L.ftnn_mm_auto_engine(typ, n, oh, ow, kn, k))
 
 
 def mm_scratch_bytes(engine, typ, n, oh, ow, kn, k):

@@ -40,8 +40,7 @@ int run(const char* version) {
         ftnn_check(ftnn_pack_gemm_operand(x.as<float>(), m, p, static_cast<int64_t*>(xp.reserve(elems / 4)), st), "ftnn_pack_gemm_operand");
         ftnn_check(ftnn_pack_gemm_operand(w.as<float>(), n, p, static_cast<int64_t*>(wp.reserve(elems / 4)), st), "ftnn_pack_gemm_operand");
         const int64_t sb = ftnn_mm_scratch_bytes(FTNN_ENGINE_AUTO, TNN, m, 1, 1, n, p_packed);
-        // without scratch AUTO multiplies the packed rows as they are, on the fp4 matrix cores
-        const int engine = sb == 0 ? FTNN_ENGINE_MFMA_F4 : ftnn_select_engine(TNN, m, 1, 1, n, p_packed);
+        const int engine = ftnn_mm_auto_engine(TNN, m, 1, 1, n, p_packed);
         void* d_scr = scratch.reserve((size_t)(sb > 0 ? sb : 16));
         float* out = static_cast<float*>(y.reserve((size_t)m * n * sizeof(float)));
         auto call = [&] {

@@ -194,9 +194,11 @@ FTNN_API int ftnn_mm(int type, const int64_t *d_a, const int64_t *d_b, int N, in
 #define FTNN_ENGINE_MFMA_I8 2 /* v_mfma_i32_32x32x32_i8 on expanded operands         */
 #define FTNN_ENGINE_MFMA_F4 3 /* v_mfma_f32_32x32x64_f8f6f4 (fp4); GEMM rows of at most 65536 words */
 
-/* the engine for this shape by its amount of work (never AUTO).  FTNN_ENGINE_AUTO takes it for products of 160 tiles of
- * 256 x 256 and more; smaller and narrower ones it runs on the fp4 matrix cores straight from their packed rows, whatever
- * this says: those are the shapes for which ftnn_mm_scratch_bytes(FTNN_ENGINE_AUTO, ...) is 0 while rows stay below 2^18 words. */
+/* the engine FTNN_ENGINE_AUTO runs this shape on: FTNN_ENGINE_MFMA_F4 also for the products that it multiplies straight from
+ * their packed rows, which are most below 160 tiles of 256 x 256 and need no scratch */
+FTNN_API int ftnn_mm_auto_engine(int type, int N, int OH, int OW, int KN, int K);
+
+/* the engine for this shape by its amount of work alone (never AUTO), for callers that keep operands expanded */
 FTNN_API int ftnn_select_engine(int type, int N, int OH, int OW, int KN, int K);
 
 /* device scratch, in bytes, that ftnn_mm_engine needs for `engine` (0 for the VALU engine; for AUTO 0 for products from packed

@@ -233,6 +233,29 @@ def test_layer_chain_refuses_unknown_flags():
     assert "flags" in lib._L.ftnn_last_error().decode()
 
 
+# (type, n, oh, ow, kernels, words) on either side of each line between packed rows and the vector ALU
+AUTO_LINES = [
+    # few results of short rows, by type and layout
+    ((0, 32, 1, 1, 512, 16), (0, 32, 1, 1, 512, 20)), ((0, 32, 1, 1, 512, 16), (0, 32, 1, 1, 513, 16)), ((0, 256, 1, 1, 128, 16), (0, 257, 1, 1, 128, 16)),
+    ((1, 256, 1, 1, 128, 64), (1, 256, 1, 1, 128, 68)), ((3, 256, 1, 1, 127, 4096), (3, 256, 1, 1, 127, 4100)), ((3, 256, 1, 1, 128, 256), (3, 256, 1, 1, 128, 260)),
+    ((0, 4, 7, 7, 668, 16), (0, 4, 7, 7, 669, 16)), ((0, 4, 7, 7, 668, 16), (0, 196, 1, 1, 668, 16)), ((0, 1, 7, 7, 1000, 16), (0, 1, 7, 7, 1001, 16)),
+    # few columns
+    ((0, 10000, 1, 1, 4, 64), (0, 10001, 1, 1, 4, 64)), ((0, 30000, 1, 1, 8, 16), (0, 30000, 1, 1, 9, 16)), ((0, 30000, 1, 1, 1, 16), (0, 30001, 1, 1, 1, 16)),
+    # one group of words
+    ((2, 1000, 1, 1, 1000, 4), (2, 1000, 1, 1, 1000, 8)), ((2, 4000, 1, 1, 97, 4), (2, 4000, 1, 1, 96, 4)), ((0, 100000, 1, 1, 48, 4), (0, 99999, 1, 1, 48, 4)),
+    ((0, 100000, 1, 1, 31, 4), (0, 100000, 1, 1, 32, 4)), ((3, 64, 28, 28, 64, 4), (3, 64, 28, 28, 64, 8)), ((2, 1, 99, 101, 100, 4), (2, 1, 100, 100, 100, 4)),
+]
+
+
+@pytest.mark.parametrize("valu,rows", AUTO_LINES)
+def test_auto_takes_the_engine_that_is_ahead(valu, rows):
+    import fastertnn_amd.lib as lib
+    assert lib.mm_auto_engine(*valu) == lib.ENGINE_VALU
+    assert lib.mm_auto_engine(*rows) == lib.ENGINE_MFMA_F4
+    assert lib.mm_scratch_bytes(lib.ENGINE_AUTO, *valu) == lib.mm_scratch_bytes(lib.ENGINE_AUTO, *rows) == 0
+    assert lib.select_engine(*valu) == lib.select_engine(*rows) == lib.ENGINE_VALU
+
+
 def test_products_from_packed_rows_ask_for_no_operand_scratch():
     """AUTO asks for none where the packed rows are multiplied as they are; the explicit fp4 engine keeps its demand: both operands as
     fragments below 160 tiles of 256 x 256, else in packed4 form, however narrow the product and beyond the other kernel's grid"""

@@ -1,6 +1,7 @@
-"""The matrix-core GEMM straight from packed rows (k_rows, what AUTO runs below 160 tiles of 256 x 256): every type,
-row-major and NCHW results, at the sizes where each of its wavefront tiles starts, ends or is ragged, with K from one group
-of words (fewer groups than wavefronts) to K tails, bit for bit against the oracle."""
+"""The matrix-core GEMM straight from packed rows (k_rows, what the explicit fp4 engine runs below 160 tiles of 256 x 256, and AUTO
+where the vector ALU is not ahead): every type, row-major and NCHW results, at the sizes where each of its wavefront
+tiles starts, ends or is ragged, with K from one group of words (fewer groups than wavefronts) to K tails, bit for bit
+against the oracle."""
 import numpy as np
 import pytest
 
@@ -32,15 +33,16 @@ def test_products_from_packed_rows(hip, oracle, typ, shape):
     print("case", TYPE_NAMES[typ], shape, flush=True)
     a, b = _operands(typ, m, kn, kw, 100 * typ + m + kn + kw)
     ku = 64 * kw - 5
-    # a sentinel past the result: nothing may be written there
-    y = torch.full((m * kn + 64,), float("nan"), dtype=torch.float32, device="cuda")
     a_d, b_d = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
     for alpha in (0.5, -0.25):
         want = oracle.mm(typ, a, b, n, oh, ow, kn, kw, alpha, ku)
-        hip.mm_engine(hip.ENGINE_AUTO, typ, a_d, b_d, n, oh, ow, kn, kw, alpha, ku, out=y)
-        got = y.cpu().numpy()
-        assert got[:m * kn].tobytes() == want.tobytes(), alpha
-        assert np.isnan(got[m * kn:]).all()
+        for engine in (hip.ENGINE_MFMA_F4, hip.ENGINE_AUTO):
+            # a sentinel past the result: nothing may be written there
+            y = torch.full((m * kn + 64,), float("nan"), dtype=torch.float32, device="cuda")
+            hip.mm_engine(engine, typ, a_d, b_d, n, oh, ow, kn, kw, alpha, ku, out=y)
+            got = y.cpu().numpy()
+            assert got[:m * kn].tobytes() == want.tobytes(), (engine, alpha)
+            assert np.isnan(got[m * kn:]).all()
 
 
 def test_rows_longer_than_the_fp4_engine_takes(hip):
@@ -82,7 +84,7 @@ def test_more_rows_than_the_smallest_tile_has_workgroups_for(hip):
     a_d = torch.randint(-2 ** 62, 2 ** 62, (m * kw,), dtype=torch.int64, device="cuda")
     b_d = torch.randint(-2 ** 62, 2 ** 62, (kw,), dtype=torch.int64, device="cuda")
     want = hip.mm_engine(hip.ENGINE_VALU, BNN, a_d, b_d, m, 1, 1, 1, kw, 0.5, 64 * kw)
-    got = hip.mm_engine(hip.ENGINE_AUTO, BNN, a_d, b_d, m, 1, 1, 1, kw, 0.5, 64 * kw)
+    got = hip.mm_engine(hip.ENGINE_MFMA_F4, BNN, a_d, b_d, m, 1, 1, 1, kw, 0.5, 64 * kw)
     assert torch.equal(got, want)
 
 
