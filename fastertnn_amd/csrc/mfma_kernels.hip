@@ -779,9 +779,9 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
 // and their im2row operand does not exist in memory.  This kernel therefore works on small tiles
 // with many wavefronts in flight and gathers its activation fragments itself:
 //   * a wavefront owns 64 kernels x 64 output pixels (2 x 2 MFMA blocks, 64 accumulator
-//     registers).  A workgroup is 4 wavefronts: S of them split the K loop of one tile (word w of
-//     the reference's K order (kh*KW + kw)*C_pack + ic goes to wavefront w % S of the tile), so
-//     it covers 4/S pixel tiles.  S = 1 for layers with 600 tiles or more (no exchange at all), 2 or
+//     registers).  A workgroup is 4 wavefronts: S of them split the K loop of one tile (each takes a
+//     run of the reference's K order (kh*KW + kw)*C_pack + ic; words dealt out in turn cost layers 0.2-0.6 us
+//     more, as every step then changes the tap), so it covers 4/S pixel tiles.  S = 1 for layers with 600 tiles or more (no exchange at all), 2 or
 //     4 where the tiles alone would leave most of the chip idle; the partial tiles then meet in
 //     LDS and each wavefront finishes 4/S of the tile's four blocks;
 //   * weights are the MFMA A side (rows = accumulator registers), pixels the B side (rows =
