@@ -1383,8 +1383,8 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
     // operand sizes: the buffer-load variants announce them in their descriptors
     const int64_t p4_bytes = (int64_t)N * cg.CP * cg.H * cg.W * 32, wf_bytes = (int64_t)((KN + 31) / 32) * KB * 1024;
     static const bool no_buf = getenv("FTNN_CONV_NO_BUFFER_LOADS") != nullptr;   // tuning aid
-    // an fp32 tile reaches over 64 kernels of its first image and as many more images as 64 pixels may touch
-    const int64_t y_span = ((int64_t)std::min(N - 1, 63 / OHW + 1) * KN + 64) * OHW * 4;
+    // an fp32 tile reaches over 64 kernels of its first image and as many more images as 64 pixels may touch, within the result
+    const int64_t y_span = std::min(((int64_t)std::min(N - 1, 63 / OHW + 1) * KN + 64) * OHW, M * KN) * 4;
     const bool buf = !no_buf && p4_bytes <= 0xf0000000LL && wf_bytes <= 0xf0000000LL && (qo.mode != 0 || y_span <= 0xf0000000LL);
     auto clip = [](int64_t v) { return (uint32_t)std::min<int64_t>(v, 0xffffffffLL); };
     const uint64_t wgs = (uint64_t)grid.x * grid.y;

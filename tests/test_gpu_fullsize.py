@@ -245,16 +245,16 @@ def test_large_layer_on_the_gemm_route_with_128x128_tiles(hip, oracle, typ):
 
 
 @pytest.mark.parametrize("typ", [TNN, BNN], ids=lambda t: TYPE_NAMES[t])
-@pytest.mark.parametrize("h", [4096, 8192])
-def test_chain_result_beyond_32_bit_offsets(hip, oracle, typ, h):
-    """the last layer of a chain, whose quantised input the layer before hands over, with an fp32 result of more than 4 GiB:
-    two images of 130 x h x 1024, whose tiles stay within 32-bit offsets (h = 4096) or do not (8192: one image alone
-    is larger).  Every element against the same layers one by one on the vector-ALU engine"""
+@pytest.mark.parametrize("n,h,w,kn", [(2, 4096, 1024, 130), (2, 8192, 1024, 130), (1, 8192, 4096, 3)])
+def test_chain_result_beyond_32_bit_offsets(hip, oracle, typ, n, h, w, kn):
+    """the last layer of a chain, whose quantised input the layer before hands over, with an fp32 result of more than 4 GiB whose
+    tiles stay within 32-bit offsets or do not (8192 x 1024: one image alone is larger), and with a small result of so
+    many pixels that 64 kernels of them would not.  Every element against the same layers one by one on the vector-ALU engine"""
     import torch
     from fastertnn_amd import synth
-    n, w, mid, kn = 2, 1024, 64, 130
-    assert n * kn * h * w * 4 > 2 ** 32
-    print("case", TYPE_NAMES[typ], h, flush=True)
+    mid = 64
+    assert (n * kn if n > 1 else 64) * h * w * 4 > 2 ** 32
+    print("case", TYPE_NAMES[typ], n, h, w, kn, flush=True)
     tern = typ == TNN
     thr = 0.5 if tern else 0.0
     rows = [(3, h, w, mid, 3, 3, 1, 1), (mid, h, w, kn, 1, 1, 0, 1)]
