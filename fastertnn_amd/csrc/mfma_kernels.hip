@@ -184,10 +184,7 @@ __device__ __forceinline__ void mfma(typename Acc<F4>::type& c, const uint4& a, 
 // it; the kernel waits for it by hand (s_waitcnt vmcnt before the barrier that publishes
 // the buffer).  M0 carries the LDS address; one wait state is required after writing M0.
 __device__ __forceinline__ void dma16(const uint4* gsrc, uint32_t lds_byte_addr) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                 :
-                 : "v"(gsrc), "s"(lds_byte_addr)
-                 : "memory", "m0");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(gsrc), "{m0}"(lds_byte_addr) : "memory");
 }
 
 // Epilogue of the GEMM kernels: r = acc - bias, then PReLU in the reference's form for the type (form 0 "f = r; if

@@ -85,20 +85,17 @@ __device__ __forceinline__ void unpack_half(const RawRow<TERN>& r, int i, v4u& e
 // LDS-direct loads: 16 bytes per lane from base + voff (base uniform); the 64 lanes land contiguously.  M0 holds the LDS
 // address (one wait state after writing it); the instruction's immediate offset moves the source and the LDS address
 // alike, so two loads into adjacent KiB share one M0 (v1 is then the source less 1024).  Inline asm, so that the compiler does
-// not order its own LDS reads against the loads; the kernel counts them by hand.  M0 is written and used within one statement and
-// declared: single loads, pairs and runs of four measured the same within 2 % from 256 x 256 to 3072 x 3072.
+// not order its own LDS reads against the loads; the kernel counts them by hand.  M0 is an operand, which the compiler sets in
+// front of the statement: single loads, pairs and runs of four measured the same within 2 % from 256 x 256 to 3072 x 3072.
 template <bool TWO>
 __device__ __forceinline__ void dma16(uint32_t lds_byte_addr, const char* b0, uint32_t v0, const char* b1, uint32_t v1) {
     if constexpr (TWO)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %3, %4 offset:1024"
+        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %3, %4 offset:1024"
                      :
-                     : "s"(lds_byte_addr), "v"(v0), "s"(b0), "v"(v1), "s"(b1)
-                     : "memory", "m0");
+                     : "{m0}"(lds_byte_addr), "v"(v0), "s"(b0), "v"(v1), "s"(b1)
+                     : "memory");
     else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     :
-                     : "s"(lds_byte_addr), "v"(v0), "s"(b0)
-                     : "memory", "m0");
+        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "{m0}"(lds_byte_addr), "v"(v0), "s"(b0) : "memory");
 }
 
 // Which tile a workgroup works on.  Workgroups go to the eight XCDs round-robin by number; XCD x takes the x-th eighth of the
