@@ -1032,7 +1032,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
                 }
                 const bool live = px0 + 32 * b + lr < M;
                 const int p0 = kn0 + 32 * a + 4 * h;
-                auto put = [&](auto whole) {
+                auto put = [&](auto whole, auto nt) {
+                    constexpr bool NT = decltype(nt)::value;
                     if constexpr (BUF) {
                         // a lane's part, and the kernel's row as a scalar; lanes past the pixels store beyond the buffer: nothing
                         const uint32_t vy =
@@ -1041,22 +1042,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
                         for (int e = 0; e < 16; e++) {
                             const int row = 8 * (e >> 2) + (e & 3);
                             if (decltype(whole)::value || p0 + row < KN)
-                                __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_uint(r[e]), brs_y, (int)vy, (int)((uint32_t)(row * 4) * (uint32_t)OHW), 0);
+                                __builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_uint(r[e]), brs_y, (int)vy, (int)((uint32_t)(row * 4) * (uint32_t)OHW), NT ? 2 : 0);
                         }
                     } else if (live) {
                         float* yq = Y + ((size_t)img[b] * KN + p0) * OHW + pix[b];
 #pragma unroll
                         for (int e = 0; e < 16; e++) {
                             const int row = 8 * (e >> 2) + (e & 3);
-                            if (decltype(whole)::value || p0 + row < KN) yq[(size_t)row * OHW] = r[e];
+                            if (decltype(whole)::value || p0 + row < KN) {
+                                if (NT) __builtin_nontemporal_store(r[e], yq + (size_t)row * OHW);
+                                else yq[(size_t)row * OHW] = r[e];
+                            }
                         }
                     }
                 };
                 // A whole block stores in a straight line.  With the check of the row beside the uniform one in a single
                 // condition, every store is a branch of its own: 0.3-0.8 us of a 4-12 us layer (1 x 64 x 56 x 56, 3 x 3:
                 // 5.5 against 4.9 us with the quantiser; 8 x 256 x 56 x 56 -> 128, 1 x 1: 12.2 against 11.4).
-                if (kn0 + 32 * a + 32 <= KN) put(std::true_type{});
-                else put(std::false_type{});
+                const bool inside = kn0 + 32 * a + 32 <= KN;
+                // A result beyond the Infinity Cache (see XcdOrder) is stored past the caches: 8 x 1024 x 1024 -> 130 behind a first
+                // layer, 3 x 3 1605 -> 1207 us, 1 x 1 1240 -> 1125; 40 x 128 x 128 -> 2048 the same within its spread (870-970).
+                if (xo.mask == 0) {
+                    if (inside) put(std::true_type{}, std::true_type{});
+                    else put(std::false_type{}, std::true_type{});
+                } else {
+                    if (inside) put(std::true_type{}, std::false_type{});
+                    else put(std::false_type{}, std::false_type{});
+                }
             }
         });
     } else {
