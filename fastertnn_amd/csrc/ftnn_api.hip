@@ -746,9 +746,9 @@ static float* host_mm(int type, int64_t* a, int64_t* b, int N, int OH, int OW, i
     return y;
 }
 
-// bytes of the two regions of the matrix-core layer path: P4 (32 bytes per pixel and 64 channels),
-// then the fp4 fragments of the weights
-int64_t conv_f4_p4_bytes(int N, int C, int H, int W) {
+// Bytes of the two regions of the matrix-core layer path: the quantised input (announced to callers at 32 bytes per pixel and 64
+// channels, of which the records take half), then the weights in engine form
+int64_t conv_f4_p2_bytes(int N, int C, int H, int W) {
     return ((int64_t)N * H * W * cpack_of(C) * 32 + 255) / 256 * 256;
 }
 
@@ -847,7 +847,7 @@ static int prepare_weights(int type, const int64_t* d_qw, int C, int KN, int KH,
             rows = d_wd;
         }
         int64_t* kept = keep_rows && fc_weights(C, KH, KW) ? reinterpret_cast<int64_t*>(static_cast<char*>(d_prepared) + tmp_off) : nullptr;
-        e = launch_mfma_expand(true, wt, rows, KN, conv_f4_weight_words(C, KH, KW), d_prepared, st, kept);
+        e = launch_expand_records(wt, dense_f4_applies(C, KH, KW), rows, KN, conv_f4_weight_words(C, KH, KW), d_prepared, st, kept);
         return e == hipSuccess ? FTNN_OK : hip_fail(e, "weight expansion launch");
     }
     if (dense) {
@@ -861,15 +861,15 @@ static int prepare_weights(int type, const int64_t* d_qw, int C, int KN, int KH,
 // operand region of the fp4 layer for this shape, whichever form it takes
 int64_t conv_f4_operand_bytes(int N, int C, int H, int W, int KH, int KW, int OH, int OW, int KN, int W_stride) {
     if (dense_f4_applies(C, KH, KW)) return conv_f4_dense_bytes(N, C, H, W, KH, KW, OH, OW);
-    int64_t bytes = conv_f4_p4_bytes(N, C, H, W);
+    int64_t bytes = conv_f4_p2_bytes(N, C, H, W);
     const int64_t M = (int64_t)N * OH * OW;
-    // the tile kernel's layout of the same input: a little larger where the width is no multiple of the stride
-    const int64_t t4 = quantize_f4_tiled_bytes(N, C, H, W, W_stride);
-    if (conv_f4_tile_route(M, KN, cpack_of(C), KH * KW, t4, 0, W_stride)) bytes = std::max(bytes, (t4 + 255) / 256 * 256);
+    // the tile kernel's layout of the same input: larger than the records where the width is no multiple of the stride
+    const int64_t t2 = quantize_f4_tiled_bytes(N, C, H, W, W_stride);
+    if (conv_f4_tile_route(M, KN, cpack_of(C), KH * KW, t2, 0, W_stride)) bytes = std::max(bytes, (t2 + 255) / 256 * 256);
     if (conv_f4_gemm_route(M, KN, cpack_of(C) * KH * KW)) {
         const int Kw = conv_f4_weight_words(C, KH, KW);
         const int64_t route = gemm_route_plane_bytes(N, C, H, W) + gemm_route_row_bytes(M, Kw) +
-                              (mfma_fragment_bytes(true, M, Kw) + 255) / 256 * 256;
+                              (record_block_bytes(M, Kw) + 255) / 256 * 256;
         if (route > bytes) bytes = route;
     }
     return bytes;
@@ -885,10 +885,10 @@ int conv_f4_weight_words(int C, int KH, int KW) {
     return round4(cpack_of(C) * KH * KW);
 }
 
-// the matrix-core layer with the weights already expanded (d_wf); d_p4 takes the quantised input
+// the matrix-core layer with the weights already expanded (d_wf); d_p2 takes the quantised input
 int conv_f4_expanded(int type, const float* d_x, const float* d_thr, const void* d_wf, int N, int C, int H,
                            int W, int KN, int KH, int KW, int H_pad, int W_pad, int H_stride, int W_stride,
-                           float prelu_alpha, void* d_p4, float* d_y, hipStream_t st, const QuantOut& qo) {
+                           float prelu_alpha, void* d_p2, float* d_y, hipStream_t st, const QuantOut& qo) {
     const int OH = out_dim(H, H_pad, KH, H_stride), OW = out_dim(W, W_pad, KW, W_stride);
     const bool act_ternary = (type == kTNN || type == kTBN);
     hipError_t e = hipSuccess;
@@ -904,28 +904,28 @@ int conv_f4_expanded(int type, const float* d_x, const float* d_thr, const void*
         }
         int T, Kd;
         dense_applies(C, KH, KW, &T, &Kd);
-        void* d_a4 = static_cast<char*>(d_p4) + dense_f4_pq_bytes(N, H, W);
-        e = launch_dense_rows_f4(act_ternary, d_x, d_thr, N, C, H, W, H_pad, W_pad, KH, KW, H_stride, W_stride, d_p4,
-                                 d_a4, st);
+        void* d_a2 = static_cast<char*>(d_p2) + dense_f4_pq_bytes(N, H, W);
+        e = launch_dense_rows_f4(act_ternary, d_x, d_thr, N, C, H, W, H_pad, W_pad, KH, KW, H_stride, W_stride, d_p2,
+                                 d_a2, st);
         if (e != hipSuccess) return hip_fail(e, "fp4 dense rows launch");
         const ConvGeom cg = {OH, OW, Kd, OH, OW, 1, Kd, 0, 0, 1, 1,
                              make_fastdiv((uint32_t)OW), make_fastdiv((uint32_t)Kd), make_fastdiv(1u)};
-        e = launch_conv_f4(type, d_a4, d_wf, cg, N, KN, C * KH * KW, prelu_alpha, d_y, st, qo);
+        e = launch_conv_f4(type, d_a2, d_wf, cg, N, KN, C * KH * KW, prelu_alpha, d_y, st, qo);
         return e == hipSuccess ? FTNN_OK : hip_fail(e, "fp4 conv launch");
     }
     const int64_t M = (int64_t)N * OH * OW;
     const bool tiles = d_x && qo.mode == 0 && conv_f4_tile_route(M, KN, cpack_of(C), KH * KW, quantize_f4_tiled_bytes(N, C, H, W, W_stride), W_pad, W_stride);
     if (d_x && qo.mode == 0 && !tiles && conv_f4_gemm_route(M, KN, cpack_of(C) * KH * KW)) {
         const int Kw = conv_f4_weight_words(C, KH, KW);
-        char* base = static_cast<char*>(d_p4);
+        char* base = static_cast<char*>(d_p2);
         int64_t* d_rows = reinterpret_cast<int64_t*>(base + gemm_route_plane_bytes(N, C, H, W));
         void* d_af = reinterpret_cast<char*>(d_rows) + gemm_route_row_bytes(M, Kw);
         e = launch_quantize_im2row(act_ternary, d_x, d_thr, N, C, H, W, H_pad, W_pad, KH, KW, H_stride, W_stride, d_rows,
                                    base, st);
         if (e != hipSuccess) return hip_fail(e, "quantise + im2row launch");
-        e = launch_mfma_expand(true, act_ternary, d_rows, (int)M, Kw, d_af, st);
+        e = launch_expand_records(act_ternary, false, d_rows, (int)M, Kw, d_af, st);
         if (e != hipSuccess) return hip_fail(e, "row expansion launch");
-        e = launch_mfma_gemm(true, type, d_af, d_wf, M, OH * OW, KN, Kw, C * KH * KW, prelu_alpha, d_y, st);
+        e = launch_records_gemm(type, d_af, d_wf, M, OH * OW, KN, Kw, C * KH * KW, prelu_alpha, d_y, st);
         return e == hipSuccess ? FTNN_OK : hip_fail(e, "matrix-core GEMM launch");
     }
     const ConvGeom cg = {H, W, cpack_of(C), OH, OW, KW, cpack_of(C) * KH * KW, H_pad, W_pad, H_stride, W_stride,
@@ -933,14 +933,14 @@ int conv_f4_expanded(int type, const float* d_x, const float* d_thr, const void*
     // many tiles, fp32 input and result: workgroup tiles staged through LDS, gathered from the quantised input in the
     // tile kernel's own layout
     if (tiles) {
-        e = launch_quantize_f4_tiled(act_ternary, d_x, d_thr, N, C, H, W, W_stride, d_p4, st);
+        e = launch_quantize_f4_tiled(act_ternary, d_x, d_thr, N, C, H, W, W_stride, d_p2, st);
         if (e != hipSuccess) return hip_fail(e, "fp4 quantize launch");
-        e = launch_conv_f4_tiles(type, d_p4, d_wf, cg, N, KN, C * KH * KW, prelu_alpha, d_y, st);
+        e = launch_conv_f4_tiles(type, d_p2, d_wf, cg, N, KN, C * KH * KW, prelu_alpha, d_y, st);
         return e == hipSuccess ? FTNN_OK : hip_fail(e, "fp4 conv tile launch");
     }
-    if (d_x) e = launch_quantize_f4(act_ternary, d_x, d_thr, N, C, H, W, d_p4, st);   // else d_p4 is ready
+    if (d_x) e = launch_quantize_f4(act_ternary, d_x, d_thr, N, C, H, W, d_p2, st);   // else d_p2 is ready
     if (e != hipSuccess) return hip_fail(e, "fp4 quantize launch");
-    e = launch_conv_f4(type, d_p4, d_wf, cg, N, KN, C * KH * KW, prelu_alpha, d_y, st, qo);
+    e = launch_conv_f4(type, d_p2, d_wf, cg, N, KN, C * KH * KW, prelu_alpha, d_y, st, qo);
     return e == hipSuccess ? FTNN_OK : hip_fail(e, "fp4 conv launch");
 }
 
@@ -1200,7 +1200,7 @@ int ftnn_expand_rows(int engine, int ternary, const int64_t* d_rows, int rows, i
         return fail(FTNN_EINVAL, "null or misaligned device pointer");
     hipError_t e = engine == FTNN_ENGINE_MFMA_F4
                        ? launch_mfma_pack4(ternary != 0, d_rows, rows, round4(K), d_out, (hipStream_t)stream)
-                       : launch_mfma_expand(false, ternary != 0, d_rows, rows, round4(K), d_out, (hipStream_t)stream);
+                       : launch_mfma_expand(ternary != 0, d_rows, rows, round4(K), d_out, (hipStream_t)stream);
     return e == hipSuccess ? FTNN_OK : hip_fail(e, "expand launch");
 }
 
@@ -1219,7 +1219,7 @@ int ftnn_mm_expanded(int engine, int type, const void* d_a_exp, const void* d_b_
     hipError_t e = engine == FTNN_ENGINE_MFMA_F4
                        ? launch_mfma_gemm_packed4(type, d_a_exp, d_b_exp, M, OH * OW, KN, round4(K), K_unpack, prelu_alpha, d_y,
                                                   (hipStream_t)stream)
-                       : launch_mfma_gemm(false, type, d_a_exp, d_b_exp, M, OH * OW, KN, round4(K), K_unpack, prelu_alpha, d_y,
+                       : launch_mfma_gemm(type, d_a_exp, d_b_exp, M, OH * OW, KN, round4(K), K_unpack, prelu_alpha, d_y,
                                           (hipStream_t)stream);
     return e == hipSuccess ? FTNN_OK : hip_fail(e, "mfma gemm launch");
 }
@@ -1299,7 +1299,7 @@ int ftnn_conv_engine(int engine, int type, const float* d_x, const float* d_thr,
             if (e != hipSuccess) return hip_fail(e, "dense weights launch");
             rows = d_wd;
         }
-        e = launch_mfma_expand(true, w_ternary, rows, KN, Kw, d_wf, (hipStream_t)stream);
+        e = launch_expand_records(w_ternary, dense_f4_applies(C, KH, KW), rows, KN, Kw, d_wf, (hipStream_t)stream);
         if (e != hipSuccess) return hip_fail(e, "weight expansion launch");
         return conv_f4_expanded(type, d_x, d_thr, d_wf, N, C, H, W, KN, KH, KW, H_pad, W_pad, H_stride, W_stride,
                                 prelu_alpha, d_scratch, d_y, (hipStream_t)stream, QuantOut());

@@ -72,10 +72,27 @@ struct ConvGeom {
     FastDiv dOW, dCP, dKW;
 };
 
+// Quantised layer operands: two bits per lane, a record of 16 bytes per 64 lanes ("P2").
+//
+// A lane in {-1, 0, +1} is an E2M1 nibble 0xA / 0x0 / 0x2, which uses bits 1 (not zero) and 3 (sign) only, so two dwords of
+// nibbles D0, D1 share one dword P = D0 | D1 >> 1 and come apart as D0 = P & 0xAAAAAAAA, D1 = (P << 1) & 0xAAAAAAAA: 1.5 vector
+// instructions per dword beside the multiplies, for half the bytes through memory, L1 and LDS and half the loads.  The
+// layer kernels are bound by those bytes (64 per cycle and compute unit come back from the L1) and not by instructions.
+// Against nibbles at four bits: see the layer kernels.
+//
+// Lane c = 32 a + 8 q + 4 h + i of a record sits in dword 2 h + a, byte q, nibble i / 2; even i in bits 1 and 3, odd i in bits
+// 0 and 2.  That is the order in which an accumulator tile holds its kernels (a: block, h: lane half, 4 q + i: register), so
+// an epilogue hands its results over without exchanging lanes.  Dwords 0, 1 feed one multiply, dwords 2, 3 the next.
+// Few-channel first layers keep their lanes in plain order (`natural`: dword j holds lanes 16 j .. 16 j + 7 as D0 and the
+// next eight as D1) in both operands: any order serves as long as both have it.
+constexpr uint32_t kP2Mask = 0xAAAAAAAAu;   // D0 of a dword
+constexpr uint32_t kP2Plus = 0x33333333u;   // +1 in every lane: the padding of binary activations
+__device__ __forceinline__ uint32_t p2_join(uint32_t d0, uint32_t d1) { return d0 | d1 >> 1; }
+
 // Fused hand-over to a following fp4 layer: instead of the fp32 result, a GEMM kernel writes the
-// next layer's quantised input, P4[n][ceil(KN/64)][pixel][32 bytes] (see launch_quantize_f4), from
+// next layer's quantised input, P2[n][ceil(KN/64)][pixel][16 bytes] (see launch_quantize_f4), from
 // the same fp32 values: mode 1 = ternary with threshold t (strict compares), 2 = binary, 0 = off.
-// Kernels past KN in the last 64-channel word get the padding nibble.
+// Kernels past KN in the last 64-channel word get the padding lane.
 //
 // cut = true: the thresholds as cuts on the integer r in front of PReLU, found on the host (make_quant_out).  PReLU does
 // not fall for a slope >= 0, so r -> sign is a staircase:
@@ -85,7 +102,7 @@ struct ConvGeom {
 // instructions, clamp(a - width, 0, 1) = p and med3(a, -1, p) (binary: one, med3(a, -1/2, 1/2)), before two of them
 // become two nibbles in one conversion (v_cvt_scalef32_pk_fp4_f32).  Other slopes and thresholds run PReLU and compare.
 struct QuantOut {
-    void* p4 = nullptr;
+    void* p2 = nullptr;
     float t = 0.0f;       // the next layer's threshold
     int mode = 0;
     bool cut = false;
@@ -94,7 +111,7 @@ struct QuantOut {
 constexpr int kMaxCutSum = 1 << 22;   // largest |r| the cuts are made for: r - lo and its half steps stay exact in fp32
 
 // alpha, form0: the producing layer's PReLU; max_sum: bound of |r|
-QuantOut make_quant_out(void* p4, int mode, float t, float alpha, int64_t max_sum);
+QuantOut make_quant_out(void* p2, int mode, float t, float alpha, int64_t max_sum);
 
 // the E2M1 nibble of one value under QuantOut mode 1 / 2 (src/tnns/ternarize2row_avx2.c:443-449,
 // src/tnns/binarize2row_avx2.c:19-21); `live` = false gives the padding lane of that mode
@@ -125,24 +142,6 @@ __device__ __forceinline__ uint32_t pack_fp4x8(const float* z) {
     return d;
 }
 
-// Lanes l and l ^ 32 hold the nibbles of one pixel for a 32-kernel block, lane half h those of kernels 8 q + 4 h + {0..3},
-// as d.x (q = 0, 1) and d.y (q = 2, 3), 16 bits per q; the block's dword q is the pair's 16 bits side by side.
-// v_permlane32_swap exchanges the upper half of its first operand with the lower half of its second.
-//
-// one block: lane half h returns dwords 2 h and 2 h + 1
-__device__ __forceinline__ uint2 exchange_halves(const uint2& d) {
-    const auto r = __builtin_amdgcn_permlane32_swap(d.x, d.y, false, false);
-    // lanes 0..31: r[0] = own d.x, r[1] = d.x of lane + 32; lanes 32..63: r[0] = d.y of lane - 32, r[1] = own d.y
-    return make_uint2((r[0] & 0xffffu) | (r[1] << 16), (r[0] >> 16) | (r[1] & 0xffff0000u));
-}
-// two blocks (the pixel's 64 kernels): lane half h returns the 16 bytes of block h
-__device__ __forceinline__ uint4 exchange_blocks(const uint2& b0, const uint2& b1) {
-    const auto r = __builtin_amdgcn_permlane32_swap(b0.x, b1.x, false, false);
-    const auto s = __builtin_amdgcn_permlane32_swap(b0.y, b1.y, false, false);
-    return make_uint4((r[0] & 0xffffu) | (r[1] << 16), (r[0] >> 16) | (r[1] & 0xffff0000u),
-                      (s[0] & 0xffffu) | (s[1] << 16), (s[0] >> 16) | (s[1] & 0xffff0000u));
-}
-
 // PReLU in the reference's two forms: "f <= 0 -> f *= alpha" (TNN, src/tnns/mm_p2_final_tnn_avx2.c:204-208; a zero
 // becomes 0 * alpha) and "r >= 0 ? r : alpha * r" (the others, src/tnns/mm_p2_final_tbn_avx2.c:73)
 template <bool FORM0>
@@ -159,33 +158,32 @@ __device__ __forceinline__ float acc_init(const QuantOut& qo, float bias) {
 }
 
 // One 32-kernel block of a pixel under the hand-over.  v[e] = this lane's 16 accumulators (started at acc_init), kernel
-// kbase + 8 (e / 4) + 4 h + e % 4 (h = lane half).  Returns the nibbles as exchange_halves / exchange_blocks take them.
+// kbase + 8 (e / 4) + 4 h + e % 4 (h = lane half).  Returns dword 2 h + a of the pixel's record (a: the block's number in its word).
 template <bool FORM0, int QMODE>
-__device__ __forceinline__ uint2 hand_over_block(const v16f& v, float alpha, const QuantOut& qo, int kbase, int h, int KN) {
+__device__ __forceinline__ uint32_t hand_over_block(const v16f& v, float alpha, const QuantOut& qo, int kbase, int h, int KN) {
     const bool whole = kbase + 32 <= KN;   // wave-uniform: the block holds real kernels only
     if (qo.cut) {
-        float z[16];
+        float z[16];   // even registers, then odd ones
 #pragma unroll
         for (int e = 0; e < 16; e++) {
-            if (QMODE == 1) z[e] = __builtin_amdgcn_fmed3f(v[e], -1.0f, __builtin_amdgcn_fmed3f(v[e] - qo.width, 0.0f, 1.0f));
-            else z[e] = __builtin_amdgcn_fmed3f(v[e], -0.5f, 0.5f);
+            float& d = z[(e >> 1) + 8 * (e & 1)];
+            if (QMODE == 1) d = __builtin_amdgcn_fmed3f(v[e], -1.0f, __builtin_amdgcn_fmed3f(v[e] - qo.width, 0.0f, 1.0f));
+            else d = __builtin_amdgcn_fmed3f(v[e], -0.5f, 0.5f);
         }
         if (!whole) {   // kernels past KN hold the padding lane
 #pragma unroll
-            for (int e = 0; e < 16; e++)
-                z[e] = kbase + 8 * (e >> 2) + 4 * h + (e & 3) < KN ? z[e] : (QMODE == 1 ? 0.0f : 0.5f);
+            for (int e = 0; e < 16; e++) {
+                float& d = z[(e >> 1) + 8 * (e & 1)];
+                d = kbase + 8 * (e >> 2) + 4 * h + (e & 3) < KN ? d : (QMODE == 1 ? 0.0f : 0.5f);
+            }
         }
-        return make_uint2(pack_fp4x8<QMODE>(z), pack_fp4x8<QMODE>(z + 8));
+        return p2_join(pack_fp4x8<QMODE>(z), pack_fp4x8<QMODE>(z + 8));
     }
-    uint32_t half[4];
+    uint32_t d[2] = {0u, 0u};
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-        half[g] = 0u;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            half[g] |= quant_nibble(prelu_ref<FORM0>(v[4 * g + i], alpha), qo.t, QMODE == 1, kbase + 8 * g + 4 * h + i < KN) << (4 * i);
-    }
-    return make_uint2(half[0] | (half[1] << 16), half[2] | (half[3] << 16));
+    for (int e = 0; e < 16; e++)
+        d[e & 1] |= quant_nibble(prelu_ref<FORM0>(v[e], alpha), qo.t, QMODE == 1, kbase + 8 * (e >> 2) + 4 * h + (e & 3) < KN) << (4 * (e >> 1));
+    return p2_join(d[0], d[1]);
 }
 
 // record a failure text for ftnn_last_error(); returns `code`
@@ -216,9 +214,9 @@ hipError_t launch_mm_implicit(int type, const void* d_p, const int64_t* d_b, con
 hipError_t launch_quantize(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
                            void* d_p, hipStream_t st);
 
-// quantise only, into fp4 nibbles: fp32 NCHW -> P4[n][C_pack][pixel][32 bytes] (operand of launch_conv_f4)
+// quantise only, into two-bit records: fp32 NCHW -> P2[n][C_pack][pixel][16 bytes] (operand of launch_conv_f4)
 hipError_t launch_quantize_f4(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
-                              void* d_p4, hipStream_t st);
+                              void* d_p2, hipStream_t st);
 // quantise only, into Packing-2 rows: fp32 [N][C] -> N rows (activations of a fully connected layer as launch_mm_rows reads them)
 hipError_t launch_quantize_rows(bool ternary, const float* d_x, const float* d_thr, int N, int C, int64_t* d_out, hipStream_t st);
 
@@ -230,8 +228,8 @@ hipError_t launch_dense_weights(bool ternary, const int64_t* d_qw, int KN, int C
                                 int64_t* d_out, hipStream_t st);
 
 // the same for the fp4 layer kernel (C <= 8): quantise to one nibble dword per pixel (d_pq,
-// dense_f4_pq_bytes), then string T taps per 64-lane word into A4[n][Kd][output pixel][32 bytes] (d_a4), the
-// operand of launch_conv_f4 for a 1x1 layer with C_pack = Kd over the OH x OW output pixels
+// dense_f4_pq_bytes), then string T taps per 64-lane word into A2[n][Kd][output pixel][16 bytes] (d_a2, natural lane
+// order), the operand of launch_conv_f4 for a 1x1 layer with C_pack = Kd over the OH x OW output pixels
 bool dense_f4_applies(int C, int KH, int KW);
 // stem_kernels.hip: the same layer in one kernel (fp32 input -> result, the rows never stored) where its input
 // patch fits the LDS: bytes of LDS it needs, 0 = does not apply
@@ -242,16 +240,27 @@ hipError_t launch_stem_f4(int type, const float* d_x, const float* d_thr, const 
 int64_t dense_f4_pq_bytes(int N, int H, int W);
 hipError_t launch_dense_rows_f4(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
                                 int H_pad, int W_pad, int kH, int kW, int H_stride, int W_stride, void* d_pq,
-                                void* d_a4, hipStream_t st);
+                                void* d_a2, hipStream_t st);
 
-// ---- mfma_kernels.hip: matrix-core formulation (int8 or fp4 operands expanded into d_scratch) ----
+// ---- mfma_kernels.hip: matrix-core formulation ----
+// Bytes of an operand brought into engine form: int8 fragments (1 KiB per 32 rows and half word), or what a layer's weights are
+// given (1 KiB per 32 rows and word; their records take half of it)
 int64_t mfma_fragment_bytes(bool f4, int64_t rows, int Kw);
-hipError_t launch_mfma_expand(bool f4, bool ternary, const int64_t* d_rows, int rows, int Kw, void* d_out,
-                              hipStream_t st, int64_t* d_kept = nullptr /* also copies the rows there */);
-hipError_t launch_mfma_gemm(bool f4, int type, const void* d_af, const void* d_bf, int64_t M, int OHW, int KN,
+// packed rows -> int8 fragments
+hipError_t launch_mfma_expand(bool ternary, const int64_t* d_rows, int rows, int Kw, void* d_out, hipStream_t st);
+// packed rows -> record blocks, 1 KiB [row block of 32][pair of K words][lane l = (word of the pair l / 32, row l % 32)][16 bytes]:
+// weights of the fp4 layer kernels, and im2row rows of the layers' GEMM route.  natural: lane order of few-channel first layers;
+// d_kept: also copies the rows there
+int64_t record_block_bytes(int64_t rows, int Kw);
+hipError_t launch_expand_records(bool ternary, bool natural, const int64_t* d_rows, int rows, int Kw, void* d_out, hipStream_t st,
+                                 int64_t* d_kept = nullptr);
+hipError_t launch_mfma_gemm(int type, const void* d_af, const void* d_bf, int64_t M, int OHW, int KN,
                             int Kw, int K_unpack, float alpha, float* d_y, hipStream_t st);
+// the layers' GEMM route: both operands as record blocks
+hipError_t launch_records_gemm(int type, const void* d_a, const void* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
+                               float alpha, float* d_y, hipStream_t st);
 // the fp4 GEMM's own operand form, two bits per lane ("packed4"): what ftnn_expand_rows / ftnn_mm_expanded /
-// ftnn_mm_engine use for FTNN_ENGINE_MFMA_F4 (the layer kernels keep the plain fragments above)
+// ftnn_mm_engine use for FTNN_ENGINE_MFMA_F4
 int64_t mfma_packed4_bytes(int64_t rows, int Kw);
 hipError_t launch_mfma_pack4(bool ternary, const int64_t* d_rows, int rows, int Kw, void* d_out, hipStream_t st);
 hipError_t launch_mfma_gemm_packed4(int type, const void* d_ac, const void* d_bc, int64_t M, int OHW, int KN, int Kw, int K_unpack,
@@ -270,35 +279,34 @@ bool mm_rows_within_limits(int64_t M, int KN, int Kw);
 hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
                           float alpha, float* d_y, hipStream_t st);
 
-// conv layer on the fp4 matrix cores: activations from launch_quantize_f4, weights as the fp4 fragments
-// launch_mfma_expand(true, ...) makes of the packed weight rows (Kw = round4(cg.K) words per row)
-hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const ConvGeom& cg, int N, int KN,
+// conv layer on the fp4 matrix cores: activations from launch_quantize_f4, weights as the record blocks
+// launch_expand_records makes of the packed weight rows (Kw = round4(cg.K) words per row)
+hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const ConvGeom& cg, int N, int KN,
                           int K_unpack, float alpha, float* d_y, hipStream_t st, const QuantOut& qo = QuantOut());
 
 
-// the same layer as workgroup tiles of 128 x 128 or 256 x 256 staged through LDS (the GEMM kernel with its activation
-// fragments gathered from T4, the quantised input in the layout of launch_quantize_f4_tiled): for layers with
-// conv_f4_tile_route() and an fp32 result
+// the same layer as workgroup tiles of 64 x 64 to 256 x 256 staged through LDS (the activation records gathered from T2, the
+// quantised input in the layout of launch_quantize_f4_tiled): for layers with conv_f4_tile_route() and an fp32 result
 int64_t quantize_f4_tiled_bytes(int N, int C, int H, int W, int W_stride);
 hipError_t launch_quantize_f4_tiled(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
-                                    int W_stride, void* d_t4, hipStream_t st);
-bool conv_f4_tile_route(int64_t M, int KN, int CP, int taps, int64_t t4_bytes, int W_pad, int W_stride);
-hipError_t launch_conv_f4_tiles(int type, const void* d_p4, const void* d_wf, const ConvGeom& cg, int N, int KN,
+                                    int W_stride, void* d_t2, hipStream_t st);
+bool conv_f4_tile_route(int64_t M, int KN, int CP, int taps, int64_t t2_bytes, int W_pad, int W_stride);
+hipError_t launch_conv_f4_tiles(int type, const void* d_t2, const void* d_wf, const ConvGeom& cg, int N, int KN,
                                 int K_unpack, float alpha, float* d_y, hipStream_t st);
 
 // ---- ftnn_api.hip ----  (arguments already validated)
-// The fp4 layer with weights expanded beforehand (d_wf: launch_mfma_expand(true, ...) of the packed rows).
-// d_x != null: the input is quantised into d_p4 (N*H*W*C_pack*32 bytes) first; d_x == null: d_p4 already
+// The fp4 layer with weights expanded beforehand (d_wf: launch_expand_records of the packed rows).
+// d_x != null: the input is quantised into d_p2 (N*H*W*C_pack*16 bytes) first; d_x == null: d_p2 already
 // holds it (written by the previous layer through its QuantOut).  qo.mode != 0: d_y is not written.
 int conv_f4_expanded(int type, const float* d_x, const float* d_thr, const void* d_wf, int N, int C, int H,
                      int W, int KN, int KH, int KW, int H_pad, int W_pad, int H_stride, int W_stride,
-                     float prelu_alpha, void* d_p4, float* d_y, hipStream_t st, const QuantOut& qo);
+                     float prelu_alpha, void* d_p2, float* d_y, hipStream_t st, const QuantOut& qo);
 // the vector-ALU layer; d_scratch as for ftnn_conv
 // (weights_prepared: for a few-channel layer d_qw already holds the re-packed rows of launch_dense_weights)
 int conv_valu(int type, const float* d_x, const float* d_thr, const int64_t* d_qw, int N, int C, int H, int W,
               int KN, int KH, int KW, int H_pad, int W_pad, int H_stride, int W_stride, float prelu_alpha,
               void* d_scratch, float* d_y, hipStream_t st, const QuantOut& qo, bool weights_prepared);
-// bytes of the fp4 layer's operand region (d_p4 above) for this shape, rounded up to 256: P4, or for a
+// bytes of the fp4 layer's operand region (d_p2 above) for this shape, rounded up to 256: P2, or for a
 // few-channel layer the nibble pixels and dense rows
 int64_t conv_f4_operand_bytes(int N, int C, int H, int W, int KH, int KW, int OH, int OW, int KN, int W_stride);
 // words per row of the weights as the fp4 layer reads them (the dense re-packing shortens them)

@@ -4,7 +4,7 @@
 // Between two layers the reference holds fp32 activations (its tnns_conv returns them and the next
 // call quantises them again).  Here a layer that feeds a layer on the fp4 matrix-core engine
 // quantises its own results in its epilogue, with the next layer's thresholds, and writes that
-// layer's operand (P4) directly: the fp32 tensor in between (e.g. 103 MB after a batch-32 stem)
+// layer's operand (P2) directly: the fp32 tensor in between (e.g. 103 MB after a batch-32 stem)
 // is neither written nor read, and the next layer needs no quantise launch.  The values compared
 // against the thresholds are the same fp32 numbers, so the chain's output is unchanged.
 #include <stdlib.h>
@@ -28,7 +28,7 @@ struct NetPart {
     // so that an image lies at the same place of its buffer in all layers of that size.  The XCD that works on it
     // (XcdOrder) then writes lines that no other XCD's L2 holds; with two buffers for all sizes the layer behind the
     // stride-2 one of the ResNet-18-like chain took 9.7 instead of 7.6 us at batch 32.
-    std::vector<void*> d_p4;
+    std::vector<void*> d_p2;
     void* d_scratch = nullptr;              // work space of the vector-ALU layers
 };
 
@@ -37,8 +37,8 @@ struct ftnn_net {
     std::vector<ftnn_layer_t> layers;
     std::vector<int> OH, OW;
     std::vector<float*> d_thr;       // per layer: batch copies of its threshold
-    std::vector<void*> d_wf;         // per layer on the fp4 engine: its weights as matrix-core fragments
-    std::vector<int> p4_buf;         // per layer: which of a part's d_p4 its quantised input lies in (-1: none)
+    std::vector<void*> d_wf;         // per layer on the fp4 engine: its weights as record blocks
+    std::vector<int> p2_buf;         // per layer: which of a part's d_p2 its quantised input lies in (-1: none)
     std::vector<char> rereads;       // per layer: its input is the leading part of the previous layer's fp32 output
     std::vector<NetPart> parts;      // one, or two that run concurrently
     hipStream_t side = nullptr;      // stream of the second part
@@ -56,9 +56,9 @@ namespace ftnn {
 
 // The cuts are found with the very fp32 products and compares the kernels would make (r * alpha rounds the same on both
 // sides), by bisection over the integers r: PReLU(r) does not fall with r for a slope >= 0.
-QuantOut make_quant_out(void* p4, int mode, float t, float alpha, int64_t max_sum) {
+QuantOut make_quant_out(void* p2, int mode, float t, float alpha, int64_t max_sum) {
     QuantOut q;
-    q.p4 = p4;
+    q.p2 = p2;
     q.mode = mode;
     q.t = t;
     const bool finite = alpha >= 0.0f && alpha <= 3.0e38f && t >= -3.0e38f && t <= 3.0e38f;
@@ -86,30 +86,30 @@ namespace {
 
 using namespace ftnn;
 
-// layer i of one part; `in` / `p4_ready` carry the part's state from layer to layer
-int enqueue_layer(ftnn_net* net, const NetPart& part, int i, const float*& in, bool& p4_ready, float* d_y,
+// layer i of one part; `in` / `p2_ready` carry the part's state from layer to layer
+int enqueue_layer(ftnn_net* net, const NetPart& part, int i, const float*& in, bool& p2_ready, float* d_y,
                   hipStream_t st) {
     const int n = (int)net->layers.size();
     const ftnn_layer_t& L = net->layers[i];
-    // the next layer takes a quantised hand-over if it is an fp4 layer that reads P4 (not a few-channel one)
+    // the next layer takes a quantised hand-over if it is an fp4 layer that reads P2 (not a few-channel one)
     const bool next_f4 = i + 1 < n && net->d_wf[i + 1] && !net->rereads[i + 1] &&
                          !dense_f4_applies(net->layers[i + 1].C, net->layers[i + 1].KH, net->layers[i + 1].KW);
     QuantOut qo;
     if (next_f4) {
         const int nt = net->layers[i + 1].type;
-        qo = make_quant_out(part.d_p4[(size_t)net->p4_buf[i + 1]], (nt == kTNN || nt == kTBN) ? 1 : 2, net->layers[i + 1].threshold,
+        qo = make_quant_out(part.d_p2[(size_t)net->p2_buf[i + 1]], (nt == kTNN || nt == kTBN) ? 1 : 2, net->layers[i + 1].threshold,
                             L.prelu_alpha, (int64_t)64 * cpack_of(L.C) * L.KH * L.KW);
     }
     float* out = next_f4 ? nullptr : ((i == n - 1) ? d_y : part.d_act[i & 1]);
     int rc;
     if (net->d_wf[i])
-        rc = conv_f4_expanded(L.type, p4_ready ? nullptr : in, net->d_thr[i], net->d_wf[i], part.batch, L.C, L.H, L.W,
+        rc = conv_f4_expanded(L.type, p2_ready ? nullptr : in, net->d_thr[i], net->d_wf[i], part.batch, L.C, L.H, L.W,
                               L.KN, L.KH, L.KW, L.pad, L.pad, L.stride, L.stride, L.prelu_alpha,
-                              part.d_p4[(size_t)net->p4_buf[i]], out, st, qo);
+                              part.d_p2[(size_t)net->p2_buf[i]], out, st, qo);
     else
         rc = conv_valu(L.type, in, net->d_thr[i], L.d_qw, part.batch, L.C, L.H, L.W, L.KN, L.KH, L.KW, L.pad, L.pad,
                        L.stride, L.stride, L.prelu_alpha, part.d_scratch, out, st, qo, false);
-    p4_ready = next_f4;
+    p2_ready = next_f4;
     in = out;
     return rc;
 }
@@ -128,7 +128,7 @@ int enqueue_layers(ftnn_net* net, const float* d_x, float* d_y, hipStream_t st) 
     }
     const float* in[2];
     float* y[2];
-    bool p4_ready[2] = {false, false};
+    bool p2_ready[2] = {false, false};
     for (size_t p = 0; p < np; p++) {
         in[p] = d_x + (size_t)net->parts[p].first * net->in_elems_per_image;
         y[p] = d_y + (size_t)net->parts[p].first * net->out_elems_per_image;
@@ -136,7 +136,7 @@ int enqueue_layers(ftnn_net* net, const float* d_x, float* d_y, hipStream_t st) 
     int rc = FTNN_OK;
     for (int i = 0; i < n && rc == FTNN_OK; i++)
         for (size_t p = 0; p < np && rc == FTNN_OK; p++)
-            rc = enqueue_layer(net, net->parts[p], i, in[p], p4_ready[p], y[p], p == 0 ? st : net->side);
+            rc = enqueue_layer(net, net->parts[p], i, in[p], p2_ready[p], y[p], p == 0 ? st : net->side);
     if (np > 1) {
         // join even after a failure: a capture in progress must see the side stream return
         e = hipEventRecord(net->join, net->side);
@@ -232,12 +232,12 @@ ftnn_net_t* ftnn_net_create_ex(int batch, int n_layers, const ftnn_layer_t* laye
     const int pb = net->parts[0].batch;
     std::vector<char> f4((size_t)n_layers, 0);
     int64_t max_act = 0, max_scratch = 256;
-    struct P4Size {
+    struct P2Size {
         int64_t image;       // bytes of one quantised image
         int64_t bytes[2];    // largest operand region among its layers, by layer parity (0: no such layer)
         int slot[2];
     };
-    std::vector<P4Size> sizes;
+    std::vector<P2Size> sizes;
     std::vector<int> size_of((size_t)n_layers, -1);
     for (int i = 0; i < n_layers; i++) {
         const ftnn_layer_t& L = layers[i];
@@ -249,12 +249,12 @@ ftnn_net_t* ftnn_net_create_ex(int batch, int n_layers, const ftnn_layer_t* laye
         // sized for the larger part; a very large layer's operand region depends on the batch in steps (the
         // im2row + GEMM form), so the smaller part is asked too
         if (f4[i]) {
-            const int64_t image = (int64_t)cpack_of(L.C) * L.H * L.W * 32;
+            const int64_t image = (int64_t)cpack_of(L.C) * L.H * L.W * 16;
             for (size_t k = 0; k < sizes.size() && size_of[i] < 0; k++)
                 if (sizes[k].image == image) size_of[i] = (int)k;
             if (size_of[i] < 0) {
                 size_of[i] = (int)sizes.size();
-                sizes.push_back(P4Size{image, {0, 0}, {-1, -1}});
+                sizes.push_back(P2Size{image, {0, 0}, {-1, -1}});
             }
         }
         for (const NetPart& part : net->parts) {
@@ -273,19 +273,19 @@ ftnn_net_t* ftnn_net_create_ex(int batch, int n_layers, const ftnn_layer_t* laye
             max_act = std::max(max_act, (int64_t)pb * layers[i - 1].KN * net->OH[i - 1] * net->OW[i - 1]);
     }
     bool good = true;
-    int n_p4 = 0;
-    for (P4Size& z : sizes)
+    int n_p2 = 0;
+    for (P2Size& z : sizes)
         for (int b = 0; b < 2; b++)
-            if (z.bytes[b] > 0) z.slot[b] = n_p4++;
-    for (int i = 0; i < n_layers; i++) net->p4_buf.push_back(f4[i] ? sizes[(size_t)size_of[i]].slot[i & 1] : -1);
+            if (z.bytes[b] > 0) z.slot[b] = n_p2++;
+    for (int i = 0; i < n_layers; i++) net->p2_buf.push_back(f4[i] ? sizes[(size_t)size_of[i]].slot[i & 1] : -1);
     for (NetPart& part : net->parts) {
-        part.d_p4.assign((size_t)n_p4, nullptr);
+        part.d_p2.assign((size_t)n_p2, nullptr);
         good = good && hipMalloc(&part.d_scratch, (size_t)max_scratch) == hipSuccess;
         for (int b = 0; b < 2 && good && max_act > 0; b++)
             good = hipMalloc((void**)&part.d_act[b], (size_t)max_act * sizeof(float)) == hipSuccess;
-        for (const P4Size& z : sizes)
+        for (const P2Size& z : sizes)
             for (int b = 0; b < 2 && good; b++)
-                if (z.slot[b] >= 0) good = hipMalloc(&part.d_p4[(size_t)z.slot[b]], (size_t)z.bytes[b]) == hipSuccess;
+                if (z.slot[b] >= 0) good = hipMalloc(&part.d_p2[(size_t)z.slot[b]], (size_t)z.bytes[b]) == hipSuccess;
     }
     if (good && nparts > 1)
         good = hipStreamCreateWithFlags(&net->side, hipStreamNonBlocking) == hipSuccess &&
@@ -307,7 +307,7 @@ ftnn_net_t* ftnn_net_create_ex(int batch, int n_layers, const ftnn_layer_t* laye
         if (!f4[i]) continue;
         const int Kw = conv_f4_weight_words(L.C, L.KH, L.KW);
         const bool wt = L.type == kTNN || L.type == kBTN;
-        good = hipMalloc(&net->d_wf[i], (size_t)mfma_fragment_bytes(true, L.KN, Kw)) == hipSuccess;
+        good = hipMalloc(&net->d_wf[i], (size_t)record_block_bytes(L.KN, Kw)) == hipSuccess;
         if (!good) break;
         const int64_t* rows = L.d_qw;
         void* d_wd = nullptr;
@@ -317,7 +317,7 @@ ftnn_net_t* ftnn_net_create_ex(int batch, int n_layers, const ftnn_layer_t* laye
                        hipSuccess;
             rows = static_cast<const int64_t*>(d_wd);
         }
-        good = good && launch_mfma_expand(true, wt, rows, L.KN, Kw, net->d_wf[i], nullptr) == hipSuccess &&
+        good = good && launch_expand_records(wt, dense_f4_applies(L.C, L.KH, L.KW), rows, L.KN, Kw, net->d_wf[i], nullptr) == hipSuccess &&
                hipStreamSynchronize(nullptr) == hipSuccess;
         if (d_wd) (void)hipFree(d_wd);
     }
@@ -338,7 +338,7 @@ void ftnn_net_destroy(ftnn_net_t* net) {
     for (NetPart& part : net->parts) {
         for (int b = 0; b < 2; b++)
             if (part.d_act[b]) (void)hipFree(part.d_act[b]);
-        for (void* p : part.d_p4)
+        for (void* p : part.d_p2)
             if (p) (void)hipFree(p);
         if (part.d_scratch) (void)hipFree(part.d_scratch);
     }

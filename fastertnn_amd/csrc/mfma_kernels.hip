@@ -8,13 +8,13 @@
 //     accumulate;
 //   * MFMA fp4   (v_mfma_f32_32x32x64_f8f6f4, E2M1): lanes become nibbles 0x2 / 0x0 / 0xA
 //     (+1.0 / 0 / -1.0), fp32 accumulate -- exact while 64*Kw < 2^24, which the host
-//     checks.  Twice the matrix rate of int8 and half the operand bytes.  This is the form
-//     of the conv layer kernels and their prepared weights; the fp4 GEMM engine itself
-//     (k_pack4, k_mfma_p4 further down) codes a lane a as (a + 1) / 2 at two bits per lane.
+//     checks.  Twice the matrix rate of int8.  The conv layers keep both operands at two bits
+//     per lane (records, see P2) and split them in registers; the fp4 GEMM engine itself
+//     (k_pack4, k_mfma_p4 further down) codes a lane a as (a + 1) / 2, also at two bits.
 //
-// The kernels of the int8 engine and of the layers' GEMM route:
+// The kernels of the int8 engine:
 //   k_expand  Packing-2 (or single-plane binary) rows -> "fragments": 1 KiB blocks
-//             holding 32 rows x 32 (int8) or 64 (fp4) lanes in exactly the register
+//             holding 32 rows x 32 lanes in exactly the register
 //             layout of an MFMA operand (lane l = (k half l/32, row l%32), 16 bytes).
 //             HBM-bound, one pass per operand.
 //   k_mfma    256 x 256 output tile per workgroup (4 wavefronts, 128 x 128 each, 256
@@ -36,10 +36,9 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
-// Ring of NS LDS buffers, each holding KF fragments (K words for fp4) per row-block: one barrier per KF fragments.
+// Ring of NS LDS buffers, each holding KF fragments per row-block: one barrier per KF fragments.
 // A workgroup of 2 x 2 wavefronts computes (64 WTP) x (64 WTQ) results, a wavefront WTP x WTQ blocks of 32 x 32:
-// 4 x 4 for problems with enough 256 x 256 tiles to fill the chip, 2 x 2 (128 x 128) below that, 4 x 2 (256 kernels x
-// 128 pixels) for conv layers on the tile kernel, whose kernel side is the cheaper one to stage.
+// 4 x 4 for problems with enough 256 x 256 tiles to fill the chip, 2 x 2 (128 x 128) below that.
 template <int WTP, int WTQ, int KF, int NS>
 struct Tile {
     static constexpr int RBP = 2 * WTP, RBQ = 2 * WTQ;   // row-blocks per operand side
@@ -57,7 +56,17 @@ struct Tile {
 // grid (row-blocks, groups / 4), block 256: thread = (row r = t%32, dword pair dq = t/32).
 // A group is 4 words (256 lanes) of a packed row: 16 dwords (8 sign, 8 zero) for ternary
 // rows, 8 dwords for binary rows.  Rows past `rows` expand to zeros.
-template <bool F4, bool TERN>
+// FORM: int8 fragments, or records of two bits per lane (see P2) as blocks [row block][pair of K words][lane l = (word of the
+// pair l / 32, row l % 32)][16 bytes], in the layers' lane order or in natural order.
+enum { FORM_I8, FORM_REC, FORM_REC_NATURAL };
+
+// four lanes per byte, bit i of a byte -> the lanes' places in a record byte (1, 0, 5, 4); shifted by two for the signs
+__device__ __forceinline__ uint32_t spread_lanes(uint32_t v) {
+    v &= 0x0F0F0F0Fu;
+    return ((v & 0x09090909u) << 1) | ((v >> 1) & 0x01010101u) | ((v << 3) & 0x20202020u);
+}
+
+template <int FORM, bool TERN>
 __device__ __forceinline__ void expand_block(const uint32_t* __restrict__ P, int rows, int G, uint4* __restrict__ out, int rb,
                                              int gy, uint32_t* stage, uint32_t* __restrict__ kept = nullptr) {
     // A workgroup expands kGPB adjacent groups of its 32 rows: 256 contiguous bytes of each ternary row (128 of a
@@ -101,22 +110,30 @@ __device__ __forceinline__ void expand_block(const uint32_t* __restrict__ P, int
         if (g >= G) break;
         const uint32_t nz = live ? ~zv[i] : 0u;
         const uint32_t s = sv[i] & nz;   // a lane flagged zero is zero whatever its sign bit says
-        if (F4) {
-            // fragment = one 64-lane word: dword dq&1 is its k half; nibble = sign<<3 | nonzero<<1
-            uint4* frag = out + ((size_t)rb * (G * 4) + (g * 4 + (dq >> 1))) * 64;
-            uint32_t o[4];
+        if constexpr (FORM != FORM_I8) {
+            const int w = g * 4 + (dq >> 1), half = dq & 1;   // this thread: 32 lanes of word w
+            uint2* rec = reinterpret_cast<uint2*>(out + ((size_t)rb * (G * 2) + (w >> 1)) * 64 + (w & 1) * 32 + r) + half;
+            if constexpr (FORM == FORM_REC) {
+                // dwords `half` and 2 + `half` of the record; the threads of the two halves of a word are lanes l and l + 32:
+                // the swap gives the lower one dwords 0 and 1, the upper one 2 and 3
+                const uint32_t d0 = spread_lanes(nz) | spread_lanes(s) << 2, d1 = spread_lanes(nz >> 4) | spread_lanes(s >> 4) << 2;
+                const auto d = __builtin_amdgcn_permlane32_swap(d0, d1, false, false);
+                *rec = make_uint2(d[0], d[1]);
+            } else {
+                uint32_t o[4];
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                uint32_t a = (s >> (8 * q)) & 0xffu, b = (nz >> (8 * q)) & 0xffu;
-                a = (a | (a << 12)) & 0x000F000Fu;
-                a = (a | (a << 6)) & 0x03030303u;
-                a = (a | (a << 3)) & 0x11111111u;
-                b = (b | (b << 12)) & 0x000F000Fu;
-                b = (b | (b << 6)) & 0x03030303u;
-                b = (b | (b << 3)) & 0x11111111u;
-                o[q] = (a << 3) | (b << 1);
+                for (int q = 0; q < 4; q++) {   // eight lanes -> eight nibbles, sign << 3 | nonzero << 1
+                    uint32_t a = (s >> (8 * q)) & 0xffu, b = (nz >> (8 * q)) & 0xffu;
+                    a = (a | (a << 12)) & 0x000F000Fu;
+                    a = (a | (a << 6)) & 0x03030303u;
+                    a = (a | (a << 3)) & 0x11111111u;
+                    b = (b | (b << 12)) & 0x000F000Fu;
+                    b = (b | (b << 6)) & 0x03030303u;
+                    b = (b | (b << 3)) & 0x11111111u;
+                    o[q] = (a << 3) | (b << 1);
+                }
+                *rec = make_uint2(p2_join(o[0], o[1]), p2_join(o[2], o[3]));
             }
-            frag[(dq & 1) * 32 + r] = make_uint4(o[0], o[1], o[2], o[3]);
         } else {
             // fragment = one 32-lane dword: its two 16-lane halves are the k halves
             uint4* frag = out + ((size_t)rb * (G * 8) + (g * 8 + dq)) * 64;
@@ -138,21 +155,21 @@ __device__ __forceinline__ void expand_block(const uint32_t* __restrict__ P, int
 }
 
 // kept: where the packed rows themselves are copied to on the way (a copy of its own costs the caller 20 us), or null
-template <bool F4, bool TERN>
+template <int FORM, bool TERN>
 __global__ __launch_bounds__(256) void k_expand(const uint32_t* __restrict__ P, int rows, int G, uint4* __restrict__ out,
                                                 uint32_t* __restrict__ kept) {
     __shared__ uint32_t stage[32 * 65];
-    expand_block<F4, TERN>(P, rows, G, out, blockIdx.x, blockIdx.y, stage, kept);
+    expand_block<FORM, TERN>(P, rows, G, out, blockIdx.x, blockIdx.y, stage, kept);
 }
 
-// both operands of a GEMM in one launch (the same K): the first ceil(rows_a / 32) workgroup columns expand A, the others B
-template <bool F4, bool TA, bool TB>
+// both int8 operands of a GEMM in one launch (the same K): the first ceil(rows_a / 32) workgroup columns expand A, the others B
+template <bool TA, bool TB>
 __global__ __launch_bounds__(256) void k_expand2(const uint32_t* __restrict__ Pa, int rows_a, uint4* __restrict__ out_a,
                                                  const uint32_t* __restrict__ Pb, int rows_b, uint4* __restrict__ out_b, int G) {
     __shared__ uint32_t stage[32 * 65];
     const int rba = (rows_a + 31) / 32;
-    if ((int)blockIdx.x < rba) expand_block<F4, TA>(Pa, rows_a, G, out_a, blockIdx.x, blockIdx.y, stage);
-    else expand_block<F4, TB>(Pb, rows_b, G, out_b, (int)blockIdx.x - rba, blockIdx.y, stage);
+    if ((int)blockIdx.x < rba) expand_block<FORM_I8, TA>(Pa, rows_a, G, out_a, blockIdx.x, blockIdx.y, stage);
+    else expand_block<FORM_I8, TB>(Pb, rows_b, G, out_b, (int)blockIdx.x - rba, blockIdx.y, stage);
 }
 
 // ----------------------------------------------------------------------- GEMM
@@ -230,25 +247,12 @@ __device__ __forceinline__ void store_tile(const typename Acc<F4>::type (&acc)[W
 // The epilogue computes r = acc - bias, then PReLU in the reference's form for the type:
 // form 0 "f = r; if (f <= 0) f *= alpha" (mm_p2_final_tnn_avx2.c:204-208), form 1
 // "r >= 0 ? r : alpha * r" (mm_p2_final_tbn_avx2.c:73).
-// IMPL (fp4, SWAP): a conv layer with implicit im2row.  Qf is then not a fragment array but the layer's quantised input
-// in the form T4[n][C_pack][half][row][column % s][column / s][16 bytes] (k_quantize_f4 with TILED): the two wavefronts
-// that stage the Q side compute, per fragment, each lane's own source address -- lane (pixel, K half) of the fragment of
-// K word w = (kh KW + kw) C_pack + ic reads its 16 bytes at input pixel (oh s + kh - p, ow s + kw - p) of plane ic, or a
-// the fill piece behind the planes (16 bytes of zeros, or of +1 nibbles for binary activations: the reference's
-// fill, src/tnns/ternarize2row_avx2.c:748-755, src/tnns/binarize2row_avx2.c:151) where that pixel lies outside the image or w is a padding word -- and the LDS-direct load drops the 64
-// lanes contiguously into the ring exactly as it drops a stored fragment.  In T4 the 32 pixels of a fragment half are
-// consecutive 16-byte pieces within an output row whatever the stride (records of 32 bytes gathered at the stride
-// took the load unit four times as many requests: 50 against 32 us on a 1024-channel 28 x 28 stride-2 layer).  The im2row rows and their expansion are never written (for a 1024-channel 56 x 56 layer:
-// 116 + 231 MB less traffic and two launches less), and everything behind the ring is the GEMM kernel unchanged.
-template <bool F4, bool SWAP, int WTP, int WTQ, int kKF, int kNS, bool IMPL = false, bool BAL = false>
+template <bool SWAP, int WTP, int WTQ, int kKF, int kNS>
 __global__ __launch_bounds__(256) void k_mfma(const uint4* __restrict__ Pf, const uint4* __restrict__ Qf,
                                               float* __restrict__ Y, int M, int KN, int OHW, int KB,
-                                              int bias, int form, float alpha, ConvGeom cg = ConvGeom(),
-                                              FastDiv dOHW = FastDiv(), int Ws = 0, FastDiv dSW = FastDiv()) {
-    static_assert(!IMPL || (F4 && SWAP), "implicit im2row: fp4 layer with the pixels along the lanes");
-    static_assert(!BAL || IMPL, "the balanced assignment of fragments is for the gathering kernel");
+                                              int bias, int form, float alpha) {
     extern __shared__ uint4 lds[];   // kNS buffers of kFR KiB
-    typedef typename Acc<F4>::type acc_t;
+    typedef Acc<false>::type acc_t;
     typedef Tile<WTP, WTQ, kKF, kNS> TL;
     constexpr int RBP = TL::RBP, RBQ = TL::RBQ, kFR = TL::FR, kFW = TL::FW, NL = TL::NL, NM = TL::NM, DPI = TL::DPI;
     constexpr int kPF = RBP * kKF;   // fragments of the P side per step
@@ -256,20 +260,7 @@ __global__ __launch_bounds__(256) void k_mfma(const uint4* __restrict__ Pf, cons
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wy = wave >> 1, wx = wave & 1;
     const int prow = SWAP ? KN : M, qrow = SWAP ? M : KN;
-    // Tile of this workgroup.  Under IMPL the kernel tiles of one pixel tile read the same part of T4; workgroups are dealt
-    // to the eight XCDs round-robin by their linear number, so the tiles are renumbered to keep those on one XCD (its L2
-    // then fetches that part once, not once per kernel tile): XCD x takes the pixel tiles x, x + 8, ...; the pixel
-    // tiles beyond the last multiple of eight keep the plain order.
-    uint32_t bx = blockIdx.x, by = blockIdx.y;
-    if constexpr (IMPL) {
-        const uint32_t kt = gridDim.x, pt8 = gridDim.y / 8 * 8, lin = bx + kt * by;
-        if (lin < kt * pt8) {
-            const uint32_t xcd = lin & 7u, slot = lin >> 3;
-            by = xcd + 8u * (slot / kt);
-            bx = slot % kt;
-        }
-    }
-    const int prb0 = bx * RBP, qrb0 = by * RBQ;
+    const int prb0 = blockIdx.x * RBP, qrb0 = blockIdx.y * RBQ;
     const int prbmax = (prow + 31) / 32 - 1, qrbmax = (qrow + 31) / 32 - 1;
     acc_t acc[WTP][WTQ];
 #pragma unroll
@@ -281,107 +272,16 @@ __global__ __launch_bounds__(256) void k_mfma(const uint4* __restrict__ Pf, cons
 
     // fragment f of a step: the P side's kPF fragments first (row-block f / kKF, k fragment f % kKF), then the Q
     // side's; row-blocks past the operand are clamped (their results are never stored)
-    // Which fragments a wavefront stages: in order (wavefront w the fragments w kFW .. w kFW + kFW - 1), or, BAL, a
-    // quarter of each side (PW fragments of the P side, then QW of the Q side), so that under IMPL every wavefront
-    // gathers the same number of fragments and none of them holds the others up at the step's barrier.
-    constexpr int PW = BAL ? kPF / 4 : 0, QW = BAL ? kFW - PW : 0;
-    static_assert(!BAL || (kPF % 4 == 0 && (QW % kKF == 0 || (QW == 1 && kKF == 2))), "a quarter of each side per wavefront");
-    auto frag_of = [&](int i) -> int {   // fragment number (its place in a stage of the ring) of the wavefront's slot i
-        if constexpr (BAL) return i < PW ? wave * PW + i : kPF + wave * QW + (i - PW);
-        else return wave * kFW + i;
-    };
     const uint4* src[kFW];
 #pragma unroll
     for (int i = 0; i < kFW; i++) {
-        const int f = frag_of(i);
+        const int f = wave * kFW + i;
         const bool qside = f >= kPF;
         const int g = qside ? f - kPF : f, rbi = g / kKF, kbi = g % kKF;
         const uint4* base = !qside ? Pf + ((size_t)min(prb0 + rbi, prbmax) * KB + kbi) * 64
                                    : Qf + ((size_t)min(qrb0 + rbi, qrbmax) * KB + kbi) * 64;
         src[i] = base + lane;
     }
-    // IMPL: the Q side's fragments are gathered.  They are the last RBQ * kKF fragments of a step, staged by wavefront
-    // 3 and, where the tile is not square, by the tail of wavefront 2; a wavefront's Q fragments cover whole row blocks
-    // of 32 pixels, at most QMAX of them, from row block qfirst on.  A wavefront issues one instruction every few
-    // cycles, so what the gather adds per fragment must stay a handful of instructions:
-    //   * a table behind the ring, one entry per K word w = (kh KW + kw) C_pack + ic, holds what does not depend on
-    //     the lane: the bit of the word's tap (0 for a padding word), and the word's part of the piece index (plane,
-    //     tap row, column class and slot offset);
-    //   * per row block a lane keeps the mask of the taps that fall inside the image for its pixel, and its pixel's
-    //     part of the piece index;
-    // a fragment's source is then one AND, one add, one select and the address.
-    static_assert(!IMPL || kKF == 2, "two table entries per read");
-    static_assert(!IMPL || BAL || (kPF % kKF == 0 && kFW % kKF == 0 && kPF >= 2 * kFW), "Q fragments in whole row blocks, on wavefronts 2 and 3 only");
-    constexpr int QMAX = BAL ? (QW + kKF - 1) / kKF : kFW / kKF;
-    const bool gathers = IMPL && (BAL || (wave + 1) * kFW > kPF);   // wave-uniform: this wavefront stages Q fragments
-    const int qfirst = BAL ? (wave * QW) / kKF : max(0, wave * kFW - kPF) / kKF;
-    uint32_t tapmask[IMPL ? QMAX : 1], pbase[IMPL ? QMAX : 1];
-    const uint32_t row16 = (uint32_t)(cg.W_stride * Ws);          // pieces per input row
-    const uint32_t half16 = (uint32_t)cg.H * row16;               // per half plane
-    const uint32_t fill_piece = (uint32_t)(cg.CP * 2) * half16 * (uint32_t)((M - 1) / OHW + 1);   // right behind the planes
-    uint2* const wtab = reinterpret_cast<uint2*>(lds + (size_t)kNS * kFR * 64);
-    if constexpr (IMPL) {
-        for (int w = tid; w < KB; w += 256) {
-            const int tap = (int)fastdiv((uint32_t)w, cg.dCP), ic = w - tap * cg.CP;
-            const int kh = (int)fastdiv((uint32_t)tap, cg.dKW), kw = tap - kh * cg.KW;
-            // column ow s + d with d = kw - pad: class d mod s, slot ow + floor(d / s) (d made non-negative by a
-            // multiple of s first: the host keeps the padding below 4096 s)
-            const uint32_t dd = (uint32_t)(kw - cg.W_pad + 4096 * cg.W_stride);
-            const uint32_t dq = fastdiv(dd, dSW), cls = dd - dq * (uint32_t)cg.W_stride;
-            wtab[w] = make_uint2(w < cg.K ? 1u << tap : 0u,
-                                 (uint32_t)ic * 2u * half16 + (uint32_t)kh * row16 + cls * (uint32_t)Ws + dq - 4096u);
-        }
-#pragma unroll
-        for (int j = 0; j < QMAX; j++) {
-            const int rb = min(qfirst + j, RBQ - 1);
-            const uint32_t q = (uint32_t)min((qrb0 + rb) * 32 + (lane & 31), M - 1);
-            const uint32_t img = fastdiv(q, dOHW);
-            const uint32_t pix = q - img * (uint32_t)OHW;
-            const int oh = (int)fastdiv(pix, cg.dOW), ow = (int)pix - oh * cg.OW;
-            const int ih0 = oh * cg.H_stride - cg.H_pad, iw0 = ow * cg.W_stride - cg.W_pad;
-            // (image, plane 0, this lane's half, row ih0, class 0, slot ow): wraps for a negative ih0, and the
-            // word's part brings it back whenever the tap is inside
-            pbase[j] = (img * (uint32_t)cg.CP * 2u + (uint32_t)(lane >> 5)) * half16 + (uint32_t)ih0 * row16 + (uint32_t)ow;
-            uint32_t m = 0u;
-            for (int kh = 0, tap = 0; kh < cg.K / (cg.CP * cg.KW); kh++)
-                for (int kw = 0; kw < cg.KW; kw++, tap++)
-                    m |= ((unsigned)(ih0 + kh) < (unsigned)cg.H && (unsigned)(iw0 + kw) < (unsigned)cg.W ? 1u : 0u) << tap;
-            tapmask[j] = m;
-        }
-        __syncthreads();   // the table is complete before the first stage is issued
-    }
-    // the table entries of the kKF words of the stage about to be issued (stages are issued strictly in order), read
-    // from LDS one stage ahead of their use (the table has two entries to spare behind its last word)
-    int g_w = kKF;
-    uint4 wt = make_uint4(0u, 0u, 0u, 0u), wt_ahead = make_uint4(0u, 0u, 0u, 0u);
-    if constexpr (IMPL) {
-        if (gathers) wt_ahead = *reinterpret_cast<const uint4*>(wtab);
-    }
-    auto next_words = [&]() {
-        wt = wt_ahead;
-        wt_ahead = *reinterpret_cast<const uint4*>(wtab + min(g_w, KB));
-        g_w += kKF;
-    };
-    // the gathered source of fragment i of wavefront W (both compile-time): its row block's slot in tapmask / pbase is
-    // then a constant
-    auto gathered = [&](auto wtag, int i) -> const uint4* {
-        constexpr int W = decltype(wtag)::value;
-        int j;
-        bool even;   // the fragment's K word within the stage
-        if constexpr (BAL) {
-            // slot i holds Q fragment w QW + (i - PW): with whole row blocks per wavefront both are compile-time; with one
-            // fragment per wavefront (QW == 1) the K word is the wavefront's parity
-            j = QW % kKF == 0 ? (i - PW) / kKF : 0;
-            even = QW % kKF == 0 ? ((i - PW) % kKF) == 0 : (wave & 1) == 0;
-        } else {
-            constexpr int first = (W * kFW > kPF ? W * kFW - kPF : 0) / kKF;
-            j = (W * kFW + i - kPF) / kKF - first;
-            even = (i % kKF) == 0;
-        }
-        const uint32_t bit = even ? wt.x : wt.z, off = even ? wt.y : wt.w;
-        const uint32_t piece = pbase[j] + off;
-        return Qf + ((tapmask[j] & bit) != 0u ? piece : fill_piece);   // a select on the index: no branch
-    };
     const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
     const int nstep = KB / kKF;
     uint4 fa[2][WTP], fb[2][WTQ];
@@ -397,89 +297,63 @@ __global__ __launch_bounds__(256) void k_mfma(const uint4* __restrict__ Pf, cons
     // square tile), in the order (a, b) = (m / WTQ, m % WTQ)
     auto mfma2 = [&](int set, int i) {
 #pragma unroll
-        for (int m = i * NM / NL; m < (i + 1) * NM / NL; m++) mfma<F4>(acc[m / WTQ][m % WTQ], fa[set][m / WTQ], fb[set][m % WTQ]);
+        for (int m = i * NM / NL; m < (i + 1) * NM / NL; m++) mfma<false>(acc[m / WTQ][m % WTQ], fa[set][m / WTQ], fb[set][m % WTQ]);
     };
+    auto stage = [&](int step) {
+        const uint32_t dst = lds0 + (uint32_t)(step % kNS) * (kFR * 1024);
+#pragma unroll
+        for (int i = 0; i < kFW; i++) dma16(src[i] + (size_t)step * kKF * 64, dst + (uint32_t)(wave * kFW + i) * 1024);
+    };
+    // prologue: the first kNS stages in flight, wait for stage 0 only
+#pragma unroll
+    for (int p = 0; p < kNS; p++)
+        if (p < nstep) stage(p);
+    if (nstep >= kNS) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFW * (kNS - 1)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NL; i++) ldone(0, 0, 0, i);
 
-    // The pipeline, instantiated per role of the wavefront so that no fragment's source is chosen at run time: role 0
-    // stages stored fragments only (every wavefront without IMPL; wavefronts 0 and 1 with it), roles 2 and 3 are
-    // wavefronts 2 and 3 under IMPL, whose Q fragments are gathered.  Every role passes the same barriers.
-    auto pipeline = [&](auto role_tag) {
-        constexpr int ROLE = decltype(role_tag)::value;
-        // source of the wavefront's fragment i for K step `step` (gathered: of the stage next_words() was last called for)
-        auto source = [&](int i, int step) -> const uint4* {
-            if constexpr (BAL) {
-                if (i >= PW) return gathered(role_tag, i);
-            } else if constexpr (ROLE != 0) {
-                if (ROLE * kFW + i >= kPF) return gathered(role_tag, i);
-            }
-            return src[i] + (size_t)step * kKF * 64;
-        };
-        auto stage = [&](int step) {
-            const uint32_t dst = lds0 + (uint32_t)(step % kNS) * (kFR * 1024);
-            if constexpr (ROLE != 0) next_words();
+    auto step_body = [&](int s, auto full_tag) {
+        constexpr bool FULL = decltype(full_tag)::value;   // FULL: s + kNS < nstep
 #pragma unroll
-            for (int i = 0; i < kFW; i++) dma16(source(i, step), dst + (uint32_t)frag_of(i) * 1024);
-        };
-        // prologue: the first kNS stages in flight, wait for stage 0 only
+        for (int k = 0; k < kKF; k++) {
+            const int set = k & 1;
+            if (k + 1 < kKF) {
 #pragma unroll
-        for (int p = 0; p < kNS; p++)
-            if (p < nstep) stage(p);
-        if (nstep >= kNS) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFW * (kNS - 1)) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+                for (int i = 0; i < NL; i++) {
+                    ldone(s % kNS, k + 1, set ^ 1, i);
+                    mfma2(set, i);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                // Last fragment of the step: all of this step is in registers.  Stage s+1 must
+                // have landed (stages s+2 .. s+kNS-1 may still be in flight); after the barrier
+                // buffer s % kNS is free for stage s+kNS.
+                if (FULL || s + kNS - 1 < nstep) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFW * (kNS - 2)) : "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+                const bool do_ld = FULL || s + 1 < nstep;
+                const uint32_t dst = lds0 + (uint32_t)(s % kNS) * (kFR * 1024);
 #pragma unroll
-        for (int i = 0; i < NL; i++) ldone(0, 0, 0, i);
-
-        auto step_body = [&](int s, auto full_tag) {
-            constexpr bool FULL = decltype(full_tag)::value;   // FULL: s + kNS < nstep
+                for (int i = 0; i < NL; i++) {
+                    if (FULL) {
 #pragma unroll
-            for (int k = 0; k < kKF; k++) {
-                const int set = k & 1;
-                if (k + 1 < kKF) {
-#pragma unroll
-                    for (int i = 0; i < NL; i++) {
-                        ldone(s % kNS, k + 1, set ^ 1, i);
-                        mfma2(set, i);
-                        __builtin_amdgcn_sched_barrier(0);
+                        for (int j = 0; j < DPI; j++)
+                            dma16(src[i * DPI + j] + (size_t)(s + kNS) * kKF * 64, dst + (uint32_t)(wave * kFW + i * DPI + j) * 1024);
                     }
-                } else {
-                    // Last fragment of the step: all of this step is in registers.  Stage s+1 must
-                    // have landed (stages s+2 .. s+kNS-1 may still be in flight); after the barrier
-                    // buffer s % kNS is free for stage s+kNS.
-                    if (FULL || s + kNS - 1 < nstep) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFW * (kNS - 2)) : "memory");
-                    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    __syncthreads();
-                    const bool do_ld = FULL || s + 1 < nstep;
-                    const uint32_t dst = lds0 + (uint32_t)(s % kNS) * (kFR * 1024);
-                    if constexpr (FULL && ROLE != 0) next_words();
-#pragma unroll
-                    for (int i = 0; i < NL; i++) {
-                        if (FULL) {
-#pragma unroll
-                            for (int j = 0; j < DPI; j++) dma16(source(i * DPI + j, s + kNS), dst + (uint32_t)frag_of(i * DPI + j) * 1024);
-                        }
-                        if (do_ld) ldone((s + 1) % kNS, 0, set ^ 1, i);
-                        mfma2(set, i);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
+                    if (do_ld) ldone((s + 1) % kNS, 0, set ^ 1, i);
+                    mfma2(set, i);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
-        };
-        int s = 0;
-        for (; s + kNS < nstep; s++) step_body(s, std::true_type{});
-        for (; s < nstep; s++) step_body(s, std::false_type{});
+        }
     };
-    if constexpr (BAL) {
-        pipeline(std::integral_constant<int, 1>{});   // every wavefront stages and gathers alike
-    } else if constexpr (IMPL) {
-        if (wave == 3) pipeline(std::integral_constant<int, 3>{});
-        else if (wave == 2) pipeline(std::integral_constant<int, 2>{});
-        else pipeline(std::integral_constant<int, 0>{});
-    } else {
-        pipeline(std::integral_constant<int, 0>{});
-    }
+    int s = 0;
+    for (; s + kNS < nstep; s++) step_body(s, std::true_type{});
+    for (; s < nstep; s++) step_body(s, std::false_type{});
 
-    store_tile<F4, SWAP, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
+    store_tile<false, SWAP, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
 }
 
 // ------------------------------------------------- fp4 operands at two bits per lane, offset codes
@@ -771,48 +645,297 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
     store_tile_offset<SWAP, WT>(acc, Y, M, KN, OHW, prb0 + wy * WT, qrb0 + wx * WT, lane, sums, wy, wx, off, form, alpha);
 }
 
+// ------------------------------------------------------------ conv layers as workgroup tiles (fp4, records)
+// Large layers.  2 x 2 wavefronts per workgroup, WTP x WTQ blocks of 32 x 32 each: (64 WTP) x (64 WTQ) results.  P side:
+// weights, Q side: pixels (SWAP; without it, for one-pixel images, P = rows of the activations and Q = weights, row-major).
+// Both operands are blocks of records: 1 KiB = 32 rows x two K words, lane l = (word of the pair l / 32, row l % 32).  A stage
+// of the LDS ring holds PPS pairs of every row block, filled by LDS-direct loads that the kernel counts by hand; a block is one
+// 16-byte read per lane, split into the nibbles of two multiplies (lanes of both words of a pair enter both, see P2).  The
+// schedule is k_mfma_p4's: the first word's multiplies run while the second one's operands are split; then (behind the barrier
+// where the stage ends) the second word's multiplies run beside the LDS reads of the next pair, each block split LAG slots
+// after its read.  These tiles are bound by what they move through the LDS: at four bits per lane a step of two K words
+// moved 72 KiB for 512 cycles of matrix pipe (256 x 128 tile) and took 1080 cycles.
+//
+// IMPL: a conv layer with implicit im2row.  Qc is then the layer's quantised input in the form T2[n][C_pack][row][column % s]
+// [column / s][16 bytes] (k_quantize_f4 with TILED): lane l of a block of K words 2 i, 2 i + 1 loads the record of its pixel at
+// the tap of word w = 2 i + l / 32 = (kh KW + kw) C_pack + ic, from input pixel (oh s + kh - p, ow s + kw - p) of plane ic, or
+// the fill record behind the planes (zeros, or +1 for binary activations: the reference's fill,
+// src/tnns/ternarize2row_avx2.c:748-755, src/tnns/binarize2row_avx2.c:151) where that pixel lies outside the image or w is a
+// padding word.  In T2 the 32 pixels are consecutive records within an output row whatever the stride.  Every wavefront stages
+// a quarter of each side, so that none holds the others up at the barrier.  A wavefront issues one instruction every few
+// cycles, so what the gather adds per block must stay a handful of instructions:
+//   * a table behind the ring, one entry per K word, holds what does not depend on the pixel: the bit of the word's tap (0
+//     for a padding word), and the word's part of the record index (plane, tap row, column class and slot offset);
+//   * per row block a lane keeps the mask of the taps that fall inside the image for its pixel, and its pixel's part of the index;
+// a block's source is then one AND, one add, one select and the address.
+template <int WTP, int WTQ, int PPS, int NS>
+struct TileRec {
+    static constexpr int RBP = 2 * WTP, RBQ = 2 * WTQ;         // row blocks per operand side
+    static constexpr int PF = RBP * PPS, FR = PF + RBQ * PPS;  // blocks per stage: the P side's, then the Q side's
+    static constexpr int PW = PF / 4, QW = RBQ * PPS / 4, FW = PW + QW;   // blocks a wavefront stages
+    static constexpr int NL = WTP + WTQ, NM = WTP * WTQ;       // LDS reads per pair of words, multiplies per word
+    static constexpr int LAG = NL >= 8 ? 4 : (NL >= 4 ? 3 : 1);
+    static constexpr size_t lds_bytes = (size_t)NS * FR * 1024;
+    static_assert(PF % 4 == 0 && (RBQ * PPS) % 4 == 0 && FW <= NL, "a quarter of each side per wavefront, one load per slot");
+    static_assert(PPS == 1 || QW == 1, "one pair per wavefront on the gathered side");
+};
+
+template <bool SWAP, int WTP, int WTQ, int PPS, int NS, bool IMPL>
+__global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, const uint4* __restrict__ Qc, float* __restrict__ Y,
+                                                 int M, int KN, int OHW, int KP /* pairs of words per row */, int nstep, int bias,
+                                                 int form, float alpha, ConvGeom cg, FastDiv dOHW, int Ws, FastDiv dSW) {
+    static_assert(!IMPL || SWAP, "implicit im2row: the pixels along the lanes");
+    extern __shared__ uint4 lds[];   // NS stages of FR KiB, then the table
+    typedef Acc<true>::type acc_t;
+    typedef TileRec<WTP, WTQ, PPS, NS> TL;
+    constexpr int RBP = TL::RBP, RBQ = TL::RBQ, PF = TL::PF, FR = TL::FR, PW = TL::PW, QW = TL::QW, FW = TL::FW;
+    constexpr int NL = TL::NL, NM = TL::NM, LAG = TL::LAG;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wy = wave >> 1, wx = wave & 1;
+    const int prow = SWAP ? KN : M, qrow = SWAP ? M : KN;
+    // Tile of this workgroup.  Under IMPL the kernel tiles of one pixel tile read the same part of T2; workgroups are dealt
+    // to the eight XCDs round-robin by their linear number, so the tiles are renumbered to keep those on one XCD (its L2
+    // then fetches that part once, not once per kernel tile): XCD x takes the pixel tiles x, x + 8, ...; the pixel
+    // tiles beyond the last multiple of eight keep the plain order.
+    uint32_t bx = blockIdx.x, by = blockIdx.y;
+    if constexpr (IMPL) {
+        const uint32_t kt = gridDim.x, pt8 = gridDim.y / 8 * 8, lin = bx + kt * by;
+        if (lin < kt * pt8) {
+            const uint32_t xcd = lin & 7u, slot = lin >> 3;
+            by = xcd + 8u * (slot / kt);
+            bx = slot % kt;
+        }
+    }
+    const int prb0 = bx * RBP, qrb0 = by * RBQ;
+    const int prbmax = (prow + 31) / 32 - 1, qrbmax = (qrow + 31) / 32 - 1;
+    acc_t acc[WTP][WTQ];
+#pragma unroll
+    for (int a = 0; a < WTP; a++)
+#pragma unroll
+        for (int b = 0; b < WTQ; b++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[a][b][e] = 0;
+
+    // Block g of a side and stage: row block g / PPS, pair g % PPS.  Wavefront w stages blocks w PW .. of the P side and w QW ..
+    // of the Q side; row blocks past the operand are clamped (their results are never stored).
+    const uint4* psrc[PW];
+#pragma unroll
+    for (int i = 0; i < PW; i++) {
+        const int g = wave * PW + i;
+        psrc[i] = Pc + ((size_t)min(prb0 + g / PPS, prbmax) * KP + g % PPS) * 64 + lane;
+    }
+    const uint4* qsrc[IMPL ? 1 : QW];
+    uint32_t tapmask[IMPL ? QW : 1], qbase[IMPL ? QW : 1];
+    const uint32_t row16 = (uint32_t)(cg.W_stride * Ws);            // records per input row
+    const uint32_t plane16 = (uint32_t)cg.H * row16;                // per plane of 64 channels
+    const uint32_t fill_rec = (uint32_t)cg.CP * plane16 * (uint32_t)((M - 1) / OHW + 1);   // right behind the planes
+    uint2* const wtab = reinterpret_cast<uint2*>(lds + (size_t)NS * FR * 64);
+    const int words = 2 * PPS * nstep;
+    if constexpr (IMPL) {
+        for (int w = tid; w < words; w += 256) {
+            const int tap = (int)fastdiv((uint32_t)w, cg.dCP), ic = w - tap * cg.CP;
+            const int kh = (int)fastdiv((uint32_t)tap, cg.dKW), kw = tap - kh * cg.KW;
+            // column ow s + d with d = kw - pad: class d mod s, slot ow + floor(d / s) (d made non-negative by a
+            // multiple of s first: the host keeps the padding below 4096 s)
+            const uint32_t dd = (uint32_t)(kw - cg.W_pad + 4096 * cg.W_stride);
+            const uint32_t dq = fastdiv(dd, dSW), cls = dd - dq * (uint32_t)cg.W_stride;
+            wtab[w] = make_uint2(w < cg.K ? 1u << tap : 0u,
+                                 (uint32_t)ic * plane16 + (uint32_t)kh * row16 + cls * (uint32_t)Ws + dq - 4096u);
+        }
+#pragma unroll
+        for (int j = 0; j < QW; j++) {
+            const int rb = (wave * QW + j) / PPS;
+            const uint32_t q = (uint32_t)min((qrb0 + rb) * 32 + (lane & 31), M - 1);
+            const uint32_t img = fastdiv(q, dOHW);
+            const uint32_t pix = q - img * (uint32_t)OHW;
+            const int oh = (int)fastdiv(pix, cg.dOW), ow = (int)pix - oh * cg.OW;
+            const int ih0 = oh * cg.H_stride - cg.H_pad, iw0 = ow * cg.W_stride - cg.W_pad;
+            // (image, plane 0, row ih0, class 0, slot ow): wraps for a negative ih0, and the word's part brings it back
+            // whenever the tap is inside
+            qbase[j] = img * (uint32_t)cg.CP * plane16 + (uint32_t)ih0 * row16 + (uint32_t)ow;
+            uint32_t m = 0u;
+            for (int kh = 0, tap = 0; kh < cg.K / (cg.CP * cg.KW); kh++)
+                for (int kw = 0; kw < cg.KW; kw++, tap++)
+                    m |= ((unsigned)(ih0 + kh) < (unsigned)cg.H && (unsigned)(iw0 + kw) < (unsigned)cg.W ? 1u : 0u) << tap;
+            tapmask[j] = m;
+        }
+        __syncthreads();   // the table is complete before the first stage is issued
+    } else {
+#pragma unroll
+        for (int i = 0; i < QW; i++) {
+            const int g = wave * QW + i;
+            qsrc[i] = Qc + ((size_t)min(qrb0 + g / PPS, qrbmax) * KP + g % PPS) * 64 + lane;
+        }
+    }
+    // this lane's word of the pair that its wavefront gathers of the stage about to be issued (stages are issued strictly in
+    // order); its table entry is read one stage ahead of its use
+    int g_w = 2 * (PPS == 1 ? 0 : wave % PPS) + (lane >> 5);
+    uint2 wt = make_uint2(0u, 0u), wt_ahead = make_uint2(0u, 0u);
+    if constexpr (IMPL) wt_ahead = wtab[g_w];
+    auto next_words = [&]() {
+        wt = wt_ahead;
+        g_w = min(g_w + 2 * PPS, words - 1);   // (past the last stage: any entry)
+        wt_ahead = wtab[g_w];
+    };
+    const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
+    auto load = [&](int i, int step) {   // slot i of the wavefront's loads for stage `step`
+        const uint32_t dst = lds0 + (uint32_t)(step % NS) * (FR * 1024);
+        if (i < PW) {
+            dma16(psrc[i] + (size_t)step * PPS * 64, dst + (uint32_t)(wave * PW + i) * 1024);
+        } else {
+            const int j = i - PW;
+            const uint32_t d = dst + (uint32_t)(PF + wave * QW + j) * 1024;
+            if constexpr (IMPL) dma16(Qc + ((tapmask[j] & wt.x) != 0u ? qbase[j] + wt.y : fill_rec), d);   // a select on the index: no branch
+            else dma16(qsrc[j] + (size_t)step * PPS * 64, d);
+        }
+    };
+    auto stage = [&](int step) {
+        if constexpr (IMPL) next_words();
+#pragma unroll
+        for (int i = 0; i < FW; i++) load(i, step);
+    };
+    // raw: the records of the pair being consumed; e[k]: its nibbles for multiply k.  Slots in the order the multiplies take
+    // them: 0: P block 0, 1 .. WTQ: Q blocks, then P blocks 1 .. WTP - 1.
+    uint4 rp[WTP], rq[WTQ], ep[2][WTP], eq[2][WTQ];
+    auto read_raw = [&](int buf, int pair, int i) {
+        const uint4* L = lds + (size_t)buf * FR * 64 + pair * 64 + lane;
+        if (i == 0) rp[0] = L[(wy * WTP + 0) * PPS * 64];
+        else if (i <= WTQ) rq[i - 1] = L[(PF + (wx * WTQ + (i - 1)) * PPS) * 64];
+        else rp[i - WTQ] = L[(wy * WTP + (i - WTQ)) * PPS * 64];
+    };
+    auto split = [&](int k, int i) {
+        const uint4& r = i == 0 ? rp[0] : (i <= WTQ ? rq[i - 1] : rp[i - WTQ]);
+        const uint32_t d0 = k == 0 ? r.x : r.z, d1 = k == 0 ? r.y : r.w;
+        const uint4 v = make_uint4(d0 & kP2Mask, (d0 << 1) & kP2Mask, d1 & kP2Mask, (d1 << 1) & kP2Mask);
+        if (i == 0) ep[k][0] = v;
+        else if (i <= WTQ) eq[k][i - 1] = v;
+        else ep[k][i - WTQ] = v;
+    };
+    // the multiplies of slot i: the NM of a word spread evenly over the NL slots, in the order (a, b) = (m / WTQ, m % WTQ)
+    auto multiply = [&](int k, int i) {
+#pragma unroll
+        for (int m = i * NM / NL; m < (i + 1) * NM / NL; m++) mfma<true>(acc[m / WTQ][m % WTQ], ep[k][m / WTQ], eq[k][m % WTQ]);
+    };
+
+    // prologue: the first NS stages in flight, wait for stage 0 only
+#pragma unroll
+    for (int p = 0; p < NS; p++)
+        if (p < nstep) stage(p);
+    if (nstep >= NS) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FW * (NS - 1)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NL; i++) read_raw(0, 0, i);
+#pragma unroll
+    for (int i = 0; i < NL; i++) split(0, i);
+
+    // A block read in slot i is split in slot i + LAG, the last LAG ones in the first slots of the next pair, ahead of their
+    // first multiply (block b: P block 0 and Q block 0 in the slot of m = 0, Q block j of m = j, P block a of m = a WTQ).
+    auto step_body = [&](int s, auto full_tag) {
+        constexpr bool FULL = decltype(full_tag)::value;   // FULL: s + NS < nstep
+#pragma unroll
+        for (int pp = 0; pp < PPS; pp++) {
+#pragma unroll
+            for (int i = 0; i < NL; i++) {
+                if (i < LAG && (s > 0 || pp > 0)) split(0, NL - LAG + i);
+                split(1, i);
+                multiply(0, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const bool last = pp == PPS - 1;
+            if (last) {
+                // Everything of this stage is in registers.  Stage s + 1 must have landed (stages s + 2 .. s + NS - 1 may
+                // still be in flight); after the barrier buffer s % NS is free for stage s + NS.
+                if (FULL || s + NS - 1 < nstep) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FW * (NS - 2)) : "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+                if constexpr (FULL && IMPL) next_words();
+            }
+            const bool do_ld = !last || FULL || s + 1 < nstep;
+#pragma unroll
+            for (int i = 0; i < NL; i++) {
+                if (do_ld) read_raw(last ? (s + 1) % NS : s % NS, last ? 0 : pp + 1, i);
+                if (FULL && last && i < FW) load(i, s + NS);
+                if (do_ld && i >= LAG) split(0, i - LAG);
+                multiply(1, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    int s = 0;
+    for (; s + NS < nstep; s++) step_body(s, std::true_type{});
+    for (; s < nstep; s++) step_body(s, std::false_type{});
+
+    store_tile<true, SWAP, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
+}
+
 // ------------------------------------------------------------ conv layer (fp4)
 // Layer-sized problems (a few GMAC, 10^3..10^5 output pixels) are latency-, not throughput-bound,
 // and their im2row operand does not exist in memory.  This kernel therefore works on small tiles
 // with many wavefronts in flight and gathers its activation fragments itself:
 //   * a wavefront owns 64 kernels x 64 output pixels (2 x 2 MFMA blocks, 64 accumulator
 //     registers).  A workgroup is 4 wavefronts: S of them split the K loop of one tile (each takes a
-//     run of the reference's K order (kh*KW + kw)*C_pack + ic; words dealt out in turn cost layers 0.2-0.6 us
-//     more, as every step then changes the tap), so it covers 4/S pixel tiles.  S = 1 for layers with 600 tiles or more (no exchange at all), 2 or
+//     run of pairs of words in the reference's K order (kh*KW + kw)*C_pack + ic; words dealt out in turn cost layers
+//     0.2-0.6 us more, as every step then changes the tap), so it covers 4/S pixel tiles.  S = 1 for layers with 600 tiles or more (no exchange at all), 2 or
 //     4 where the tiles alone would leave most of the chip idle; the partial tiles then meet in
 //     LDS and each wavefront finishes 4/S of the tile's four blocks;
 //   * weights are the MFMA A side (rows = accumulator registers), pixels the B side (rows =
 //     lanes), so a store instruction writes 32 consecutive pixels of one NCHW plane;
-//   * an activation fragment is 32 pixels x 64 channels of one kernel tap: lane (pixel, half)
-//     loads its 16 bytes straight from P4 (k_quantize_f4's output) at the tap's input pixel,
-//     or takes the padding value: zeros for ternary inputs, +1 nibbles for binary ones (the
-//     reference's fill, src/tnns/ternarize2row_avx2.c:748-755, src/tnns/binarize2row_avx2.c:151);
-//   * the padding words that round K up to a multiple of 4 are skipped: their products are zero
-//     except for BNN, whose epilogue constant counts the real words only.
+//   * both operands come as records of two bits per lane (P2): lane (row or pixel, hw) loads the 16 bytes of word 2 i + hw of its
+//     row, which hold the operands of two multiplies; a load instruction moves two K words of 32 rows.  What bounds the
+//     K loop is the return path of vector memory, 64 bytes per cycle and compute unit over all its wavefronts: at four
+//     bits per lane a K word of a 64 x 64 tile took a wavefront 540-620 cycles, for 128 of matrix pipe;
+//   * the two words of a pair are two planes of one tap where C_pack is even (the tap is then the same for all lanes and
+//     changes every C_pack / 2 pairs), else any two neighbouring words: each lane half walks its own taps;
+//   * a tap outside the image contributes zeros for ternary inputs, +1 lanes for binary ones (the reference's fill,
+//     src/tnns/ternarize2row_avx2.c:748-755, src/tnns/binarize2row_avx2.c:151);
+//   * the words that round K up to a multiple of 4 are skipped, but for the one that makes up the last pair of an odd K: its
+//     activation lanes are zeros (BNN's epilogue constant counts the real words only).
 // ABIN: binary activations (padding value +1).  FORM0: the TNN form of PReLU, "f <= 0 -> f *= alpha"
 // (mm_p2_final_tnn_avx2.c:204-208), else "r >= 0 ? r : alpha * r" (mm_p2_final_tbn_avx2.c:73).
 // QMODE: 0 = fp32 NCHW result, 1 / 2 = ternary / binary hand-over to the next layer (QuantOut).
 // All three are compile-time so that the per-element epilogue carries no selects for them.
 // TA x TB: blocks of 32 kernels x 32 pixels per wavefront.  2 x 2, or 1 x 1 with S = 4 for layers with few tiles: a
-// wavefront moves a bounded number of bytes per cycle from a cold L2 whatever its prefetch depth (600-700 cycles per K word
-// of a 64 x 64 tile, measured), so a small layer gets faster only with more wavefronts, on more compute units.  Kernel
-// tiles of 32 come in pairs under the hand-over (a pixel's 64-channel word is written by two workgroups, 16 bytes each; a
-// tile past KN writes padding lanes).
+// wavefront moves a bounded number of bytes per cycle from a cold L2 whatever its prefetch depth, so a small layer gets faster
+// only with more wavefronts, on more compute units.  Kernel tiles of 32 come in pairs under the hand-over (a pixel's
+// record is written by two workgroups, 8 bytes each; a tile past KN writes padding lanes).
 // The unsplit hand-over variants are the ones launched with several thousand wavefronts (stems,
 // first stages): they are asked to fit three wavefronts per SIMD, which they do without scratch.
 // BUF: fragments arrive through buffer loads.  Their offsets are 32-bit, the place of a word within the operand is a
-// scalar offset, and for ternary activations an offset beyond the buffer returns zeros, which is what a
-// tap outside the image must contribute: no select on the loaded data (binary activations pad with +1 and keep the select).
-// Needs both operands below 4 GiB (p4_bytes, wf_bytes: the sizes the descriptors announce).  fp32 results leave through buffer
+// scalar offset, and an offset beyond the buffer returns zeros, which is what a tap outside the image must contribute for
+// ternary activations (binary ones or the +1 lanes in while splitting the record).
+// Needs both operands below 4 GiB (p2_bytes, wf_bytes: the sizes the descriptors announce).  fp32 results leave through buffer
 // stores too, relative to the tile's first image and kernel: y_span bounds what a tile reaches from there, whatever the size
 // of the result.
+// How a lane's word moves on when its run of pairs ends.  C_pack even: a run is the C_pack / 2 pairs of a tap, `stride` bytes
+// apart, then the next tap.  C_pack odd: every pair is a run, and both halves move on by two words = (kh, kw, ic).
+struct PairWalk {
+    int even, run, NP;       // NP: pairs per row, ceil(K / 2)
+    int dkh, dkw, dic, KH;
+    FastDiv dRun;            // C_pack / 2
+};
+inline PairWalk make_pair_walk(const ConvGeom& cg) {
+    PairWalk p;
+    p.even = cg.CP % 2 == 0;
+    p.run = p.even ? cg.CP / 2 : 1;
+    p.NP = (cg.K + 1) / 2;
+    const int taps = p.even ? 1 : 2 / cg.CP;
+    p.dic = p.even ? 0 : 2 % cg.CP;
+    p.dkh = taps / cg.KW;
+    p.dkw = taps % cg.KW;
+    p.KH = cg.K / (cg.CP * cg.KW);
+    p.dRun = make_fastdiv((uint32_t)p.run);
+    return p;
+}
+
 template <bool ABIN, bool FORM0, int QMODE, int TA, int TB, int S, bool BUF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && QMODE != 0) ? 3 : 1, 8))) void k_conv_f4(
-    const uint4* __restrict__ P4, const uint4* __restrict__ Wf, float* __restrict__ Y, int M, int KN, int OHW, int KB, int bias,
-    float alpha, FastDiv dOHW, ConvGeom cg, QuantOut qo, uint32_t p4_bytes, uint32_t wf_bytes, uint32_t y_span, XcdOrder xo, uint32_t grid_x, uint32_t grid_y) {
+    const uint4* __restrict__ P2, const uint4* __restrict__ Wf, float* __restrict__ Y, int M, int KN, int OHW, int KP /* pairs a weight row is stored at */,
+    int bias, float alpha, FastDiv dOHW, ConvGeom cg, PairWalk pw, QuantOut qo, uint32_t p2_bytes, uint32_t wf_bytes, uint32_t y_span, XcdOrder xo, uint32_t grid_x, uint32_t grid_y) {
     constexpr int WPB = 4;                // wavefronts per workgroup (single-wavefront workgroups for S = 1
                                           // measured slower: neighbours no longer share weight fragments in L1)
-    constexpr int NB = 3;                 // register sets of fragments: NB - 1 words of loads in flight; more measured no faster
+    constexpr int NB = 3;                 // register sets of records: NB - 1 pairs of loads in flight; four and six measured slower
     constexpr int NBLK = TA * TB;
     constexpr int PUB = NBLK == 1 ? 1 : 4 - 4 / S;   // blocks a wavefront hands to the others of its tile
     __shared__ float4 red[S > 1 ? 4 * PUB * 4 * 64 : 1];   // [wavefront][slot][e / 4][lane]
@@ -830,7 +953,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
     const int px0 = ((int)bx * (WPB / S) + pt) * 32 * TB, kn0 = (int)by * 32 * TA;
 
     int ih0[TB], iw0[TB];
-    uint32_t img[TB], pix[TB], xrec[TB];   // xrec: record of (image, plane 0, pixel (ih0, iw0)) in P4[n][C_pack][pixel]
+    uint32_t img[TB], pix[TB], xrec[TB];   // xrec: record of (image, plane 0, pixel (ih0, iw0)) in P2[n][C_pack][pixel]
 #pragma unroll
     for (int b = 0; b < TB; b++) {
         const uint32_t q = (uint32_t)min(px0 + 32 * b + lr, M - 1);
@@ -844,48 +967,67 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
     const int HWin = cg.H * cg.W;
     const int rbmax = (KN + 31) / 32 - 1;
 
-    // The words of this wavefront, [w, w1) of the reference's K order (kh * KW + kw) * C_pack + ic: a word is a step of
-    // one plane within a tap, so the lanes compute addresses and borders once per tap and everything else is scalar.
-    int w = S == 1 ? 0 : (int)((uint32_t)(cg.K * ks) / S);
-    const int w1 = S == 1 ? cg.K : (int)((uint32_t)(cg.K * (ks + 1)) / S);
-    const int words = w1 - w;
-    int kh = 0, kw = 0, ic = 0;
-    if constexpr (S > 1) {
-        const int tap = (int)fastdiv((uint32_t)w, cg.dCP);
-        ic = w - tap * cg.CP;
+    // The pairs of this wavefront, [p, p1).  A lane's word is 2 p + h = (kh, kw, ic) of the reference's K order; addresses and
+    // borders are computed when a run of pairs ends (PairWalk), within one everything is scalar.
+    int p = S == 1 ? 0 : (int)((uint32_t)(pw.NP * ks) / S);
+    const int p1 = S == 1 ? pw.NP : (int)((uint32_t)(pw.NP * (ks + 1)) / S);
+    const int pairs = p1 - p;
+    int kh, kw, ic, left = pw.run, soff = 0;   // pairs left in the run, scalar part of the input's byte offset
+    if (pw.even) {
+        int tap = 0;
+        if constexpr (S > 1) {
+            tap = (int)fastdiv((uint32_t)p, pw.dRun);
+            const int j = p - tap * pw.run;
+            left -= j;
+            soff = j * HWin * 32;
+        }
+        kh = S > 1 ? (int)fastdiv((uint32_t)tap, cg.dKW) : 0;
+        kw = tap - kh * cg.KW;
+        ic = h;
+    } else {
+        const uint32_t w = (uint32_t)(2 * p + h);
+        const int tap = (int)fastdiv(w, cg.dCP);
+        ic = (int)w - tap * cg.CP;
         kh = (int)fastdiv((uint32_t)tap, cg.dKW);
         kw = tap - kh * cg.KW;
     }
-    struct Frag {
+    struct Rec {
         v4i w[TA], x[TB];
-        bool in[TB];   // x[b] holds a real input pixel (else the padding value replaces it)
+        uint32_t fill[TB];   // ABIN: the nibbles that a tap outside the image is replaced by (0: none)
+        bool in[TB];         // (without BUF) x[b] holds a real input pixel
     };
-    uint32_t vx[TB];   // the tap's record (BUF: byte offset) for this lane's pixels
+    uint32_t vx[TB], fill[TB];   // the lane's record (BUF: byte offset) at its present word
     bool in[TB];
     auto tap = [&]() {
+        const bool real = kh < pw.KH;   // the word that makes up the last pair of an odd K is none
+        const uint32_t off = (uint32_t)(ic * HWin + kh * cg.W + kw);
 #pragma unroll
         for (int b = 0; b < TB; b++) {
-            in[b] = (unsigned)(ih0[b] + kh) < (unsigned)cg.H && (unsigned)(iw0[b] + kw) < (unsigned)cg.W;
-            const uint32_t rec = xrec[b] + (uint32_t)(kh * cg.W + kw);   // wraps to the right value whenever the tap is inside
-            // a tap outside the image: an offset beyond the buffer returns zeros, the padding of ternary activations;
-            // binary ones read record 0 and take the padding value in compute()
-            if (BUF) vx[b] = in[b] ? rec * 32u + 16u * (uint32_t)h : (ABIN ? 0u : 0xffffff00u);
-            else vx[b] = in[b] ? rec : 0u;
+            const bool inside = (unsigned)(ih0[b] + kh) < (unsigned)cg.H && (unsigned)(iw0[b] + kw) < (unsigned)cg.W;
+            const bool valid = inside && real;
+            if constexpr (ABIN) fill[b] = real && !inside ? 0x22222222u : 0u;   // (vx last, as in the other branch below: no register behind a pointer)
+            const uint32_t rec = xrec[b] + off;   // wraps to the right value whenever the tap is inside
+            if constexpr (BUF) {
+                vx[b] = valid ? rec * 16u : 0xffffff00u;   // an offset beyond the buffer returns zeros
+            } else {
+                vx[b] = valid ? rec : 0u;
+                in[b] = valid;
+            }
         }
     };
     tap();
     // buffer descriptors (base; stride 0; bytes; raw 32-bit data format)
-    const __amdgpu_buffer_rsrc_t brs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(P4), 0, (int)p4_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t brs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(P2), 0, (int)p2_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t brs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(Wf), 0, (int)wf_bytes, 0x00020000);
-    // All loads of a word are unconditional and are issued two words ahead of the one being multiplied.  They are ordinary
+    // All loads of a pair are unconditional and are issued two pairs ahead of the one being multiplied.  They are ordinary
     // loads (plain, or buffer-load builtins), so the compiler owns the dependency between a load and the use of its
     // registers and places every s_waitcnt vmcnt itself; what keeps a load where the code issues it -- and not next to
-    // its use, where the scheduler would sink it -- is the scheduling fence after each word's loads.
+    // its use, where the scheduler would sink it -- is the scheduling fence after each pair's loads.
     uint32_t vw = (uint32_t)lane * 16u;
-    auto load = [&](Frag& f) {   // word w, then on to the next one
+    auto load = [&](Rec& f) {   // pair p, then on to the next one
 #pragma unroll
         for (int a = 0; a < TA; a++) {
-            const uint32_t block = (uint32_t)min(kn0 / 32 + a, rbmax) * (uint32_t)KB + (uint32_t)w;
+            const uint32_t block = (uint32_t)min(kn0 / 32 + a, rbmax) * (uint32_t)KP + (uint32_t)p;
             if constexpr (BUF) {
                 const v4u v = __builtin_amdgcn_raw_buffer_load_b128(brs_w, (int)vw, (int)(block * 1024u), 0);
                 f.w[a] = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
@@ -896,24 +1038,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
 #pragma unroll
         for (int b = 0; b < TB; b++) {
             if constexpr (BUF) {
-                const v4u v = __builtin_amdgcn_raw_buffer_load_b128(brs_x, (int)vx[b], ic * HWin * 32, 0);
+                const v4u v = __builtin_amdgcn_raw_buffer_load_b128(brs_x, (int)vx[b], soff, 0);
                 f.x[b] = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
             } else {
-                f.x[b] = *reinterpret_cast<const v4i*>(P4 + (size_t)(vx[b] + (uint32_t)(in[b] ? ic * HWin : 0)) * 2 + h);
+                f.x[b] = *reinterpret_cast<const v4i*>(P2 + ((size_t)vx[b] + (size_t)(in[b] ? (uint32_t)soff / 16u : 0u)));
             }
-            f.in[b] = in[b];
+            if constexpr (!BUF) f.in[b] = in[b];
         }
-        if (w + 1 < w1) {
-            w++;
-            if (++ic == cg.CP) {
-                ic = 0;
-                if (++kw == cg.KW) {
-                    kw = 0;
-                    kh++;
-                }
+#pragma unroll
+        for (int b = 0; b < TB; b++)
+            if constexpr (ABIN) f.fill[b] = fill[b];
+        if (p + 1 < p1) {
+            p++;
+            soff += HWin * 32;
+            if (--left == 0) {
+                left = pw.run;
+                soff = 0;
+                ic += pw.dic;
+                const bool c = ic >= cg.CP;
+                ic -= c ? cg.CP : 0;
+                kw += pw.dkw + (c ? 1 : 0);
+                const bool d = kw >= cg.KW;
+                kw -= d ? cg.KW : 0;
+                kh += pw.dkh + (d ? 1 : 0);
                 tap();
             }
-        } else if (BUF) {   // past the end: offsets beyond the buffers, which move no data (else the last word is read again)
+        } else if (BUF) {   // past the end: offsets beyond the buffers, which move no data (else the last pair is read again)
             vw = 0xffffff00u;
 #pragma unroll
             for (int b = 0; b < TB; b++) vx[b] = 0xffffff00u;
@@ -921,27 +1071,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
         __builtin_amdgcn_sched_barrier(0);   // these loads stay in front of the multiplies that follow
     };
     v16f acc[TA][TB];
-    auto compute = [&](const Frag& f) {
-        v8i x[TB], wv[TA];
+    auto compute = [&](const Rec& f) {
 #pragma unroll
-        for (int b = 0; b < TB; b++) {
+        for (int k = 0; k < 2; k++) {   // dwords 0 and 1 of the records, then 2 and 3
+            v8i x[TB], wv[TA];
 #pragma unroll
-            for (int i = 0; i < 4; i++) x[b][i] = ((BUF && !ABIN) || f.in[b]) ? f.x[b][i] : (ABIN ? 0x22222222 : 0);
+            for (int b = 0; b < TB; b++) {
 #pragma unroll
-            for (int i = 4; i < 8; i++) x[b][i] = 0;
+                for (int i = 0; i < 2; i++) {
+                    const uint32_t d = BUF || f.in[b] ? (uint32_t)f.x[b][2 * k + i] : 0u;
+                    const uint32_t fl = ABIN ? f.fill[b] : 0u;
+                    x[b][2 * i] = (int)((d & kP2Mask) | fl);
+                    x[b][2 * i + 1] = (int)(((d << 1) & kP2Mask) | fl);
+                }
+#pragma unroll
+                for (int i = 4; i < 8; i++) x[b][i] = 0;
+            }
+#pragma unroll
+            for (int a = 0; a < TA; a++) {
+                const uint32_t d0 = (uint32_t)f.w[a][2 * k], d1 = (uint32_t)f.w[a][2 * k + 1];
+                wv[a] = v8i{(int)(d0 & kP2Mask), (int)((d0 << 1) & kP2Mask), (int)(d1 & kP2Mask), (int)((d1 << 1) & kP2Mask), 0, 0, 0, 0};
+            }
+            // cbsz = blgp = 4: both operands E2M1, unscaled (see mfma<true>)
+#pragma unroll
+            for (int a = 0; a < TA; a++)
+#pragma unroll
+                for (int b = 0; b < TB; b++)
+                    acc[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wv[a], x[b], acc[a][b], 4, 4, 0, 0, 0, 0);
         }
-#pragma unroll
-        for (int a = 0; a < TA; a++) wv[a] = v8i{f.w[a][0], f.w[a][1], f.w[a][2], f.w[a][3], 0, 0, 0, 0};
-        // cbsz = blgp = 4: both operands E2M1, unscaled (see mfma<true>)
-#pragma unroll
-        for (int a = 0; a < TA; a++)
-#pragma unroll
-            for (int b = 0; b < TB; b++)
-                acc[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wv[a], x[b], acc[a][b], 4, 4, 0, 0, 0, 0);
     };
 
-    // The register sets rotate by name (the loop is unrolled by NB); loads past the last word are not multiplied.
-    Frag f[NB];
+    // The register sets rotate by name (the loop is unrolled by NB); loads past the last pair are not multiplied.
+    Rec f[NB];
 #pragma unroll
     for (int j = 0; j < NB - 1; j++) load(f[j]);
     {   // the accumulators are cleared while the first loads are on their way
@@ -953,11 +1114,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
 #pragma unroll
                 for (int e = 0; e < 16; e++) acc[a][b][e] = init;
     }
-    for (int i = 0; i < words; i += NB) {   // (a share of K is empty where K < S)
+    for (int i = 0; i < pairs; i += NB) {   // (a share of K is empty where there are fewer pairs than S)
 #pragma unroll
         for (int j = 0; j < NB; j++) {
             load(f[(j + NB - 1) % NB]);
-            if (j == 0 || i + j < words) compute(f[j]);
+            if (j == 0 || i + j < pairs) compute(f[j]);
         }
     }
 
@@ -1072,30 +1233,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
             }
         });
     } else {
-        // Hand-over to an fp4 layer: a pixel's 64-channel word is 32 bytes, 16 per 32-kernel block
+        // Hand-over to an fp4 layer: dwords 2 h and 2 h + 1 of a pixel's record are lane half h of its two 32-kernel blocks
         const uint32_t KT = TA == 2 ? grid_y : grid_y >> 1, kt = TA == 2 ? by : by >> 1;
-        auto out_word = [&](int b) {
-            return static_cast<unsigned char*>(qo.p4) + (((size_t)img[b] * KT + kt) * (uint32_t)OHW + pix[b]) * 32;
+        auto out_rec = [&](int b) {
+            return static_cast<unsigned char*>(qo.p2) + (((size_t)img[b] * KT + kt) * (uint32_t)OHW + pix[b]) * 16 + 8 * h;
         };
-        if constexpr (NBLK == 4 && S < 4) {   // the wavefront finishes both kernel blocks of a pixel block: lane half h stores block h
+        if constexpr (NBLK == 4 && S < 4) {   // the wavefront finishes both kernel blocks of a pixel block
             auto pixel_block = [&](auto b_tag) {
                 constexpr int b = decltype(b_tag)::value;
                 if (b % S == ks) {
-                    const uint2 d0 = hand_over_block<FORM0, QMODE>(total(b_tag), alpha, qo, kn0, h, KN);
-                    const uint2 d1 = hand_over_block<FORM0, QMODE>(total(std::integral_constant<int, TB + b>{}), alpha, qo, kn0 + 32, h, KN);
-                    const uint4 out = exchange_blocks(d0, d1);
-                    if (px0 + 32 * b + lr < M) *reinterpret_cast<uint4*>(out_word(b) + 16 * h) = out;
+                    const uint32_t d0 = hand_over_block<FORM0, QMODE>(total(b_tag), alpha, qo, kn0, h, KN);
+                    const uint32_t d1 = hand_over_block<FORM0, QMODE>(total(std::integral_constant<int, TB + b>{}), alpha, qo, kn0 + 32, h, KN);
+                    if (px0 + 32 * b + lr < M) *reinterpret_cast<uint2*>(out_rec(b)) = make_uint2(d0, d1);
                 }
             };
             pixel_block(std::integral_constant<int, 0>{});
             pixel_block(std::integral_constant<int, 1>{});
-        } else {   // one block: lane half h stores 8 bytes
+        } else {   // one block
             for_blocks([&](auto blk_tag) {
                 constexpr int BLK = decltype(blk_tag)::value, a = BLK / TB, b = BLK % TB;
                 if (BLK % S == ks) {
-                    const uint2 out = exchange_halves(hand_over_block<FORM0, QMODE>(total(blk_tag), alpha, qo, kn0 + 32 * a, h, KN));
+                    const uint32_t d = hand_over_block<FORM0, QMODE>(total(blk_tag), alpha, qo, kn0 + 32 * a, h, KN);
                     const int part = TA == 2 ? a : (int)(by & 1u);
-                    if (px0 + 32 * b + lr < M) *reinterpret_cast<uint2*>(out_word(b) + 16 * part + 8 * h) = out;
+                    if (px0 + 32 * b + lr < M) *reinterpret_cast<uint32_t*>(out_rec(b) + 4 * part) = d;
                 }
             });
         }
@@ -1111,16 +1271,16 @@ inline int64_t mfma_small_tile_below() {
     return v;
 }
 
-template <bool F4, bool SWAP, int WTP, int WTQ, int KF, int NS>
+template <bool SWAP, int WTP, int WTQ, int KF, int NS>
 hipError_t launch_gemm_tile(const uint4* Pf, const uint4* Qf, float* Y, int M, int KN, int OHW, int KB,
                             int bias, int form, float alpha, hipStream_t st) {
-    auto kern = k_mfma<F4, SWAP, WTP, WTQ, KF, NS>;
+    auto kern = k_mfma<SWAP, WTP, WTQ, KF, NS>;
     constexpr size_t lds_bytes = Tile<WTP, WTQ, KF, NS>::lds_bytes;
     // the opt-in to more than 64 KiB of dynamic LDS is per kernel; done once, thread-safe
     // The kernel counts its LDS-direct loads by hand (s_waitcnt vmcnt(N)); a scratch access would be one more
     // vector-memory operation inside those windows, so a build of it that spills is refused (once per variant).
     static const hipError_t configured = []() {
-        const void* kern = reinterpret_cast<const void*>(&k_mfma<F4, SWAP, WTP, WTQ, KF, NS>);
+        const void* kern = reinterpret_cast<const void*>(&k_mfma<SWAP, WTP, WTQ, KF, NS>);
         hipFuncAttributes attr;
         hipError_t e = hipFuncGetAttributes(&attr, kern);
         if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
@@ -1131,38 +1291,33 @@ hipError_t launch_gemm_tile(const uint4* Pf, const uint4* Qf, float* Y, int M, i
     const int prow = SWAP ? KN : M, qrow = SWAP ? M : KN;
     dim3 grid((prow + 64 * WTP - 1) / (64 * WTP), (qrow + 64 * WTQ - 1) / (64 * WTQ));
     if (grid.y > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, ConvGeom(), FastDiv(), 0,
-                       FastDiv());
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha);
     return hipGetLastError();
 }
 
-template <bool F4, bool SWAP>
+template <bool SWAP>
 hipError_t launch_gemm(const uint4* Pf, const uint4* Qf, float* Y, int M, int KN, int OHW, int KB,
                        int bias, int form, float alpha, hipStream_t st) {
     // 256 x 256 tiles re-read the operands least, but a problem must have enough of them for the chip's
     // 256 compute units; below that, 128 x 128 tiles (two workgroups fit a compute unit)
     const int64_t big = (((int64_t)M + 255) / 256) * ((KN + 255) / 256);
     bool small = big < mfma_small_tile_below();
-    // two fragments per step and a ring of four: four fragments per step with a ring of two (the same LDS, half
-    // the barriers) measured 0.87 against 0.76 ms on 8192 x 8192 x 32768 -- the ring then no longer covers the loads
-    if constexpr (!F4) {
-        // Fewer than 112 tiles of 128 x 128 leave most compute units idle: tiles of 64 x 64 then, four K words per step
-        // (from 144 tiles on the larger tile is faster; tiles of 128 x 64 lose everywhere).  fp4 comes here from the layers'
-        // GEMM route only, which starts at 256 tiles.  FTNN_MFMA_TINY_BELOW = n moves the threshold (tuning aid).
-        static const int tiny_below = getenv("FTNN_MFMA_TINY_BELOW") ? atoi(getenv("FTNN_MFMA_TINY_BELOW")) : 112;
-        const int64_t mid = (((int64_t)M + 127) / 128) * ((KN + 127) / 128);
-        if (small && mid < tiny_below) return launch_gemm_tile<F4, SWAP, 1, 1, 4, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st);
-    }
-    return small ? launch_gemm_tile<F4, SWAP, 2, 2, 2, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st)
-                 : launch_gemm_tile<F4, SWAP, 4, 4, 2, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st);
+    // Fewer than 112 tiles of 128 x 128 leave most compute units idle: tiles of 64 x 64 then, four fragments per step
+    // (from 144 tiles on the larger tile is faster; tiles of 128 x 64 lose everywhere).
+    // FTNN_MFMA_TINY_BELOW = n moves the threshold (tuning aid).
+    static const int tiny_below = getenv("FTNN_MFMA_TINY_BELOW") ? atoi(getenv("FTNN_MFMA_TINY_BELOW")) : 112;
+    const int64_t mid = (((int64_t)M + 127) / 128) * ((KN + 127) / 128);
+    if (small && mid < tiny_below) return launch_gemm_tile<SWAP, 1, 1, 4, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st);
+    return small ? launch_gemm_tile<SWAP, 2, 2, 2, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st)
+                 : launch_gemm_tile<SWAP, 4, 4, 2, 4>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st);
 }
 
-template <bool F4>
+template <int FORM>
 hipError_t launch_expand(bool tern, const uint32_t* rows_ptr, int rows, int G, uint4* out, uint32_t* kept, hipStream_t st) {
     dim3 grid((rows + 31) / 32, (G + 3) / 4);   // 4 groups per workgroup (kGPB in the kernel)
     if (grid.y > 65535) return hipErrorInvalidValue;
-    if (tern) hipLaunchKernelGGL((k_expand<F4, true>), grid, dim3(256), 0, st, rows_ptr, rows, G, out, kept);
-    else hipLaunchKernelGGL((k_expand<F4, false>), grid, dim3(256), 0, st, rows_ptr, rows, G, out, kept);
+    if (tern) hipLaunchKernelGGL((k_expand<FORM, true>), grid, dim3(256), 0, st, rows_ptr, rows, G, out, kept);
+    else hipLaunchKernelGGL((k_expand<FORM, false>), grid, dim3(256), 0, st, rows_ptr, rows, G, out, kept);
     return hipGetLastError();
 }
 
@@ -1203,31 +1358,31 @@ int64_t mfma_fragment_bytes(bool f4, int64_t rows, int Kw) {
     return ((rows + 31) / 32) * (int64_t)(f4 ? Kw : 2 * Kw) * 1024;
 }
 
-hipError_t launch_mfma_expand(bool f4, bool ternary, const int64_t* d_rows, int rows, int Kw, void* d_out,
-                              hipStream_t st, int64_t* d_kept) {
+hipError_t launch_mfma_expand(bool ternary, const int64_t* d_rows, int rows, int Kw, void* d_out, hipStream_t st) {
+    return launch_expand<FORM_I8>(ternary, reinterpret_cast<const uint32_t*>(d_rows), rows, Kw / 4, static_cast<uint4*>(d_out), nullptr, st);
+}
+
+int64_t record_block_bytes(int64_t rows, int Kw) { return ((rows + 31) / 32) * (int64_t)(Kw / 2) * 1024; }
+
+hipError_t launch_expand_records(bool ternary, bool natural, const int64_t* d_rows, int rows, int Kw, void* d_out, hipStream_t st,
+                                 int64_t* d_kept) {
     const uint32_t* R = reinterpret_cast<const uint32_t*>(d_rows);
     uint4* out = static_cast<uint4*>(d_out);
     uint32_t* kept = reinterpret_cast<uint32_t*>(d_kept);
-    return f4 ? launch_expand<true>(ternary, R, rows, Kw / 4, out, kept, st)
-              : launch_expand<false>(ternary, R, rows, Kw / 4, out, kept, st);
+    return natural ? launch_expand<FORM_REC_NATURAL>(ternary, R, rows, Kw / 4, out, kept, st)
+                   : launch_expand<FORM_REC>(ternary, R, rows, Kw / 4, out, kept, st);
 }
 
-hipError_t launch_mfma_gemm(bool f4, int type, const void* d_af, const void* d_bf, int64_t M, int OHW, int KN,
+hipError_t launch_mfma_gemm(int type, const void* d_af, const void* d_bf, int64_t M, int OHW, int KN,
                             int Kw, int K_unpack, float alpha, float* d_y, hipStream_t st) {
-    const int KB = f4 ? Kw : 2 * Kw;
     const uint4* Af = static_cast<const uint4*>(d_af);
     const uint4* Bf = static_cast<const uint4*>(d_bf);
     // BNN: the lanes past K_unpack are +1 in both operands and add 64*Kw - K_unpack to the dot
     // product; the reference's K_unpack - 2*popc(a^b) leaves them out (mm_p2_final_bnn_avx2.c:55-58)
     const int bias = type == kBNN ? 64 * Kw - K_unpack : 0;
     const int form = type == kTNN ? 0 : 1;
-    const bool swap = OHW > 1;
-    if (f4) {
-        return swap ? launch_gemm<true, true>(Bf, Af, d_y, (int)M, KN, OHW, KB, bias, form, alpha, st)
-                    : launch_gemm<true, false>(Af, Bf, d_y, (int)M, KN, OHW, KB, bias, form, alpha, st);
-    }
-    return swap ? launch_gemm<false, true>(Bf, Af, d_y, (int)M, KN, OHW, KB, bias, form, alpha, st)
-                : launch_gemm<false, false>(Af, Bf, d_y, (int)M, KN, OHW, KB, bias, form, alpha, st);
+    return OHW > 1 ? launch_gemm<true>(Bf, Af, d_y, (int)M, KN, OHW, 2 * Kw, bias, form, alpha, st)
+                   : launch_gemm<false>(Af, Bf, d_y, (int)M, KN, OHW, 2 * Kw, bias, form, alpha, st);
 }
 
 // ---- packed4: the fp4 GEMM's operands at two bits per lane in offset codes (Kw a multiple of 4, as everywhere) ----
@@ -1276,18 +1431,19 @@ hipError_t launch_mfma_gemm_packed4(int type, const void* d_ac, const void* d_bc
 }
 
 namespace {
-constexpr int kMaxTileRouteWords = 2040;   // K words per row the tile kernel keeps a table entry for (16 KiB of LDS with the two spare ones)
-template <int WTP, int WTQ, int NS, bool BAL>
-hipError_t launch_conv_tiles_wt(const uint4* Wf, const uint4* P4, float* Y, int M, int KN, int OHW, int KB, int bias, int form,
-                                float alpha, const ConvGeom& cg, hipStream_t st) {
-    auto kern = k_mfma<true, true, WTP, WTQ, 2, NS, true, BAL>;
-    typedef Tile<WTP, WTQ, 2, NS> TL;
+constexpr int kMaxTileRouteWords = 2040;   // K words per row the tile kernel keeps a table entry for (16 KiB of LDS)
+template <bool SWAP, int WTP, int WTQ, int PPS, int NS, bool IMPL>
+hipError_t launch_records_tile(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, int pairs, int bnn_k, int form,
+                               float alpha, const ConvGeom& cg, hipStream_t st) {
+    auto kern = k_mfma_s2<SWAP, WTP, WTQ, PPS, NS, IMPL>;
+    typedef TileRec<WTP, WTQ, PPS, NS> TL;
     constexpr size_t kLdsMax = 160u << 10;   // LDS of a compute unit
-    const size_t lds_bytes = TL::lds_bytes + (size_t)(KB + 2) * 8;   // the ring, then the table of K words (+ 2 read ahead)
-    if (KB > kMaxTileRouteWords || lds_bytes > kLdsMax) return hipErrorInvalidValue;
+    const int nstep = (pairs + PPS - 1) / PPS;   // (a row is stored at an even number of pairs)
+    const size_t lds_bytes = TL::lds_bytes + (IMPL ? (size_t)nstep * PPS * 2 * 8 : 0);   // the ring, then the table of K words
+    if (lds_bytes > kLdsMax) return hipErrorInvalidValue;
     // as launch_gemm_tile: hand-counted LDS-direct loads, so no scratch; the LDS opt-in is per kernel
     static const hipError_t configured = []() {
-        const void* k = reinterpret_cast<const void*>(&k_mfma<true, true, WTP, WTQ, 2, NS, true, BAL>);
+        const void* k = reinterpret_cast<const void*>(&k_mfma_s2<SWAP, WTP, WTQ, PPS, NS, IMPL>);
         hipFuncAttributes attr;
         hipError_t e = hipFuncGetAttributes(&attr, k);
         if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
@@ -1295,13 +1451,33 @@ hipError_t launch_conv_tiles_wt(const uint4* Wf, const uint4* P4, float* Y, int 
         return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
     }();
     if (configured != hipSuccess) return configured;
-    dim3 grid((KN + 64 * WTP - 1) / (64 * WTP), (M + 64 * WTQ - 1) / (64 * WTQ));   // P = weights, Q = pixels
+    const int prow = SWAP ? KN : M, qrow = SWAP ? M : KN;
+    dim3 grid((prow + 64 * WTP - 1) / (64 * WTP), (qrow + 64 * WTQ - 1) / (64 * WTQ));
     if (grid.y > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Wf, P4, Y, M, KN, OHW, KB, bias, form, alpha, cg,
-                       make_fastdiv((uint32_t)OHW), (cg.W + cg.W_stride - 1) / cg.W_stride, make_fastdiv((uint32_t)cg.W_stride));
+    // BNN: every lane that is no real (channel, tap) is +1 x +1 in both operands, padding words included
+    const int bias = bnn_k ? 128 * nstep * PPS - bnn_k : 0;
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Pc, Qc, Y, M, KN, OHW, KP, nstep, bias, form, alpha, cg,
+                       make_fastdiv((uint32_t)OHW), IMPL ? (cg.W + cg.W_stride - 1) / cg.W_stride : 0, make_fastdiv(IMPL ? (uint32_t)cg.W_stride : 1u));
     return hipGetLastError();
 }
+
+template <bool SWAP>
+hipError_t launch_records(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int Kw, int bnn_k, int form, float alpha,
+                          hipStream_t st) {
+    const int64_t big = (((int64_t)M + 255) / 256) * ((KN + 255) / 256);
+    return big < mfma_small_tile_below()
+               ? launch_records_tile<SWAP, 2, 2, 1, 4, false>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, ConvGeom(), st)
+               : launch_records_tile<SWAP, 4, 4, 1, 4, false>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, ConvGeom(), st);
+}
 }  // namespace
+
+hipError_t launch_records_gemm(int type, const void* d_a, const void* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
+                               float alpha, float* d_y, hipStream_t st) {
+    const uint4 *A = static_cast<const uint4*>(d_a), *B = static_cast<const uint4*>(d_b);
+    const int bnn_k = type == kBNN ? K_unpack : 0, form = type == kTNN ? 0 : 1;
+    return OHW > 1 ? launch_records<true>(B, A, d_y, (int)M, KN, OHW, Kw, bnn_k, form, alpha, st)
+                   : launch_records<false>(A, B, d_y, (int)M, KN, OHW, Kw, bnn_k, form, alpha, st);
+}
 
 // A layer goes to the tile kernel with implicit im2row from 90 tiles of 128 x 128 on, if its rows have at least 16
 // words and it has at least 512 output pixels.  Measured on MI355X, the reference's batch-8 stride-2 layers, quantiser
@@ -1311,38 +1487,36 @@ hipError_t launch_conv_tiles_wt(const uint4* Wf, const uint4* P4, float* Y, int 
 // 64 x 64 are faster than both (16.5 and 28.4 us); with 52 tiles (512 channels at 28 x 28) a tie, below that the layer
 // kernels win.  FTNN_CONV_TILES_FROM = n: tuning aid; it sets the tile count and drops the conditions on words and pixels.
 namespace {
-// the tile kernel's limits: a tap mask of 32 bits per pixel, a table entry per K word, 32-bit piece indices into T4,
+// the tile kernel's limits: a tap mask of 32 bits per pixel, a table entry per K word, 32-bit record indices into T2,
 // pixel indices below 2^31 and its way of keeping kw - pad non-negative
-bool conv_tiles_within_limits(int64_t M, int CP, int taps, int64_t t4_bytes, int W_pad, int W_stride) {
+bool conv_tiles_within_limits(int64_t M, int CP, int taps, int64_t t2_bytes, int W_pad, int W_stride) {
     const int64_t K = (int64_t)CP * taps;
-    return taps <= 32 && (K + 3) / 4 * 4 <= kMaxTileRouteWords && M <= 0x7fffff00LL && t4_bytes / 16 <= 0x7fffffffLL &&
+    return taps <= 32 && (K + 3) / 4 * 4 <= kMaxTileRouteWords && M <= 0x7fffff00LL && t2_bytes / 16 <= 0x7fffffffLL &&
            W_pad < 4096 * (int64_t)W_stride;
 }
 }  // namespace
 
-bool conv_f4_tile_route(int64_t M, int KN, int CP, int taps, int64_t t4_bytes, int W_pad, int W_stride) {
+bool conv_f4_tile_route(int64_t M, int KN, int CP, int taps, int64_t t2_bytes, int W_pad, int W_stride) {
     static const char* tune = getenv("FTNN_CONV_TILES_FROM");
     static const int64_t from = tune ? atoll(tune) : 90;
     const int64_t tiles = ((M + 127) / 128) * ((KN + 127) / 128);
     const int64_t K = (int64_t)CP * taps;
-    return tiles >= from && (tune || (K >= 16 && M >= 512)) && conv_tiles_within_limits(M, CP, taps, t4_bytes, W_pad, W_stride);
+    return tiles >= from && (tune || (K >= 16 && M >= 512)) && conv_tiles_within_limits(M, CP, taps, t2_bytes, W_pad, W_stride);
 }
 
-// A large conv layer as workgroup tiles staged through LDS, the activation fragments gathered from T4
-// (launch_quantize_f4_tiled; k_mfma with IMPL): fp32 NCHW result only.  d_wf: the weights as fp4 fragments
-// (KB = round4(cg.K) words per row).
-hipError_t launch_conv_f4_tiles(int type, const void* d_p4, const void* d_wf, const ConvGeom& cg, int N, int KN, int K_unpack,
+// A large conv layer as workgroup tiles staged through LDS, the activation records gathered from T2
+// (launch_quantize_f4_tiled; k_mfma_s2 with IMPL): fp32 NCHW result only.  d_wf: the weights as record blocks
+// (round4(cg.K) words per row).
+hipError_t launch_conv_f4_tiles(int type, const void* d_t2, const void* d_wf, const ConvGeom& cg, int N, int KN, int K_unpack,
                                 float alpha, float* d_y, hipStream_t st) {
     const int OHW = cg.OH * cg.OW;
     const int64_t M = (int64_t)N * OHW;
-    const int KB = round4(cg.K);
+    const int KP = round4(cg.K) / 2, pairs = (cg.K + 1) / 2;
     if (!conv_tiles_within_limits(M, cg.CP, cg.K / cg.CP, quantize_f4_tiled_bytes(N, cg.CP * 64, cg.H, cg.W, cg.W_stride), cg.W_pad, cg.W_stride))
         return hipErrorInvalidValue;
-    // BNN: every lane that is no real (channel, tap) is +1 x +1 in both operands, padding words included
-    const int bias = type == kBNN ? 64 * KB - K_unpack : 0;
-    const int form = type == kTNN ? 0 : 1;
+    const int bnn_k = type == kBNN ? K_unpack : 0, form = type == kTNN ? 0 : 1;
     const uint4* Wf = static_cast<const uint4*>(d_wf);
-    const uint4* P4 = static_cast<const uint4*>(d_p4);
+    const uint4* T2 = static_cast<const uint4*>(d_t2);
     // tile shape (kernels x pixels): FTNN_CONV_TILE_SHAPE = 11 | 22 | 42 | 44 forces one (tuning aid)
     static const int tune = getenv("FTNN_CONV_TILE_SHAPE") ? atoi(getenv("FTNN_CONV_TILE_SHAPE")) : 0;
     // 256 x 256 tiles once they fill the chip; 256 kernels x 128 pixels where those fill most of it in one round (the
@@ -1352,20 +1526,18 @@ hipError_t launch_conv_f4_tiles(int type, const void* d_p4, const void* d_wf, co
     const int64_t sq = ((M + 127) / 128) * ((KN + 127) / 128);
     int shape = big >= mfma_small_tile_below() ? 44 : (mid >= 180 ? 42 : (sq >= 150 ? 22 : 11));
     if (tune == 11 || tune == 22 || tune == 42 || tune == 44) shape = tune;
-    // 128 x 128 and 256 x 128 tiles: every wavefront gathers a quarter of the activation fragments (1024 channels at
-    // 56 x 56, batch 8: 60.2 -> 57.4 us; 512 channels: 27.3 -> 26.8); on 64 x 64 tiles the two gathering wavefronts of the
-    // plain order are faster (28.3 against 29.0 us), and 256 x 256 tiles have no registers to spare for four gatherers
-    if (shape == 44) return launch_conv_tiles_wt<4, 4, 4, false>(Wf, P4, d_y, (int)M, KN, OHW, KB, bias, form, alpha, cg, st);
-    if (shape == 42) return launch_conv_tiles_wt<4, 2, 4, true>(Wf, P4, d_y, (int)M, KN, OHW, KB, bias, form, alpha, cg, st);
-    if (shape == 11) return launch_conv_tiles_wt<1, 1, 4, false>(Wf, P4, d_y, (int)M, KN, OHW, KB, bias, form, alpha, cg, st);
-    return launch_conv_tiles_wt<2, 2, 4, true>(Wf, P4, d_y, (int)M, KN, OHW, KB, bias, form, alpha, cg, st);
+    if (shape == 44) return launch_records_tile<true, 4, 4, 1, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
+    if (shape == 42) return launch_records_tile<true, 4, 2, 1, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
+    if (shape == 11) return launch_records_tile<true, 1, 1, 2, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
+    return launch_records_tile<true, 2, 2, 1, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
 }
 
-hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const ConvGeom& cg, int N, int KN,
+hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const ConvGeom& cg, int N, int KN,
                           int K_unpack, float alpha, float* d_y, hipStream_t st, const QuantOut& qo) {
     const int OHW = cg.OH * cg.OW;
     const int64_t M = (int64_t)N * OHW;
-    const int KB = round4(cg.K);
+    const int KP = round4(cg.K) / 2;
+    const PairWalk pw = make_pair_walk(cg);
     // BNN: the channel lanes past C are +1 in both operands (see launch_mfma_gemm); padding words are skipped
     const int bias = type == kBNN ? 64 * cg.K - K_unpack : 0;
     // K split: enough wavefronts to occupy the chip's 1024 SIMDs, but no exchange where the tiles
@@ -1378,7 +1550,7 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
         return (v == 1 || v == 2 || v == 4) ? v : 0;
     }();
     if (tune) split = tune;
-    while (split > 1 && cg.K < split) split /= 2;   // no wavefront without K words of its own, forced or not
+    while (split > 1 && pw.NP < split) split /= 2;   // no wavefront without K words of its own, forced or not
     const int wpb = 4, tpb = wpb / split;   // wavefronts and pixel tiles per workgroup (see the kernel)
     // few 64 x 64 tiles: tiles of 32 x 32, four times the workgroups
     static const int small_below = getenv("FTNN_CONV_SMALL_BELOW") ? atoi(getenv("FTNN_CONV_SMALL_BELOW")) : 150;
@@ -1386,15 +1558,15 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
     dim3 grid((unsigned)(((M + 63) / 64 + tpb - 1) / tpb), (unsigned)((KN + 63) / 64));
     if (small) grid = dim3((unsigned)((M + 31) / 32), (unsigned)(qo.mode != 0 ? 2 * ((KN + 63) / 64) : (KN + 31) / 32));
     if (M > 0x7fffff00LL || grid.y > 65535) return hipErrorInvalidValue;   // pixel indices stay below 2^31
-    const uint4* P4 = static_cast<const uint4*>(d_p4);
+    const uint4* P2 = static_cast<const uint4*>(d_p2);
     const uint4* Wf = static_cast<const uint4*>(d_wf);
     const FastDiv dOHW = make_fastdiv((uint32_t)OHW);
     // operand sizes: the buffer-load variants announce them in their descriptors
-    const int64_t p4_bytes = (int64_t)N * cg.CP * cg.H * cg.W * 32, wf_bytes = (int64_t)((KN + 31) / 32) * KB * 1024;
+    const int64_t p2_bytes = (int64_t)N * cg.CP * cg.H * cg.W * 16, wf_bytes = (int64_t)((KN + 31) / 32) * KP * 1024;
     static const bool no_buf = getenv("FTNN_CONV_NO_BUFFER_LOADS") != nullptr;   // tuning aid
     // an fp32 tile reaches over 64 kernels of its first image and as many more images as 64 pixels may touch, within the result
     const int64_t y_span = std::min(((int64_t)std::min(N - 1, 63 / OHW + 1) * KN + 64) * OHW, M * KN) * 4;
-    const bool buf = !no_buf && p4_bytes <= 0xf0000000LL && wf_bytes <= 0xf0000000LL && (qo.mode != 0 || y_span <= 0xf0000000LL);
+    const bool buf = !no_buf && p2_bytes <= 0xf0000000LL && wf_bytes <= 0xf0000000LL && (qo.mode != 0 || y_span <= 0xf0000000LL);
     auto clip = [](int64_t v) { return (uint32_t)std::min<int64_t>(v, 0xffffffffLL); };
     const uint64_t wgs = (uint64_t)grid.x * grid.y;
     if (wgs > 0xffffffffull) return hipErrorInvalidValue;   // (no such result fits in memory)
@@ -1405,8 +1577,8 @@ hipError_t launch_conv_f4(int type, const void* d_p4, const void* d_wf, const Co
         constexpr bool A = decltype(abin)::value, F = decltype(form0)::value;
         constexpr int Q = decltype(qmode)::value, T = decltype(blocks)::value, SP = decltype(sp)::value;
         auto go = [&](auto kern) -> hipError_t {
-            hipLaunchKernelGGL(kern, grid, dim3(64 * wpb), 0, st, P4, Wf, d_y, (int)M, KN, OHW, KB, bias, alpha, dOHW, cg, qo,
-                               clip(p4_bytes), clip(wf_bytes), clip(y_span), xo, grid.x, grid.y);
+            hipLaunchKernelGGL(kern, grid, dim3(64 * wpb), 0, st, P2, Wf, d_y, (int)M, KN, OHW, KP, bias, alpha, dOHW, cg, pw, qo,
+                               clip(p2_bytes), clip(wf_bytes), clip(y_span), xo, grid.x, grid.y);
             return hipGetLastError();
         };
         return buf ? go(k_conv_f4<A, F, Q, T, T, SP, true>) : go(k_conv_f4<A, F, Q, T, T, SP, false>);
@@ -1485,7 +1657,7 @@ hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* 
         if (grid.y > 65535) return hipErrorInvalidValue;
         const uint32_t *Ra = reinterpret_cast<const uint32_t*>(d_a), *Rb = reinterpret_cast<const uint32_t*>(d_b);
         uint4 *Oa = static_cast<uint4*>(Af), *Ob = static_cast<uint4*>(Bf);
-#define FTNN_EXP2(TA_, TB_) hipLaunchKernelGGL((k_expand2<false, TA_, TB_>), grid, dim3(256), 0, st, Ra, (int)M, Oa, Rb, KN, Ob, Kw / 4)
+#define FTNN_EXP2(TA_, TB_) hipLaunchKernelGGL((k_expand2<TA_, TB_>), grid, dim3(256), 0, st, Ra, (int)M, Oa, Rb, KN, Ob, Kw / 4)
         if (a_tern && b_tern) FTNN_EXP2(true, true);
         else if (a_tern) FTNN_EXP2(true, false);
         else if (b_tern) FTNN_EXP2(false, true);
@@ -1494,7 +1666,7 @@ hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* 
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    return launch_mfma_gemm(false, type, Af, Bf, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
+    return launch_mfma_gemm(type, Af, Bf, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
 }
 
 }  // namespace ftnn

@@ -388,24 +388,22 @@ __global__ __launch_bounds__(KS ? 64 * KS : 256) void k_mm(const uint32_t* __res
         const int64_t i = row0 + lane + 64 * a;
         if (i < M) {
             if (!TR && qo.mode != 0) {
-                // hand-over to an fp4 layer: this lane's TN kernels are TN consecutive nibbles of one pixel
+                // hand-over to an fp4 layer: this lane's TN kernels are one or two bytes of a pixel's record, four kernels each
                 const uint32_t img = fastdiv((uint32_t)i, dOHW);
                 const uint32_t pix = (uint32_t)i - img * (uint32_t)OHW;
                 const float t = qo.t;
-                uint32_t dw = 0u;
-                const bool tern = qo.mode == 1;
-                if (col0 + TN <= KN) {   // uniform: all of this wavefront's columns are real kernels
-#pragma unroll
-                    for (int b = 0; b < TN; b++) dw |= quant_nibble(finish(a, b), t, tern, true) << (4 * b);
-                } else {
-#pragma unroll
-                    for (int b = 0; b < TN; b++) dw |= quant_nibble(finish(a, b), t, tern, col0 + b < KN) << (4 * b);
-                }
+                const bool tern = qo.mode == 1, whole = col0 + TN <= KN;   // uniform: all of this wavefront's columns are real kernels
                 const size_t word = ((size_t)img * ((KN + 63) / 64) + (col0 >> 6)) * OHW + pix;
-                unsigned char* dst = static_cast<unsigned char*>(qo.p4) + word * 32 + ((col0 & 63) >> 1);
-                if (TN == 8) *reinterpret_cast<uint32_t*>(dst) = dw;
-                else if (TN == 4) *reinterpret_cast<unsigned short*>(dst) = (unsigned short)dw;
-                else *dst = (unsigned char)dw;
+                unsigned char* dst = static_cast<unsigned char*>(qo.p2) + word * 16 + 4 * ((col0 >> 5) & 1) + ((col0 >> 3) & 3);
+                if constexpr (TN >= 4) {   // (the launcher takes no narrower tile: two kernels are half a byte)
+#pragma unroll
+                    for (int b = 0; b < TN; b += 4) {
+                        uint32_t n[4];
+#pragma unroll
+                        for (int j = 0; j < 4; j++) n[j] = quant_nibble(finish(a, b + j), t, tern, whole || col0 + b + j < KN);
+                        dst[8 * (((col0 + b) >> 2) & 1)] = (unsigned char)(p2_join(n[0], n[1]) | p2_join(n[2], n[3]) << 4);
+                    }
+                }
             } else if (TR) {   // consecutive lanes write consecutive floats of one output row
 #pragma unroll
                 for (int b = 0; b < TN; b++) {
@@ -464,7 +462,8 @@ hipError_t launch_mode(const uint32_t* A, const uint32_t* B, float* Y, int64_t M
         sscanf(force, "%d,%d", &tm, &tn);
 #define FTNN_TRY(TM_, TN_) \
     if (tm == TM_ && tn == TN_) return launch_cfg<MODE, TM_, TN_, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
-        FTNN_TRY(2, 8) FTNN_TRY(1, 8) FTNN_TRY(1, 4) FTNN_TRY(1, 2)
+        FTNN_TRY(2, 8) FTNN_TRY(1, 8) FTNN_TRY(1, 4)
+        if (qo.mode == 0) { FTNN_TRY(1, 2) }
 #undef FTNN_TRY
     }
     // Few tiles and a K loop worth splitting: the wavefronts of a workgroup share K (KS in the kernel).  Measured on
@@ -486,7 +485,8 @@ hipError_t launch_mode(const uint32_t* A, const uint32_t* B, float* Y, int64_t M
     }
     if (wgs(2, 8) >= 3072) return launch_cfg<MODE, 2, 8, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
     if (wgs(1, 8) >= 1536) return launch_cfg<MODE, 1, 8, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
-    if (wgs(1, 4) >= 2048) return launch_cfg<MODE, 1, 4, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
+    // (a hand-over writes whole bytes of four kernels)
+    if (wgs(1, 4) >= 2048 || qo.mode != 0) return launch_cfg<MODE, 1, 4, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
     return launch_cfg<MODE, 1, 2, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
 }
 

@@ -78,77 +78,76 @@ __global__ __launch_bounds__(256) void k_quantize_pixels(const float* __restrict
     }
 }
 
-// Quantise straight into the operand form of the fp4 matrix-core layer kernel: one E2M1 nibble
-// per channel (0x2 = +1, 0x0 = 0, 0xA = -1; low nibble = even channel), 32 bytes per pixel and
-// 64 channels, in planes of 64 channels: P4[n][C_pack][pixel][32 bytes], so that the 32
-// consecutive pixels of a matrix-core fragment are (for stride 1) one contiguous KiB.  Channels past C read as the reference's padding
-// lanes: zero for ternary inputs (src/tnns/ternarize2row_avx2.c:440-441), +1 for binary ones
-// (cleared bits, src/tnns/binarize2row_avx2.c:151).  Same block shape and loads as
-// k_quantize_pixels; a thread's 8 channels are one dword, transposed through LDS so that a
-// pixel's 32 bytes leave contiguously.
-// TILED: the operand of the tile kernel with implicit im2row instead (k_mfma, IMPL): the two 16-byte halves of a record in
-// planes of their own, and the columns of an image row sorted by column % stride_w, T4[n][C_pack][half][row][column %
-// s][column / s][16 bytes] with ceil(W / s) slots per class: the 32 lanes of a fragment half -- consecutive output
-// pixels, i.e. input columns s apart -- then read consecutive 16-byte pieces within an output row, whatever the stride.
-template <bool TERN, bool TILED = false>
+// Quantise straight into the operand form of the fp4 layer kernels: two bits per channel, a record of 16 bytes per pixel and 64
+// channels (see P2), in planes of 64 channels: P2[n][C_pack][pixel][16 bytes].  Channels past C read as the reference's padding
+// lanes: zero for ternary inputs (src/tnns/ternarize2row_avx2.c:440-441), +1 for binary ones (cleared bits,
+// src/tnns/binarize2row_avx2.c:151).  grid (pixels / PX, C_pack, N); the records leave through LDS as one contiguous piece.
+// Bound by reading the fp32 input: PX = 64, where a thread makes one dword of a record out of 16 channels with 16 coalesced loads
+// in flight (8 x 1024 x 56 x 56: 17.0 us against 18.1 on PX = 32).  Small inputs, which last no longer than a launch, have twice the
+// wavefronts with PX = 32, a thread making half a dword out of 8 channels.
+// TILED: the operand of the tile kernel with implicit im2row instead (k_mfma_s2, IMPL): the columns of an image row sorted by
+// column % stride_w, T2[n][C_pack][row][column % s][column / s][16 bytes] with ceil(W / s) slots per class: the 32 lanes of a
+// fragment half -- consecutive output pixels, i.e. input columns s apart -- then read consecutive records within an output
+// row, whatever the stride.
+template <bool TERN, bool TILED, int PX>
 __global__ __launch_bounds__(256) void k_quantize_f4(const float* __restrict__ x,
                                                      const float* __restrict__ thr, int C, int HW,
-                                                     int CP, uint32_t* __restrict__ P4, int W = 0, int SW = 1, int Ws = 0,
-                                                     FastDiv dW = FastDiv(), FastDiv dSW = FastDiv()) {
-    __shared__ uint32_t s_dw[32 * 9];
-    const int px = threadIdx.x & 31, oct = threadIdx.x >> 5;
-    const int p = blockIdx.x * 32 + px;
+                                                     int CP, uint4* __restrict__ P2, int W, int SW, int Ws,
+                                                     FastDiv dW, FastDiv dSW) {
+    static_assert(PX == 64 || PX == 32, "a dword or half a dword of a record per thread");
+    constexpr int NC = PX / 4;   // channels of a thread
+    __shared__ uint32_t s_dw[PX * 5];
+    const int px = threadIdx.x % PX;
+    const int part = PX == 64 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / PX)) : (int)(threadIdx.x / PX);
+    const int j = PX == 64 ? part : part >> 1, q0 = PX == 64 ? 0 : 2 * (part & 1);   // dword 2 h + a of the record, its first byte
+    const int p = blockIdx.x * PX + px;
     const int ic = blockIdx.y, n = blockIdx.z;
     const float t = thr[n];
-    const int c0 = ic * 64 + oct * 8;
-    uint32_t dw = TERN ? 0u : 0x22222222u;
+    const int c0 = ic * 64 + 32 * (j & 1) + 4 * (j >> 1) + 8 * q0;   // channels c0 + 8 q + i
     if (p < HW) {
         const float* xp = x + ((size_t)n * C + c0) * HW + p;
-        float v[8];
+        float v[NC];
 #pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = (c0 + j < C) ? xp[(size_t)j * HW] : 0.0f;
-        dw = 0u;
+        for (int e = 0; e < NC; e++) {
+            const int d = 8 * (e >> 2) + (e & 3);
+            v[e] = c0 + d < C ? xp[(size_t)d * HW] : 0.0f;
+        }
+        uint32_t dw = 0u;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            uint32_t nib;
+        for (int e = 0; e < NC; e++) {
+            const bool real = c0 + 8 * (e >> 2) + (e & 3) < C;
+            uint32_t code;   // bit 0: not zero, bit 2: negative
             if (TERN) {
                 // strict compares, src/tnns/ternarize2row_avx2.c:443-449
-                nib = v[j] < -t ? 0xAu : (v[j] > t ? 0x2u : 0x0u);
-                if (c0 + j >= C) nib = 0x0u;
+                code = v[e] < -t ? 5u : (v[e] > t ? 1u : 0u);
+                if (!real) code = 0u;
             } else {
                 // src/tnns/binarize2row_avx2.c:19-21
-                nib = v[j] < t ? 0xAu : 0x2u;
-                if (c0 + j >= C) nib = 0x2u;
+                code = v[e] < t ? 5u : 1u;
+                if (!real) code = 1u;
             }
-            dw |= nib << (4 * j);
+            dw |= code << (4 * (e >> 1) + 1 - (e & 1));
         }
+        if constexpr (PX == 64) s_dw[px * 5 + j] = dw;
+        else reinterpret_cast<uint16_t*>(s_dw)[(px * 5 + j) * 2 + (part & 1)] = (uint16_t)dw;
     }
-    s_dw[px * 9 + oct] = dw;
     __syncthreads();
+    if (threadIdx.x < PX && p < HW) {
+        const uint32_t* d = s_dw + px * 5;
+        size_t piece = ((size_t)n * CP + ic) * HW + p;
+        if constexpr (TILED) {
+            const uint32_t ih = fastdiv((uint32_t)p, dW), iw = (uint32_t)p - ih * (uint32_t)W;
+            const uint32_t cls_q = fastdiv(iw, dSW), cls = iw - cls_q * (uint32_t)SW;
+            piece = (((size_t)n * CP + ic) * (HW / W) + ih) * ((size_t)SW * Ws) + (size_t)cls * Ws + cls_q;
+        }
+        P2[piece] = make_uint4(d[0], d[1], d[2], d[3]);
+    }
     if constexpr (TILED) {
-        // thread (pixel, half) stores the half record's 16 bytes
-        if (threadIdx.x < 64) {
-            const int wp = threadIdx.x & 31, half = threadIdx.x >> 5;
-            const int q = blockIdx.x * 32 + wp;
-            if (q < HW) {
-                const uint32_t ih = fastdiv((uint32_t)q, dW), iw = (uint32_t)q - ih * (uint32_t)W;
-                const uint32_t cls_q = fastdiv(iw, dSW), cls = iw - cls_q * (uint32_t)SW;
-                const int H = HW / W;
-                const size_t piece = ((((size_t)n * CP + ic) * 2 + half) * H + ih) * ((size_t)SW * Ws) + (size_t)cls * Ws + cls_q;
-                const uint32_t* d = s_dw + wp * 9 + half * 4;
-                reinterpret_cast<uint4*>(P4)[piece] = make_uint4(d[0], d[1], d[2], d[3]);
-            }
-        }
-        // the fill piece right behind the planes: what a tap outside the image contributes (0, or +1 for binary inputs)
+        // the fill record right behind the planes: what a tap outside the image contributes (0, or +1 for binary inputs)
         if (threadIdx.x == 64 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
-            const uint32_t f = TERN ? 0u : 0x22222222u;
-            const int H = HW / W;
-            reinterpret_cast<uint4*>(P4)[(size_t)gridDim.z * CP * 2 * H * ((size_t)SW * Ws)] = make_uint4(f, f, f, f);
+            const uint32_t f = TERN ? 0u : kP2Plus;
+            P2[(size_t)gridDim.z * CP * (HW / W) * ((size_t)SW * Ws)] = make_uint4(f, f, f, f);
         }
-    } else {
-        const int wp = threadIdx.x >> 3, wo = threadIdx.x & 7;
-        const int q = blockIdx.x * 32 + wp;
-        if (q < HW) P4[(((size_t)n * CP + ic) * HW + q) * 8 + wo] = s_dw[wp * 9 + wo];
     }
 }
 
@@ -374,15 +373,15 @@ __global__ __launch_bounds__(256) void k_quantize_nib(const float* __restrict__ 
 // nibbles together, T = 64 / C taps per 64-lane word (lane (tap % T)*C + c, as in k_dense_rows), the
 // lanes left over holding the padding lane of the type like taps outside the image.  C is a template
 // parameter: every shift and every position in the word's eight dwords is then a constant, the word
-// is assembled in registers and leaves as two 16-byte stores (32 contiguous bytes per pixel,
-// neighbouring pixels next to each other).
+// is assembled in registers and leaves as a record of 16 bytes in natural lane order (neighbouring pixels
+// next to each other).
 // Output = the fp4 layer kernel's operand for a 1x1 layer over the output pixels with Kd words per
-// pixel: A4[n][d][pixel][32 bytes].
+// pixel: A2[n][d][pixel][16 bytes].
 template <bool TERN, int C>
 __global__ __launch_bounds__(256) void k_dense_rows_f4(const uint32_t* __restrict__ Pq, int H, int W, int OHW,
                                                        int OW, int KW, int taps, int Kd, int H_pad, int W_pad,
                                                        int H_stride, int W_stride, FastDiv dOW,
-                                                       uint4* __restrict__ A4) {
+                                                       uint4* __restrict__ A2) {
     constexpr int T = 64 / C;
     constexpr uint32_t padv = TERN ? 0u : 0x22222222u;
     constexpr uint32_t cmask = C >= 8 ? 0xffffffffu : ((1u << (4 * (C & 7))) - 1u);
@@ -417,9 +416,8 @@ __global__ __launch_bounds__(256) void k_dense_rows_f4(const uint32_t* __restric
                 o[lo + 1] = (o[lo + 1] & ~(cmask >> rest)) | (v >> rest);
             }
         }
-        uint4* dst = A4 + (((size_t)n * Kd + d) * OHW + pix) * 2;
-        dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
-        dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
+        A2[((size_t)n * Kd + d) * OHW + pix] =
+            make_uint4(p2_join(o[0], o[1]), p2_join(o[2], o[3]), p2_join(o[4], o[5]), p2_join(o[6], o[7]));
     }
 }
 
@@ -430,7 +428,7 @@ __global__ __launch_bounds__(256) void k_dense_rows_f4(const uint32_t* __restric
 template <bool TERN, int C, int KH, int KW>
 __global__ __launch_bounds__(256) void k_dense_rows_f4_win(const uint32_t* __restrict__ Pq, int H, int W, int OHW,
                                                            int OW, int H_pad, int W_pad, int H_stride, int W_stride,
-                                                           FastDiv dOW, uint4* __restrict__ A4) {
+                                                           FastDiv dOW, uint4* __restrict__ A2) {
     constexpr int T = 64 / C, taps = KH * KW, Kd = (taps + T - 1) / T;
     constexpr uint32_t padv = TERN ? 0u : 0x22222222u;
     constexpr uint32_t cmask = C >= 8 ? 0xffffffffu : ((1u << (4 * (C & 7))) - 1u);
@@ -480,9 +478,8 @@ __global__ __launch_bounds__(256) void k_dense_rows_f4_win(const uint32_t* __res
             if (32 * i >= used) o[i] |= padv;
             else if (32 * (i + 1) > used) o[i] |= padv & ~((1u << (used - 32 * i)) - 1u);
         }
-        uint4* dst = A4 + (((size_t)n * Kd + d) * OHW + pix) * 2;
-        dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
-        dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
+        A2[((size_t)n * Kd + d) * OHW + pix] =
+            make_uint4(p2_join(o[0], o[1]), p2_join(o[2], o[3]), p2_join(o[4], o[5]), p2_join(o[6], o[7]));
     }
 }
 
@@ -556,14 +553,14 @@ int64_t dense_f4_pq_bytes(int N, int H, int W) { return ((int64_t)N * H * W * 4 
 
 hipError_t launch_dense_rows_f4(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
                                 int H_pad, int W_pad, int kH, int kW, int H_stride, int W_stride, void* d_pq,
-                                void* d_a4, hipStream_t st) {
+                                void* d_a2, hipStream_t st) {
     int T, Kd;
     dense_applies(C, kH, kW, &T, &Kd);
     const int OH = out_dim(H, H_pad, kH, H_stride), OW = out_dim(W, W_pad, kW, W_stride);
     const int HW = H * W, OHW = OH * OW;
     if (N > 65535 || Kd > 65535) return hipErrorInvalidValue;
     uint32_t* Pq = static_cast<uint32_t*>(d_pq);
-    uint4* A4 = static_cast<uint4*>(d_a4);
+    uint4* A2 = static_cast<uint4*>(d_a2);
     dim3 gq((HW + 255) / 256, N), gr((OHW + 255) / 256, N);
     const FastDiv dOW = make_fastdiv((uint32_t)OW);
     (void)T;
@@ -571,12 +568,12 @@ hipError_t launch_dense_rows_f4(bool ternary, const float* d_x, const float* d_t
     else hipLaunchKernelGGL((k_quantize_nib<false>), gq, dim3(256), 0, st, d_x, d_thr, C, HW, Pq);
 #define FTNN_DENSE_WIN(TERN_, C_, K_)                                                                             \
     hipLaunchKernelGGL((k_dense_rows_f4_win<TERN_, C_, K_, K_>), gr, dim3(256), 0, st, Pq, H, W, OHW, OW, H_pad, W_pad, \
-                       H_stride, W_stride, dOW, A4)
+                       H_stride, W_stride, dOW, A2)
 #define FTNN_DENSE_T(TERN_, C_)                                                                                     \
     if (kH == 3 && kW == 3) FTNN_DENSE_WIN(TERN_, C_, 3);                                                           \
     else if (kH == 7 && kW == 7) FTNN_DENSE_WIN(TERN_, C_, 7);                                                      \
     else hipLaunchKernelGGL((k_dense_rows_f4<TERN_, C_>), gr, dim3(256), 0, st, Pq, H, W, OHW, OW, kW, kH * kW, Kd,    \
-                            H_pad, W_pad, H_stride, W_stride, dOW, A4)
+                            H_pad, W_pad, H_stride, W_stride, dOW, A2)
 #define FTNN_DENSE(C_)                                                                                              \
     case C_:                                                                                                        \
         if (ternary) { FTNN_DENSE_T(true, C_); }                                                                    \
@@ -635,14 +632,31 @@ hipError_t launch_quantize(bool ternary, const float* d_x, const float* d_thr, i
     return hipGetLastError();
 }
 
+namespace {
+// PX: the larger workgroup tile from 1024 workgroups on, where the input comes from HBM
+hipError_t launch_quantize_records(bool ternary, bool tiled, const float* d_x, const float* d_thr, int N, int C, int H, int W, int SW,
+                                   void* d_out, hipStream_t st) {
+    const int CP = cpack_of(C), HW = H * W, Ws = (W + SW - 1) / SW;
+    const bool large = (int64_t)((HW + 63) / 64) * CP * N >= 1024;
+    const int px = large ? 64 : 32;
+    const dim3 grid((HW + px - 1) / px, CP, N);
+    const FastDiv dW = make_fastdiv((uint32_t)W), dSW = make_fastdiv((uint32_t)SW);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, d_x, d_thr, C, HW, CP, static_cast<uint4*>(d_out), W, SW, Ws, dW, dSW);
+        return hipGetLastError();
+    };
+    if (ternary) {
+        if (tiled) return large ? go(k_quantize_f4<true, true, 64>) : go(k_quantize_f4<true, true, 32>);
+        return large ? go(k_quantize_f4<true, false, 64>) : go(k_quantize_f4<true, false, 32>);
+    }
+    if (tiled) return large ? go(k_quantize_f4<false, true, 64>) : go(k_quantize_f4<false, true, 32>);
+    return large ? go(k_quantize_f4<false, false, 64>) : go(k_quantize_f4<false, false, 32>);
+}
+}  // namespace
+
 hipError_t launch_quantize_f4(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
-                              void* d_p4, hipStream_t st) {
-    const int CP = cpack_of(C), HW = H * W;
-    dim3 grid((HW + 31) / 32, CP, N);
-    uint32_t* P4 = static_cast<uint32_t*>(d_p4);
-    if (ternary) hipLaunchKernelGGL((k_quantize_f4<true>), grid, dim3(256), 0, st, d_x, d_thr, C, HW, CP, P4, 0, 1, 0, FastDiv(), FastDiv());
-    else hipLaunchKernelGGL((k_quantize_f4<false>), grid, dim3(256), 0, st, d_x, d_thr, C, HW, CP, P4, 0, 1, 0, FastDiv(), FastDiv());
-    return hipGetLastError();
+                              void* d_p2, hipStream_t st) {
+    return launch_quantize_records(ternary, false, d_x, d_thr, N, C, H, W, 1, d_p2, st);
 }
 
 // fp32 rows -> Packing-2 rows of round4(ceil(C / 64)) words, the pad words filled as the im2row operand's: a row per image of a
@@ -657,21 +671,15 @@ hipError_t launch_quantize_rows(bool ternary, const float* d_x, const float* d_t
     return hipGetLastError();
 }
 
-// bytes of T4 (k_quantize_f4 with TILED) for this input and column stride
+// bytes of T2 (k_quantize_f4 with TILED) for this input and column stride
 int64_t quantize_f4_tiled_bytes(int N, int C, int H, int W, int W_stride) {
-    return (int64_t)N * cpack_of(C) * 2 * H * W_stride * ((W + W_stride - 1) / W_stride) * 16 + 16;   // + the fill piece
+    return (int64_t)N * cpack_of(C) * H * W_stride * ((W + W_stride - 1) / W_stride) * 16 + 16;   // + the fill record
 }
 
 hipError_t launch_quantize_f4_tiled(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
-                                    int W_stride, void* d_t4, hipStream_t st) {
-    const int CP = cpack_of(C), HW = H * W, Ws = (W + W_stride - 1) / W_stride;
-    dim3 grid((HW + 31) / 32, CP, N);
-    uint32_t* T4 = static_cast<uint32_t*>(d_t4);
-    const FastDiv dW = make_fastdiv((uint32_t)W), dSW = make_fastdiv((uint32_t)W_stride);
+                                    int W_stride, void* d_t2, hipStream_t st) {
     // slots of a class past its last column (W % s != 0) are never read: the gather reads real columns only
-    if (ternary) hipLaunchKernelGGL((k_quantize_f4<true, true>), grid, dim3(256), 0, st, d_x, d_thr, C, HW, CP, T4, W, W_stride, Ws, dW, dSW);
-    else hipLaunchKernelGGL((k_quantize_f4<false, true>), grid, dim3(256), 0, st, d_x, d_thr, C, HW, CP, T4, W, W_stride, Ws, dW, dSW);
-    return hipGetLastError();
+    return launch_quantize_records(ternary, true, d_x, d_thr, N, C, H, W, W_stride, d_t2, st);
 }
 
 hipError_t launch_quantize_im2row(bool ternary, const float* d_x, const float* d_thr, int N, int C,

@@ -41,7 +41,7 @@ struct StemGeom {
 // ABIN / FORM0 / QMODE as in k_conv_f4; C is compile-time so that every shift below is a constant.
 template <bool ABIN, bool FORM0, int QMODE, int C>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_stem_f4(
-    const float* __restrict__ x, const float* __restrict__ thr, const uint4* __restrict__ Wf, float* __restrict__ Y,
+    const float* __restrict__ x, const float* __restrict__ thr, const uint2* __restrict__ Wf, float* __restrict__ Y,
     int KN, int KB, int bias, float alpha, StemGeom g, QuantOut qo) {
     constexpr int T = 64 / C;                    // taps per word
     constexpr int J1 = 32 / C;                   // first tap that reaches into the upper half of a word
@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     const int PP = g.PH * g.PW;
     uint32_t* patch = lds;                 // [0, PP): the quantised patch; [PP, 2 PP): padding nibbles
     uint32_t* toff = lds + 2 * PP;         // [Kd][TT]: byte offset of a tap in the patch (or into the padding)
-    // [Kd][2] weight fragments of this kernel tile, 16-byte aligned behind the table
+    // [Kd][2] weight fragments of this kernel tile (nibbles), 16-byte aligned behind the table
     uint4* wl = reinterpret_cast<uint4*>(lds + (2 * PP + g.Kd * TT + 3) / 4 * 4);
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -82,13 +82,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         const float t = thr[n];
         const int ihb = oh0 * g.H_stride - g.H_pad, iwb = ow0 * g.W_stride - g.W_pad;
         const float* xn = x + (size_t)n * C * HW;
-        uint4 wreg[kWR];
-#pragma unroll
-        for (int k = 0; k < kWR; k++) {
-            const int i = min(tid + NT * k, nwf - 1);
+        // piece i of the fragments = word d, block a, lane (K half, row): half of the row's record, unpacked on the way into LDS
+        auto wsrc = [&](int i) {
             const int d = i >> 7, a = (i >> 6) & 1, l = i & 63;
-            wreg[k] = Wf[((size_t)min(kn0 / 32 + a, rbm) * KB + d) * 64 + l];
-        }
+            return Wf[(((size_t)min(kn0 / 32 + a, rbm) * (KB >> 1) + (d >> 1)) * 64 + (d & 1) * 32 + (l & 31)) * 2 + (l >> 5)];
+        };
+        auto nibbles = [](const uint2& r) {
+            return make_uint4(r.x & kP2Mask, (r.x << 1) & kP2Mask, r.y & kP2Mask, (r.y << 1) & kP2Mask);
+        };
+        uint2 wreg[kWR];
+#pragma unroll
+        for (int k = 0; k < kWR; k++) wreg[k] = wsrc(min(tid + NT * k, nwf - 1));
         // kCH patch pixels per thread and round, all their loads issued before the first is used: the fill is a
         // chain of memory latencies otherwise (one round covers the 37 x 37 patch of a stride-2 7x7 layer)
         constexpr int kCH = 6;
@@ -127,11 +131,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         }
 #pragma unroll
         for (int k = 0; k < kWR; k++)
-            if (tid + NT * k < nwf) wl[tid + NT * k] = wreg[k];
-        for (int i = tid + NT * kWR; i < nwf; i += NT) {   // more than 4 words: the rest, one by one
-            const int d = i >> 7, a = (i >> 6) & 1, l = i & 63;
-            wl[i] = Wf[((size_t)min(kn0 / 32 + a, rbm) * KB + d) * 64 + l];
-        }
+            if (tid + NT * k < nwf) wl[tid + NT * k] = nibbles(wreg[k]);
+        for (int i = tid + NT * kWR; i < nwf; i += NT) wl[i] = nibbles(wsrc(i));   // more than 4 words: the rest, one by one
         for (int idx = tid; idx < g.Kd * TT; idx += NT) {
             const int d = idx / TT, j = idx - d * TT;
             const int tap = d * T + j;
@@ -232,12 +233,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
                 }
             }
         } else {
-            // as in k_conv_f4: lane half h ends up with bytes 16 h .. 16 h + 15 of the pixel's 64-channel word
-            const uint2 d0 = hand_over_block<FORM0, QMODE>(acc[0][b], alpha, qo, kn0, h, KN);
-            const uint2 d1 = hand_over_block<FORM0, QMODE>(acc[1][b], alpha, qo, kn0 + 32, h, KN);
+            // as in k_conv_f4: lane half h holds dwords 2 h and 2 h + 1 of the pixel's record
+            const uint2 out = make_uint2(hand_over_block<FORM0, QMODE>(acc[0][b], alpha, qo, kn0, h, KN),
+                                         hand_over_block<FORM0, QMODE>(acc[1][b], alpha, qo, kn0 + 32, h, KN));
             const size_t word = ((size_t)n * g.kn_tiles + kt) * OHW + pix;
-            const uint4 out = exchange_blocks(d0, d1);
-            if (live) *reinterpret_cast<uint4*>(static_cast<unsigned char*>(qo.p4) + word * 32 + 16 * h) = out;
+            if (live) *reinterpret_cast<uint2*>(static_cast<unsigned char*>(qo.p2) + word * 16 + 8 * h) = out;
         }
     }
 }
@@ -292,7 +292,7 @@ hipError_t launch_stem_f4(int type, const float* d_x, const float* d_thr, const 
     g.dTiles = make_fastdiv((uint32_t)tiles);
     g.xo = make_xcd_order((uint64_t)N, (uint32_t)(tiles * kn_tiles), qo.mode == 0 && (int64_t)N * KN * OH * OW * 4 > kXcdOrderResultBytes);
     const dim3 grid((unsigned)tiles, (unsigned)kn_tiles, (unsigned)N);   // (in one dimension 2^32 threads would bound it)
-    const uint4* Wf = static_cast<const uint4*>(d_wf);
+    const uint2* Wf = static_cast<const uint2*>(d_wf);
     const int KB = round4(Kd);
     // BNN: every lane of the Kd words that is not a real (tap, channel) is +1 in both operands
     const int bias = type == kBNN ? 64 * Kd - C * taps : 0;
