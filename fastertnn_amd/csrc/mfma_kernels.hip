@@ -208,7 +208,7 @@ __device__ __forceinline__ void dma16(const uint4* gsrc, uint32_t lds_byte_addr)
 // (f <= 0) f *= alpha", mm_p2_final_tnn_avx2.c:204-208; form 1 "r >= 0 ? r : alpha * r", mm_p2_final_tbn_avx2.c:73), stored
 // row-major (SWAP = false, OHW == 1) or in NCHW order.  Accumulator e of block (a, b): P row = 32 * (prb + a) + 8 * (e / 4)
 // + 4 * (lane / 32) + e % 4, Q row = 32 * (qrb + b) + lane % 32.
-template <bool F4, bool SWAP, int WTP, int WTQ>
+template <bool F4, bool SWAP, bool NT, int WTP, int WTQ>
 __device__ __forceinline__ void store_tile(const typename Acc<F4>::type (&acc)[WTP][WTQ], float* __restrict__ Y, int M, int KN,
                                            int OHW, int prb, int qrb, int lane, int bias, int form, float alpha) {
     const bool le_form = form == 0;
@@ -235,7 +235,10 @@ __device__ __forceinline__ void store_tile(const typename Acc<F4>::type (&acc)[W
                 const bool scale = le_form ? (fr <= 0.0f) : (r < 0);
                 const float f = scale ? fr * alpha : fr;
                 const size_t o = SWAP ? qoff + (size_t)p * OHW : (size_t)p * KN + qoff;
-                if (qok && p < (SWAP ? KN : M)) __builtin_nontemporal_store(f, &Y[o]);
+                if (qok && p < (SWAP ? KN : M)) {
+                    if (NT) __builtin_nontemporal_store(f, &Y[o]);
+                    else Y[o] = f;
+                }
             }
         }
 }
@@ -247,7 +250,7 @@ __device__ __forceinline__ void store_tile(const typename Acc<F4>::type (&acc)[W
 // The epilogue computes r = acc - bias, then PReLU in the reference's form for the type:
 // form 0 "f = r; if (f <= 0) f *= alpha" (mm_p2_final_tnn_avx2.c:204-208), form 1
 // "r >= 0 ? r : alpha * r" (mm_p2_final_tbn_avx2.c:73).
-template <bool SWAP, int WTP, int WTQ, int kKF, int kNS>
+template <bool SWAP, bool NT, int WTP, int WTQ, int kKF, int kNS>
 __global__ __launch_bounds__(256) void k_mfma(const uint4* __restrict__ Pf, const uint4* __restrict__ Qf,
                                               float* __restrict__ Y, int M, int KN, int OHW, int KB,
                                               int bias, int form, float alpha) {
@@ -353,7 +356,7 @@ __global__ __launch_bounds__(256) void k_mfma(const uint4* __restrict__ Pf, cons
     for (; s + kNS < nstep; s++) step_body(s, std::true_type{});
     for (; s < nstep; s++) step_body(s, std::false_type{});
 
-    store_tile<false, SWAP, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
+    store_tile<false, SWAP, NT, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
 }
 
 // ------------------------------------------------- fp4 operands at two bits per lane, offset codes
@@ -474,7 +477,7 @@ __device__ __forceinline__ uint4 unpack4(uint32_t p0, uint32_t p1) {
 // The epilogue of the offset form: dot = 4 acc - sum of the P row - sum of the Q row - lanes, then as store_tile
 // (off = lanes + the BNN bias).  sums: the tile's row sums in LDS, RB * 32 of the P side, then RB * 32 of the Q side
 // (zero for rows past the operand, which store nothing).
-template <bool SWAP, int WT>
+template <bool SWAP, bool NT, int WT>
 __device__ __forceinline__ void store_tile_offset(const Acc<true>::type (&acc)[WT][WT], float* __restrict__ Y, int M, int KN, int OHW,
                                                   int prb, int qrb, int lane, const int* sums, int wy, int wx, int off, int form,
                                                   float alpha) {
@@ -509,7 +512,10 @@ __device__ __forceinline__ void store_tile_offset(const Acc<true>::type (&acc)[W
                 const bool scale = le_form ? (fr <= 0.0f) : (r < 0);
                 const float f = scale ? fr * alpha : fr;
                 const size_t o = SWAP ? qoff + (size_t)p * OHW : (size_t)p * KN + qoff;
-                if (qok && p < prow) __builtin_nontemporal_store(f, &Y[o]);
+                if (qok && p < prow) {
+                    if (NT) __builtin_nontemporal_store(f, &Y[o]);
+                    else Y[o] = f;
+                }
             }
         }
     }
@@ -521,7 +527,7 @@ __device__ __forceinline__ void store_tile_offset(const Acc<true>::type (&acc)[W
 // then the barrier; the second K word's multiplies run beside the loads of stage s + kNS and the LDS reads of stage
 // s + 1, one read per slot of two multiplies (a 16-byte LDS read holds the wavefront's issue for 16 cycles), each block
 // unpacked LAG slots after its read -- the last LAG blocks in the first slots of the next step.
-template <bool SWAP, int WT, int kNS>
+template <bool SWAP, bool NT, int WT, int kNS>
 __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, const uint4* __restrict__ Qc, float* __restrict__ Y,
                                                  int M, int KN, int OHW, int KP, const int* __restrict__ sP,
                                                  const int* __restrict__ sQ, int off, int form, float alpha) {
@@ -642,7 +648,7 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
         sums[RB * 32 + tid] = qr < qrow ? sQ[qr] : 0;
     }
     __syncthreads();
-    store_tile_offset<SWAP, WT>(acc, Y, M, KN, OHW, prb0 + wy * WT, qrb0 + wx * WT, lane, sums, wy, wx, off, form, alpha);
+    store_tile_offset<SWAP, NT, WT>(acc, Y, M, KN, OHW, prb0 + wy * WT, qrb0 + wx * WT, lane, sums, wy, wx, off, form, alpha);
 }
 
 // ------------------------------------------------------------ conv layers as workgroup tiles (fp4, records)
@@ -867,7 +873,7 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
     for (; s + NS < nstep; s++) step_body(s, std::true_type{});
     for (; s < nstep; s++) step_body(s, std::false_type{});
 
-    store_tile<true, SWAP, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
+    store_tile<true, SWAP, true, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
 }
 
 // ------------------------------------------------------------ conv layer (fp4)
@@ -1271,16 +1277,21 @@ inline int64_t mfma_small_tile_below() {
     return v;
 }
 
-template <bool SWAP, int WTP, int WTQ, int KF, int NS>
-hipError_t launch_gemm_tile(const uint4* Pf, const uint4* Qf, float* Y, int M, int KN, int OHW, int KB,
+// Two workgroups of the smaller tiles share a compute unit: where rows are long, one's stores go on beside the other's multiplies,
+// and only the write-back at the end of a launch through the caches is left (stores_past_caches).  Operands kept, us past / through
+// the caches: 30000 x 150 x 4096 (64 words) 23.2 / 19.9, x 16384 55.3 / 55.2, 5905 x 1474 x 27904 121 / 129.
+inline bool tile_hides_stores(int WT, int Kw) { return WT < 4 && Kw > 128; }
+
+template <bool SWAP, bool NT, int WTP, int WTQ, int KF, int NS>
+hipError_t launch_gemm_tile_as(const uint4* Pf, const uint4* Qf, float* Y, int M, int KN, int OHW, int KB,
                             int bias, int form, float alpha, hipStream_t st) {
-    auto kern = k_mfma<SWAP, WTP, WTQ, KF, NS>;
+    auto kern = k_mfma<SWAP, NT, WTP, WTQ, KF, NS>;
     constexpr size_t lds_bytes = Tile<WTP, WTQ, KF, NS>::lds_bytes;
     // the opt-in to more than 64 KiB of dynamic LDS is per kernel; done once, thread-safe
     // The kernel counts its LDS-direct loads by hand (s_waitcnt vmcnt(N)); a scratch access would be one more
     // vector-memory operation inside those windows, so a build of it that spills is refused (once per variant).
     static const hipError_t configured = []() {
-        const void* kern = reinterpret_cast<const void*>(&k_mfma<SWAP, WTP, WTQ, KF, NS>);
+        const void* kern = reinterpret_cast<const void*>(&k_mfma<SWAP, NT, WTP, WTQ, KF, NS>);
         hipFuncAttributes attr;
         hipError_t e = hipFuncGetAttributes(&attr, kern);
         if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
@@ -1293,6 +1304,14 @@ hipError_t launch_gemm_tile(const uint4* Pf, const uint4* Qf, float* Y, int M, i
     if (grid.y > 65535) return hipErrorInvalidValue;
     hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha);
     return hipGetLastError();
+}
+
+template <bool SWAP, int WTP, int WTQ, int KF, int NS>
+hipError_t launch_gemm_tile(const uint4* Pf, const uint4* Qf, float* Y, int M, int KN, int OHW, int KB,
+                            int bias, int form, float alpha, hipStream_t st) {
+    return stores_past_caches(SWAP ? OHW : KN, M, KN) || tile_hides_stores(WTP, KB / 2)
+               ? launch_gemm_tile_as<SWAP, true, WTP, WTQ, KF, NS>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st)
+               : launch_gemm_tile_as<SWAP, false, WTP, WTQ, KF, NS>(Pf, Qf, Y, M, KN, OHW, KB, bias, form, alpha, st);
 }
 
 template <bool SWAP>
@@ -1321,14 +1340,14 @@ hipError_t launch_expand(bool tern, const uint32_t* rows_ptr, int rows, int G, u
     return hipGetLastError();
 }
 
-template <bool SWAP, int WT, int NS>
-hipError_t launch_gemm_p4_tile(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, const int* sP,
+template <bool SWAP, bool NT, int WT, int NS>
+hipError_t launch_gemm_p4_tile_as(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, const int* sP,
                                const int* sQ, int off, int form, float alpha, hipStream_t st) {
-    auto kern = k_mfma_p4<SWAP, WT, NS>;
+    auto kern = k_mfma_p4<SWAP, NT, WT, NS>;
     constexpr size_t lds_bytes = (size_t)NS * 4 * WT * 1024;
     // hand-counted LDS-direct loads: no scratch (see launch_gemm_tile); the opt-in to more than 64 KiB of LDS is per kernel
     static const hipError_t configured = []() {
-        const void* k = reinterpret_cast<const void*>(&k_mfma_p4<SWAP, WT, NS>);
+        const void* k = reinterpret_cast<const void*>(&k_mfma_p4<SWAP, NT, WT, NS>);
         hipFuncAttributes attr;
         hipError_t e = hipFuncGetAttributes(&attr, k);
         if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
@@ -1341,6 +1360,14 @@ hipError_t launch_gemm_p4_tile(const uint4* Pc, const uint4* Qc, float* Y, int M
     if (grid.y > 65535) return hipErrorInvalidValue;
     hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha);
     return hipGetLastError();
+}
+
+template <bool SWAP, int WT, int NS>
+hipError_t launch_gemm_p4_tile(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, const int* sP,
+                               const int* sQ, int off, int form, float alpha, hipStream_t st) {
+    return stores_past_caches(SWAP ? OHW : KN, M, KN) || tile_hides_stores(WT, 2 * KP)
+               ? launch_gemm_p4_tile_as<SWAP, true, WT, NS>(Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha, st)
+               : launch_gemm_p4_tile_as<SWAP, false, WT, NS>(Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha, st);
 }
 
 template <bool SWAP>
