@@ -266,7 +266,7 @@ FTNN_API int ftnn_conv_static(int type, const float *d_x, const float *d_thr, co
 /*
  * The same layer on an explicit engine (no counterpart in the reference; same bits on either):
  * FTNN_ENGINE_VALU      quantise to bit planes, vector-ALU popcount GEMM with implicit im2row;
- * FTNN_ENGINE_MFMA_F4   quantise to fp4 nibbles, expand the weights into matrix-core fragments
+ * FTNN_ENGINE_MFMA_F4   quantise to two bits per lane, bring the weights into the same form
  *                       (in d_scratch) and run the fp4 matrix-core layer kernel;
  * FTNN_ENGINE_AUTO      what ftnn_conv does: ftnn_select_conv_engine()'s choice.
  * ftnn_conv_scratch_bytes() covers every engine.
