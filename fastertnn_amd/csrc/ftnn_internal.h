@@ -94,7 +94,6 @@ struct ConvGeom {
 // Few-channel first layers keep their lanes in plain order (`natural`: dword j holds lanes 16 j .. 16 j + 7 as D0 and the
 // next eight as D1) in both operands: any order serves as long as both have it.
 constexpr uint32_t kP2Mask = 0xAAAAAAAAu;   // D0 of a dword
-constexpr uint32_t kP2Plus = 0x33333333u;   // +1 in every lane: the padding of binary activations
 __device__ __forceinline__ uint32_t p2_join(uint32_t d0, uint32_t d1) { return d0 | d1 >> 1; }
 
 // Fused hand-over to a following fp4 layer: instead of the fp32 result, a GEMM kernel writes the
