@@ -65,8 +65,8 @@ inline XcdOrder make_xcd_order(uint64_t outer, uint32_t inner, bool plain) {   /
     return x;
 }
 
-// The workgroup tiles (k_mfma, k_mfma_p4, k_mfma_s2) and layers with results beyond the Infinity Cache (k_conv_f4) store rows of 32 results,
-// `row` values apart: past the caches (non-temporal) where those are whole sectors of 64 bytes, and where the result is small;
+// The GEMM tiles (k_mfma, k_mfma_p4) and layers with results beyond the Infinity Cache (k_conv_f4) store rows of 32 results, `row`
+// values apart: past the caches (non-temporal) where those are whole sectors of 64 bytes, and where the result is small;
 // through the caches a launch ends with their write-back.  Large results of other rows go through the caches, which put the parts
 // of a sector together; past them each part is a read and a write of memory.  Whole calls, us, past / through the caches: TNN
 // 4096 x 4096 x 4096 44 / 52, x 4112 columns 65 / 72, x 4111 92 / 71; 6016 x 6016 x 512 58 / 72, 6001 x 6001 124 / 72; operands kept,
@@ -94,6 +94,7 @@ struct ConvGeom {
 // Few-channel first layers keep their lanes in plain order (`natural`: dword j holds lanes 16 j .. 16 j + 7 as D0 and the
 // next eight as D1) in both operands: any order serves as long as both have it.
 constexpr uint32_t kP2Mask = 0xAAAAAAAAu;   // D0 of a dword
+constexpr uint32_t kP2Plus = 0x33333333u;   // +1 in every lane: the padding of binary activations
 __device__ __forceinline__ uint32_t p2_join(uint32_t d0, uint32_t d1) { return d0 | d1 >> 1; }
 
 // Fused hand-over to a following fp4 layer: instead of the fp32 result, a GEMM kernel writes the
@@ -291,6 +292,16 @@ hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int6
 hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const ConvGeom& cg, int N, int KN,
                           int K_unpack, float alpha, float* d_y, hipStream_t st, const QuantOut& qo = QuantOut());
 
+
+// the same layer as workgroup tiles of 128 x 128 or 256 x 128 staged through LDS (the activation records gathered from T2, the
+// quantised input in the layout of launch_quantize_f4_tiled): for layers with conv_f4_tile_route() and an fp32 result
+int64_t quantize_f4_tiled_bytes(int N, int C, int H, int W, int W_stride);
+hipError_t launch_quantize_f4_tiled(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
+                                    int W_stride, void* d_t2, hipStream_t st);
+bool conv_f4_tile_route(int64_t M, int KN, int CP, int taps, int64_t t2_bytes, int W_pad, int W_stride);
+hipError_t launch_conv_f4_tiles(int type, const void* d_t2, const void* d_wf, const ConvGeom& cg, int N, int KN,
+                                int K_unpack, float alpha, float* d_y, hipStream_t st);
+
 // ---- ftnn_api.hip ----  (arguments already validated)
 // The fp4 layer with weights expanded beforehand (d_wf: launch_expand_records of the packed rows).
 // d_x != null: the input is quantised into d_p2 (N*H*W*C_pack*16 bytes) first; d_x == null: d_p2 already
@@ -305,7 +316,7 @@ int conv_valu(int type, const float* d_x, const float* d_thr, const int64_t* d_q
               void* d_scratch, float* d_y, hipStream_t st, const QuantOut& qo, bool weights_prepared);
 // bytes of the fp4 layer's operand region (d_p2 above) for this shape, rounded up to 256: P2, or for a
 // few-channel layer the nibble pixels and dense rows
-int64_t conv_f4_operand_bytes(int N, int C, int H, int W, int KH, int KW, int OH, int OW, int KN);
+int64_t conv_f4_operand_bytes(int N, int C, int H, int W, int KH, int KW, int OH, int OW, int KN, int W_stride);
 // words per row of the weights as the fp4 layer reads them (the dense re-packing shortens them)
 int conv_f4_weight_words(int C, int KH, int KW);
 

@@ -261,7 +261,7 @@ ftnn_net_t* ftnn_net_create_ex(int batch, int n_layers, const ftnn_layer_t* laye
             if (f4[i]) {
                 int64_t& bytes = sizes[(size_t)size_of[i]].bytes[i & 1];
                 bytes = std::max(bytes, conv_f4_operand_bytes(part.batch, L.C, L.H, L.W, L.KH, L.KW, net->OH[i], net->OW[i],
-                                                              L.KN));
+                                                              L.KN, L.stride));
             } else
                 max_scratch = std::max(max_scratch, ftnn_conv_scratch_bytes(L.type, part.batch, L.C, L.H, L.W, L.KN, L.KH,
                                                                             L.KW, L.pad, L.pad, L.stride, L.stride));

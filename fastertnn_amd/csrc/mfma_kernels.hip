@@ -651,8 +651,8 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
     store_tile_offset<SWAP, NT, WT>(acc, Y, M, KN, OHW, prb0 + wy * WT, qrb0 + wx * WT, lane, sums, wy, wx, off, form, alpha);
 }
 
-// ------------------------------------------------------------ product of record blocks (fp4)
-// Layers of few pixels and many kernels, from im2row rows.  2 x 2 wavefronts per workgroup, WTP x WTQ blocks of 32 x 32 each: (64 WTP) x (64 WTQ) results.  P side:
+// ------------------------------------------------------------ conv layers as workgroup tiles (fp4, records)
+// Large layers.  2 x 2 wavefronts per workgroup, WTP x WTQ blocks of 32 x 32 each: (64 WTP) x (64 WTQ) results.  P side:
 // weights, Q side: pixels (SWAP; without it, for one-pixel images, P = rows of the activations and Q = weights, row-major).
 // Both operands are blocks of records: 1 KiB = 32 rows x two K words, lane l = (word of the pair l / 32, row l % 32).  A stage
 // of the LDS ring holds PPS pairs of every row block, filled by LDS-direct loads that the kernel counts by hand; a block is one
@@ -661,6 +661,19 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
 // where the stage ends) the second word's multiplies run beside the LDS reads of the next pair, each block split LAG slots
 // after its read.  These tiles are bound by what they move through the LDS: at four bits per lane a step of two K words
 // moved 72 KiB for 512 cycles of matrix pipe (256 x 128 tile) and took 1080 cycles.
+//
+// IMPL: a conv layer with implicit im2row.  Qc is then the layer's quantised input in the form T2[n][C_pack][row][column % s]
+// [column / s][16 bytes] (k_quantize_f4 with TILED): lane l of a block of K words 2 i, 2 i + 1 loads the record of its pixel at
+// the tap of word w = 2 i + l / 32 = (kh KW + kw) C_pack + ic, from input pixel (oh s + kh - p, ow s + kw - p) of plane ic, or
+// the fill record behind the planes (zeros, or +1 for binary activations: the reference's fill,
+// src/tnns/ternarize2row_avx2.c:748-755, src/tnns/binarize2row_avx2.c:151) where that pixel lies outside the image or w is a
+// padding word.  In T2 the 32 pixels are consecutive records within an output row whatever the stride.  Every wavefront stages
+// a quarter of each side, so that none holds the others up at the barrier.  A wavefront issues one instruction every few
+// cycles, so what the gather adds per block must stay a handful of instructions:
+//   * a table behind the ring, one entry per K word, holds what does not depend on the pixel: the bit of the word's tap (0
+//     for a padding word), and the word's part of the record index (plane, tap row, column class and slot offset);
+//   * per row block a lane keeps the mask of the taps that fall inside the image for its pixel, and its pixel's part of the index;
+// a block's source is then one AND, one add, one select and the address.
 template <int WTP, int WTQ, int PPS, int NS>
 struct TileRec {
     static constexpr int RBP = 2 * WTP, RBQ = 2 * WTQ;         // row blocks per operand side
@@ -670,13 +683,15 @@ struct TileRec {
     static constexpr int LAG = NL >= 8 ? 4 : (NL >= 4 ? 3 : 1);
     static constexpr size_t lds_bytes = (size_t)NS * FR * 1024;
     static_assert(PF % 4 == 0 && (RBQ * PPS) % 4 == 0 && FW <= NL, "a quarter of each side per wavefront, one load per slot");
+    static_assert(PPS == 1 || QW == 1, "one pair per wavefront on the gathered side");
 };
 
-template <bool SWAP, bool NT, int WTP, int WTQ, int PPS, int NS>
+template <bool SWAP, int WTP, int WTQ, int PPS, int NS, bool IMPL>
 __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, const uint4* __restrict__ Qc, float* __restrict__ Y,
                                                  int M, int KN, int OHW, int KP /* pairs of words per row */, int nstep, int bias,
-                                                 int form, float alpha) {
-    extern __shared__ uint4 lds[];   // NS stages of FR KiB
+                                                 int form, float alpha, ConvGeom cg, FastDiv dOHW, int Ws, FastDiv dSW) {
+    static_assert(!IMPL || SWAP, "implicit im2row: the pixels along the lanes");
+    extern __shared__ uint4 lds[];   // NS stages of FR KiB, then the table
     typedef Acc<true>::type acc_t;
     typedef TileRec<WTP, WTQ, PPS, NS> TL;
     constexpr int RBP = TL::RBP, RBQ = TL::RBQ, PF = TL::PF, FR = TL::FR, PW = TL::PW, QW = TL::QW, FW = TL::FW;
@@ -685,7 +700,20 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wy = wave >> 1, wx = wave & 1;
     const int prow = SWAP ? KN : M, qrow = SWAP ? M : KN;
-    const int prb0 = blockIdx.x * RBP, qrb0 = blockIdx.y * RBQ;
+    // Tile of this workgroup.  Under IMPL the kernel tiles of one pixel tile read the same part of T2; workgroups are dealt
+    // to the eight XCDs round-robin by their linear number, so the tiles are renumbered to keep those on one XCD (its L2
+    // then fetches that part once, not once per kernel tile): XCD x takes the pixel tiles x, x + 8, ...; the pixel
+    // tiles beyond the last multiple of eight keep the plain order.
+    uint32_t bx = blockIdx.x, by = blockIdx.y;
+    if constexpr (IMPL) {
+        const uint32_t kt = gridDim.x, pt8 = gridDim.y / 8 * 8, lin = bx + kt * by;
+        if (lin < kt * pt8) {
+            const uint32_t xcd = lin & 7u, slot = lin >> 3;
+            by = xcd + 8u * (slot / kt);
+            bx = slot % kt;
+        }
+    }
+    const int prb0 = bx * RBP, qrb0 = by * RBQ;
     const int prbmax = (prow + 31) / 32 - 1, qrbmax = (qrow + 31) / 32 - 1;
     acc_t acc[WTP][WTQ];
 #pragma unroll
@@ -703,12 +731,59 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
         const int g = wave * PW + i;
         psrc[i] = Pc + ((size_t)min(prb0 + g / PPS, prbmax) * KP + g % PPS) * 64 + lane;
     }
-    const uint4* qsrc[QW];
+    const uint4* qsrc[IMPL ? 1 : QW];
+    uint32_t tapmask[IMPL ? QW : 1], qbase[IMPL ? QW : 1];
+    const uint32_t row16 = (uint32_t)(cg.W_stride * Ws);            // records per input row
+    const uint32_t plane16 = (uint32_t)cg.H * row16;                // per plane of 64 channels
+    const uint32_t fill_rec = (uint32_t)cg.CP * plane16 * (uint32_t)((M - 1) / OHW + 1);   // right behind the planes
+    uint2* const wtab = reinterpret_cast<uint2*>(lds + (size_t)NS * FR * 64);
+    const int words = 2 * PPS * nstep;
+    if constexpr (IMPL) {
+        for (int w = tid; w < words; w += 256) {
+            const int tap = (int)fastdiv((uint32_t)w, cg.dCP), ic = w - tap * cg.CP;
+            const int kh = (int)fastdiv((uint32_t)tap, cg.dKW), kw = tap - kh * cg.KW;
+            // column ow s + d with d = kw - pad: class d mod s, slot ow + floor(d / s) (d made non-negative by a
+            // multiple of s first: the host keeps the padding below 4096 s)
+            const uint32_t dd = (uint32_t)(kw - cg.W_pad + 4096 * cg.W_stride);
+            const uint32_t dq = fastdiv(dd, dSW), cls = dd - dq * (uint32_t)cg.W_stride;
+            wtab[w] = make_uint2(w < cg.K ? 1u << tap : 0u,
+                                 (uint32_t)ic * plane16 + (uint32_t)kh * row16 + cls * (uint32_t)Ws + dq - 4096u);
+        }
 #pragma unroll
-    for (int i = 0; i < QW; i++) {
-        const int g = wave * QW + i;
-        qsrc[i] = Qc + ((size_t)min(qrb0 + g / PPS, qrbmax) * KP + g % PPS) * 64 + lane;
+        for (int j = 0; j < QW; j++) {
+            const int rb = (wave * QW + j) / PPS;
+            const uint32_t q = (uint32_t)min((qrb0 + rb) * 32 + (lane & 31), M - 1);
+            const uint32_t img = fastdiv(q, dOHW);
+            const uint32_t pix = q - img * (uint32_t)OHW;
+            const int oh = (int)fastdiv(pix, cg.dOW), ow = (int)pix - oh * cg.OW;
+            const int ih0 = oh * cg.H_stride - cg.H_pad, iw0 = ow * cg.W_stride - cg.W_pad;
+            // (image, plane 0, row ih0, class 0, slot ow): wraps for a negative ih0, and the word's part brings it back
+            // whenever the tap is inside
+            qbase[j] = img * (uint32_t)cg.CP * plane16 + (uint32_t)ih0 * row16 + (uint32_t)ow;
+            uint32_t m = 0u;
+            for (int kh = 0, tap = 0; kh < cg.K / (cg.CP * cg.KW); kh++)
+                for (int kw = 0; kw < cg.KW; kw++, tap++)
+                    m |= ((unsigned)(ih0 + kh) < (unsigned)cg.H && (unsigned)(iw0 + kw) < (unsigned)cg.W ? 1u : 0u) << tap;
+            tapmask[j] = m;
+        }
+        __syncthreads();   // the table is complete before the first stage is issued
+    } else {
+#pragma unroll
+        for (int i = 0; i < QW; i++) {
+            const int g = wave * QW + i;
+            qsrc[i] = Qc + ((size_t)min(qrb0 + g / PPS, qrbmax) * KP + g % PPS) * 64 + lane;
+        }
     }
+    // this lane's word of the pair that its wavefront gathers of the stage about to be issued (stages are issued strictly in
+    // order); its table entry is read one stage ahead of its use
+    int g_w = 2 * (PPS == 1 ? 0 : wave % PPS) + (lane >> 5);
+    uint2 wt = make_uint2(0u, 0u), wt_ahead = make_uint2(0u, 0u);
+    if constexpr (IMPL) wt_ahead = wtab[g_w];
+    auto next_words = [&]() {
+        wt = wt_ahead;
+        g_w = min(g_w + 2 * PPS, words - 1);   // (past the last stage: any entry)
+        wt_ahead = wtab[g_w];
+    };
     const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
     auto load = [&](int i, int step) {   // slot i of the wavefront's loads for stage `step`
         const uint32_t dst = lds0 + (uint32_t)(step % NS) * (FR * 1024);
@@ -717,10 +792,12 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
         } else {
             const int j = i - PW;
             const uint32_t d = dst + (uint32_t)(PF + wave * QW + j) * 1024;
-            dma16(qsrc[j] + (size_t)step * PPS * 64, d);
+            if constexpr (IMPL) dma16(Qc + ((tapmask[j] & wt.x) != 0u ? qbase[j] + wt.y : fill_rec), d);   // a select on the index: no branch
+            else dma16(qsrc[j] + (size_t)step * PPS * 64, d);
         }
     };
     auto stage = [&](int step) {
+        if constexpr (IMPL) next_words();
 #pragma unroll
         for (int i = 0; i < FW; i++) load(i, step);
     };
@@ -779,6 +856,7 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
                 if (FULL || s + NS - 1 < nstep) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FW * (NS - 2)) : "memory");
                 else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __syncthreads();
+                if constexpr (FULL && IMPL) next_words();
             }
             const bool do_ld = !last || FULL || s + 1 < nstep;
 #pragma unroll
@@ -795,7 +873,7 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
     for (; s + NS < nstep; s++) step_body(s, std::true_type{});
     for (; s < nstep; s++) step_body(s, std::false_type{});
 
-    store_tile<true, SWAP, NT, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
+    store_tile<true, SWAP, true, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
 }
 
 // ------------------------------------------------------------ conv layer (fp4)
@@ -1381,17 +1459,19 @@ hipError_t launch_mfma_gemm_packed4(int type, const void* d_ac, const void* d_bc
 }
 
 namespace {
-template <bool SWAP, bool NT, int WTP, int WTQ, int PPS, int NS>
+constexpr int kMaxTileRouteWords = 2040;   // K words per row the tile kernel keeps a table entry for (16 KiB of LDS)
+template <bool SWAP, int WTP, int WTQ, int PPS, int NS, bool IMPL>
 hipError_t launch_records_tile(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, int pairs, int bnn_k, int form,
-                               float alpha, hipStream_t st) {
-    auto kern = k_mfma_s2<SWAP, NT, WTP, WTQ, PPS, NS>;
+                               float alpha, const ConvGeom& cg, hipStream_t st) {
+    auto kern = k_mfma_s2<SWAP, WTP, WTQ, PPS, NS, IMPL>;
     typedef TileRec<WTP, WTQ, PPS, NS> TL;
     constexpr size_t kLdsMax = 160u << 10;   // LDS of a compute unit
     const int nstep = (pairs + PPS - 1) / PPS;   // (a row is stored at an even number of pairs)
-    static_assert(TL::lds_bytes <= kLdsMax, "the ring");
+    const size_t lds_bytes = TL::lds_bytes + (IMPL ? (size_t)nstep * PPS * 2 * 8 : 0);   // the ring, then the table of K words
+    if (lds_bytes > kLdsMax) return hipErrorInvalidValue;
     // as launch_gemm_tile: hand-counted LDS-direct loads, so no scratch; the LDS opt-in is per kernel
     static const hipError_t configured = []() {
-        const void* k = reinterpret_cast<const void*>(&k_mfma_s2<SWAP, NT, WTP, WTQ, PPS, NS>);
+        const void* k = reinterpret_cast<const void*>(&k_mfma_s2<SWAP, WTP, WTQ, PPS, NS, IMPL>);
         hipFuncAttributes attr;
         hipError_t e = hipFuncGetAttributes(&attr, k);
         if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
@@ -1404,7 +1484,8 @@ hipError_t launch_records_tile(const uint4* Pc, const uint4* Qc, float* Y, int M
     if (grid.y > 65535) return hipErrorInvalidValue;
     // BNN: every lane that is no real (channel, tap) is +1 x +1 in both operands, padding words included
     const int bias = bnn_k ? 128 * nstep * PPS - bnn_k : 0;
-    hipLaunchKernelGGL(kern, grid, dim3(256), TL::lds_bytes, st, Pc, Qc, Y, M, KN, OHW, KP, nstep, bias, form, alpha);
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Pc, Qc, Y, M, KN, OHW, KP, nstep, bias, form, alpha, cg,
+                       make_fastdiv((uint32_t)OHW), IMPL ? (cg.W + cg.W_stride - 1) / cg.W_stride : 0, make_fastdiv(IMPL ? (uint32_t)cg.W_stride : 1u));
     return hipGetLastError();
 }
 
@@ -1412,13 +1493,9 @@ template <bool SWAP>
 hipError_t launch_records(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int Kw, int bnn_k, int form, float alpha,
                           hipStream_t st) {
     const int64_t big = (((int64_t)M + 255) / 256) * ((KN + 255) / 256);
-    const bool small = big < mfma_small_tile_below();
-    auto go = [&](auto nt) {
-        constexpr bool NT = decltype(nt)::value;
-        return small ? launch_records_tile<SWAP, NT, 2, 2, 1, 4>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, st)
-                     : launch_records_tile<SWAP, NT, 4, 4, 1, 4>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, st);
-    };
-    return stores_past_caches(SWAP ? OHW : KN, M, KN) || tile_hides_stores(small ? 2 : 4, Kw) ? go(std::true_type{}) : go(std::false_type{});
+    return big < mfma_small_tile_below()
+               ? launch_records_tile<SWAP, 2, 2, 1, 4, false>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, ConvGeom(), st)
+               : launch_records_tile<SWAP, 4, 4, 1, 4, false>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, ConvGeom(), st);
 }
 }  // namespace
 
@@ -1428,6 +1505,53 @@ hipError_t launch_records_gemm(int type, const void* d_a, const void* d_b, int64
     const int bnn_k = type == kBNN ? K_unpack : 0, form = type == kTNN ? 0 : 1;
     return OHW > 1 ? launch_records<true>(B, A, d_y, (int)M, KN, OHW, Kw, bnn_k, form, alpha, st)
                    : launch_records<false>(A, B, d_y, (int)M, KN, OHW, Kw, bnn_k, form, alpha, st);
+}
+
+// Large layers with a stride and long rows go to the tile kernel with implicit im2row: the layer kernel gathers records a stride
+// apart, so it moves twice the cache lines per record and its L1 is what bounds it; T2 keeps them side by side.  8 x 1024 x 56 x 56 ->
+// 1024, 3 x 3 stride 2 (1568 tiles of 64 x 64, 144 words) under sustained load 51.7 us, 56.5 on the layer kernel.  Elsewhere the
+// layer kernel is ahead on 920 random layers: at stride 1 by 5 to 50 %, at stride 2 with short rows (1216 tiles, 72
+// words 36 / 32 us) or fewer tiles (848, 325 words 83 / 78).  FTNN_CONV_TILES_FROM = n: tuning aid; it sets the tile count and drops the
+// other conditions.
+namespace {
+// the tile kernel's limits: a tap mask of 32 bits per pixel, a table entry per K word, 32-bit record indices into T2,
+// pixel indices below 2^31 and its way of keeping kw - pad non-negative
+bool conv_tiles_within_limits(int64_t M, int CP, int taps, int64_t t2_bytes, int W_pad, int W_stride) {
+    const int64_t K = (int64_t)CP * taps;
+    return taps <= 32 && (K + 3) / 4 * 4 <= kMaxTileRouteWords && M <= 0x7fffff00LL && t2_bytes / 16 <= 0x7fffffffLL &&
+           W_pad < 4096 * (int64_t)W_stride;
+}
+}  // namespace
+
+bool conv_f4_tile_route(int64_t M, int KN, int CP, int taps, int64_t t2_bytes, int W_pad, int W_stride) {
+    static const char* tune = getenv("FTNN_CONV_TILES_FROM");
+    static const int64_t from = tune ? atoll(tune) : 1500;
+    const int64_t tiles = ((M + 63) / 64) * ((KN + 63) / 64);
+    return tiles >= from && (tune || (W_stride > 1 && (int64_t)CP * taps >= 100 && M >= 512)) &&
+           conv_tiles_within_limits(M, CP, taps, t2_bytes, W_pad, W_stride);
+}
+
+// A large conv layer as workgroup tiles staged through LDS, the activation records gathered from T2
+// (launch_quantize_f4_tiled; k_mfma_s2 with IMPL): fp32 NCHW result only.  d_wf: the weights as record blocks
+// (round4(cg.K) words per row).
+hipError_t launch_conv_f4_tiles(int type, const void* d_t2, const void* d_wf, const ConvGeom& cg, int N, int KN, int K_unpack,
+                                float alpha, float* d_y, hipStream_t st) {
+    const int OHW = cg.OH * cg.OW;
+    const int64_t M = (int64_t)N * OHW;
+    const int KP = round4(cg.K) / 2, pairs = (cg.K + 1) / 2;
+    if (!conv_tiles_within_limits(M, cg.CP, cg.K / cg.CP, quantize_f4_tiled_bytes(N, cg.CP * 64, cg.H, cg.W, cg.W_stride), cg.W_pad, cg.W_stride))
+        return hipErrorInvalidValue;
+    const int bnn_k = type == kBNN ? K_unpack : 0, form = type == kTNN ? 0 : 1;
+    const uint4* Wf = static_cast<const uint4*>(d_wf);
+    const uint4* T2 = static_cast<const uint4*>(d_t2);
+    // tiles of 256 kernels x 128 pixels where those fill most of the chip in one round (the layer above: 196 workgroups, 53.9 us against
+    // 55.6 on 392 tiles of 128 x 128), else 128 x 128.  FTNN_CONV_TILE_SHAPE = 22 | 42 forces one (tuning aid)
+    static const int tune = getenv("FTNN_CONV_TILE_SHAPE") ? atoi(getenv("FTNN_CONV_TILE_SHAPE")) : 0;
+    const int64_t mid = ((M + 127) / 128) * ((KN + 255) / 256);
+    int shape = mid >= 180 && mid <= 256 ? 42 : 22;
+    if (tune == 22 || tune == 42) shape = tune;
+    if (shape == 42) return launch_records_tile<true, 4, 2, 1, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
+    return launch_records_tile<true, 2, 2, 1, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
 }
 
 hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const ConvGeom& cg, int N, int KN,

@@ -85,10 +85,15 @@ __global__ __launch_bounds__(256) void k_quantize_pixels(const float* __restrict
 // Bound by reading the fp32 input: PX = 64, where a thread makes one dword of a record out of 16 channels with 16 coalesced loads
 // in flight (8 x 1024 x 56 x 56: 17.0 us against 18.1 on PX = 32).  Small inputs, which last no longer than a launch, have twice the
 // wavefronts with PX = 32, a thread making half a dword out of 8 channels.
-template <bool TERN, int PX>
+// TILED: the operand of the tile kernel with implicit im2row instead (k_mfma_s2, IMPL): the columns of an image row sorted by
+// column % stride_w, T2[n][C_pack][row][column % s][column / s][16 bytes] with ceil(W / s) slots per class: the 32 lanes of a
+// fragment half -- consecutive output pixels, i.e. input columns s apart -- then read consecutive records within an output
+// row, whatever the stride.
+template <bool TERN, bool TILED, int PX>
 __global__ __launch_bounds__(256) void k_quantize_f4(const float* __restrict__ x,
                                                      const float* __restrict__ thr, int C, int HW,
-                                                     int CP, uint4* __restrict__ P2) {
+                                                     int CP, uint4* __restrict__ P2, int W, int SW, int Ws,
+                                                     FastDiv dW, FastDiv dSW) {
     static_assert(PX == 64 || PX == 32, "a dword or half a dword of a record per thread");
     constexpr int NC = PX / 4;   // channels of a thread
     __shared__ uint32_t s_dw[PX * 5];
@@ -129,7 +134,20 @@ __global__ __launch_bounds__(256) void k_quantize_f4(const float* __restrict__ x
     __syncthreads();
     if (threadIdx.x < PX && p < HW) {
         const uint32_t* d = s_dw + px * 5;
-        P2[((size_t)n * CP + ic) * HW + p] = make_uint4(d[0], d[1], d[2], d[3]);
+        size_t piece = ((size_t)n * CP + ic) * HW + p;
+        if constexpr (TILED) {
+            const uint32_t ih = fastdiv((uint32_t)p, dW), iw = (uint32_t)p - ih * (uint32_t)W;
+            const uint32_t cls_q = fastdiv(iw, dSW), cls = iw - cls_q * (uint32_t)SW;
+            piece = (((size_t)n * CP + ic) * (HW / W) + ih) * ((size_t)SW * Ws) + (size_t)cls * Ws + cls_q;
+        }
+        P2[piece] = make_uint4(d[0], d[1], d[2], d[3]);
+    }
+    if constexpr (TILED) {
+        // the fill record right behind the planes: what a tap outside the image contributes (0, or +1 for binary inputs)
+        if (threadIdx.x == 64 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
+            const uint32_t f = TERN ? 0u : kP2Plus;
+            P2[(size_t)gridDim.z * CP * (HW / W) * ((size_t)SW * Ws)] = make_uint4(f, f, f, f);
+        }
     }
 }
 
@@ -614,19 +632,31 @@ hipError_t launch_quantize(bool ternary, const float* d_x, const float* d_thr, i
     return hipGetLastError();
 }
 
+namespace {
 // PX: the larger workgroup tile from 1024 workgroups on, where the input comes from HBM
-hipError_t launch_quantize_f4(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
-                              void* d_p2, hipStream_t st) {
-    const int CP = cpack_of(C), HW = H * W;
+hipError_t launch_quantize_records(bool ternary, bool tiled, const float* d_x, const float* d_thr, int N, int C, int H, int W, int SW,
+                                   void* d_out, hipStream_t st) {
+    const int CP = cpack_of(C), HW = H * W, Ws = (W + SW - 1) / SW;
     const bool large = (int64_t)((HW + 63) / 64) * CP * N >= 1024;
     const int px = large ? 64 : 32;
     const dim3 grid((HW + px - 1) / px, CP, N);
+    const FastDiv dW = make_fastdiv((uint32_t)W), dSW = make_fastdiv((uint32_t)SW);
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, d_x, d_thr, C, HW, CP, static_cast<uint4*>(d_p2));
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, d_x, d_thr, C, HW, CP, static_cast<uint4*>(d_out), W, SW, Ws, dW, dSW);
         return hipGetLastError();
     };
-    if (ternary) return large ? go(k_quantize_f4<true, 64>) : go(k_quantize_f4<true, 32>);
-    return large ? go(k_quantize_f4<false, 64>) : go(k_quantize_f4<false, 32>);
+    if (ternary) {
+        if (tiled) return large ? go(k_quantize_f4<true, true, 64>) : go(k_quantize_f4<true, true, 32>);
+        return large ? go(k_quantize_f4<true, false, 64>) : go(k_quantize_f4<true, false, 32>);
+    }
+    if (tiled) return large ? go(k_quantize_f4<false, true, 64>) : go(k_quantize_f4<false, true, 32>);
+    return large ? go(k_quantize_f4<false, false, 64>) : go(k_quantize_f4<false, false, 32>);
+}
+}  // namespace
+
+hipError_t launch_quantize_f4(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
+                              void* d_p2, hipStream_t st) {
+    return launch_quantize_records(ternary, false, d_x, d_thr, N, C, H, W, 1, d_p2, st);
 }
 
 // fp32 rows -> Packing-2 rows of round4(ceil(C / 64)) words, the pad words filled as the im2row operand's: a row per image of a
@@ -639,6 +669,17 @@ hipError_t launch_quantize_rows(bool ternary, const float* d_x, const float* d_t
     if (ternary) hipLaunchKernelGGL((k_quantize_ballot<0, true>), grid, dim3(256), 0, st, d_x, d_thr, C, Kw, out);
     else hipLaunchKernelGGL((k_quantize_ballot<1, false>), grid, dim3(256), 0, st, d_x, d_thr, C, Kw, out);
     return hipGetLastError();
+}
+
+// bytes of T2 (k_quantize_f4 with TILED) for this input and column stride
+int64_t quantize_f4_tiled_bytes(int N, int C, int H, int W, int W_stride) {
+    return (int64_t)N * cpack_of(C) * H * W_stride * ((W + W_stride - 1) / W_stride) * 16 + 16;   // + the fill record
+}
+
+hipError_t launch_quantize_f4_tiled(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W,
+                                    int W_stride, void* d_t2, hipStream_t st) {
+    // slots of a class past its last column (W % s != 0) are never read: the gather reads real columns only
+    return launch_quantize_records(ternary, true, d_x, d_thr, N, C, H, W, W_stride, d_t2, st);
 }
 
 hipError_t launch_quantize_im2row(bool ternary, const float* d_x, const float* d_thr, int N, int C,

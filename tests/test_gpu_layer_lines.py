@@ -13,6 +13,25 @@ LAYERS = [(1, 64, t, 64, 64, 3) for t in (299, 300, 519, 520, 1023, 1024)] + [(1
          [(1, 896, t, 64, 64, 3) for t in (149, 150)] + [(2, 64, 256, 256, 530, 1), (2, 64, 255, 255, 535, 1), (2, 64, 1, 65537, 530, 1)]
 
 
+# stride 2, 108 words: on both sides of the 1500 tiles from which such a layer runs as workgroup tiles, on both of their shapes
+STRIDED = [(1, 768, 185, 127, 1000, 3), (1, 768, 189, 127, 1000, 3), (1, 768, 299, 255, 300, 3)]
+
+
+@pytest.mark.parametrize("typ", range(4), ids=[TYPE_NAMES[t] for t in range(4)])
+@pytest.mark.parametrize("layer", STRIDED, ids=lambda v: "x".join(map(str, v)))
+def test_strided_lines(hip, typ, layer):
+    n, c, h, w, kn, k = layer
+    print("case", TYPE_NAMES[typ], layer, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(17 + typ)
+    wt = weight_is_ternary(typ)
+    x = torch.randn((n, c, h, w), generator=g, device="cuda")
+    thr = torch.full((n,), 0.5 if act_is_ternary(typ) else 0.0, device="cuda")
+    qw = hip.pack_weights(torch.randn((kn, c, k, k), generator=g, device="cuda"), torch.full((kn,), 0.5 if wt else 0.0, device="cuda"), wt)
+    got = hip.conv(typ, x, thr, qw, kn, k, k, 1, 2, -0.25, engine=hip.ENGINE_MFMA_F4)
+    want = hip.conv(typ, x, thr, qw, kn, k, k, 1, 2, -0.25, engine=hip.ENGINE_VALU)
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
 @pytest.mark.parametrize("typ", range(4), ids=[TYPE_NAMES[t] for t in range(4)])
 @pytest.mark.parametrize("layer", LAYERS, ids=lambda v: "x".join(map(str, v)))
 def test_lines(hip, typ, layer):
