@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pair_walk.h"
+
 namespace ftnn {
 
 constexpr int kTNN = 0, kTBN = 1, kBTN = 2, kBNN = 3;
@@ -12,24 +14,6 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 inline int cpack_of(int C) { return (int)(((int64_t)C + 63) / 64); }
 inline int round4(int k) { return 4 * ((k + 3) / 4); }
 inline int out_dim(int in, int pad, int k, int stride) { return (in + 2 * pad - k) / stride + 1; }
-
-// Division of a 32-bit unsigned n by a fixed d without the ~25-instruction expansion of "/":
-// m = floor(2^32 / d) (saturated for d = 1) under-estimates the quotient by at most one, which one
-// compare fixes.  Exact for every n < 2^32, d >= 1.
-struct FastDiv {
-    uint32_t d, m;
-};
-inline FastDiv make_fastdiv(uint32_t d) {
-    FastDiv f;
-    f.d = d;
-    f.m = d <= 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d);
-    return f;
-}
-__device__ __forceinline__ uint32_t fastdiv(uint32_t n, const FastDiv& f) {
-    uint32_t q = __umulhi(n, f.m);
-    if (n - q * f.d >= f.d) q++;
-    return q;
-}
 
 // Which tile of outer x inner ones a workgroup of the layer kernels takes.  Workgroups go to the eight XCDs round-robin by
 // their linear number; XCD x takes the x-th eighth of the tiles, walked inner index first.  With the pixels as the outer
@@ -72,13 +56,6 @@ inline XcdOrder make_xcd_order(uint64_t outer, uint32_t inner, bool plain) {   /
 // 4096 x 4096 x 4096 44 / 52, x 4112 columns 65 / 72, x 4111 92 / 71; 6016 x 6016 x 512 58 / 72, 6001 x 6001 124 / 72; operands kept,
 // 30000 x 150 x 512 (17 MiB) 14.1 / 10.2.
 inline __host__ __device__ bool stores_past_caches(int row, int64_t M, int KN) { return row % 16 == 0 || M * KN <= (4 << 20); }
-
-// geometry of one conv layer as the implicit-im2row GEMM needs it
-struct ConvGeom {
-    int H, W, CP, OH, OW, KW, K;   // K = C_pack*KH*KW words per plane before rounding
-    int H_pad, W_pad, H_stride, W_stride;
-    FastDiv dOW, dCP, dKW;
-};
 
 // Quantised layer operands: two bits per lane, a record of 16 bytes per 64 lanes ("P2").
 //

@@ -914,27 +914,6 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
 // Needs both operands below 4 GiB (p2_bytes, wf_bytes: the sizes the descriptors announce).  fp32 results leave through buffer
 // stores too, relative to the tile's first image and kernel: y_span bounds what a tile reaches from there, whatever the size
 // of the result.
-// How a lane's word moves on when its run of pairs ends.  C_pack even: a run is the C_pack / 2 pairs of a tap, `stride` bytes
-// apart, then the next tap.  C_pack odd: every pair is a run, and both halves move on by two words = (kh, kw, ic).
-struct PairWalk {
-    int even, run, NP;       // NP: pairs per row, ceil(K / 2)
-    int dkh, dkw, dic, KH;
-    FastDiv dRun;            // C_pack / 2
-};
-inline PairWalk make_pair_walk(const ConvGeom& cg) {
-    PairWalk p;
-    p.even = cg.CP % 2 == 0;
-    p.run = p.even ? cg.CP / 2 : 1;
-    p.NP = (cg.K + 1) / 2;
-    const int taps = p.even ? 1 : 2 / cg.CP;
-    p.dic = p.even ? 0 : 2 % cg.CP;
-    p.dkh = taps / cg.KW;
-    p.dkw = taps % cg.KW;
-    p.KH = cg.K / (cg.CP * cg.KW);
-    p.dRun = make_fastdiv((uint32_t)p.run);
-    return p;
-}
-
 template <bool ABIN, bool FORM0, int QMODE, int TA, int TB, int S, bool BUF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && QMODE != 0) ? 3 : 1, 8))) void k_conv_f4(
     const uint4* __restrict__ P2, const uint4* __restrict__ Wf, float* __restrict__ Y, int M, int KN, int OHW, int KP /* pairs a weight row is stored at */,
@@ -970,7 +949,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
         iw0[b] = ow * cg.W_stride - cg.W_pad;
         xrec[b] = img[b] * (uint32_t)(cg.CP * cg.H * cg.W) + (uint32_t)(ih0[b] * cg.W + iw0[b]);
     }
-    const int HWin = cg.H * cg.W;
     const int rbmax = (KN + 31) / 32 - 1;
 
     // The pairs of this wavefront, [p, p1).  A lane's word is 2 p + h = (kh, kw, ic) of the reference's K order; addresses and
@@ -978,25 +956,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
     int p = S == 1 ? 0 : (int)((uint32_t)(pw.NP * ks) / S);
     const int p1 = S == 1 ? pw.NP : (int)((uint32_t)(pw.NP * (ks + 1)) / S);
     const int pairs = p1 - p;
-    int kh, kw, ic, left = pw.run, soff = 0;   // pairs left in the run, scalar part of the input's byte offset
-    if (pw.even) {
-        int tap = 0;
-        if constexpr (S > 1) {
-            tap = (int)fastdiv((uint32_t)p, pw.dRun);
-            const int j = p - tap * pw.run;
-            left -= j;
-            soff = j * HWin * 32;
-        }
-        kh = S > 1 ? (int)fastdiv((uint32_t)tap, cg.dKW) : 0;
-        kw = tap - kh * cg.KW;
-        ic = h;
-    } else {
-        const uint32_t w = (uint32_t)(2 * p + h);
-        const int tap = (int)fastdiv(w, cg.dCP);
-        ic = (int)w - tap * cg.CP;
-        kh = (int)fastdiv((uint32_t)tap, cg.dKW);
-        kw = tap - kh * cg.KW;
-    }
+    // (the scalar part of its place in bytes for buffer loads, whose operand is below 3.75 GiB, and in records for any operand)
+    PairPos<BUF ? 16u : 1u> pos;
+    pos.template start<S == 1>(pw, cg, p, h);
     struct Rec {
         v4i w[TA], x[TB];
         uint32_t fill[TB];   // ABIN: the nibbles that a tap outside the image is replaced by (0: none)
@@ -1005,11 +967,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
     uint32_t vx[TB], fill[TB];   // the lane's record (BUF: byte offset) at its present word
     bool in[TB];
     auto tap = [&]() {
-        const bool real = kh < pw.KH;   // the word that makes up the last pair of an odd K is none
-        const uint32_t off = (uint32_t)(ic * HWin + kh * cg.W + kw);
+        const bool real = pos.kh < pw.KH;   // the word that makes up the last pair of an odd K is none
+        const uint32_t off = pos.off(cg);
 #pragma unroll
         for (int b = 0; b < TB; b++) {
-            const bool inside = (unsigned)(ih0[b] + kh) < (unsigned)cg.H && (unsigned)(iw0[b] + kw) < (unsigned)cg.W;
+            const bool inside = (unsigned)(ih0[b] + pos.kh) < (unsigned)cg.H && (unsigned)(iw0[b] + pos.kw) < (unsigned)cg.W;
             const bool valid = inside && real;
             if constexpr (ABIN) fill[b] = real && !inside ? 0x22222222u : 0u;   // (vx last, as in the other branch below: no register behind a pointer)
             const uint32_t rec = xrec[b] + off;   // wraps to the right value whenever the tap is inside
@@ -1044,10 +1006,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
 #pragma unroll
         for (int b = 0; b < TB; b++) {
             if constexpr (BUF) {
-                const v4u v = __builtin_amdgcn_raw_buffer_load_b128(brs_x, (int)vx[b], soff, 0);
+                const v4u v = __builtin_amdgcn_raw_buffer_load_b128(brs_x, (int)vx[b], (int)pos.soff, 0);
                 f.x[b] = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
             } else {
-                f.x[b] = *reinterpret_cast<const v4i*>(P2 + ((size_t)vx[b] + (size_t)(in[b] ? (uint32_t)soff / 16u : 0u)));
+                f.x[b] = *reinterpret_cast<const v4i*>(P2 + ((size_t)vx[b] + (in[b] ? pos.soff : 0u)));
             }
             if constexpr (!BUF) f.in[b] = in[b];
         }
@@ -1056,19 +1018,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
             if constexpr (ABIN) f.fill[b] = fill[b];
         if (p + 1 < p1) {
             p++;
-            soff += HWin * 32;
-            if (--left == 0) {
-                left = pw.run;
-                soff = 0;
-                ic += pw.dic;
-                const bool c = ic >= cg.CP;
-                ic -= c ? cg.CP : 0;
-                kw += pw.dkw + (c ? 1 : 0);
-                const bool d = kw >= cg.KW;
-                kw -= d ? cg.KW : 0;
-                kh += pw.dkh + (d ? 1 : 0);
-                tap();
-            }
+            if (pos.next(pw, cg)) tap();
         } else if (BUF) {   // past the end: offsets beyond the buffers, which move no data (else the last pair is read again)
             vw = 0xffffff00u;
 #pragma unroll

@@ -276,6 +276,39 @@ def test_chain_result_beyond_32_bit_offsets(hip, oracle, typ, n, h, w, kn):
     assert torch.equal(y, want)
 
 
+@pytest.mark.parametrize("typ", [TNN, BNN], ids=lambda t: TYPE_NAMES[t])
+def test_chain_input_beyond_32_bit_offsets_within_an_image(hip, oracle, typ):
+    """the last layer of a chain reads ten words of channels of an 8192 x 4096 image, 5 GiB of records that the layer before hands
+    over: the planes of the upper words lie more than 4 GiB from the image's first.  Bands of rows at the top, in the middle and at
+    the bottom against the same layers on the vector-ALU engine (the second layer is 1 x 1, so a band needs one row of halo)"""
+    import torch
+    from fastertnn_amd import synth
+    h, w, mid, kn = 8192, 4096, 640, 3
+    assert (mid // 64 - 2) * h * w * 16 >= 2 ** 32
+    print("case", TYPE_NAMES[typ], flush=True)
+    tern = typ == TNN
+    thr = 0.5 if tern else 0.0
+    rows = [(3, h, w, mid, 3, 3, 1, 1), (mid, h, w, kn, 1, 1, 0, 1)]
+    qws = []
+    for i, (c, _, _, k, ks, _, _, _) in enumerate(rows):
+        wt = (synth.ternary if tern else synth.binary)(80 + i, (k, c, ks, ks))
+        qws.append(torch.from_numpy(oracle.pack_weights(wt, np.full(k, 0.5 if tern else 0.0, np.float32), tern)).cuda())
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9)
+    x = torch.randn((1, 3, h, w), generator=g, device="cuda")
+    thr_d = torch.full((1,), thr, device="cuda")
+    net = hip.Net(1, [dict(type=typ, shape=r, threshold=thr, alpha=0.5, qw=q) for r, q in zip(rows, qws)])
+    y = torch.full(net.out_shape, float("nan"), device="cuda")
+    net.run(x, out=y)
+    torch.cuda.synchronize()
+    net.close()
+    for first, last in ((0, 40), (h // 2 - 13, h // 2 + 20), (h - 40, h)):
+        lo, hi = max(first - 1, 0), min(last + 1, h)
+        a = hip.conv(typ, x[:, :, lo:hi].contiguous(), thr_d, qws[0], mid, 3, 3, 1, 1, 0.5, engine=hip.ENGINE_VALU)
+        want = hip.conv(typ, a[:, :, first - lo:last - lo].contiguous(), thr_d, qws[1], kn, 1, 1, 0, 1, 0.5, engine=hip.ENGINE_VALU)
+        assert torch.equal(y[:, :, first:last], want), (first, last)
+
+
 @pytest.mark.parametrize("typ", [TNN, TBN, BTN, BNN], ids=lambda t: TYPE_NAMES[t])
 @pytest.mark.parametrize("c", [3, 64], ids=["first-layer", "layer"])
 def test_layers_with_results_beyond_256_mib(hip, oracle, typ, c):
