@@ -917,7 +917,7 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
 template <bool ABIN, bool FORM0, int QMODE, int TA, int TB, int S, bool BUF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && QMODE != 0) ? 3 : 1, 8))) void k_conv_f4(
     const uint4* __restrict__ P2, const uint4* __restrict__ Wf, float* __restrict__ Y, int M, int KN, int OHW, int KP /* pairs a weight row is stored at */,
-    int bias, float alpha, FastDiv dOHW, ConvGeom cg, PairWalk pw, QuantOut qo, uint32_t p2_bytes, uint32_t wf_bytes, uint32_t y_span, XcdOrder xo, uint32_t grid_x, uint32_t grid_y) {
+    int bias, float alpha, FastDiv dOHW, ConvGeom cg, PairWalk pw, QuantOut qo, uint32_t p2_bytes, uint32_t wf_bytes, uint32_t y_span, XcdOrder xo, uint32_t launched_x, uint32_t kernel_tiles) {
     constexpr int WPB = 4;                // wavefronts per workgroup (single-wavefront workgroups for S = 1
                                           // measured slower: neighbours no longer share weight fragments in L1)
     constexpr int NB = 3;                 // register sets of records: NB - 1 pairs of loads in flight; four and six measured slower
@@ -929,7 +929,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
     const int ks = wave % S, pt = wave / S;   // K share and pixel tile of this wavefront
     const int h = lane >> 5, lr = lane & 31;
     uint32_t bx, by;   // pixel tiles, kernel tile
-    xo.tile<QMODE == 0>(blockIdx.x + grid_x * blockIdx.y, bx, by);   // (gridDim would bring 256 bytes of hidden arguments: 0.1 us a launch)
+    xo.tile<QMODE == 0>(blockIdx.x + launched_x * blockIdx.y, bx, by);   // (gridDim would bring 256 bytes of hidden arguments: 0.1 us a launch)
     if (QMODE == 0 && xo.mask == 0) {   // plain: pixel tiles are the inner index
         const uint32_t t = bx;
         bx = by;
@@ -1191,7 +1191,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
         });
     } else {
         // Hand-over to an fp4 layer: dwords 2 h and 2 h + 1 of a pixel's record are lane half h of its two 32-kernel blocks
-        const uint32_t KT = TA == 2 ? grid_y : grid_y >> 1, kt = TA == 2 ? by : by >> 1;
+        const uint32_t KT = TA == 2 ? kernel_tiles : kernel_tiles >> 1, kt = TA == 2 ? by : by >> 1;
         auto out_rec = [&](int b) {
             return static_cast<unsigned char*>(qo.p2) + (((size_t)img[b] * KT + kt) * (uint32_t)OHW + pix[b]) * 16 + 8 * h;
         };
@@ -1535,7 +1535,10 @@ hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const Co
     const bool small = tiles < (tune_small >= 0 ? tune_small : qo.mode == 0 && cg.K < 120 ? 300 : 150);
     dim3 grid((unsigned)(((M + 63) / 64 + tpb - 1) / tpb), (unsigned)((KN + 63) / 64));
     if (small) grid = dim3((unsigned)((M + 31) / 32), (unsigned)(qo.mode != 0 ? 2 * ((KN + 63) / 64) : (KN + 31) / 32));
-    if (M > 0x7fffff00LL || grid.y > 65535) return hipErrorInvalidValue;   // pixel indices stay below 2^31
+    if (M > 0x7fffff00LL) return hipErrorInvalidValue;   // pixel indices stay below 2^31
+    // A launch takes 65535 workgroups in y: from 65536 kernel tiles on they go in x.  The kernel goes by the linear number.
+    const dim3 launched = grid.y > 65535 ? dim3(grid.y, grid.x) : grid;
+    if (launched.y > 65535) return hipErrorInvalidValue;
     const uint4* P2 = static_cast<const uint4*>(d_p2);
     const uint4* Wf = static_cast<const uint4*>(d_wf);
     const FastDiv dOHW = make_fastdiv((uint32_t)OHW);
@@ -1555,8 +1558,8 @@ hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const Co
         constexpr bool A = decltype(abin)::value, F = decltype(form0)::value;
         constexpr int Q = decltype(qmode)::value, T = decltype(blocks)::value, SP = decltype(sp)::value;
         auto go = [&](auto kern) -> hipError_t {
-            hipLaunchKernelGGL(kern, grid, dim3(64 * wpb), 0, st, P2, Wf, d_y, (int)M, KN, OHW, KP, bias, alpha, dOHW, cg, pw, qo,
-                               clip(p2_bytes), clip(wf_bytes), clip(y_span), xo, grid.x, grid.y);
+            hipLaunchKernelGGL(kern, launched, dim3(64 * wpb), 0, st, P2, Wf, d_y, (int)M, KN, OHW, KP, bias, alpha, dOHW, cg, pw, qo,
+                               clip(p2_bytes), clip(wf_bytes), clip(y_span), xo, launched.x, grid.y);
             return hipGetLastError();
         };
         return buf ? go(k_conv_f4<A, F, Q, T, T, SP, true>) : go(k_conv_f4<A, F, Q, T, T, SP, false>);

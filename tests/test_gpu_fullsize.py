@@ -309,6 +309,36 @@ def test_chain_input_beyond_32_bit_offsets_within_an_image(hip, oracle, typ):
         assert torch.equal(y[:, :, first:last], want), (first, last)
 
 
+@pytest.mark.parametrize("typ", [TNN, BNN], ids=lambda t: TYPE_NAMES[t])
+def test_more_kernel_tiles_than_a_launch_takes_in_y(hip, typ):
+    """65537 tiles of 64 kernels on 23 x 23 pixels (a result of 8.3 GiB), on the engine and with prepared weights, against the vector-ALU
+    engine on quarters of the kernels"""
+    import torch
+    from fastertnn_amd import weight_is_ternary
+    kn, c, hw = 65536 * 64 + 1, 64, 23
+    assert (kn + 63) // 64 > 65535 and hw * hw >= 512
+    print("case", TYPE_NAMES[typ], flush=True)
+    wt = weight_is_ternary(typ)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(10)
+    x = torch.randn((1, c, hw, hw), generator=g, device="cuda")
+    thr = torch.full((1,), 0.5 if typ == TNN else 0.0, device="cuda")
+    qw = hip.pack_weights(torch.randn((kn, c, 1, 1), generator=g, device="cuda"), torch.full((kn,), 0.5 if wt else 0.0, device="cuda"), wt)
+    words = qw.numel() // kn
+    out = torch.full((1, kn, hw, hw), float("nan"), device="cuda")
+    for prepared in (False, True):
+        if prepared:
+            out.fill_(float("nan"))
+            hip.conv_prepared(typ, x, thr, hip.prepare_conv_weights(typ, qw, c, kn, 1, 1), kn, 1, 1, 0, 1, 0.5, out=out)
+        else:
+            hip.conv(typ, x, thr, qw, kn, 1, 1, 0, 1, 0.5, engine=hip.ENGINE_MFMA_F4, out=out)
+        for lo in range(0, kn, kn // 4 + 1):
+            hi = min(lo + kn // 4 + 1, kn)
+            part = qw[lo * words:hi * words].contiguous()
+            want = hip.conv(typ, x, thr, part, hi - lo, 1, 1, 0, 1, 0.5, engine=hip.ENGINE_VALU)
+            assert torch.equal(out[:, lo:hi], want), (prepared, lo)
+
+
 @pytest.mark.parametrize("typ", [TNN, TBN, BTN, BNN], ids=lambda t: TYPE_NAMES[t])
 @pytest.mark.parametrize("c", [3, 64], ids=["first-layer", "layer"])
 def test_layers_with_results_beyond_256_mib(hip, oracle, typ, c):
