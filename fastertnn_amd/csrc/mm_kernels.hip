@@ -379,6 +379,30 @@ __global__ __launch_bounds__(KS ? 64 * KS : 256) void k_mm(const uint32_t* __res
         // src/tnns/mm_p2_final_tbn_avx2.c:72-73
         return r >= 0 ? (float)r : alpha * r;
     };
+    // Hand-over to an fp4 layer: kernels col0 + b and col0 + b + 1 of this lane's pixel, half a byte of its record
+    const bool tern = qo.mode == 1, whole = col0 + TN <= KN;   // uniform: all of this wavefront's columns are real kernels
+    auto half_byte = [&](int a, int b) -> uint32_t {
+        return p2_join(quant_nibble(finish(a, b), qo.t, tern, whole || col0 + b < KN),
+                       quant_nibble(finish(a, b + 1), qo.t, tern, whole || col0 + b + 1 < KN));
+    };
+    auto record_of = [&](int64_t i) -> unsigned char* {   // the bytes of kernels col0 .. of pixel i: four kernels each, eight bytes apart
+        const uint32_t img = fastdiv((uint32_t)i, dOHW);
+        const uint32_t pix = (uint32_t)i - img * (uint32_t)OHW;
+        const size_t word = ((size_t)img * ((KN + 63) / 64) + (col0 >> 6)) * OHW + pix;
+        return static_cast<unsigned char*>(qo.p2) + word * 16 + 4 * ((col0 >> 5) & 1) + ((col0 >> 3) & 3);
+    };
+    if constexpr (TN == 2 && !TR && !KS) {
+        if (qo.mode != 0) {   // two wavefronts make a byte: they meet in the operand buffers, behind the partial zero counts
+            static_assert(TM == 1 && (MODE == kTBN ? 4 * BM : 0) + 4 * 64 <= 2 * BM * LDW, "the half bytes fit the operand buffers");
+            uint32_t* met = &lds[0][0] + (MODE == kTBN ? 4 * BM : 0);
+            const uint32_t own = half_byte(0, 0);
+            met[wave * 64 + lane] = own;
+            __syncthreads();
+            const int64_t i = row0 + lane;
+            if ((wave & 1) == 0 && i < M) record_of(i)[8 * ((col0 >> 2) & 1)] = (unsigned char)(own | met[(wave + 1) * 64 + lane] << 4);
+            return;
+        }
+    }
     // Row-major result (OHW == 1, the GEMM entry points): a lane's TN columns are contiguous, so they
     // leave as 16-byte stores (full 32-byte sectors) instead of TN scattered dwords.
     const bool vec = TN % 4 == 0 && OHW == 1 && (KN & 3) == 0 && col0 + TN <= KN &&
@@ -388,21 +412,10 @@ __global__ __launch_bounds__(KS ? 64 * KS : 256) void k_mm(const uint32_t* __res
         const int64_t i = row0 + lane + 64 * a;
         if (i < M) {
             if (!TR && qo.mode != 0) {
-                // hand-over to an fp4 layer: this lane's TN kernels are one or two bytes of a pixel's record, four kernels each
-                const uint32_t img = fastdiv((uint32_t)i, dOHW);
-                const uint32_t pix = (uint32_t)i - img * (uint32_t)OHW;
-                const float t = qo.t;
-                const bool tern = qo.mode == 1, whole = col0 + TN <= KN;   // uniform: all of this wavefront's columns are real kernels
-                const size_t word = ((size_t)img * ((KN + 63) / 64) + (col0 >> 6)) * OHW + pix;
-                unsigned char* dst = static_cast<unsigned char*>(qo.p2) + word * 16 + 4 * ((col0 >> 5) & 1) + ((col0 >> 3) & 3);
-                if constexpr (TN >= 4) {   // (the launcher takes no narrower tile: two kernels are half a byte)
+                if constexpr (TN >= 4) {
+                    unsigned char* dst = record_of(i);
 #pragma unroll
-                    for (int b = 0; b < TN; b += 4) {
-                        uint32_t n[4];
-#pragma unroll
-                        for (int j = 0; j < 4; j++) n[j] = quant_nibble(finish(a, b + j), t, tern, whole || col0 + b + j < KN);
-                        dst[8 * (((col0 + b) >> 2) & 1)] = (unsigned char)(p2_join(n[0], n[1]) | p2_join(n[2], n[3]) << 4);
-                    }
+                    for (int b = 0; b < TN; b += 4) dst[8 * (((col0 + b) >> 2) & 1)] = (unsigned char)(half_byte(a, b) | half_byte(a, b + 2) << 4);
                 }
             } else if (TR) {   // consecutive lanes write consecutive floats of one output row
 #pragma unroll
@@ -462,8 +475,7 @@ hipError_t launch_mode(const uint32_t* A, const uint32_t* B, float* Y, int64_t M
         sscanf(force, "%d,%d", &tm, &tn);
 #define FTNN_TRY(TM_, TN_) \
     if (tm == TM_ && tn == TN_) return launch_cfg<MODE, TM_, TN_, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
-        FTNN_TRY(2, 8) FTNN_TRY(1, 8) FTNN_TRY(1, 4)
-        if (qo.mode == 0) { FTNN_TRY(1, 2) }
+        FTNN_TRY(2, 8) FTNN_TRY(1, 8) FTNN_TRY(1, 4) FTNN_TRY(1, 2)
 #undef FTNN_TRY
     }
     // Few tiles and a K loop worth splitting: the wavefronts of a workgroup share K (KS in the kernel).  Measured on
@@ -485,8 +497,9 @@ hipError_t launch_mode(const uint32_t* A, const uint32_t* B, float* Y, int64_t M
     }
     if (wgs(2, 8) >= 3072) return launch_cfg<MODE, 2, 8, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
     if (wgs(1, 8) >= 1536) return launch_cfg<MODE, 1, 8, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
-    // (a hand-over writes whole bytes of four kernels)
-    if (wgs(1, 4) >= 2048 || qo.mode != 0) return launch_cfg<MODE, 1, 4, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
+    // A hand-over goes by whole bytes of four kernels, two wavefronts to a byte on tiles of two.  Chains of a few-channel layer and a 1 x 1
+    // layer, us, tiles of two / four kernels: 52 workgroups of four 12.9 / 13.5, 208 13.6 / 14.1, 784 TBN 15.3 / 15.0, BTN 17.1 / 17.5.
+    if (wgs(1, 4) >= (qo.mode != 0 ? 512 : 2048)) return launch_cfg<MODE, 1, 4, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
     return launch_cfg<MODE, 1, 2, 1, IMPL, TR>(A, B, Y, M, KN, OHW, G, K_unpack, alpha, cg, st, qo);
 }
 

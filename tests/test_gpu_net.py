@@ -197,6 +197,20 @@ def test_random_chains_match_the_oracle(hip, oracle):
         done += 1
 
 
+@pytest.mark.parametrize("kn", [1, 2, 3, 4, 6, 7, 9, 33, 62, 63, 66, 130])
+@pytest.mark.parametrize("typ", [TNN, TBN, BTN, BNN], ids=lambda t: TYPE_NAMES[t])
+def test_small_hand_over_of_the_vector_alu(hip, oracle, typ, kn):
+    """few-channel layers of few pixels run on tiles of two kernels, where two wavefronts make a byte of the record they hand over:
+    kernel counts around the four of a byte and the eight of a workgroup, ragged pixel counts, to a ternary and a binary layer"""
+    import torch
+    print("case", TYPE_NAMES[typ], kn, flush=True)
+    for c, h, w, nxt in ((12, 9, 11, TNN), (21, 5, 13, BTN)):
+        net, host = build(hip, oracle, 2, [(typ, (c, h, w, kn, 3, 3, 1, 1)), (nxt, (kn, h, w, 40, 1, 1, 0, 1))])
+        x = synth.normal(70 + kn, (2, c, h, w))
+        assert net.run(torch.from_numpy(x).cuda()).cpu().numpy().tobytes() == oracle_chain(oracle, host, x).tobytes()
+        net.close()
+
+
 def test_resnet18_like_stack_at_batch_32(hip, oracle):
     """The end-to-end configuration at its stated size: batch 32, 3 x 224 x 224 fp32 N(0,1) input, the 19 layers of
     the ResNet-18-like TNN stack (thresholds 0.5, uniform ternary weights, PReLU 0.5), chained on the device with the
