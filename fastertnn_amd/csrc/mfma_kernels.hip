@@ -1465,10 +1465,10 @@ hipError_t launch_records_gemm(int type, const void* d_a, const void* d_b, int64
 // other conditions.
 namespace {
 // the tile kernel's limits: a tap mask of 32 bits per pixel, a table entry per K word, 32-bit record indices into T2,
-// pixel indices below 2^31 and its way of keeping kw - pad non-negative
+// its tiles of 128 pixels in y of a launch, which takes 65535, and its way of keeping kw - pad non-negative
 bool conv_tiles_within_limits(int64_t M, int CP, int taps, int64_t t2_bytes, int W_pad, int W_stride) {
     const int64_t K = (int64_t)CP * taps;
-    return taps <= 32 && (K + 3) / 4 * 4 <= kMaxTileRouteWords && M <= 0x7fffff00LL && t2_bytes / 16 <= 0x7fffffffLL &&
+    return taps <= 32 && (K + 3) / 4 * 4 <= kMaxTileRouteWords && (M + 127) / 128 <= 65535 && t2_bytes / 16 <= 0x7fffffffLL &&
            W_pad < 4096 * (int64_t)W_stride;
 }
 }  // namespace

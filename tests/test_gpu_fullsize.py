@@ -339,6 +339,25 @@ def test_more_kernel_tiles_than_a_launch_takes_in_y(hip, typ):
             assert torch.equal(out[:, lo:hi], want), (prepared, lo)
 
 
+@pytest.mark.parametrize("typ", [TNN, BNN], ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("n", [166, 168], ids=["65072_tiles", "65856_tiles"])
+def test_strided_layer_on_both_sides_of_what_a_launch_takes_in_y(hip, typ, n):
+    """256 x 448 x 448, 5 x 5 stride 2 (100 words): the tile kernel's tiles of 128 pixels go in y of a launch, which takes 65535.  Against
+    the vector-ALU engine on every element"""
+    import torch
+    from fastertnn_amd import weight_is_ternary
+    c, hw, kn = 256, 448, 8
+    print("case", TYPE_NAMES[typ], n, flush=True)
+    wt = weight_is_ternary(typ)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(11)
+    x = torch.randn((n, c, hw, hw), generator=g, device="cuda")
+    thr = torch.full((n,), 0.5 if typ == TNN else 0.0, device="cuda")
+    qw = hip.pack_weights(torch.randn((kn, c, 5, 5), generator=g, device="cuda"), torch.full((kn,), 0.5 if wt else 0.0, device="cuda"), wt)
+    got, want = (hip.conv(typ, x, thr, qw, kn, 5, 5, 2, 2, 0.5, engine=e) for e in (hip.ENGINE_MFMA_F4, hip.ENGINE_VALU))
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("typ", [TNN, TBN, BTN, BNN], ids=lambda t: TYPE_NAMES[t])
 @pytest.mark.parametrize("c", [3, 64], ids=["first-layer", "layer"])
 def test_layers_with_results_beyond_256_mib(hip, oracle, typ, c):
