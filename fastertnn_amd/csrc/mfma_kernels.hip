@@ -686,7 +686,7 @@ struct TileRec {
     static_assert(PPS == 1 || QW == 1, "one pair per wavefront on the gathered side");
 };
 
-template <bool SWAP, int WTP, int WTQ, int PPS, int NS, bool IMPL>
+template <bool SWAP, bool NT, int WTP, int WTQ, int PPS, int NS, bool IMPL>
 __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, const uint4* __restrict__ Qc, float* __restrict__ Y,
                                                  int M, int KN, int OHW, int KP /* pairs of words per row */, int nstep, int bias,
                                                  int form, float alpha, ConvGeom cg, FastDiv dOHW, int Ws, FastDiv dSW) {
@@ -873,7 +873,7 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
     for (; s + NS < nstep; s++) step_body(s, std::true_type{});
     for (; s < nstep; s++) step_body(s, std::false_type{});
 
-    store_tile<true, SWAP, true, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
+    store_tile<true, SWAP, NT, WTP, WTQ>(acc, Y, M, KN, OHW, prb0 + wy * WTP, qrb0 + wx * WTQ, lane, bias, form, alpha);
 }
 
 // ------------------------------------------------------------ conv layer (fp4)
@@ -1410,10 +1410,10 @@ hipError_t launch_mfma_gemm_packed4(int type, const void* d_ac, const void* d_bc
 
 namespace {
 constexpr int kMaxTileRouteWords = 2040;   // K words per row the tile kernel keeps a table entry for (16 KiB of LDS)
-template <bool SWAP, int WTP, int WTQ, int PPS, int NS, bool IMPL>
-hipError_t launch_records_tile(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, int pairs, int bnn_k, int form,
+template <bool SWAP, bool NT, int WTP, int WTQ, int PPS, int NS, bool IMPL>
+hipError_t launch_records_tile_as(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, int pairs, int bnn_k, int form,
                                float alpha, const ConvGeom& cg, hipStream_t st) {
-    auto kern = k_mfma_s2<SWAP, WTP, WTQ, PPS, NS, IMPL>;
+    auto kern = k_mfma_s2<SWAP, NT, WTP, WTQ, PPS, NS, IMPL>;
     typedef TileRec<WTP, WTQ, PPS, NS> TL;
     constexpr size_t kLdsMax = 160u << 10;   // LDS of a compute unit
     const int nstep = (pairs + PPS - 1) / PPS;   // (a row is stored at an even number of pairs)
@@ -1421,7 +1421,7 @@ hipError_t launch_records_tile(const uint4* Pc, const uint4* Qc, float* Y, int M
     if (lds_bytes > kLdsMax) return hipErrorInvalidValue;
     // as launch_gemm_tile: hand-counted LDS-direct loads, so no scratch; the LDS opt-in is per kernel
     static const hipError_t configured = []() {
-        const void* k = reinterpret_cast<const void*>(&k_mfma_s2<SWAP, WTP, WTQ, PPS, NS, IMPL>);
+        const void* k = reinterpret_cast<const void*>(&k_mfma_s2<SWAP, NT, WTP, WTQ, PPS, NS, IMPL>);
         hipFuncAttributes attr;
         hipError_t e = hipFuncGetAttributes(&attr, k);
         if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
@@ -1437,6 +1437,20 @@ hipError_t launch_records_tile(const uint4* Pc, const uint4* Qc, float* Y, int M
     hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Pc, Qc, Y, M, KN, OHW, KP, nstep, bias, form, alpha, cg,
                        make_fastdiv((uint32_t)OHW), IMPL ? (cg.W + cg.W_stride - 1) / cg.W_stride : 0, make_fastdiv(IMPL ? (uint32_t)cg.W_stride : 1u));
     return hipGetLastError();
+}
+
+// The larger tiles store as those of the GEMM do (stores_past_caches).  Strided layers on 256 x 128, under sustained load, us, past / through
+// the caches: whole sectors 50.2 / 52.3 (8 x 1024 x 56 x 56 -> 1024), 137 / 142, 114 / 118; other rows 65.3 / 57.5 (34 x 1024 x 28 x 28 -> 1024),
+// 118 / 112, 95.9 / 90.5, 192 / 185.  Of 128 x 128 two workgroups share a compute unit, one's stores go on beside the other's
+// multiplies: past the caches 0.94 to 1.08 of the time through them on other rows, 0.87 to 0.99 on whole sectors.
+template <bool SWAP, int WTP, int WTQ, int PPS, int NS, bool IMPL>
+hipError_t launch_records_tile(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, int pairs, int bnn_k, int form,
+                               float alpha, const ConvGeom& cg, hipStream_t st) {
+    if constexpr (WTP >= 4) {
+        if (!stores_past_caches(SWAP ? OHW : KN, M, KN))
+            return launch_records_tile_as<SWAP, false, WTP, WTQ, PPS, NS, IMPL>(Pc, Qc, Y, M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
+    }
+    return launch_records_tile_as<SWAP, true, WTP, WTQ, PPS, NS, IMPL>(Pc, Qc, Y, M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
 }
 
 template <bool SWAP>
@@ -1494,8 +1508,10 @@ hipError_t launch_conv_f4_tiles(int type, const void* d_t2, const void* d_wf, co
     const int bnn_k = type == kBNN ? K_unpack : 0, form = type == kTNN ? 0 : 1;
     const uint4* Wf = static_cast<const uint4*>(d_wf);
     const uint4* T2 = static_cast<const uint4*>(d_t2);
-    // tiles of 256 kernels x 128 pixels where those fill most of the chip in one round (the layer above: 196 workgroups, 53.9 us against
-    // 55.6 on 392 tiles of 128 x 128), else 128 x 128.  FTNN_CONV_TILE_SHAPE = 22 | 42 forces one (tuning aid)
+    // Tiles of 256 kernels x 128 pixels where those fill most of the chip in one round, else 128 x 128.  Ten layers of 1500 tiles of
+    // 64 x 64 and more with 196 to 252 of them, under sustained load, 128 x 128 / 256 x 128: 8 x 1024 x 56 x 56 -> 1024 (196) 51.4 / 50.2 us,
+    // 34 x 1024 x 28 x 28 -> 1024 (212) 59.6 / 57.5, 6 x 2105 x 56 x 87 -> 1024 (232) 120 / 114, the others 0.94 to 0.99; from 258 on 217 / 193
+    // and up to 1.4.  FTNN_CONV_TILE_SHAPE = 22 | 42 forces one (tuning aid)
     static const int tune = getenv("FTNN_CONV_TILE_SHAPE") ? atoi(getenv("FTNN_CONV_TILE_SHAPE")) : 0;
     const int64_t mid = ((M + 127) / 128) * ((KN + 255) / 256);
     int shape = mid >= 180 && mid <= 256 ? 42 : 22;

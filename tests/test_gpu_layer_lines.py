@@ -13,8 +13,9 @@ LAYERS = [(1, 64, t, 64, 64, 3) for t in (299, 300, 519, 520, 1023, 1024)] + [(1
          [(1, 896, t, 64, 64, 3) for t in (149, 150)] + [(2, 64, 256, 256, 530, 1), (2, 64, 255, 255, 535, 1), (2, 64, 1, 65537, 530, 1)]
 
 
-# stride 2, 108 words: on both sides of the 1500 tiles from which such a layer runs as workgroup tiles, on both of their shapes
-STRIDED = [(1, 768, 185, 127, 1000, 3), (1, 768, 189, 127, 1000, 3), (1, 768, 299, 255, 300, 3)]
+# stride 2, 108 words: on both sides of the 1500 tiles from which such a layer runs as workgroup tiles, on both of their shapes; then
+# results of more than 4 Mi values whose rows are no whole sectors, on both shapes
+STRIDED = [(1, 768, 185, 127, 1000, 3), (1, 768, 189, 127, 1000, 3), (1, 768, 299, 255, 300, 3), (5, 768, 75, 71, 1000, 3), (8, 768, 75, 71, 1000, 3)]
 
 
 @pytest.mark.parametrize("typ", range(4), ids=[TYPE_NAMES[t] for t in range(4)])
