@@ -655,10 +655,10 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
 // Large layers.  2 x 2 wavefronts per workgroup, WTP x WTQ blocks of 32 x 32 each: (64 WTP) x (64 WTQ) results.  P side:
 // weights, Q side: pixels (SWAP; without it, for one-pixel images, P = rows of the activations and Q = weights, row-major).
 // Both operands are blocks of records: 1 KiB = 32 rows x two K words, lane l = (word of the pair l / 32, row l % 32).  A stage
-// of the LDS ring holds PPS pairs of every row block, filled by LDS-direct loads that the kernel counts by hand; a block is one
+// of the LDS ring holds one pair of every row block, filled by LDS-direct loads that the kernel counts by hand; a block is one
 // 16-byte read per lane, split into the nibbles of two multiplies (lanes of both words of a pair enter both, see P2).  The
-// schedule is k_mfma_p4's: the first word's multiplies run while the second one's operands are split; then (behind the barrier
-// where the stage ends) the second word's multiplies run beside the LDS reads of the next pair, each block split LAG slots
+// schedule is k_mfma_p4's: the first word's multiplies run while the second one's operands are split; then, behind the barrier, the
+// second word's multiplies run beside the LDS reads of the next pair, each block split LAG slots
 // after its read.  These tiles are bound by what they move through the LDS: at four bits per lane a step of two K words
 // moved 72 KiB for 512 cycles of matrix pipe (256 x 128 tile) and took 1080 cycles.
 //
@@ -674,27 +674,26 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
 //     for a padding word), and the word's part of the record index (plane, tap row, column class and slot offset);
 //   * per row block a lane keeps the mask of the taps that fall inside the image for its pixel, and its pixel's part of the index;
 // a block's source is then one AND, one add, one select and the address.
-template <int WTP, int WTQ, int PPS, int NS>
+template <int WTP, int WTQ, int NS>
 struct TileRec {
     static constexpr int RBP = 2 * WTP, RBQ = 2 * WTQ;         // row blocks per operand side
-    static constexpr int PF = RBP * PPS, FR = PF + RBQ * PPS;  // blocks per stage: the P side's, then the Q side's
-    static constexpr int PW = PF / 4, QW = RBQ * PPS / 4, FW = PW + QW;   // blocks a wavefront stages
+    static constexpr int FR = RBP + RBQ;                       // blocks per stage: the P side's, then the Q side's
+    static constexpr int PW = RBP / 4, QW = RBQ / 4, FW = PW + QW;   // blocks a wavefront stages
     static constexpr int NL = WTP + WTQ, NM = WTP * WTQ;       // LDS reads per pair of words, multiplies per word
-    static constexpr int LAG = NL >= 8 ? 4 : (NL >= 4 ? 3 : 1);
+    static constexpr int LAG = NL >= 8 ? 4 : 3;
     static constexpr size_t lds_bytes = (size_t)NS * FR * 1024;
-    static_assert(PF % 4 == 0 && (RBQ * PPS) % 4 == 0 && FW <= NL, "a quarter of each side per wavefront, one load per slot");
-    static_assert(PPS == 1 || QW == 1, "one pair per wavefront on the gathered side");
+    static_assert(RBP % 4 == 0 && RBQ % 4 == 0 && FW <= NL, "a quarter of each side per wavefront, one load per slot");
 };
 
-template <bool SWAP, bool NT, int WTP, int WTQ, int PPS, int NS, bool IMPL>
+template <bool SWAP, bool NT, int WTP, int WTQ, int NS, bool IMPL>
 __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, const uint4* __restrict__ Qc, float* __restrict__ Y,
                                                  int M, int KN, int OHW, int KP /* pairs of words per row */, int nstep, int bias,
                                                  int form, float alpha, ConvGeom cg, FastDiv dOHW, int Ws, FastDiv dSW) {
     static_assert(!IMPL || SWAP, "implicit im2row: the pixels along the lanes");
     extern __shared__ uint4 lds[];   // NS stages of FR KiB, then the table
     typedef Acc<true>::type acc_t;
-    typedef TileRec<WTP, WTQ, PPS, NS> TL;
-    constexpr int RBP = TL::RBP, RBQ = TL::RBQ, PF = TL::PF, FR = TL::FR, PW = TL::PW, QW = TL::QW, FW = TL::FW;
+    typedef TileRec<WTP, WTQ, NS> TL;
+    constexpr int RBP = TL::RBP, RBQ = TL::RBQ, FR = TL::FR, PW = TL::PW, QW = TL::QW, FW = TL::FW;
     constexpr int NL = TL::NL, NM = TL::NM, LAG = TL::LAG;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -723,21 +722,17 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[a][b][e] = 0;
 
-    // Block g of a side and stage: row block g / PPS, pair g % PPS.  Wavefront w stages blocks w PW .. of the P side and w QW ..
-    // of the Q side; row blocks past the operand are clamped (their results are never stored).
+    // Wavefront w stages row blocks w PW .. of the P side and w QW .. of the Q side; row blocks past the operand are clamped (their results are never stored).
     const uint4* psrc[PW];
 #pragma unroll
-    for (int i = 0; i < PW; i++) {
-        const int g = wave * PW + i;
-        psrc[i] = Pc + ((size_t)min(prb0 + g / PPS, prbmax) * KP + g % PPS) * 64 + lane;
-    }
+    for (int i = 0; i < PW; i++) psrc[i] = Pc + (size_t)min(prb0 + wave * PW + i, prbmax) * KP * 64 + lane;
     const uint4* qsrc[IMPL ? 1 : QW];
     uint32_t tapmask[IMPL ? QW : 1], qbase[IMPL ? QW : 1];
     const uint32_t row16 = (uint32_t)(cg.W_stride * Ws);            // records per input row
     const uint32_t plane16 = (uint32_t)cg.H * row16;                // per plane of 64 channels
     const uint32_t fill_rec = (uint32_t)cg.CP * plane16 * (uint32_t)((M - 1) / OHW + 1);   // right behind the planes
     uint2* const wtab = reinterpret_cast<uint2*>(lds + (size_t)NS * FR * 64);
-    const int words = 2 * PPS * nstep;
+    const int words = 2 * nstep;
     if constexpr (IMPL) {
         for (int w = tid; w < words; w += 256) {
             const int tap = (int)fastdiv((uint32_t)w, cg.dCP), ic = w - tap * cg.CP;
@@ -751,7 +746,7 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
         }
 #pragma unroll
         for (int j = 0; j < QW; j++) {
-            const int rb = (wave * QW + j) / PPS;
+            const int rb = wave * QW + j;
             const uint32_t q = (uint32_t)min((qrb0 + rb) * 32 + (lane & 31), M - 1);
             const uint32_t img = fastdiv(q, dOHW);
             const uint32_t pix = q - img * (uint32_t)OHW;
@@ -769,31 +764,28 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
         __syncthreads();   // the table is complete before the first stage is issued
     } else {
 #pragma unroll
-        for (int i = 0; i < QW; i++) {
-            const int g = wave * QW + i;
-            qsrc[i] = Qc + ((size_t)min(qrb0 + g / PPS, qrbmax) * KP + g % PPS) * 64 + lane;
-        }
+        for (int i = 0; i < QW; i++) qsrc[i] = Qc + (size_t)min(qrb0 + wave * QW + i, qrbmax) * KP * 64 + lane;
     }
     // this lane's word of the pair that its wavefront gathers of the stage about to be issued (stages are issued strictly in
     // order); its table entry is read one stage ahead of its use
-    int g_w = 2 * (PPS == 1 ? 0 : wave % PPS) + (lane >> 5);
+    int g_w = lane >> 5;
     uint2 wt = make_uint2(0u, 0u), wt_ahead = make_uint2(0u, 0u);
     if constexpr (IMPL) wt_ahead = wtab[g_w];
     auto next_words = [&]() {
         wt = wt_ahead;
-        g_w = min(g_w + 2 * PPS, words - 1);   // (past the last stage: any entry)
+        g_w = min(g_w + 2, words - 1);   // (past the last stage: any entry)
         wt_ahead = wtab[g_w];
     };
     const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
     auto load = [&](int i, int step) {   // slot i of the wavefront's loads for stage `step`
         const uint32_t dst = lds0 + (uint32_t)(step % NS) * (FR * 1024);
         if (i < PW) {
-            dma16(psrc[i] + (size_t)step * PPS * 64, dst + (uint32_t)(wave * PW + i) * 1024);
+            dma16(psrc[i] + (size_t)step * 64, dst + (uint32_t)(wave * PW + i) * 1024);
         } else {
             const int j = i - PW;
-            const uint32_t d = dst + (uint32_t)(PF + wave * QW + j) * 1024;
+            const uint32_t d = dst + (uint32_t)(RBP + wave * QW + j) * 1024;
             if constexpr (IMPL) dma16(Qc + ((tapmask[j] & wt.x) != 0u ? qbase[j] + wt.y : fill_rec), d);   // a select on the index: no branch
-            else dma16(qsrc[j] + (size_t)step * PPS * 64, d);
+            else dma16(qsrc[j] + (size_t)step * 64, d);
         }
     };
     auto stage = [&](int step) {
@@ -804,11 +796,11 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
     // raw: the records of the pair being consumed; e[k]: its nibbles for multiply k.  Slots in the order the multiplies take
     // them: 0: P block 0, 1 .. WTQ: Q blocks, then P blocks 1 .. WTP - 1.
     uint4 rp[WTP], rq[WTQ], ep[2][WTP], eq[2][WTQ];
-    auto read_raw = [&](int buf, int pair, int i) {
-        const uint4* L = lds + (size_t)buf * FR * 64 + pair * 64 + lane;
-        if (i == 0) rp[0] = L[(wy * WTP + 0) * PPS * 64];
-        else if (i <= WTQ) rq[i - 1] = L[(PF + (wx * WTQ + (i - 1)) * PPS) * 64];
-        else rp[i - WTQ] = L[(wy * WTP + (i - WTQ)) * PPS * 64];
+    auto read_raw = [&](int buf, int i) {
+        const uint4* L = lds + (size_t)buf * FR * 64 + lane;
+        if (i == 0) rp[0] = L[(wy * WTP + 0) * 64];
+        else if (i <= WTQ) rq[i - 1] = L[(RBP + wx * WTQ + (i - 1)) * 64];
+        else rp[i - WTQ] = L[(wy * WTP + (i - WTQ)) * 64];
     };
     auto split = [&](int k, int i) {
         const uint4& r = i == 0 ? rp[0] : (i <= WTQ ? rq[i - 1] : rp[i - WTQ]);
@@ -832,7 +824,7 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NL; i++) read_raw(0, 0, i);
+    for (int i = 0; i < NL; i++) read_raw(0, i);
 #pragma unroll
     for (int i = 0; i < NL; i++) split(0, i);
 
@@ -841,32 +833,26 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
     auto step_body = [&](int s, auto full_tag) {
         constexpr bool FULL = decltype(full_tag)::value;   // FULL: s + NS < nstep
 #pragma unroll
-        for (int pp = 0; pp < PPS; pp++) {
+        for (int i = 0; i < NL; i++) {
+            if (i < LAG && s > 0) split(0, NL - LAG + i);
+            split(1, i);
+            multiply(0, i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // Everything of this stage is in registers.  Stage s + 1 must have landed (stages s + 2 .. s + NS - 1 may still be in
+        // flight); after the barrier buffer s % NS is free for stage s + NS.
+        if (FULL || s + NS - 1 < nstep) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FW * (NS - 2)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if constexpr (FULL && IMPL) next_words();
+        const bool do_ld = FULL || s + 1 < nstep;
 #pragma unroll
-            for (int i = 0; i < NL; i++) {
-                if (i < LAG && (s > 0 || pp > 0)) split(0, NL - LAG + i);
-                split(1, i);
-                multiply(0, i);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            const bool last = pp == PPS - 1;
-            if (last) {
-                // Everything of this stage is in registers.  Stage s + 1 must have landed (stages s + 2 .. s + NS - 1 may
-                // still be in flight); after the barrier buffer s % NS is free for stage s + NS.
-                if (FULL || s + NS - 1 < nstep) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FW * (NS - 2)) : "memory");
-                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                __syncthreads();
-                if constexpr (FULL && IMPL) next_words();
-            }
-            const bool do_ld = !last || FULL || s + 1 < nstep;
-#pragma unroll
-            for (int i = 0; i < NL; i++) {
-                if (do_ld) read_raw(last ? (s + 1) % NS : s % NS, last ? 0 : pp + 1, i);
-                if (FULL && last && i < FW) load(i, s + NS);
-                if (do_ld && i >= LAG) split(0, i - LAG);
-                multiply(1, i);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+        for (int i = 0; i < NL; i++) {
+            if (do_ld) read_raw((s + 1) % NS, i);
+            if (FULL && i < FW) load(i, s + NS);
+            if (do_ld && i >= LAG) split(0, i - LAG);
+            multiply(1, i);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     int s = 0;
@@ -1410,18 +1396,17 @@ hipError_t launch_mfma_gemm_packed4(int type, const void* d_ac, const void* d_bc
 
 namespace {
 constexpr int kMaxTileRouteWords = 2040;   // K words per row the tile kernel keeps a table entry for (16 KiB of LDS)
-template <bool SWAP, bool NT, int WTP, int WTQ, int PPS, int NS, bool IMPL>
-hipError_t launch_records_tile_as(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, int pairs, int bnn_k, int form,
+template <bool SWAP, bool NT, int WTP, int WTQ, int NS, bool IMPL>
+hipError_t launch_records_tile_as(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, int nstep, int bnn_k, int form,
                                float alpha, const ConvGeom& cg, hipStream_t st) {
-    auto kern = k_mfma_s2<SWAP, NT, WTP, WTQ, PPS, NS, IMPL>;
-    typedef TileRec<WTP, WTQ, PPS, NS> TL;
+    auto kern = k_mfma_s2<SWAP, NT, WTP, WTQ, NS, IMPL>;
+    typedef TileRec<WTP, WTQ, NS> TL;
     constexpr size_t kLdsMax = 160u << 10;   // LDS of a compute unit
-    const int nstep = (pairs + PPS - 1) / PPS;   // (a row is stored at an even number of pairs)
-    const size_t lds_bytes = TL::lds_bytes + (IMPL ? (size_t)nstep * PPS * 2 * 8 : 0);   // the ring, then the table of K words
+    const size_t lds_bytes = TL::lds_bytes + (IMPL ? (size_t)nstep * 2 * 8 : 0);   // the ring, then the table of K words
     if (lds_bytes > kLdsMax) return hipErrorInvalidValue;
     // as launch_gemm_tile: hand-counted LDS-direct loads, so no scratch; the LDS opt-in is per kernel
     static const hipError_t configured = []() {
-        const void* k = reinterpret_cast<const void*>(&k_mfma_s2<SWAP, NT, WTP, WTQ, PPS, NS, IMPL>);
+        const void* k = reinterpret_cast<const void*>(&k_mfma_s2<SWAP, NT, WTP, WTQ, NS, IMPL>);
         hipFuncAttributes attr;
         hipError_t e = hipFuncGetAttributes(&attr, k);
         if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
@@ -1433,7 +1418,7 @@ hipError_t launch_records_tile_as(const uint4* Pc, const uint4* Qc, float* Y, in
     dim3 grid((prow + 64 * WTP - 1) / (64 * WTP), (qrow + 64 * WTQ - 1) / (64 * WTQ));
     if (grid.y > 65535) return hipErrorInvalidValue;
     // BNN: every lane that is no real (channel, tap) is +1 x +1 in both operands, padding words included
-    const int bias = bnn_k ? 128 * nstep * PPS - bnn_k : 0;
+    const int bias = bnn_k ? 128 * nstep - bnn_k : 0;
     hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Pc, Qc, Y, M, KN, OHW, KP, nstep, bias, form, alpha, cg,
                        make_fastdiv((uint32_t)OHW), IMPL ? (cg.W + cg.W_stride - 1) / cg.W_stride : 0, make_fastdiv(IMPL ? (uint32_t)cg.W_stride : 1u));
     return hipGetLastError();
@@ -1443,14 +1428,14 @@ hipError_t launch_records_tile_as(const uint4* Pc, const uint4* Qc, float* Y, in
 // the caches: whole sectors 50.2 / 52.3 (8 x 1024 x 56 x 56 -> 1024), 137 / 142, 114 / 118; other rows 65.3 / 57.5 (34 x 1024 x 28 x 28 -> 1024),
 // 118 / 112, 95.9 / 90.5, 192 / 185.  Of 128 x 128 two workgroups share a compute unit, one's stores go on beside the other's
 // multiplies: past the caches 0.94 to 1.08 of the time through them on other rows, 0.87 to 0.99 on whole sectors.
-template <bool SWAP, int WTP, int WTQ, int PPS, int NS, bool IMPL>
-hipError_t launch_records_tile(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, int pairs, int bnn_k, int form,
+template <bool SWAP, int WTP, int WTQ, int NS, bool IMPL>
+hipError_t launch_records_tile(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, int nstep, int bnn_k, int form,
                                float alpha, const ConvGeom& cg, hipStream_t st) {
     if constexpr (WTP >= 4) {
         if (!stores_past_caches(SWAP ? OHW : KN, M, KN))
-            return launch_records_tile_as<SWAP, false, WTP, WTQ, PPS, NS, IMPL>(Pc, Qc, Y, M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
+            return launch_records_tile_as<SWAP, false, WTP, WTQ, NS, IMPL>(Pc, Qc, Y, M, KN, OHW, KP, nstep, bnn_k, form, alpha, cg, st);
     }
-    return launch_records_tile_as<SWAP, true, WTP, WTQ, PPS, NS, IMPL>(Pc, Qc, Y, M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
+    return launch_records_tile_as<SWAP, true, WTP, WTQ, NS, IMPL>(Pc, Qc, Y, M, KN, OHW, KP, nstep, bnn_k, form, alpha, cg, st);
 }
 
 template <bool SWAP>
@@ -1458,8 +1443,8 @@ hipError_t launch_records(const uint4* Pc, const uint4* Qc, float* Y, int M, int
                           hipStream_t st) {
     const int64_t big = (((int64_t)M + 255) / 256) * ((KN + 255) / 256);
     return big < mfma_small_tile_below()
-               ? launch_records_tile<SWAP, 2, 2, 1, 4, false>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, ConvGeom(), st)
-               : launch_records_tile<SWAP, 4, 4, 1, 4, false>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, ConvGeom(), st);
+               ? launch_records_tile<SWAP, 2, 2, 4, false>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, ConvGeom(), st)
+               : launch_records_tile<SWAP, 4, 4, 4, false>(Pc, Qc, Y, M, KN, OHW, Kw / 2, Kw / 2, bnn_k, form, alpha, ConvGeom(), st);
 }
 }  // namespace
 
@@ -1516,8 +1501,8 @@ hipError_t launch_conv_f4_tiles(int type, const void* d_t2, const void* d_wf, co
     const int64_t mid = ((M + 127) / 128) * ((KN + 255) / 256);
     int shape = mid >= 180 && mid <= 256 ? 42 : 22;
     if (tune == 22 || tune == 42) shape = tune;
-    if (shape == 42) return launch_records_tile<true, 4, 2, 1, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
-    return launch_records_tile<true, 2, 2, 1, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
+    if (shape == 42) return launch_records_tile<true, 4, 2, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
+    return launch_records_tile<true, 2, 2, 4, true>(Wf, T2, d_y, (int)M, KN, OHW, KP, pairs, bnn_k, form, alpha, cg, st);
 }
 
 hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const ConvGeom& cg, int N, int KN,
