@@ -186,10 +186,14 @@ def test_size_limits_need_no_device():
     assert lib.conv_scratch_bytes(0, 1, 1, 8192, 8191, 1, 1, 1, 0, 1) > 0         # just below 2^26 pixels per plane
     assert lib.conv_scratch_bytes(0, 1, 1, 8192, 8192, 1, 1, 1, 0, 1) == 0        # 2^26: refused
     assert lib.conv_scratch_bytes(0, 65536, 1, 4, 4, 1, 1, 1, 0, 1) == 0          # batch above 65535
-    # a very large layer sizes its scratch for the im2row + GEMM form: planes + rows + fragments
+    # more kernels need more scratch: the weights in engine form
     big = lib.conv_scratch_bytes(0, 8, 1024, 56, 56, 1024, 3, 3, 1, 2)
     small = lib.conv_scratch_bytes(0, 8, 1024, 56, 56, 128, 3, 3, 1, 2)
     assert big > small > 0
+    # a layer of few pixels and many kernels sizes its scratch for the im2row + GEMM form too: the rows beside the weights (half as
+    # many kernels do not take that form)
+    big, small = (lib.conv_scratch_bytes(0, 8, 512, 7, 7, kn, 3, 3, 1, 1) for kn in (8192, 4096))
+    assert big - small > (8192 - 4096) // 32 * 72 * 1024 + 8 * 49 * 72 * 16
     # shape arithmetic that would overflow 32 bits is refused, not wrapped
     assert lib.conv_scratch_bytes(0, 1, 1, 8, 8, 1, 3, 3, 2 ** 30, 1) == 0          # padding of 2^30
     assert lib.conv_scratch_bytes(0, 1, 2 ** 31 - 1, 8, 8, 1, 3, 3, 1, 1) == 0      # channels near 2^31

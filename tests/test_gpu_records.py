@@ -1,6 +1,6 @@
 """Layer operands at two bits per lane: a pair of K words per load, the two words being planes of one tap (an even number of
-64-channel words) or any neighbours (an odd number), the last pair of an odd K half empty; on the layer kernel and on the tile
-kernel, and behind both quantiser tiles.  Bit for bit against the oracle."""
+64-channel words) or any neighbours (an odd number), the last pair of an odd K half empty; on the layer kernel, split
+ways and whole, and behind both quantiser tiles.  Bit for bit against the oracle."""
 import numpy as np
 import pytest
 
@@ -10,8 +10,8 @@ from tests.cases import make_layer
 pytestmark = pytest.mark.gpu
 
 # (C, IH, IW, KN, KW, KH, pad, stride), batch: 1, 2, 3 and 5 words of channels, 1 to 9 taps in windows of one column, one row and both,
-# every K from one word on, ragged kernel counts; images of one pixel and of more than one; the last three run as tiles
-# (64 x 64, 128 x 128) with an odd number of pairs and of words, the very last quantised by the larger workgroups
+# every K from one word on, ragged kernel counts; images of small and of ragged sizes; the last three have 290, 522 and
+# 2376 tiles of 64 x 64, an odd number of words or of pairs, and the very last is quantised by the larger workgroups
 SHAPES = [((64, 9, 7, 40, 1, 1, 0, 1), 2), ((64, 9, 7, 40, 1, 3, 1, 1), 2), ((64, 9, 7, 70, 2, 1, 1, 1), 3), ((64, 11, 11, 64, 3, 3, 1, 2), 3),
           ((128, 9, 9, 33, 3, 3, 1, 1), 2), ((130, 8, 9, 65, 1, 1, 0, 1), 2), ((130, 8, 9, 65, 3, 3, 1, 1), 2), ((190, 5, 5, 96, 2, 2, 0, 1), 4),
           ((300, 6, 6, 100, 1, 1, 0, 1), 3), ((300, 6, 6, 34, 3, 1, 2, 1), 1), ((257, 3, 3, 20, 3, 3, 0, 1), 5),
