@@ -760,14 +760,15 @@ int64_t conv_f4_dense_bytes(int N, int C, int H, int W, int KH, int KW, int OH, 
 }
 
 // Layers of few output pixels and so many kernels that these alone fill the chip run as quantise + im2row + expansion + the
-// workgroup tiles of k_mfma_s2.  With operands at two bits per lane the layer kernel has passed this route here as everywhere
-// (us, route / layer kernel: 8 x 512 x 7 x 7 -> 8192, 3 x 3 27.5 / 18.0; 1 x 2048 x 14 x 14 -> 16384 50 / 40; 2 x 1024 x 14 x 14 ->
-// 16384, 1 x 1 14.2 / 14.2); what the route leaves in the caller's scratch is pinned by a test, so it keeps these layers.
+// workgroup tiles of k_mfma_s2, if they have more than 256 pixels.  At up to 256 the layer kernel is ahead on all 33 layers measured
+// (0.47 to 0.96 of the route's time; us, route / layer kernel: 1 x 2048 x 14 x 14 -> 16384, 3 x 3 46.5 / 37.7, 10 x 1024 x 5 x 5 -> 19865
+// 47 / 32).  Beyond, it depends on how many rounds the tiles of either take: 8 x 512 x 7 x 7 -> 8192 25.5 / 17.2, 4 x 512 x 9 x 9 -> 13965 31.5 / 20.4,
+// but 2 x 2048 x 12 x 12 -> 19590 73 / 88, 11 x 2048 x 6 x 6 -> 24768 102 / 120 (10 of 39 layers at 257 to 511 pixels are ahead on the route).
 bool conv_f4_gemm_route(int64_t M, int KN, int K) {
     static const bool off = getenv("FTNN_CONV_NO_GEMM_ROUTE") != nullptr;   // tuning aid
     // enough 128 x 128 tiles for every compute unit, and enough work to pay for the three extra passes
     const int64_t tiles = ((M + 127) / 128) * ((KN + 127) / 128);
-    return !off && M < 512 && tiles >= 256 && (double)M * KN * 64.0 * K >= 1.2e10;
+    return !off && M > 256 && M < 512 && tiles >= 256 && (double)M * KN * 64.0 * K >= 1.2e10;
 }
 
 // its buffers: channel-packed planes, Packing-2 rows, the rows as matrix-core fragments (each 256-byte aligned)

@@ -194,6 +194,9 @@ def test_size_limits_need_no_device():
     # many kernels do not take that form)
     big, small = (lib.conv_scratch_bytes(0, 8, 512, 7, 7, kn, 3, 3, 1, 1) for kn in (8192, 4096))
     assert big - small > (8192 - 4096) // 32 * 72 * 1024 + 8 * 49 * 72 * 16
+    # up to 256 pixels they run on the layer kernel: nothing but the weights grows
+    big, small = (lib.conv_scratch_bytes(0, 1, 2048, 14, 14, kn, 3, 3, 1, 1) for kn in (16384, 8192))
+    assert big - small == (16384 - 8192) // 32 * 288 * 1024
     # shape arithmetic that would overflow 32 bits is refused, not wrapped
     assert lib.conv_scratch_bytes(0, 1, 1, 8, 8, 1, 3, 3, 2 ** 30, 1) == 0          # padding of 2^30
     assert lib.conv_scratch_bytes(0, 1, 2 ** 31 - 1, 8, 8, 1, 3, 3, 1, 1) == 0      # channels near 2^31
