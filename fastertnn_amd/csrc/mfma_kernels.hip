@@ -1531,9 +1531,13 @@ hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const Co
     if (tune) split = tune;
     while (split > 1 && pw.NP < split) split /= 2;   // no wavefront without K words of its own, forced or not
     const int wpb = 4, tpb = wpb / split;   // wavefronts and pixel tiles per workgroup (see the kernel)
-    // few 64 x 64 tiles: tiles of 32 x 32, four times the workgroups
+    // Few 64 x 64 tiles: tiles of 32 x 32, four times the workgroups.  fp32 results of fewer than 120 words up to 300 tiles; but where 190 to
+    // 256 tiles give most of the 256 compute units one workgroup each and a row is long (72 words), those are ahead unless the last
+    // kernel tile is half empty.  Layer and quantiser in a graph, us, 64 x 64 split four ways / 32 x 32: 216 tiles x 108 words 9.8 / 10.4,
+    // 240 x 99 11.2 / 11.7, 208 x 117 12.5 / 13.5 (20 such layers 3 % ahead in the mean); 160 x 99 10.8 / 10.2, 280 x 90 11.3 / 10.9, 196 x 36 7.3 / 7.2.
+    const bool one_round = cg.K >= 72 && tiles >= 190 && tiles <= 256 && (KN + 31) / 32 % 2 == 0;
     static const int64_t tune_small = getenv("FTNN_CONV_SMALL_BELOW") ? atoi(getenv("FTNN_CONV_SMALL_BELOW")) : -1;
-    const bool small = tiles < (tune_small >= 0 ? tune_small : qo.mode == 0 && cg.K < 120 ? 300 : 150);
+    const bool small = tiles < (tune_small >= 0 ? tune_small : qo.mode == 0 && cg.K < 120 && !one_round ? 300 : 150);
     dim3 grid((unsigned)(((M + 63) / 64 + tpb - 1) / tpb), (unsigned)((KN + 63) / 64));
     if (small) grid = dim3((unsigned)((M + 31) / 32), (unsigned)(qo.mode != 0 ? 2 * ((KN + 63) / 64) : (KN + 31) / 32));
     if (M > 0x7fffff00LL) return hipErrorInvalidValue;   // pixel indices stay below 2^31

@@ -11,6 +11,8 @@ pytestmark = pytest.mark.gpu
 # 126: 150; then 264 MiB results of rows that are whole sectors and that are not, the last with one pixel past a tile
 LAYERS = [(1, 64, t, 64, 64, 3) for t in (299, 300, 519, 520, 1023, 1024)] + [(1, 320, t, 64, 64, 3) for t in (299, 300, 799, 800, 1499, 1500)] + \
          [(1, 896, t, 64, 64, 3) for t in (149, 150)] + [(2, 64, 256, 256, 530, 1), (2, 64, 255, 255, 535, 1), (2, 64, 1, 65537, 530, 1)]
+# 72 words: between 190 and 256 tiles on tiles of 64 x 64, outside and where the last one would be half empty on 32 x 32
+LAYERS += [(1, 512, t, 64, 64, 3) for t in (189, 190, 256, 257)] + [(1, 512, 64, 95, 90, 3)]
 # few pixels and many kernels, on both sides of the 256 pixels from which they run as im2row + GEMM
 LAYERS += [(1, 512, 16, 16, 16384, 3), (1, 512, 1, 257, 11000, 3)]
 
