@@ -568,13 +568,13 @@ static int area_of_slot(int slot) {
 
 // ---- weights of tnns_conv, kept in engine form across calls ----
 // The reference's layer functions read the packed weights where they lie; here they must reach the device and, for
-// the matrix-core engine, be re-arranged into fragments: an upload, a launch and their latencies on every call for
+// the matrix-core engine, be brought into engine form: an upload, a launch and their latencies on every call for
 // data that a network never changes.  tnns_conv therefore keeps the prepared weights of the layers it has seen,
 // found again by byte count, layer shape and a 128-bit hash of the CONTENTS, recomputed on every call: rows that are
 // rewritten in place, or another layer's rows packed into memory that malloc hands out again, give another hash and
 // a fresh upload; the same rows packed again at another address are found.  The host address is not part of the
 // identity.  The hash must cost less than the upload it saves: it runs on AES rounds where the CPU has them (limited
-// by memory bandwidth: 35 GB/s on one thread of the GPU box's host against 15 GB/s for multiply-rotate lanes) and rows
+// by memory bandwidth: 35 GB/s on one thread of an MI355X host against 15 GB/s for multiply-rotate lanes) and rows
 // of 1 MiB and more are hashed in slices on the copy threads (64 MiB in 0.36 ms, against 1.6 ms for their upload).
 // Entries are dropped least recently used first beyond 512 entries or the byte cap (1 GiB of device memory;
 // FTNN_HOST_WEIGHT_CACHE_MB = n sets it, FTNN_HOST_NO_WEIGHT_CACHE = 1 or a cap of 0 switches the cache off; a layer
@@ -771,16 +771,16 @@ bool conv_f4_gemm_route(int64_t M, int KN, int K) {
     return !off && M > 256 && M < 512 && tiles >= 256 && (double)M * KN * 64.0 * K >= 1.2e10;
 }
 
-// its buffers: channel-packed planes, Packing-2 rows, the rows as matrix-core fragments (each 256-byte aligned)
+// its buffers: channel-packed planes, Packing-2 rows, the rows as record blocks (each 256-byte aligned)
 static int64_t gemm_route_plane_bytes(int N, int C, int H, int W) {
     return (ftnn_pack_scratch_bytes(N, C, H, W, 1) + 255) / 256 * 256;
 }
 static int64_t gemm_route_row_bytes(int64_t M, int Kw) { return (M * Kw * 16 + 255) / 256 * 256; }
 
-// Fully connected layers (1 x 1 kernels on one pixel per image) run as a product of packed rows (k_rows): the fragments of
-// the fp4 layer kernels take twice the bytes, and a layer over few images does little but read its weights; over many images
+// Fully connected layers (1 x 1 kernels on one pixel per image) run as a product of packed rows (k_rows): a layer over
+// few images does little but read its weights, and these lie in the order the product reads them; over many images
 // the layer kernels scatter their results, a column of them per image.  Whole call, weights prepared and read from beyond the
-// L2, fragments / rows on MI355X: 8 images of 16384 -> 16384 31.5 / 15.4 us (64 MiB of weights: 5.4 TB/s beside the quantiser's
+// L2, layer kernel (at four bits per lane) / rows on MI355X: 8 images of 16384 -> 16384 31.5 / 15.4 us (64 MiB of weights: 5.4 TB/s beside the quantiser's
 // launch), 64 57.9 / 21.9, 8 of 4096 -> 4096 8.0 / 6.1, 8 of 512 -> 1000 5.6 / 5.0, 1024 of 4096 -> 4096 120 / 23, 4096 of
 // 1000 -> 16000 1854 / 145: ahead from 1 to 4096 images on every size tried.  Up to 64 channels the rows, four words at least,
 // would be larger than the layer's operand region, and a row is mostly padding: those stay with the layer kernels.
@@ -812,8 +812,8 @@ static int select_conv_engine(int type, int N, int C, int H, int W, int KN, int 
 }
 
 // Weights in the form the layer's engine reads them, made once per layer instead of once per call.  keep_rows: for layers that
-// may be fully connected, the packed rows behind the fragments (ftnn_conv_prepare_weights does not know the image size; the
-// 1 x 1 layers on larger images leave them unread).  tmp_off: where what lies behind the fragments starts.
+// may be fully connected, the packed rows behind the records (ftnn_conv_prepare_weights does not know the image size; the
+// 1 x 1 layers on larger images leave them unread).  tmp_off: where what lies behind the records' region starts.
 static int64_t prepared_bytes(int type, int C, int KN, int KH, int KW, bool keep_rows, int64_t* tmp_off) {
     const bool wt = (type == kTNN || type == kBTN);
     const int engine = select_conv_engine(type, 1, C, KH, KW, KN, KH, KW, 1, 1);
@@ -825,7 +825,7 @@ static int64_t prepared_bytes(int type, int C, int KN, int KH, int KW, bool keep
         if (tmp_off) *tmp_off = frag;
         // the dense path expands the re-packed rows, which need a place of their own
         if (dense_f4_applies(C, KH, KW)) return frag + (int64_t)KN * round4(Kd) * (wt ? 16 : 8);
-        // the packed rows as they are, behind the fragments: operand of conv_fc_rows
+        // the packed rows as they are, behind the records: operand of conv_fc_rows
         return frag + (keep_rows && fc_weights(C, KH, KW) ? (int64_t)KN * round4(cpack_of(C)) * (wt ? 16 : 8) : 0);
     }
     return (int64_t)KN * (dense ? round4(Kd) : round4(cpack_of(C) * KH * KW)) * (wt ? 16 : 8);
@@ -986,7 +986,7 @@ int conv_valu(int type, const float* d_x, const float* d_thr, const int64_t* d_q
 // ---- the scratch memory of ftnn_conv_static ----
 // Device memory that exists from the moment the code object is loaded until the process ends, one copy per GPU,
 // so that a caller who may not allocate (a stream under graph capture, a serving loop, a harness that forbids
-// hipMalloc) still has somewhere to put a layer's quantised input and weight fragments.  `scratch` is the
+// hipMalloc) still has somewhere to put a layer's quantised input and weights in engine form.  `scratch` is the
 // host-side handle of that array, not a device address: the address of each GPU's copy comes from
 // hipGetSymbolAddress, once per device, and is what every launch below is given.
 constexpr int64_t kStaticScratchBytes = FTNN_STATIC_SCRATCH_BYTES;
@@ -1073,7 +1073,7 @@ int64_t ftnn_conv_scratch_bytes(int type, int N, int C, int H, int W, int KN, in
         bytes += (int64_t)KN * round4(Kd) * (wt ? 16 : 8);
     }
     // enough for either engine, so that one buffer serves ftnn_conv and ftnn_conv_engine
-    // fp4: operand region, fragments of the weights and, on the dense path, the re-packed weight rows
+    // fp4: operand region, weights in engine form and, on the dense path, the re-packed weight rows
     int64_t f4 = conv_f4_operand_bytes(N, C, H, W, KH, KW, OH, OW, KN, W_stride) +
                  (mfma_fragment_bytes(true, KN, conv_f4_weight_words(C, KH, KW)) + 255) / 256 * 256;
     if (dense_f4_applies(C, KH, KW)) f4 += (int64_t)KN * conv_f4_weight_words(C, KH, KW) * (wt ? 16 : 8);

@@ -53,7 +53,7 @@ inline XcdOrder make_xcd_order(uint64_t outer, uint32_t inner, bool plain) {   /
 // values apart: past the caches (non-temporal) where those are whole sectors of 64 bytes, and where the result is small;
 // through the caches a launch ends with their write-back.  Large results of other rows go through the caches, which put the parts
 // of a sector together; past them each part is a read and a write of memory.  Whole calls, us, past / through the caches: TNN
-// 4096 x 4096 x 4096 44 / 52, x 4112 columns 65 / 72, x 4111 92 / 71; 6016 x 6016 x 512 58 / 72, 6001 x 6001 124 / 72; operands kept,
+// 4096 x 4096 x 4096 44 / 52, x 4112 columns 65 / 72, x 4111 92 / 68; 6016 x 6016 x 512 58 / 72, 6001 x 6001 124 / 60; operands kept,
 // 30000 x 150 x 512 (17 MiB) 14.1 / 10.2.
 inline __host__ __device__ bool stores_past_caches(int row, int64_t M, int KN) { return row % 16 == 0 || M * KN <= (4 << 20); }
 

@@ -360,7 +360,7 @@ __global__ __launch_bounds__(256) void k_mfma(const uint4* __restrict__ Pf, cons
 }
 
 // ------------------------------------------------- fp4 operands at two bits per lane, offset codes
-// The fp4 GEMM above is bound by power, not by its schedule.  The same instruction stream runs a quarter faster on
+// The fp4 GEMM is bound by power, not by its schedule.  The same instruction stream runs a quarter faster on
 // operands that are all zero, and a chain of nothing but these MFMAs on registers holds 2.39 GHz on zeros, 2.25 GHz on
 // lanes of {0, 0.5, 1} and 1.97 GHz on lanes of {-1, 0, +1}: it is the mixed signs in the adder trees and the operand
 // bytes on the move (L2 -> LDS -> registers) that hold the clock down.  The GEMM's own operand form answers both:
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256) void k_mfma(const uint4* __restrict__ Pf, cons
 //
 // Layout ("packed4"): 1 KiB blocks [row block of 32][pair of K words][lane l = (k half l / 32, row l % 32)][16 bytes], the
 // 16 bytes of a lane being (P0, P1) of the even K word and (P0, P1) of the odd one, P0 = D0 | D1 << 2, P1 = D2 | D3 << 2
-// with D0..D3 the lane's 16 bytes of the plain fragment layout above in offset codes.  One LDS-direct load of 16 bytes
+// with D0 .. D3 the 32 lanes of the lane's k half as nibbles in offset codes, eight to a dword.  One LDS-direct load of 16 bytes
 // per lane moves a row block's two K words.  Behind the blocks: one int32 per row (rows rounded up to 32), sum of the
 // row's lanes.
 
@@ -389,7 +389,7 @@ __global__ void k_zero_i32(int* __restrict__ p, int n, int* __restrict__ q, int 
     else if (i - n < m) q[i - n] = 0;
 }
 
-// grid (row blocks, groups / 4), block 256: as k_expand<true, TERN>, writing the packed4 layout (Kw words per row) and
+// grid (row blocks, groups / 4), block 256: as k_expand, writing the packed4 layout (Kw words per row) and
 // adding the lanes of its rows into sums (zeroed before the launch)
 template <bool TERN>
 __device__ __forceinline__ void pack4_block(const uint32_t* __restrict__ P, int rows, int G, uint2* __restrict__ out,
@@ -659,8 +659,10 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
 // 16-byte read per lane, split into the nibbles of two multiplies (lanes of both words of a pair enter both, see P2).  The
 // schedule is k_mfma_p4's: the first word's multiplies run while the second one's operands are split; then, behind the barrier, the
 // second word's multiplies run beside the LDS reads of the next pair, each block split LAG slots
-// after its read.  These tiles are bound by what they move through the LDS: at four bits per lane a step of two K words
-// moved 72 KiB for 512 cycles of matrix pipe (256 x 128 tile) and took 1080 cycles.
+// after its read.  At four bits per lane a step of two K words moved 72 KiB through the LDS for 512 cycles of matrix pipe (256 x 128
+// tile) and took 1080 cycles, bound by that; at two it moves 36 KiB.  What bounds it now is one wavefront per SIMD: counters of
+// 8 x 1024 x 56 x 56 -> 1024, 3 x 3 stride 2 (76400 cycles per wavefront, 72 steps, matrix pipe busy for 48 %): per step 16 multiplies, 110 other
+// vector, 20 scalar, 7 LDS and 3 load instructions, about 700 cycles of issue, and 27 % of the time in waits; no bank conflict.
 //
 // IMPL: a conv layer with implicit im2row.  Qc is then the layer's quantised input in the form T2[n][C_pack][row][column % s]
 // [column / s][16 bytes] (k_quantize_f4 with TILED): lane l of a block of K words 2 i, 2 i + 1 loads the record of its pixel at
@@ -869,8 +871,8 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
 //   * a wavefront owns 64 kernels x 64 output pixels (2 x 2 MFMA blocks, 64 accumulator
 //     registers).  A workgroup is 4 wavefronts: S of them split the K loop of one tile (each takes a
 //     run of pairs of words in the reference's K order (kh*KW + kw)*C_pack + ic; words dealt out in turn cost layers
-//     0.2-0.6 us more, as every step then changes the tap), so it covers 4/S pixel tiles.  S = 1 for layers with 600 tiles or more (no exchange at all), 2 or
-//     4 where the tiles alone would leave most of the chip idle; the partial tiles then meet in
+//     0.2-0.6 us more, as every step then changes the tap), so it covers 4/S pixel tiles.  S = 1 where there are tiles enough (no exchange at all), 2 or
+//     4 where they alone would leave most of the chip idle (launch_conv_f4 has the lines); the partial tiles then meet in
 //     LDS and each wavefront finishes 4/S of the tile's four blocks;
 //   * weights are the MFMA A side (rows = accumulator registers), pixels the B side (rows =
 //     lanes), so a store instruction writes 32 consecutive pixels of one NCHW plane;
@@ -1457,11 +1459,13 @@ hipError_t launch_records_gemm(int type, const void* d_a, const void* d_b, int64
 }
 
 // Large layers with a stride and long rows go to the tile kernel with implicit im2row: the layer kernel gathers records a stride
-// apart, so it moves twice the cache lines per record and its L1 is what bounds it; T2 keeps them side by side.  8 x 1024 x 56 x 56 ->
-// 1024, 3 x 3 stride 2 (1568 tiles of 64 x 64, 144 words) under sustained load 51.7 us, 56.5 on the layer kernel.  Elsewhere the
-// layer kernel is ahead on 920 random layers: at stride 1 by 5 to 50 %, at stride 2 with short rows (1216 tiles, 72
-// words 36 / 32 us) or fewer tiles (848, 325 words 83 / 78).  FTNN_CONV_TILES_FROM = n: tuning aid; it sets the tile count and drops the
-// other conditions.
+// apart, so it moves twice the cache lines per record and its L1 is what bounds it; T2 keeps them side by side.  90 random layers of
+// 900 to 6000 tiles of 64 x 64 and 60 to 400 words with strides of 2 to 4, both kernels under sustained load in turn, quantiser included: from
+// 1500 tiles and 100 words on the tile kernel takes 0.93 of the layer kernel's time in the mean (0.78 to 1.11, ahead on 34 of 38; us, tiles /
+// layer kernel: 2032 tiles x 243 words 109 / 119, 2760 x 153 at stride 4 126 / 161, 2688 x 125 at stride 3 91 / 104, 3056 x 225 109 / 119; 3488 x 126
+// 95 / 86), with shorter rows 1.06 (2496 x 63 56 / 42, 4875 x 72 80 / 70), with fewer tiles 1.02 (1104 x 144 54 / 47, 1056 x 92 487 / 486, 1088 x 369
+// at stride 3 118 / 127).  At stride 1 the layer kernel is ahead by 5 to 50 %.  FTNN_CONV_TILES_FROM = n: tuning aid; it sets the tile
+// count and drops the other conditions.
 namespace {
 // the tile kernel's limits: a tap mask of 32 bits per pixel, a table entry per K word, 32-bit record indices into T2,
 // its tiles of 128 pixels in y of a launch, which takes 65535, and its way of keeping kw - pad non-negative

@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256) void k_quantize_pixels(const float* __restrict
 // wavefronts with PX = 32, a thread making half a dword out of 8 channels.
 // TILED: the operand of the tile kernel with implicit im2row instead (k_mfma_s2, IMPL): the columns of an image row sorted by
 // column % stride_w, T2[n][C_pack][row][column % s][column / s][16 bytes] with ceil(W / s) slots per class: the 32 lanes of a
-// fragment half -- consecutive output pixels, i.e. input columns s apart -- then read consecutive records within an output
+// record block -- consecutive output pixels, i.e. input columns s apart -- then read consecutive records within an output
 // row, whatever the stride.
 template <bool TERN, bool TILED, int PX>
 __global__ __launch_bounds__(256) void k_quantize_f4(const float* __restrict__ x,

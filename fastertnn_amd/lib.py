@@ -3,8 +3,8 @@
 Device-memory entry points take torch CUDA tensors (used only as device buffers)
 and run on torch's current stream.  Host-memory entry points are the reference's
 own (`tnns_conv`, `tnns_gemm`, `t2r_p2_opt`, `b2r`, `mm_*`): they take numpy
-arrays, and the heap buffer each one returns is copied into numpy and freed, as a
-C caller would free it.
+arrays, and the heap buffer each one returns is the result's memory: freed with the
+last array over it, as a C caller would free it.
 """
 import ctypes as C
 import os

@@ -281,7 +281,7 @@ FTNN_API int ftnn_conv_engine(int engine, int type, const float *d_x, const floa
 /*
  * Weights prepared once per layer (no counterpart in the reference, whose packed rows are final):
  * ftnn_conv_prepare_weights turns the packed rows of ftnn_pack_weights / the reference's
- * quantized_kernel_packing2 into the form the layer's engine reads -- matrix-core fragments (for 1 x 1
+ * quantized_kernel_packing2 into the form the layer's engine reads -- records of two bits per lane (for 1 x 1
  * kernels with more than 64 channels the packed rows behind them, which a fully connected layer reads), or
  * the dense re-packing of a few-channel layer -- so that ftnn_conv_prepared does not repeat that
  * work on every call.  d_prepared: ftnn_conv_weights_bytes() bytes, 16-byte aligned; its layout belongs to the
