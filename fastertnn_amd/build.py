@@ -1,7 +1,9 @@
-"""Build libftnn_hip.so in-tree with hipcc for gfx950 (cross-compiles without a GPU)."""
+"""Build libftnn_hip.so in-tree with hipcc for gfx950 (cross-compiles without a GPU), and the Python module over it."""
+import importlib.machinery
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -42,8 +44,24 @@ def check_no_scratch(src, remarks):
                                        "no resource remarks found for %s" % missing))
 
 
+BINDING = os.path.join(HERE, "_call" + importlib.machinery.EXTENSION_SUFFIXES[0])
+
+
+def binding_command():
+    """the compiler call that makes _call from csrc/py_call.cpp (host code only)"""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    inc = [sysconfig.get_paths()["include"], os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           os.path.join(rocm, "include")]
+    return ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+             "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI] + ["-isystem" + d for d in inc] +
+            [os.path.join(CSRC, "py_call.cpp"), "-o", BINDING, "-L" + HERE, "-lftnn_hip", "-Wl,-rpath,$ORIGIN", "-L" + os.path.join(root, "lib"),
+             "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"])
+
+
 def build_library(verbose=False):
-    """Compile every HIP source and link the shared library; returns its path."""
+    """Compile every HIP source and link the shared library, then the Python module; returns the library's path."""
     objs = []
     procs = []
     for src in SOURCES:
@@ -70,6 +88,7 @@ def build_library(verbose=False):
             print(out)
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", LIB]
     subprocess.run(cmd, check=True)
+    subprocess.run(binding_command(), check=True)
     return LIB
 
 

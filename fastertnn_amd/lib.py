@@ -1,4 +1,5 @@
-"""ctypes binding of libftnn_hip.so (the C ABI declared in include/ftnn.h).
+"""Python binding of libftnn_hip.so (the C ABI declared in include/ftnn.h): ctypes, and for the calls made once per layer or
+product csrc/py_call.cpp.
 
 Device-memory entry points take torch CUDA tensors (used only as device buffers)
 and run on torch's current stream.  Host-memory entry points are the reference's
@@ -119,14 +120,25 @@ def pack_scratch_bytes(n, c, h, w, ternary):
 
 # A call queues 2.5 us of launch work per kernel; what the binding adds must stay below that.  torch is imported once, on
 # the first device call (importing it inside every wrapper costs 0.3 us), and the stream is asked for as the bare handle
-# (0.1 us; the Stream object of torch.cuda.current_stream() costs 2.7).
+# (0.1 us; the Stream object of torch.cuda.current_stream() costs 2.7).  The calls that a program makes once per layer or
+# product go through `_call` (csrc/py_call.cpp), which takes plain arguments and answers None to anything else; what follows
+# in their wrappers is then the way through ctypes.
 torch = None
+_call = None
 
 
 def _torch():
     global torch
     import torch
     return torch
+
+
+def _native():
+    global _call
+    _torch()
+    if _call is None:
+        from . import _call   # links against torch, which has to be loaded first
+    return _call
 
 
 def _stream():
@@ -177,6 +189,11 @@ def quantize_im2row(x, thr, kh, kw, pad, stride, ternary, out=None, scratch=None
 
 def mm(typ, a, b, n, oh, ow, kn, k, alpha, k_unpack=0, out=None):
     """mm_tnn / mm_tbn / mm_btn / mm_bnn on device tensors; returns fp32 (n, kn, oh, ow)."""
+    rc = (_call or _native()).mm(typ, a, b, n, oh, ow, kn, k, alpha, k_unpack, out)
+    if rc == 0:
+        return out
+    if rc is not None:
+        _check(rc)
     if out is None:
         out = _empty((n, kn, oh, ow), "float32", a.device)
     _check(_L.ftnn_mm(typ, _dev(a), _dev(b), n, oh, ow, kn, k, k_unpack, alpha, _f32(out),
@@ -202,6 +219,11 @@ def mm_scratch_bytes(engine, typ, n, oh, ow, kn, k):
 
 def mm_engine(engine, typ, a, b, n, oh, ow, kn, k, alpha, k_unpack=0, out=None, scratch=None):
     """ftnn_mm_engine: the GEMM on an explicit engine (or AUTO); scratch is allocated if not given."""
+    rc = (_call or _native()).mm_engine(engine, typ, a, b, n, oh, ow, kn, k, alpha, k_unpack, out, scratch)
+    if rc == 0:
+        return out
+    if rc is not None:
+        _check(rc)
     if out is None:
         out = _empty((n, kn, oh, ow), "float32", a.device)
     if scratch is None:
@@ -225,6 +247,11 @@ def expand_rows(engine, rows_t, n_rows, k, ternary, out=None):
 
 def mm_expanded(engine, typ, a_exp, b_exp, n, oh, ow, kn, k, alpha, k_unpack=0, out=None):
     """ftnn_mm_expanded: the matrix-core GEMM on two expanded operands."""
+    rc = (_call or _native()).mm_expanded(engine, typ, a_exp, b_exp, n, oh, ow, kn, k, alpha, k_unpack, out)
+    if rc == 0:
+        return out
+    if rc is not None:
+        _check(rc)
     if out is None:
         out = _empty((n, kn, oh, ow), "float32", a_exp.device)
     _check(_L.ftnn_mm_expanded(engine, typ, _dev(a_exp), _dev(b_exp), n, oh, ow, kn, k, k_unpack, alpha,
@@ -238,6 +265,12 @@ def select_conv_engine(typ, n, c, h, w, kn, kh, kw, pad, stride):
 
 def conv(typ, x, thr, qw, kn, kh, kw, pad, stride, alpha, scratch=None, out=None, engine=ENGINE_AUTO):
     """One conv layer (tnn_conv_p2 & co.) on device tensors; engine: AUTO, VALU or MFMA_F4."""
+    if engine == ENGINE_AUTO:
+        rc = (_call or _native()).conv(typ, x, thr, qw, kn, kh, kw, pad, stride, alpha, scratch, out)
+        if rc == 0:
+            return out
+        if rc is not None:
+            _check(rc)
     n, c, h, w = x.shape
     if scratch is None:
         scratch = _empty(conv_scratch_bytes(typ, n, c, h, w, kn, kh, kw, pad, stride), "uint8", x.device)
@@ -254,6 +287,11 @@ STATIC_SCRATCH_BYTES = int(_L.ftnn_static_scratch_bytes())   # FTNN_STATIC_SCRAT
 
 def conv_static(typ, x, thr, qw, kn, kh, kw, pad, stride, alpha, out):
     """ftnn_conv_static: the layer on the library's own fixed work space; allocates nothing (out is required)."""
+    rc = (_call or _native()).conv_static(typ, x, thr, qw, kn, kh, kw, pad, stride, alpha, out)
+    if rc == 0:
+        return out
+    if rc is not None:
+        _check(rc)
     n, c, h, w = x.shape
     _check(_L.ftnn_conv_static(typ, _f32(x), _f32(thr), _dev(qw), n, c, h, w, kn, kh,
                                kw, pad, pad, stride, stride, alpha, _f32(out), _stream()))
@@ -269,6 +307,11 @@ def prepare_conv_weights(typ, qw, c, kn, kh, kw):
 
 def conv_prepared(typ, x, thr, prepared, kn, kh, kw, pad, stride, alpha, scratch=None, out=None):
     """ftnn_conv_prepared: one conv layer with weights from prepare_conv_weights."""
+    rc = (_call or _native()).conv_prepared(typ, x, thr, prepared, kn, kh, kw, pad, stride, alpha, scratch, out)
+    if rc == 0:
+        return out
+    if rc is not None:
+        _check(rc)
     n, c, h, w = x.shape
     if scratch is None:
         scratch = _empty(conv_scratch_bytes(typ, n, c, h, w, kn, kh, kw, pad, stride), "uint8", x.device)
@@ -337,6 +380,11 @@ class Net:
         assert int(_L.ftnn_net_output_elems(self._h)) == int(np.prod(self.out_shape))
 
     def run(self, x, out=None, graph=False):
+        rc = (_call or _native()).net_run(self._h, x, out, int(graph))
+        if rc == 0:
+            return out
+        if rc is not None:
+            _check(rc)
         if out is None:
             out = _empty(self.out_shape, "float32", x.device)
         _check(_L.ftnn_net_run(self._h, _f32(x), _f32(out), int(graph), _stream()))
