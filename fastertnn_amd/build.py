@@ -8,8 +8,8 @@ import sysconfig
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libftnn_hip.so")
-SOURCES = ["ftnn_api.hip", "pack_kernels.hip", "mm_kernels.hip", "mfma_kernels.hip", "rows_kernels.hip", "stem_kernels.hip", "ftnn_net.hip",
-           "host_hash.cpp"]   # the last one is plain host C++
+SOURCES = ["ftnn_api.hip", "pack_kernels.hip", "mm_kernels.hip", "mfma_kernels.hip", "rows_kernels.hip", "stem_kernels.hip",
+           "direct_kernels.hip", "ftnn_net.hip", "host_hash.cpp"]   # the last one is plain host C++
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -22,7 +22,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hi
 # use ordinary loads that the compiler counts; scratch there would only be slow, and is refused as a performance guard.
 # Source -> name fragments.
 NO_SCRATCH = {"mfma_kernels.hip": ("k_conv_f4", "k_mfma"),   # "k_mfma" covers k_mfma_p4 as well
-              "rows_kernels.hip": ("k_rows",)}
+              "rows_kernels.hip": ("k_rows",), "direct_kernels.hip": ("k_direct_f4",)}
 
 
 def check_no_scratch(src, remarks):

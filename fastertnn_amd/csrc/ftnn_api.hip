@@ -915,6 +915,10 @@ int conv_f4_expanded(int type, const float* d_x, const float* d_thr, const void*
         return e == hipSuccess ? FTNN_OK : hip_fail(e, "fp4 conv launch");
     }
     const int64_t M = (int64_t)N * OH * OW;
+    const ConvGeom cg = {H, W, cpack_of(C), OH, OW, KW, cpack_of(C) * KH * KW, H_pad, W_pad, H_stride, W_stride,
+                         make_fastdiv((uint32_t)OW), make_fastdiv((uint32_t)cpack_of(C)), make_fastdiv((uint32_t)KW)};
+    if (d_x && qo.mode == 0 && launch_direct_f4(type, d_x, d_thr, d_wf, cg, C, N, KN, C * KH * KW, prelu_alpha, d_y, st, &e))
+        return e == hipSuccess ? FTNN_OK : hip_fail(e, "fp4 small-layer launch");
     const bool tiles = d_x && qo.mode == 0 && conv_f4_tile_route(M, KN, cpack_of(C), KH * KW, quantize_f4_tiled_bytes(N, C, H, W, W_stride), W_pad, W_stride);
     if (d_x && qo.mode == 0 && !tiles && conv_f4_gemm_route(M, KN, cpack_of(C) * KH * KW)) {
         const int Kw = conv_f4_weight_words(C, KH, KW);
@@ -929,8 +933,6 @@ int conv_f4_expanded(int type, const float* d_x, const float* d_thr, const void*
         e = launch_records_gemm(type, d_af, d_wf, M, OH * OW, KN, Kw, C * KH * KW, prelu_alpha, d_y, st);
         return e == hipSuccess ? FTNN_OK : hip_fail(e, "matrix-core GEMM launch");
     }
-    const ConvGeom cg = {H, W, cpack_of(C), OH, OW, KW, cpack_of(C) * KH * KW, H_pad, W_pad, H_stride, W_stride,
-                         make_fastdiv((uint32_t)OW), make_fastdiv((uint32_t)cpack_of(C)), make_fastdiv((uint32_t)KW)};
     // many tiles, fp32 input and result: workgroup tiles staged through LDS, gathered from the quantised input in the
     // tile kernel's own layout
     if (tiles) {
@@ -1344,6 +1346,10 @@ int ftnn_conv_prepared(int type, const float* d_x, const float* d_thr, const voi
             (int64_t)N * OH * OW * conv_f4_weight_words(C, KH, KW) > 0x7fffffffLL)
             return fail(FTNN_EINVAL, "more than 2^31-1 input pixel words");
         if (fc_from_rows(C, H, W, KH, KW, H_pad, W_pad)) {
+            const ConvGeom cg = {1, 1, cpack_of(C), 1, 1, 1, cpack_of(C), 0, 0, 1, 1, make_fastdiv(1u), make_fastdiv((uint32_t)cpack_of(C)), make_fastdiv(1u)};
+            hipError_t e;
+            if (launch_direct_f4(type, d_x, d_thr, d_prepared, cg, C, N, KN, C, prelu_alpha, d_y, (hipStream_t)stream, &e))
+                return e == hipSuccess ? FTNN_OK : hip_fail(e, "fp4 small-layer launch");
             int64_t rows_off;
             prepared_bytes(type, C, KN, KH, KW, true, &rows_off);
             const char* rows = static_cast<const char*>(d_prepared) + rows_off;

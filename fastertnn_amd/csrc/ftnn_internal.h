@@ -279,6 +279,12 @@ bool conv_f4_tile_route(int64_t M, int KN, int CP, int taps, int64_t t2_bytes, i
 hipError_t launch_conv_f4_tiles(int type, const void* d_t2, const void* d_wf, const ConvGeom& cg, int N, int KN,
                                 int K_unpack, float alpha, float* d_y, hipStream_t st);
 
+// ---- direct_kernels.hip ----
+// A small layer from its fp32 input in one launch, no scratch; d_wf: its weights as record blocks.  False where the layer is none of
+// those it is meant for: nothing has been done then.
+bool launch_direct_f4(int type, const float* d_x, const float* d_thr, const void* d_wf, const ConvGeom& cg, int C, int N, int KN,
+                      int K_unpack, float alpha, float* d_y, hipStream_t st, hipError_t* err);
+
 // ---- ftnn_api.hip ----  (arguments already validated)
 // The fp4 layer with weights expanded beforehand (d_wf: launch_expand_records of the packed rows).
 // d_x != null: the input is quantised into d_p2 (N*H*W*C_pack*16 bytes) first; d_x == null: d_p2 already
