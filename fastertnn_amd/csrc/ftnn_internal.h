@@ -264,6 +264,11 @@ bool mm_rows_within_limits(int64_t M, int KN, int Kw);
 hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
                           float alpha, float* d_y, hipStream_t st);
 
+// The same for operands in packed4 form (launch_mfma_pack4) with their rows' sums.  False where workgroup tiles through LDS are ahead:
+// nothing has been done then.
+bool launch_mm_packed(int type, const void* d_ac, const void* d_bc, const int* sA, const int* sB, int64_t M, int OHW, int KN, int Kw,
+                      int K_unpack, float alpha, float* d_y, hipStream_t st, hipError_t* err);
+
 // conv layer on the fp4 matrix cores: activations from launch_quantize_f4, weights as the record blocks
 // launch_expand_records makes of the packed weight rows (Kw = round4(cg.K) words per row)
 hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const ConvGeom& cg, int N, int KN,

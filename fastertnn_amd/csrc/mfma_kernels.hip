@@ -1392,6 +1392,12 @@ hipError_t launch_mfma_gemm_packed4(int type, const void* d_ac, const void* d_bc
     const int bias = type == kBNN ? 64 * Kw - K_unpack : 0;   // as launch_mfma_gemm
     const int off = 64 * Kw + bias;                           // the lanes of a row pair, padding included
     const int form = type == kTNN ? 0 : 1;
+    // below 160 tiles of 256 x 256, and for products narrower than half of such a tile, the wavefronts of a workgroup split K, but for short
+    // rows with many results
+    hipError_t e;
+    if (((M + 255) / 256 * ((KN + 255) / 256) < mfma_small_tile_below() || KN < 128 || M < 128) &&
+        launch_mm_packed(type, d_ac, d_bc, sA, sB, M, OHW, KN, Kw, K_unpack, alpha, d_y, st, &e))
+        return e;
     return OHW > 1 ? launch_gemm_p4<true>(Bc, Ac, d_y, (int)M, KN, OHW, Kw / 2, sB, sA, off, form, alpha, st)
                    : launch_gemm_p4<false>(Ac, Bc, d_y, (int)M, KN, OHW, Kw / 2, sA, sB, off, form, alpha, st);
 }

@@ -130,6 +130,79 @@ struct RowsOut {
     float bias, lim, alpha;   // r = sum - bias; PReLU scales r < lim by alpha
 };
 
+// Blocks that meet in LDS at a time
+constexpr int meeting_blocks(int nm, int ks) { return nm * ks * 4 > 144 ? nm / 2 : nm; }
+
+// The end of a product whose wavefronts split K: the partial tiles meet in LDS and the result is stored.
+// Accumulator e of block (a, b): P row 32 (prb0 + a) + 8 (e / 4) + 4 h + e % 4, Q row 32 (qrb0 + b) + lr.  Four of them
+// (a quad) are one 16-byte piece per lane in LDS; wavefront ks sums the quads ks, ks + KS, ... over all wavefronts.
+// PReLU in the reference's two forms, "f <= 0 -> f *= alpha" (mm_p2_final_tnn_avx2.c:204-208) and "r >= 0 ? r : alpha * r"
+// (mm_p2_final_tbn_avx2.c:73): results are integers below 2^24, so both are one compare, against 0.5 or 0.
+// result(sum, P row, Q row) is what is stored.
+template <int WTP, int WTQ, int KS, typename F>
+__device__ __forceinline__ void meet_and_store(v16f (&acc)[WTP][WTQ], float4* lds, const RowsOut& ro, int prb0, int qrb0, int prow, int qrow,
+                                               int ks, int lane, F&& result) {
+    constexpr int NM = WTP * WTQ, R = meeting_blocks(NM, KS), QUADS = R * 4 < KS ? 1 : R * 4 / KS;
+    static_assert(KS % 4 == 0 && (R * 4 < KS || R * 4 % KS == 0) && NM % R == 0, "whole quads per wavefront");
+    const int lr = lane & 31, h = lane >> 5;
+    const size_t stride = ro.p_stride;
+    const bool inside = (prb0 + WTP) * 32 <= prow && (qrb0 + WTQ) * 32 <= qrow;   // uniform
+    auto put4 = [&](const float4& t, int p0, int b, auto whole) {   // P rows p0 + 4 h .. + 3 (p0 uniform) of Q block b
+        const uint32_t q = (uint32_t)((qrb0 + b) * 32 + lr), img = fastdiv(q, ro.img);
+        float* const d = ro.y + (size_t)p0 * stride;
+        const size_t lo = (size_t)img * (size_t)ro.img_stride + (q - img * ro.img.d) + (size_t)(4 * h) * stride;
+        if constexpr (decltype(whole)::value) {
+            const int p = p0 + 4 * h;
+            __builtin_nontemporal_store(result(t.x, p, (int)q), d + lo);
+            __builtin_nontemporal_store(result(t.y, p + 1, (int)q), d + stride + lo);
+            __builtin_nontemporal_store(result(t.z, p + 2, (int)q), d + 2 * stride + lo);
+            __builtin_nontemporal_store(result(t.w, p + 3, (int)q), d + 3 * stride + lo);
+        } else if (q < (uint32_t)qrow) {
+            const int p = p0 + 4 * h;
+            if (p < prow) __builtin_nontemporal_store(result(t.x, p, (int)q), d + lo);
+            if (p + 1 < prow) __builtin_nontemporal_store(result(t.y, p + 1, (int)q), d + stride + lo);
+            if (p + 2 < prow) __builtin_nontemporal_store(result(t.z, p + 2, (int)q), d + 2 * stride + lo);
+            if (p + 3 < prow) __builtin_nontemporal_store(result(t.w, p + 3, (int)q), d + 3 * stride + lo);
+        }
+    };
+#pragma unroll
+    for (int r0 = 0; r0 < NM; r0 += R) {
+        __syncthreads();   // every wavefront is done with its ring, or with the round before
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+            const v16f& c = acc[(r0 + j) / WTQ][(r0 + j) % WTQ];
+#pragma unroll
+            for (int e4 = 0; e4 < 4; e4++)
+                lds[((ks * R + j) * 4 + e4) * 64 + lane] = make_float4(c[4 * e4], c[4 * e4 + 1], c[4 * e4 + 2], c[4 * e4 + 3]);
+        }
+        __syncthreads();
+        if (R * 4 < KS && ks >= R * 4) continue;   // no quad of its own (and no further round)
+        float4 t[QUADS];   // all sums before the first store: the branch around the stores would hold the reads back
+#pragma unroll
+        for (int i = 0; i < QUADS; i++) {
+            const int quad = i * KS + ks;
+            t[i] = lds[quad * 64 + lane];
+#pragma unroll
+            for (int v = 1; v < KS; v++) {
+                const float4 u = lds[(v * R * 4 + quad) * 64 + lane];
+                t[i].x += u.x;
+                t[i].y += u.y;
+                t[i].z += u.z;
+                t[i].w += u.w;
+            }
+        }
+        auto put_all = [&](auto whole) {
+#pragma unroll
+            for (int i = 0; i < QUADS; i++) {
+                const int blk = r0 + i * (KS / 4) + (KS == 4 ? 0 : ks >> 2), sub = KS == 4 ? ks : ks & 3;   // of quad i KS + ks
+                put4(t[i], (prb0 + blk / WTQ) * 32 + 8 * sub, blk % WTQ, whole);
+            }
+        };
+        if (inside) put_all(std::true_type{});
+        else put_all(std::false_type{});
+    }
+}
+
 // A wavefront's tile is WTP x WTQ blocks of 32 x 32, a workgroup's the same tile: its KS wavefronts split K.
 template <bool TP, bool TQ, int WTP, int WTQ, int KS>
 struct RowsTile {
@@ -137,7 +210,7 @@ struct RowsTile {
     static constexpr int NM = WTP * WTQ, NB = WTP + WTQ;
     static constexpr int LP = TP ? 2 : 1, LQ = TQ ? 2 : 1;   // KiB (and loads) per row block and group
     static constexpr int LPG = WTP * LP + WTQ * LQ;          // per wavefront and group
-    static constexpr int R = NM * KS * 4 > 144 ? NM / 2 : NM;   // blocks that meet in LDS at a time
+    static constexpr int R = meeting_blocks(NM, KS);
     static constexpr size_t ring = (size_t)KS * NS * LPG * 1024, red = (size_t)R * KS * 4096;
     static constexpr size_t lds = ring > red ? ring : red;
     static_assert(lds <= (160u << 10), "LDS of a compute unit");
@@ -295,70 +368,92 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in the LDS that the partial tiles take now
 
-    // Accumulator e of block (a, b): P row 32 (prb0 + a) + 8 (e / 4) + 4 h + e % 4, Q row 32 (qrb0 + b) + lr.  Four of them
-    // (a quad) are one 16-byte piece per lane in LDS; wavefront ks sums the quads ks, ks + KS, ... over all wavefronts.
-    // PReLU in the reference's two forms, "f <= 0 -> f *= alpha" (mm_p2_final_tnn_avx2.c:204-208) and "r >= 0 ? r : alpha * r"
-    // (mm_p2_final_tbn_avx2.c:73): results are integers below 2^24, so both are one compare, against 0.5 or 0.
-    auto result = [&](float v) {
+    auto result = [&](float v, int, int) {
         const float r = v - ro.bias;
         return r < ro.lim ? r * ro.alpha : r;
     };
-    const size_t stride = ro.p_stride;
-    const bool inside = (prb0 + WTP) * 32 <= prow && (qrb0 + WTQ) * 32 <= qrow;   // uniform
-    auto put4 = [&](const float4& t, int p0, int b, auto whole) {   // P rows p0 + 4 h .. + 3 (p0 uniform) of Q block b
-        const uint32_t q = (uint32_t)((qrb0 + b) * 32 + lr), img = fastdiv(q, ro.img);
-        float* const d = ro.y + (size_t)p0 * stride;
-        const size_t lo = (size_t)img * (size_t)ro.img_stride + (q - img * ro.img.d) + (size_t)(4 * h) * stride;
-        if constexpr (decltype(whole)::value) {
-            __builtin_nontemporal_store(result(t.x), d + lo);
-            __builtin_nontemporal_store(result(t.y), d + stride + lo);
-            __builtin_nontemporal_store(result(t.z), d + 2 * stride + lo);
-            __builtin_nontemporal_store(result(t.w), d + 3 * stride + lo);
-        } else if (q < (uint32_t)qrow) {
-            const int p = p0 + 4 * h;
-            if (p < prow) __builtin_nontemporal_store(result(t.x), d + lo);
-            if (p + 1 < prow) __builtin_nontemporal_store(result(t.y), d + stride + lo);
-            if (p + 2 < prow) __builtin_nontemporal_store(result(t.z), d + 2 * stride + lo);
-            if (p + 3 < prow) __builtin_nontemporal_store(result(t.w), d + 3 * stride + lo);
-        }
+    meet_and_store<WTP, WTQ, KS>(acc, lds, ro, prb0, qrb0, prow, qrow, ks, lane, result);
+}
+
+// The same product of operands kept in packed4 form (mfma_kernels.hip: 1 KiB blocks of 32 rows x two K words, lane l's 16 bytes
+// the words' nibbles at two bits per lane in offset codes; sP, sQ: the rows' sums).
+//
+// A block is one contiguous load of a wavefront and a word's operand six vector instructions beside WTP x WTQ multiplies, so the
+// wavefronts read registers straight from memory: a ring of NB sets of blocks, each asked for NB - 1 pairs of words ahead (ordinary
+// loads, counted by the compiler, held in place by scheduling fences).  While one word's operands are multiplied the next one's are
+// unpacked, between the multiplies.
+template <int WTP, int WTQ, int KS, int NB>
+__global__ __launch_bounds__(64 * KS) void k_packed(const uint4* __restrict__ Pc, const uint4* __restrict__ Qc, int prow, int qrow, int KP,
+                                                    const int* __restrict__ sP, const int* __restrict__ sQ, int off, RowsOrder od, RowsOut ro) {
+    extern __shared__ float4 lds[];
+    constexpr int NM = WTP * WTQ, NO = WTP + WTQ;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int tx, ty;
+    if (!od.tile(blockIdx.x, &tx, &ty)) return;   // past the last tile (the whole workgroup)
+    const int prb0 = tx * WTP, qrb0 = ty * WTQ;
+    const int prbmax = (prow + 31) / 32 - 1, qrbmax = (qrow + 31) / 32 - 1;
+    // row blocks past the operand are clamped (their results are never stored)
+    const uint4* src[NO];   // uniform
+#pragma unroll
+    for (int f = 0; f < NO; f++)
+        src[f] = f < WTP ? Pc + (size_t)min(prb0 + f, prbmax) * KP * 64 : Qc + (size_t)min(qrb0 + (f - WTP), qrbmax) * KP * 64;
+    v4u raw[NB][NO];
+    v4u e[2][NO];   // a word's operands: P blocks, then Q blocks
+    auto load = [&](int set, int pair) {   // (past the end: the last pair, not used)
+        const size_t at = (size_t)min(pair, KP - 1) * 64;
+#pragma unroll
+        for (int f = 0; f < NO; f++) raw[set][f] = *reinterpret_cast<const v4u*>(src[f] + at + lane);
     };
-    constexpr int R = TL::R, QUADS = R * 4 / KS;
-    static_assert(R * 4 % KS == 0 && NM % R == 0, "whole quads per wavefront");
+    auto unpack = [&](int set, int word, int f) {
+        constexpr uint32_t m = 0x33333333u;
+        const uint32_t a = raw[set][f][2 * word], b = raw[set][f][2 * word + 1];
+        e[word][f] = v4u{a & m, (a >> 2) & m, b & m, (b >> 2) & m};
+    };
+    v16f acc[WTP][WTQ];
+    // word `word` of the pair in the operand set multiplied, and word `nword` of the pair in set `nset` unpacked
+    auto step = [&](auto word, int nset) {
+        constexpr int W = decltype(word)::value;
+        static_for<NM>([&](auto mtag) {
+            constexpr int m = decltype(mtag)::value;
+            mfma_f4(acc[m / WTQ][m % WTQ], e[W][m / WTQ], e[W][WTP + m % WTQ]);
+            static_for<(m + 1) * NO / NM - m * NO / NM>([&](auto ktag) { unpack(nset, 1 - W, m * NO / NM + decltype(ktag)::value); });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    const int n = (KP - ks + KS - 1) / KS;   // pairs ks, ks + KS, ... of this wavefront (0 or less: none)
 #pragma unroll
-    for (int r0 = 0; r0 < NM; r0 += R) {
-        __syncthreads();   // every wavefront is done with its ring, or with the round before
+    for (int a = 0; a < WTP; a++)
 #pragma unroll
-        for (int j = 0; j < R; j++) {
-            const v16f& c = acc[(r0 + j) / WTQ][(r0 + j) % WTQ];
+        for (int b = 0; b < WTQ; b++)
 #pragma unroll
-            for (int e4 = 0; e4 < 4; e4++)
-                lds[((ks * R + j) * 4 + e4) * 64 + lane] = make_float4(c[4 * e4], c[4 * e4 + 1], c[4 * e4 + 2], c[4 * e4 + 3]);
+            for (int i = 0; i < 16; i++) acc[a][b][i] = 0.0f;
+    if (n > 0) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) load(j, ks + j * KS);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int f = 0; f < NO; f++) unpack(0, 0, f);
+        int pair = ks + NB * KS;   // the next one to ask for
+        for (int i = 0; i < n; i += NB) {
+            static_for<NB>([&](auto jtag) {
+                constexpr int j = decltype(jtag)::value;
+                if (j == 0 || i + j < n) {
+                    step(std::integral_constant<int, 0>{}, j);
+                    load(j, pair);
+                    pair += KS;
+                    __builtin_amdgcn_sched_barrier(0);
+                    step(std::integral_constant<int, 1>{}, (j + 1) % NB);
+                }
+            });
         }
-        __syncthreads();
-        float4 t[QUADS];   // all sums before the first store: the branch around the stores would hold the reads back
-#pragma unroll
-        for (int i = 0; i < QUADS; i++) {
-            const int quad = i * KS + ks;
-            t[i] = lds[quad * 64 + lane];
-#pragma unroll
-            for (int v = 1; v < KS; v++) {
-                const float4 u = lds[(v * R * 4 + quad) * 64 + lane];
-                t[i].x += u.x;
-                t[i].y += u.y;
-                t[i].z += u.z;
-                t[i].w += u.w;
-            }
-        }
-        auto put_all = [&](auto whole) {
-#pragma unroll
-            for (int i = 0; i < QUADS; i++) {
-                const int quad = i * KS + ks, blk = r0 + (quad >> 2);
-                put4(t[i], (prb0 + blk / WTQ) * 32 + 8 * (quad & 3), blk % WTQ, whole);
-            }
-        };
-        if (inside) put_all(std::true_type{});
-        else put_all(std::false_type{});
     }
+    // dot = 4 sum - sum of the P row - sum of the Q row - lanes (off: with BNN's constant), all of it below 2^24
+    auto result = [&](float v, int p, int q) {
+        const float r = (float)((int)(v * 4.0f) - sP[p] - sQ[q] - off);
+        return r < ro.lim ? r * ro.alpha : r;
+    };
+    meet_and_store<WTP, WTQ, KS>(acc, lds, ro, prb0, qrb0, prow, qrow, ks, lane, result);
 }
 
 // A grid dimension holds fewer than 2^32 threads: tiles, rounded up to whole eighths, times the 256 of a workgroup.  It also
@@ -423,6 +518,28 @@ hipError_t launch_rows_types(const char* P, const char* Q, int64_t prow, int64_t
     }
 }
 
+
+template <int WTP, int WTQ, int KS, int NB>
+hipError_t launch_packed_tile(const uint4* P, const uint4* Q, int64_t prow, int64_t qrow, int KP, const int* sP, const int* sQ, int off,
+                              const RowsOut& ro, hipStream_t st) {
+    constexpr int lds_bytes = meeting_blocks(WTP * WTQ, KS) * KS * 4096;
+    static_assert(lds_bytes <= (160 << 10), "LDS of a compute unit");
+    static const hipError_t configured =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_packed<WTP, WTQ, KS, NB>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (configured != hipSuccess) return configured;
+    const int64_t px = (prow + 32 * WTP - 1) / (32 * WTP), qy = (qrow + 32 * WTQ - 1) / (32 * WTQ);
+    if (px * qy > kMaxRowsTiles) return hipErrorInvalidValue;
+    RowsOrder od;
+    od.tiles = (uint32_t)(px * qy);
+    od.per_xcd = (od.tiles + 7) / 8;
+    od.px = (uint32_t)px;
+    od.band = make_fastdiv((uint32_t)(4 * qy));
+    od.last = make_fastdiv((uint32_t)(px % 4 ? px % 4 : 4));
+    hipLaunchKernelGGL((k_packed<WTP, WTQ, KS, NB>), dim3(8 * od.per_xcd), dim3(64 * KS), lds_bytes, st, P, Q, (int)prow, (int)qrow, KP, sP, sQ,
+                       off, od, ro);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 bool mm_rows_within_limits(int64_t M, int KN, int Kw) {
@@ -450,6 +567,70 @@ hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int6
     if (tp) return launch_rows_types<true, false>(P, Q, prow, qrow, Kw, ro, st);
     if (tq) return launch_rows_types<false, true>(P, Q, prow, qrow, Kw, ro, st);
     return launch_rows_types<false, false>(P, Q, prow, qrow, Kw, ro, st);
+}
+
+namespace {
+// Tiles of 32 x 32 to 128 x 128 by estimate, or none: workgroup tiles of 128 x 128 through LDS (k_mfma_p4) are ahead then.  Estimates (us) of
+// n rounds of 256 workgroups, w pairs of words per wavefront and r million results, fits to 240 products from 32 x 32 x 256 to 8192 x 8192 x
+// 32768 with every form measured: the choice is 1.2 % from the best form in the mean (1.22 at worst) and takes 0.47 of the time of
+// k_mfma_p4, which these all ran on (1.02 at worst).  k_mfma_p4 / here, us: 256 x 256 x 4096 11.5 / 4.7, 36 x 246 x 15616 30.5 / 6.8,
+// 182 x 1444 x 26624 48.6 / 12.5, 1024 x 1024 x 8192 20.3 / 7.8, 2048 x 2048 x 16384 37.0 / 27.6, 1999 x 1733 x 14592 34.9 / 31.2; the other way
+// 917 x 3773 x 768 10.0 / 10.4.  Tiles of 32 x 32 and 64 x 64 are bound by the L1 (46 bytes per cycle and compute unit), 128 x 128 by the
+// matrix pipe (1040 cycles per pair of words for 1024 of multiplies).
+struct PackedForm {
+    int p, q, ks;                 // blocks of 32 per side, wavefronts
+    double a, b, c, d, e;         // a + b (n - 1) + w (c + d (n - 1)) + e r
+};
+constexpr PackedForm kPackedForms[] = {
+    {1, 1, 4, 3.9, 0.11, 0.088, 0.080, 1.41}, {1, 1, 8, 4.25, 0.30, 0.143, 0.172, 2.46}, {1, 2, 4, 4.5, 0.0, 0.126, 0.120, 1.25},
+    {2, 1, 4, 4.7, 0.21, 0.126, 0.110, 0.99}, {2, 2, 4, 6.05, 0.85, 0.168, 0.188, 0.76}, {3, 3, 4, 9.65, 3.4, 0.315, 0.350, 1.06},
+    {4, 4, 4, 13.7, 7.0, 0.494, 0.536, 0.76}, {4, 4, 1, 6.25, 0.0, 0.208, 0.139, 0.67} /* k_mfma_p4 */};
+int packed_form_of(int64_t prow, int64_t qrow, int KP) {
+    int best = -1;
+    double least = 1e30;
+    for (int i = 0; i < (int)(sizeof kPackedForms / sizeof *kPackedForms); i++) {
+        const PackedForm& f = kPackedForms[i];
+        const int64_t tiles = ((prow + 32 * f.p - 1) / (32 * f.p)) * ((qrow + 32 * f.q - 1) / (32 * f.q));
+        if (f.ks != 1 && tiles > kMaxRowsTiles) continue;
+        const double n1 = (double)((tiles + 255) / 256 - 1), w = (double)KP / f.ks;
+        const double t = f.a + f.b * n1 + w * (f.c + f.d * n1) + f.e * 1e-6 * (double)prow * (double)qrow;
+        if (t < least) least = t, best = i;
+    }
+    return best;
+}
+
+}  // namespace
+
+bool launch_mm_packed(int type, const void* d_ac, const void* d_bc, const int* sA, const int* sB, int64_t M, int OHW, int KN, int Kw,
+                      int K_unpack, float alpha, float* d_y, hipStream_t st, hipError_t* err) {
+    const bool nchw = OHW > 1;
+    RowsOut ro;
+    ro.y = d_y;
+    ro.img_stride = (int64_t)KN * OHW;
+    ro.p_stride = (uint32_t)(nchw ? OHW : KN);
+    ro.img = make_fastdiv(nchw ? (uint32_t)OHW : 0xffffffffu);
+    ro.bias = 0.0f;
+    ro.lim = type == kTNN ? 0.5f : 0.0f;
+    ro.alpha = alpha;
+    const int off = 64 * Kw + (type == kBNN ? 64 * Kw - K_unpack : 0);   // the lanes of a row pair, padding included, and BNN's constant
+    const uint4 *P = static_cast<const uint4*>(nchw ? d_bc : d_ac), *Q = static_cast<const uint4*>(nchw ? d_ac : d_bc);
+    const int *sP = nchw ? sB : sA, *sQ = nchw ? sA : sB;
+    const int64_t prow = nchw ? KN : M, qrow = nchw ? M : KN;
+    const int KP = Kw / 2;
+    auto go = [&](hipError_t e) {
+        *err = e;
+        return true;
+    };
+    switch (packed_form_of(prow, qrow, KP)) {
+        case 0: return go(launch_packed_tile<1, 1, 4, 8>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
+        case 1: return go(launch_packed_tile<1, 1, 8, 8>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
+        case 2: return go(launch_packed_tile<1, 2, 4, 6>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
+        case 3: return go(launch_packed_tile<2, 1, 4, 6>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
+        case 4: return go(launch_packed_tile<2, 2, 4, 6>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
+        case 5: return go(launch_packed_tile<3, 3, 4, 4>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
+        case 6: return go(launch_packed_tile<4, 4, 4, 3>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
+        default: return false;
+    }
 }
 
 }  // namespace ftnn
