@@ -7,7 +7,8 @@
 // tile of 4 x 4 blocks of 32 x 32 spends 6 issue slots per multiply of 8 slots.
 //
 //   * The wavefronts of a workgroup work on ONE output tile and split K: wavefront w takes the groups of four words
-//     w, w + KS, ...  Nothing is shared in the K loop, so it has no barrier; the partial tiles meet in LDS at the end.
+//     w, w + KS, ...  Nothing is shared in the K loop, so it has no barrier; the partial tiles meet in LDS at the end.  Where rows are
+//     short and results many, that end is most of the time: four wavefronts work on tiles of their own then, on all of K.
 //   * A group travels global -> LDS by LDS-direct loads into a ring of the wavefront's own, four lanes on the 64 contiguous
 //     bytes of a ternary row (two on the 32 of a binary one), and from there to registers in the operand's order.
 //     Loaded straight into that order, 64 lanes touch 64 pieces of cache lines per instruction and the L1 delivers
@@ -21,8 +22,8 @@
 // cycles of matrix pipe (the LDS-direct loads and LDS reads of a group add 14 cycles each to a slot's multiply), at the
 // clock that sustained multiplies of mixed signs allow (1.9 GHz on all compute units).  Device time of a whole call from
 // packed rows, before (expansion launch + k_mfma, or the vector ALU) and now: 256 x 256 x 4096 4.8 -> 3.6 us,
-// 512 x 512 x 4096 10.2 -> 3.8, 1024 x 1024 x 8192 17.8 -> 7.8, 1500 x 1500 x 12032 32.6 -> 18.1, 2048 x 2048 x 16384 44.1 ->
-// 31.5, 8 x 16384 x 16384 57.8 -> 12.3.
+// 512 x 512 x 4096 10.2 -> 3.8, 1024 x 1024 x 8192 17.8 -> 7.6, 1500 x 1500 x 12032 32.6 -> 17.5, 2048 x 2048 x 16384 44.1 ->
+// 31, 8 x 16384 x 16384 57.8 -> 12.3.
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -128,43 +129,50 @@ struct RowsOut {
     uint32_t p_stride;
     FastDiv img;
     float bias, lim, alpha;   // r = sum - bias; PReLU scales r < lim by alpha
+    bool past_caches;         // (host) how results leave, by stores_past_caches; the kernels' NT
 };
 
 // Blocks that meet in LDS at a time
 constexpr int meeting_blocks(int nm, int ks) { return nm * ks * 4 > 144 ? nm / 2 : nm; }
 
-// The end of a product whose wavefronts split K: the partial tiles meet in LDS and the result is stored.
-// Accumulator e of block (a, b): P row 32 (prb0 + a) + 8 (e / 4) + 4 h + e % 4, Q row 32 (qrb0 + b) + lr.  Four of them
-// (a quad) are one 16-byte piece per lane in LDS; wavefront ks sums the quads ks, ks + KS, ... over all wavefronts.
+// Where a product's results go.  Accumulator e of block (a, b): P row 32 (prb0 + a) + 8 (e / 4) + 4 h + e % 4, Q row 32 (qrb0 + b) + lr; four
+// of them are a quad.  result(quad of sums, P row, Q row) is what is stored, for a P row within the operand.
 // PReLU in the reference's two forms, "f <= 0 -> f *= alpha" (mm_p2_final_tnn_avx2.c:204-208) and "r >= 0 ? r : alpha * r"
 // (mm_p2_final_tbn_avx2.c:73): results are integers below 2^24, so both are one compare, against 0.5 or 0.
-// result(sum, P row, Q row) is what is stored.
-template <int WTP, int WTQ, int KS, typename F>
+template <bool WHOLE, bool NT, typename F>
+__device__ __forceinline__ void put_quad(const float4& sum, int p0, int qrb, const RowsOut& ro, int prow, int qrow, int lane, F&& result) {
+    const int lr = lane & 31, h = lane >> 5;   // P rows p0 + 4 h .. + 3 (p0 uniform) of Q block qrb
+    const size_t stride = ro.p_stride;
+    const uint32_t q = (uint32_t)(qrb * 32 + lr), img = fastdiv(q, ro.img);
+    float* const d = ro.y + (size_t)p0 * stride;
+    const size_t lo = (size_t)img * (size_t)ro.img_stride + (q - img * ro.img.d) + (size_t)(4 * h) * stride;
+    auto put = [](float v, float* at) {
+        if constexpr (NT) __builtin_nontemporal_store(v, at);
+        else *at = v;
+    };
+    const int p = p0 + 4 * h;
+    if (WHOLE || (q < (uint32_t)qrow && p < prow)) {
+        const float4 t = result(sum, p, (int)q);
+        put(t.x, d + lo);
+        if (WHOLE || p + 1 < prow) put(t.y, d + stride + lo);
+        if (WHOLE || p + 2 < prow) put(t.z, d + 2 * stride + lo);
+        if (WHOLE || p + 3 < prow) put(t.w, d + 3 * stride + lo);
+    }
+}
+// fn(whether all of a tile of P blocks prb0 .. and Q blocks qrb0 .. lies inside) (uniform)
+template <int WTP, int WTQ, typename F>
+__device__ __forceinline__ void by_wholeness(int prb0, int qrb0, int prow, int qrow, F&& fn) {
+    if ((prb0 + WTP) * 32 <= prow && (qrb0 + WTQ) * 32 <= qrow) fn(std::true_type{});
+    else fn(std::false_type{});
+}
+
+// The end of a product whose wavefronts split K: the partial tiles meet in LDS, wavefront ks sums the quads ks, ks + KS, ... over all
+// wavefronts and stores them.
+template <int WTP, int WTQ, int KS, bool NT, typename F>
 __device__ __forceinline__ void meet_and_store(v16f (&acc)[WTP][WTQ], float4* lds, const RowsOut& ro, int prb0, int qrb0, int prow, int qrow,
                                                int ks, int lane, F&& result) {
     constexpr int NM = WTP * WTQ, R = meeting_blocks(NM, KS), QUADS = R * 4 < KS ? 1 : R * 4 / KS;
     static_assert(KS % 4 == 0 && (R * 4 < KS || R * 4 % KS == 0) && NM % R == 0, "whole quads per wavefront");
-    const int lr = lane & 31, h = lane >> 5;
-    const size_t stride = ro.p_stride;
-    const bool inside = (prb0 + WTP) * 32 <= prow && (qrb0 + WTQ) * 32 <= qrow;   // uniform
-    auto put4 = [&](const float4& t, int p0, int b, auto whole) {   // P rows p0 + 4 h .. + 3 (p0 uniform) of Q block b
-        const uint32_t q = (uint32_t)((qrb0 + b) * 32 + lr), img = fastdiv(q, ro.img);
-        float* const d = ro.y + (size_t)p0 * stride;
-        const size_t lo = (size_t)img * (size_t)ro.img_stride + (q - img * ro.img.d) + (size_t)(4 * h) * stride;
-        if constexpr (decltype(whole)::value) {
-            const int p = p0 + 4 * h;
-            __builtin_nontemporal_store(result(t.x, p, (int)q), d + lo);
-            __builtin_nontemporal_store(result(t.y, p + 1, (int)q), d + stride + lo);
-            __builtin_nontemporal_store(result(t.z, p + 2, (int)q), d + 2 * stride + lo);
-            __builtin_nontemporal_store(result(t.w, p + 3, (int)q), d + 3 * stride + lo);
-        } else if (q < (uint32_t)qrow) {
-            const int p = p0 + 4 * h;
-            if (p < prow) __builtin_nontemporal_store(result(t.x, p, (int)q), d + lo);
-            if (p + 1 < prow) __builtin_nontemporal_store(result(t.y, p + 1, (int)q), d + stride + lo);
-            if (p + 2 < prow) __builtin_nontemporal_store(result(t.z, p + 2, (int)q), d + 2 * stride + lo);
-            if (p + 3 < prow) __builtin_nontemporal_store(result(t.w, p + 3, (int)q), d + 3 * stride + lo);
-        }
-    };
 #pragma unroll
     for (int r0 = 0; r0 < NM; r0 += R) {
         __syncthreads();   // every wavefront is done with its ring, or with the round before
@@ -191,42 +199,60 @@ __device__ __forceinline__ void meet_and_store(v16f (&acc)[WTP][WTQ], float4* ld
                 t[i].w += u.w;
             }
         }
-        auto put_all = [&](auto whole) {
+        by_wholeness<WTP, WTQ>(prb0, qrb0, prow, qrow, [&](auto whole) {
 #pragma unroll
             for (int i = 0; i < QUADS; i++) {
                 const int blk = r0 + i * (KS / 4) + (KS == 4 ? 0 : ks >> 2), sub = KS == 4 ? ks : ks & 3;   // of quad i KS + ks
-                put4(t[i], (prb0 + blk / WTQ) * 32 + 8 * sub, blk % WTQ, whole);
+                put_quad<decltype(whole)::value, NT>(t[i], (prb0 + blk / WTQ) * 32 + 8 * sub, qrb0 + blk % WTQ, ro, prow, qrow, lane, result);
             }
-        };
-        if (inside) put_all(std::true_type{});
-        else put_all(std::false_type{});
+        });
     }
 }
 
-// A wavefront's tile is WTP x WTQ blocks of 32 x 32, a workgroup's the same tile: its KS wavefronts split K.
+// the same for a wavefront with whole sums
+template <int WTP, int WTQ, bool NT, typename F>
+__device__ __forceinline__ void store_whole_sums(v16f (&acc)[WTP][WTQ], const RowsOut& ro, int prb0, int qrb0, int prow, int qrow, int lane, F&& result) {
+    by_wholeness<WTP, WTQ>(prb0, qrb0, prow, qrow, [&](auto whole) {
+#pragma unroll
+        for (int blk = 0; blk < WTP * WTQ; blk++) {
+            const v16f& c = acc[blk / WTQ][blk % WTQ];
+#pragma unroll
+            for (int e4 = 0; e4 < 4; e4++)
+                put_quad<decltype(whole)::value, NT>(make_float4(c[4 * e4], c[4 * e4 + 1], c[4 * e4 + 2], c[4 * e4 + 3]),
+                                                 (prb0 + blk / WTQ) * 32 + 8 * e4, qrb0 + blk % WTQ, ro, prow, qrow, lane, result);
+        }
+    });
+}
+
+// A wavefront's tile is WTP x WTQ blocks of 32 x 32, a workgroup's the same tile: its KS wavefronts split K.  KS = 1: four wavefronts, 2 x 2
+// of these tiles, each on all of K.
 template <bool TP, bool TQ, int WTP, int WTQ, int KS>
 struct RowsTile {
+    static constexpr int WV = KS == 1 ? 2 : 1, NW = KS == 1 ? 4 : KS;   // tiles per side of a workgroup, wavefronts
     static constexpr int NS = 2;                             // ring slots: deeper rings (where they fit) measured no faster
     static constexpr int NM = WTP * WTQ, NB = WTP + WTQ;
     static constexpr int LP = TP ? 2 : 1, LQ = TQ ? 2 : 1;   // KiB (and loads) per row block and group
     static constexpr int LPG = WTP * LP + WTQ * LQ;          // per wavefront and group
     static constexpr int R = meeting_blocks(NM, KS);
-    static constexpr size_t ring = (size_t)KS * NS * LPG * 1024, red = (size_t)R * KS * 4096;
+    static constexpr size_t ring = (size_t)NW * NS * LPG * 1024, red = KS == 1 ? 0 : (size_t)R * KS * 4096;
     static constexpr size_t lds = ring > red ? ring : red;
     static_assert(lds <= (160u << 10), "LDS of a compute unit");
 };
 
-template <bool TP, bool TQ, int WTP, int WTQ, int KS>
-__global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, const char* __restrict__ Q, int prow, int qrow, int G,
+template <bool TP, bool TQ, int WTP, int WTQ, int KS, bool NT>
+__global__ __launch_bounds__(64 * (KS == 1 ? 4 : KS)) void k_rows(const char* __restrict__ P, const char* __restrict__ Q, int prow, int qrow, int G,
                                                   RowsOrder od, RowsOut ro) {
     extern __shared__ float4 lds[];
     typedef RowsTile<TP, TQ, WTP, WTQ, KS> TL;
     constexpr int NM = TL::NM, NB = TL::NB, NS = TL::NS, LP = TL::LP, LQ = TL::LQ, LPG = TL::LPG;
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, h = lane >> 5;
-    const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int WV = TL::WV;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ks = KS == 1 ? 0 : wave;
     int tx, ty;
     if (!od.tile(blockIdx.x, &tx, &ty)) return;   // past the last tile (the whole workgroup)
-    const int prb0 = tx * WTP, qrb0 = ty * WTQ;   // first row blocks: within the operands
+    // first row blocks: within the operands
+    const int prb0 = (tx * WV + (KS == 1 ? wave >> 1 : 0)) * WTP, qrb0 = (ty * WV + (KS == 1 ? wave & 1 : 0)) * WTQ;
+    if (KS == 1 && (prb0 * 32 >= prow || qrb0 * 32 >= qrow)) return;   // no such tile (these wavefronts never wait for each other)
     constexpr uint32_t GP = TP ? 64u : 32u, GQ = TQ ? 64u : 32u;   // bytes of a group of 4 words
     const uint32_t rbp = (uint32_t)G * GP, rbq = (uint32_t)G * GQ;  // bytes of a row
 
@@ -257,7 +283,7 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
         return (uint32_t)(tern ? lr * 64 + (piece ^ ((lr >> 2) & 3)) * 16 : lr * 32 + (piece ^ ((lr >> 3) & 1)) * 16);
     };
     const uint32_t rd_ts = piece_at(true, h), rd_tz = piece_at(true, 2 + h), rd_b = piece_at(false, h);
-    const uint32_t ring0 = (uint32_t)ks * (NS * LPG * 1024);
+    const uint32_t ring0 = (uint32_t)wave * (NS * LPG * 1024);
     const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
     const char* const ring = reinterpret_cast<const char*>(lds) + ring0;
 
@@ -368,11 +394,15 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in the LDS that the partial tiles take now
 
-    auto result = [&](float v, int, int) {
-        const float r = v - ro.bias;
-        return r < ro.lim ? r * ro.alpha : r;
+    auto result = [&](const float4& t, int, int) {
+        auto prelu = [&](float v) {
+            const float r = v - ro.bias;
+            return r < ro.lim ? r * ro.alpha : r;
+        };
+        return make_float4(prelu(t.x), prelu(t.y), prelu(t.z), prelu(t.w));
     };
-    meet_and_store<WTP, WTQ, KS>(acc, lds, ro, prb0, qrb0, prow, qrow, ks, lane, result);
+    if constexpr (KS == 1) store_whole_sums<WTP, WTQ, NT>(acc, ro, prb0, qrb0, prow, qrow, lane, result);
+    else meet_and_store<WTP, WTQ, KS, NT>(acc, lds, ro, prb0, qrb0, prow, qrow, ks, lane, result);
 }
 
 // The same product of operands kept in packed4 form (mfma_kernels.hip: 1 KiB blocks of 32 rows x two K words, lane l's 16 bytes
@@ -382,16 +412,18 @@ __global__ __launch_bounds__(64 * KS) void k_rows(const char* __restrict__ P, co
 // wavefronts read registers straight from memory: a ring of NB sets of blocks, each asked for NB - 1 pairs of words ahead (ordinary
 // loads, counted by the compiler, held in place by scheduling fences).  While one word's operands are multiplied the next one's are
 // unpacked, between the multiplies.
-template <int WTP, int WTQ, int KS, int NB>
-__global__ __launch_bounds__(64 * KS) void k_packed(const uint4* __restrict__ Pc, const uint4* __restrict__ Qc, int prow, int qrow, int KP,
+template <int WTP, int WTQ, int KS, int NB, bool NT>
+__global__ __launch_bounds__(64 * (KS == 1 ? 4 : KS)) void k_packed(const uint4* __restrict__ Pc, const uint4* __restrict__ Qc, int prow, int qrow, int KP,
                                                     const int* __restrict__ sP, const int* __restrict__ sQ, int off, RowsOrder od, RowsOut ro) {
     extern __shared__ float4 lds[];
     constexpr int NM = WTP * WTQ, NO = WTP + WTQ;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int WV = KS == 1 ? 2 : 1;   // as k_rows
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ks = KS == 1 ? 0 : wave;
     int tx, ty;
     if (!od.tile(blockIdx.x, &tx, &ty)) return;   // past the last tile (the whole workgroup)
-    const int prb0 = tx * WTP, qrb0 = ty * WTQ;
+    const int prb0 = (tx * WV + (KS == 1 ? wave >> 1 : 0)) * WTP, qrb0 = (ty * WV + (KS == 1 ? wave & 1 : 0)) * WTQ;
+    if (KS == 1 && (prb0 * 32 >= prow || qrb0 * 32 >= qrow)) return;
     const int prbmax = (prow + 31) / 32 - 1, qrbmax = (qrow + 31) / 32 - 1;
     // row blocks past the operand are clamped (their results are never stored)
     const uint4* src[NO];   // uniform
@@ -448,12 +480,19 @@ __global__ __launch_bounds__(64 * KS) void k_packed(const uint4* __restrict__ Pc
             });
         }
     }
-    // dot = 4 sum - sum of the P row - sum of the Q row - lanes (off: with BNN's constant), all of it below 2^24
-    auto result = [&](float v, int p, int q) {
-        const float r = (float)((int)(v * 4.0f) - sP[p] - sQ[q] - off);
-        return r < ro.lim ? r * ro.alpha : r;
+    // dot = 4 sum - sum of the P row - sum of the Q row - lanes (off: with BNN's constant), all of it below 2^24; the sums are there for
+    // whole blocks of rows
+    auto result = [&](const float4& t, int p, int q) {
+        const int4 s = *reinterpret_cast<const int4*>(sP + p);
+        const int o = sQ[q] + off;
+        auto prelu = [&](float v, int sp) {
+            const float r = (float)((int)(v * 4.0f) - sp - o);
+            return r < ro.lim ? r * ro.alpha : r;
+        };
+        return make_float4(prelu(t.x, s.x), prelu(t.y, s.y), prelu(t.z, s.z), prelu(t.w, s.w));
     };
-    meet_and_store<WTP, WTQ, KS>(acc, lds, ro, prb0, qrb0, prow, qrow, ks, lane, result);
+    if constexpr (KS == 1) store_whole_sums<WTP, WTQ, NT>(acc, ro, prb0, qrb0, prow, qrow, lane, result);
+    else meet_and_store<WTP, WTQ, KS, NT>(acc, lds, ro, prb0, qrb0, prow, qrow, ks, lane, result);
 }
 
 // A grid dimension holds fewer than 2^32 threads: tiles, rounded up to whole eighths, times the 256 of a workgroup.  It also
@@ -461,15 +500,14 @@ __global__ __launch_bounds__(64 * KS) void k_packed(const uint4* __restrict__ Pc
 constexpr int64_t kMaxRowsTiles = (1 << 24) - 8;
 int64_t rows_tiles(int64_t prow, int64_t qrow, int edge) { return ((prow + edge - 1) / edge) * ((qrow + edge - 1) / edge); }
 
-template <bool TP, bool TQ, int WT>
-hipError_t launch_rows_tile(const char* P, const char* Q, int64_t prow, int64_t qrow, int G, const RowsOut& ro, hipStream_t st) {
-    constexpr int KS = 4;   // 8 wavefronts measured no faster on any tile
+template <bool TP, bool TQ, int WT, int KS, bool NT>
+hipError_t launch_rows_kernel(const char* P, const char* Q, int64_t prow, int64_t qrow, int G, const RowsOut& ro, hipStream_t st) {
     typedef RowsTile<TP, TQ, WT, WT, KS> TL;
-    auto kern = k_rows<TP, TQ, WT, WT, KS>;
+    auto kern = k_rows<TP, TQ, WT, WT, KS, NT>;
     // the loads are counted by hand (s_waitcnt vmcnt(N)): a build with scratch accesses is refused; the opt-in to more than
     // 64 KiB of dynamic LDS is per kernel
     static const hipError_t configured = []() {
-        const void* k = reinterpret_cast<const void*>(&k_rows<TP, TQ, WT, WT, KS>);
+        const void* k = reinterpret_cast<const void*>(&k_rows<TP, TQ, WT, WT, KS, NT>);
         hipFuncAttributes attr;
         hipError_t e = hipFuncGetAttributes(&attr, k);
         if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
@@ -477,7 +515,8 @@ hipError_t launch_rows_tile(const char* P, const char* Q, int64_t prow, int64_t 
         return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)TL::lds);
     }();
     if (configured != hipSuccess) return configured;
-    const int64_t px = (prow + 32 * WT - 1) / (32 * WT), qy = (qrow + 32 * WT - 1) / (32 * WT);
+    constexpr int edge = 32 * WT * TL::WV;
+    const int64_t px = (prow + edge - 1) / edge, qy = (qrow + edge - 1) / edge;
     if (px * qy > kMaxRowsTiles) return hipErrorInvalidValue;
     RowsOrder od;
     od.tiles = (uint32_t)(px * qy);
@@ -485,49 +524,75 @@ hipError_t launch_rows_tile(const char* P, const char* Q, int64_t prow, int64_t 
     od.px = (uint32_t)px;
     od.band = make_fastdiv((uint32_t)(4 * qy));
     od.last = make_fastdiv((uint32_t)(px % 4 ? px % 4 : 4));
-    hipLaunchKernelGGL(kern, dim3(8 * od.per_xcd), dim3(64 * KS), TL::lds, st, P, Q, (int)prow, (int)qrow, G, od, ro);
+    hipLaunchKernelGGL(kern, dim3(8 * od.per_xcd), dim3(64 * TL::NW), TL::lds, st, P, Q, (int)prow, (int)qrow, G, od, ro);
     return hipGetLastError();
 }
-
-// Wavefront tile of a product: blocks of 32 x 32 per side.  Small tiles fill the chip with little work and pay less for the
-// meeting of the partial tiles, large ones spend fewer instructions and bytes per multiply.  The estimates (us) are
-// fits to sweeps from 32 x 32 x 256 to 4096 x 4096 x 32768 on MI355X (n rounds of 256 tiles, w words per wavefront); where
-// two tiles are within 15 % of each other either may be picked.  A tile too small for the grid counts as endless.
-int rows_tile_of(int64_t prow, int64_t qrow, int Kw) {
-    auto rounds = [&](int edge) {
-        const int64_t n = rows_tiles(prow, qrow, edge);
-        return n > kMaxRowsTiles ? 1e30 : (double)((n + 255) / 256);
-    };
-    const double w = Kw / 4.0;
-    const double n1 = rounds(32), n2 = rounds(64), n3 = rounds(96), n4 = rounds(128);
-    const double t1 = 2.65 + 0.42 * (n1 - 1) + w * (0.06 + 0.039 * (n1 - 1));
-    const double t2 = 3.55 + 1.33 * (n2 - 1) + w * (0.118 + 0.145 * (n2 - 1));
-    const double t3 = 5.0 + 4.0 * (n3 - 1) + 0.25 * n3 * w;
-    const double t4 = 8.0 + 5.5 * (n4 - 1) + 0.35 * n4 * w;
-    const double best = std::min(std::min(t1, t2), std::min(t3, t4));
-    return best == t1 ? 1 : best == t2 ? 2 : best == t3 ? 3 : 4;
+// A kernel per kind of store: deciding in the kernel costs a workgroup's end 0.1 us.  Whole calls from packed rows, us, past the caches only / by
+// stores_past_caches: TBN 22240 x 1537 x 256 79 / 25, BNN 20021 x 2017 x 256 87 / 29, 12309 x 5416 x 512 142 / 55.
+template <bool TP, bool TQ, int WT, int KS>
+hipError_t launch_rows_tile(const char* P, const char* Q, int64_t prow, int64_t qrow, int G, const RowsOut& ro, hipStream_t st) {
+    if constexpr (KS != 8)   // (256 tiles at most: small results)
+        if (!ro.past_caches) return launch_rows_kernel<TP, TQ, WT, KS, false>(P, Q, prow, qrow, G, ro, st);
+    return launch_rows_kernel<TP, TQ, WT, KS, true>(P, Q, prow, qrow, G, ro, st);
 }
+
+// How a product is cut: blocks of 32 x 32 per wavefront, and the wavefronts that split K (1: four of them on tiles of their own).  Small
+// tiles fill the chip with little work, large ones spend fewer instructions and bytes per multiply; wavefronts on tiles of their own need no
+// meeting, which is most of the time where rows are short.  The choice goes by estimates in us, a + b (n - 1) + w (c + d (n - 1)) + e r for n
+// rounds of 256 workgroups, w words (pairs of words) per wavefront and r million results.  Eight wavefronts are for tiles that leave compute
+// units idle: from a second round on four are ahead (8 x 16384 -> 16384, weights from memory, 13.9 / 14.9).
+struct ProductForm {
+    int p, q, ks;
+    double a, b, c, d, e;
+};
+constexpr int64_t kOwnTilesFrom = 650000;   // results from which wavefronts have tiles of their own; 3045 x 188 x 512 4.0 split / 4.7, 169 x 4816 x 512 5.5 / 4.4
+template <int NF>
+int form_of(const ProductForm (&forms)[NF], int64_t prow, int64_t qrow, int words) {
+    const int64_t pb = (prow + 31) / 32, qb = (qrow + 31) / 32;
+    int best = -1;
+    double least = 1e30;
+    for (int i = 0; i < NF; i++) {
+        const ProductForm& f = forms[i];
+        const int own = f.ks == 1 ? 2 : 1;   // 2 x 2 tiles per workgroup
+        const int64_t tiles = ((pb + f.p * own - 1) / (f.p * own)) * ((qb + f.q * own - 1) / (f.q * own));
+        if (tiles > kMaxRowsTiles || (f.ks == 1 && f.p == 1 && prow * qrow < kOwnTilesFrom) || (f.ks == 8 && tiles > 256)) continue;
+        const double n1 = (double)((tiles + 255) / 256 - 1), w = (double)words / f.ks;
+        const double t = f.a + f.b * n1 + w * (f.c + f.d * n1) + f.e * 1e-6 * (double)prow * (double)qrow;
+        if (t < least) least = t, best = i;
+    }
+    return best;
+}
+
+// Fits to 430 products below 160 tiles of 256 x 256, 32 x 32 x 256 to 8192 x 8192 x 32768 and all types, every form measured: the choice is 0.6 %
+// from the best form in the mean and takes 0.95 of the time of the squares on four wavefronts alone.  us, before / now: 332 x 8180 x 256
+// BTN 8.2 / 5.3, 534 x 4978 x 768 9.1 / 6.5, 2506 x 1365 x 512 BNN 9.3 / 6.5, 190 x 5514 x 26368 37.5 / 27.3, 1446 x 725 x 20736 TBN 24.8 / 21.3; the other
+// way 1020 x 398 x 27392 13.6 / 15.6, 158 x 2048 x 18688 11.8 / 13.0.
+constexpr ProductForm kRowsForms[] = {{1, 1, 4, 3.39, 0.005, 0.0578, 0.0486, 1.03}, {2, 2, 4, 4.27, 0.32, 0.1143, 0.1157, 0.94},
+                                      {3, 3, 4, 6.18, 3.07, 0.1792, 0.2319, 0.81},  {4, 4, 4, 8.61, 5.10, 0.2513, 0.3557, 0.66},
+                                      {1, 1, 1, 3.45, 0.0, 0.0616, 0.0364, 0.57},   {1, 1, 8, 3.56, 0.10, 0.0927, 0.1047, 1.51}};
 
 template <bool TP, bool TQ>
 hipError_t launch_rows_types(const char* P, const char* Q, int64_t prow, int64_t qrow, int Kw, const RowsOut& ro, hipStream_t st) {
-    switch (rows_tile_of(prow, qrow, Kw)) {
-        case 1: return launch_rows_tile<TP, TQ, 1>(P, Q, prow, qrow, Kw / 4, ro, st);
-        case 2: return launch_rows_tile<TP, TQ, 2>(P, Q, prow, qrow, Kw / 4, ro, st);
-        case 3: return launch_rows_tile<TP, TQ, 3>(P, Q, prow, qrow, Kw / 4, ro, st);
-        default: return launch_rows_tile<TP, TQ, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
+    switch (form_of(kRowsForms, prow, qrow, Kw)) {
+        case 0: return launch_rows_tile<TP, TQ, 1, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
+        case 1: return launch_rows_tile<TP, TQ, 2, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
+        case 2: return launch_rows_tile<TP, TQ, 3, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
+        case 4: return launch_rows_tile<TP, TQ, 1, 1>(P, Q, prow, qrow, Kw / 4, ro, st);
+        case 5: return launch_rows_tile<TP, TQ, 1, 8>(P, Q, prow, qrow, Kw / 4, ro, st);
+        default: return launch_rows_tile<TP, TQ, 4, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
     }
 }
 
-
-template <int WTP, int WTQ, int KS, int NB>
-hipError_t launch_packed_tile(const uint4* P, const uint4* Q, int64_t prow, int64_t qrow, int KP, const int* sP, const int* sQ, int off,
+template <int WTP, int WTQ, int KS, int NB, bool NT>
+hipError_t launch_packed_kernel(const uint4* P, const uint4* Q, int64_t prow, int64_t qrow, int KP, const int* sP, const int* sQ, int off,
                               const RowsOut& ro, hipStream_t st) {
-    constexpr int lds_bytes = meeting_blocks(WTP * WTQ, KS) * KS * 4096;
+    constexpr int WV = KS == 1 ? 2 : 1, EP = 32 * WTP * WV, EQ = 32 * WTQ * WV;
+    constexpr int lds_bytes = KS == 1 ? 0 : meeting_blocks(WTP * WTQ, KS) * KS * 4096;
     static_assert(lds_bytes <= (160 << 10), "LDS of a compute unit");
     static const hipError_t configured =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_packed<WTP, WTQ, KS, NB>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_packed<WTP, WTQ, KS, NB, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (configured != hipSuccess) return configured;
-    const int64_t px = (prow + 32 * WTP - 1) / (32 * WTP), qy = (qrow + 32 * WTQ - 1) / (32 * WTQ);
+    const int64_t px = (prow + EP - 1) / EP, qy = (qrow + EQ - 1) / EQ;
     if (px * qy > kMaxRowsTiles) return hipErrorInvalidValue;
     RowsOrder od;
     od.tiles = (uint32_t)(px * qy);
@@ -535,9 +600,16 @@ hipError_t launch_packed_tile(const uint4* P, const uint4* Q, int64_t prow, int6
     od.px = (uint32_t)px;
     od.band = make_fastdiv((uint32_t)(4 * qy));
     od.last = make_fastdiv((uint32_t)(px % 4 ? px % 4 : 4));
-    hipLaunchKernelGGL((k_packed<WTP, WTQ, KS, NB>), dim3(8 * od.per_xcd), dim3(64 * KS), lds_bytes, st, P, Q, (int)prow, (int)qrow, KP, sP, sQ,
+    hipLaunchKernelGGL((k_packed<WTP, WTQ, KS, NB, NT>), dim3(8 * od.per_xcd), dim3(64 * (KS == 1 ? 4 : KS)), lds_bytes, st, P, Q, (int)prow, (int)qrow, KP, sP, sQ,
                        off, od, ro);
     return hipGetLastError();
+}
+template <int WTP, int WTQ, int KS, int NB>
+hipError_t launch_packed_tile(const uint4* P, const uint4* Q, int64_t prow, int64_t qrow, int KP, const int* sP, const int* sQ, int off,
+                              const RowsOut& ro, hipStream_t st) {
+    if constexpr (KS != 8)
+        if (!ro.past_caches) return launch_packed_kernel<WTP, WTQ, KS, NB, false>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st);
+    return launch_packed_kernel<WTP, WTQ, KS, NB, true>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st);
 }
 
 }  // namespace
@@ -559,6 +631,7 @@ hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int6
     ro.bias = type == kBNN ? (float)(64 * Kw - K_unpack) : 0.0f;
     ro.lim = type == kTNN ? 0.5f : 0.0f;
     ro.alpha = alpha;
+    ro.past_caches = stores_past_caches(nchw ? OHW : KN, M, KN);
     const char* P = reinterpret_cast<const char*>(nchw ? d_b : d_a);
     const char* Q = reinterpret_cast<const char*>(nchw ? d_a : d_b);
     const int64_t prow = nchw ? KN : M, qrow = nchw ? M : KN;
@@ -570,34 +643,16 @@ hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int6
 }
 
 namespace {
-// Tiles of 32 x 32 to 128 x 128 by estimate, or none: workgroup tiles of 128 x 128 through LDS (k_mfma_p4) are ahead then.  Estimates (us) of
-// n rounds of 256 workgroups, w pairs of words per wavefront and r million results, fits to 240 products from 32 x 32 x 256 to 8192 x 8192 x
-// 32768 with every form measured: the choice is 1.2 % from the best form in the mean (1.22 at worst) and takes 0.47 of the time of
-// k_mfma_p4, which these all ran on (1.02 at worst).  k_mfma_p4 / here, us: 256 x 256 x 4096 11.5 / 4.7, 36 x 246 x 15616 30.5 / 6.8,
-// 182 x 1444 x 26624 48.6 / 12.5, 1024 x 1024 x 8192 20.3 / 7.8, 2048 x 2048 x 16384 37.0 / 27.6, 1999 x 1733 x 14592 34.9 / 31.2; the other way
-// 917 x 3773 x 768 10.0 / 10.4.  Tiles of 32 x 32 and 64 x 64 are bound by the L1 (46 bytes per cycle and compute unit), 128 x 128 by the
-// matrix pipe (1040 cycles per pair of words for 1024 of multiplies).
-struct PackedForm {
-    int p, q, ks;                 // blocks of 32 per side, wavefronts
-    double a, b, c, d, e;         // a + b (n - 1) + w (c + d (n - 1)) + e r
-};
-constexpr PackedForm kPackedForms[] = {
-    {1, 1, 4, 3.9, 0.11, 0.088, 0.080, 1.41}, {1, 1, 8, 4.25, 0.30, 0.143, 0.172, 2.46}, {1, 2, 4, 4.5, 0.0, 0.126, 0.120, 1.25},
-    {2, 1, 4, 4.7, 0.21, 0.126, 0.110, 0.99}, {2, 2, 4, 6.05, 0.85, 0.168, 0.188, 0.76}, {3, 3, 4, 9.65, 3.4, 0.315, 0.350, 1.06},
-    {4, 4, 4, 13.7, 7.0, 0.494, 0.536, 0.76}, {4, 4, 1, 6.25, 0.0, 0.208, 0.139, 0.67} /* k_mfma_p4 */};
-int packed_form_of(int64_t prow, int64_t qrow, int KP) {
-    int best = -1;
-    double least = 1e30;
-    for (int i = 0; i < (int)(sizeof kPackedForms / sizeof *kPackedForms); i++) {
-        const PackedForm& f = kPackedForms[i];
-        const int64_t tiles = ((prow + 32 * f.p - 1) / (32 * f.p)) * ((qrow + 32 * f.q - 1) / (32 * f.q));
-        if (f.ks != 1 && tiles > kMaxRowsTiles) continue;
-        const double n1 = (double)((tiles + 255) / 256 - 1), w = (double)KP / f.ks;
-        const double t = f.a + f.b * n1 + w * (f.c + f.d * n1) + f.e * 1e-6 * (double)prow * (double)qrow;
-        if (t < least) least = t, best = i;
-    }
-    return best;
-}
+// Operands kept: the forms above, or none: workgroup tiles of 128 x 128 through LDS (k_mfma_p4, the last estimate) are ahead then.  Fits to the same
+// 430 products; the choice is 0.6 % from the best form in the mean.  k_mfma_p4, which these all ran on before, and now, us: 256 x 256 x 4096
+// 11.5 / 4.3, 36 x 246 x 15616 30.5 / 6.2, 182 x 1444 x 26624 48.6 / 12.3, 1024 x 1024 x 8192 20.3 / 7.2, 2048 x 2048 x 16384 37.0 / 27, 534 x 4978 x 768
+// 9.3 / 6.9.  Tiles of 32 x 32 and 64 x 64 are bound by the L1 (46 bytes per cycle and compute unit), 128 x 128 by the matrix pipe (1040
+// cycles per pair of words for 1024 of multiplies).
+constexpr ProductForm kPackedForms[] = {{1, 1, 4, 3.65, 0.18, 0.0887, 0.0753, 1.27}, {1, 1, 8, 3.92, 0.60, 0.1519, 0.1587, 1.36},
+                                        {1, 2, 4, 3.90, 0.13, 0.1243, 0.1206, 1.00}, {2, 1, 4, 4.00, 0.23, 0.1297, 0.1112, 0.96},
+                                        {2, 2, 4, 4.81, 0.63, 0.1699, 0.1837, 0.72}, {3, 3, 4, 6.66, 3.11, 0.3229, 0.3832, 0.73},
+                                        {4, 4, 4, 9.58, 5.15, 0.5087, 0.5714, 0.62}, {1, 1, 1, 3.86, 0.0, 0.0954, 0.0537, 0.75},
+                                        {2, 2, 1, 6.41, 0.0, 0.2050, 0.1193, 0.57} /* k_mfma_p4 */};
 
 }  // namespace
 
@@ -612,6 +667,7 @@ bool launch_mm_packed(int type, const void* d_ac, const void* d_bc, const int* s
     ro.bias = 0.0f;
     ro.lim = type == kTNN ? 0.5f : 0.0f;
     ro.alpha = alpha;
+    ro.past_caches = stores_past_caches(nchw ? OHW : KN, M, KN);
     const int off = 64 * Kw + (type == kBNN ? 64 * Kw - K_unpack : 0);   // the lanes of a row pair, padding included, and BNN's constant
     const uint4 *P = static_cast<const uint4*>(nchw ? d_bc : d_ac), *Q = static_cast<const uint4*>(nchw ? d_ac : d_bc);
     const int *sP = nchw ? sB : sA, *sQ = nchw ? sA : sB;
@@ -621,7 +677,7 @@ bool launch_mm_packed(int type, const void* d_ac, const void* d_bc, const int* s
         *err = e;
         return true;
     };
-    switch (packed_form_of(prow, qrow, KP)) {
+    switch (form_of(kPackedForms, prow, qrow, KP)) {
         case 0: return go(launch_packed_tile<1, 1, 4, 8>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         case 1: return go(launch_packed_tile<1, 1, 8, 8>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         case 2: return go(launch_packed_tile<1, 2, 4, 6>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
@@ -629,6 +685,7 @@ bool launch_mm_packed(int type, const void* d_ac, const void* d_bc, const int* s
         case 4: return go(launch_packed_tile<2, 2, 4, 6>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         case 5: return go(launch_packed_tile<3, 3, 4, 4>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         case 6: return go(launch_packed_tile<4, 4, 4, 3>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
+        case 7: return go(launch_packed_tile<1, 1, 1, 6>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         default: return false;
     }
 }

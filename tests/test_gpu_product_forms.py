@@ -1,0 +1,41 @@
+"""Products on wavefronts with tiles of their own and on eight that split K, and results stored through the caches (k_rows and k_packed
+in fastertnn_amd/csrc/rows_kernels.hip): tiles with one row or column inside, wavefronts whose tile lies outside the product, shares of K of
+every remainder, row-major and NCHW results, all types, bit for bit against the vector-ALU engine, with nothing written past the
+result."""
+import pytest
+import torch
+
+from fastertnn_amd import TYPE_NAMES, act_is_ternary, weight_is_ternary
+
+pytestmark = pytest.mark.gpu
+
+# (images, OH, OW, columns, words): a tile per wavefront, rows of one to seven groups; 33 and 97 leave one row or column to a
+# workgroup's second wavefronts or none, 1025 to the first ones
+SHAPES = [(33, 1, 1, 20000, 4), (20000, 1, 1, 33, 8), (1025, 1, 1, 897, 4), (897, 1, 1, 1025, 12), (2, 23, 31, 961, 16), (97, 7, 97, 65, 4), (1, 1, 700000, 1, 4),
+          (700000, 1, 1, 1, 4), (1600, 1, 1, 1601, 28),
+          # eight wavefronts that split K
+          (1, 1, 1, 1, 128), (31, 1, 1, 97, 260), (3, 5, 7, 129, 300), (65, 1, 1, 33, 1000), (257, 1, 1, 131, 452),
+          # rows that are no whole sectors of results beyond 4 Mi: through the caches, on the wavefronts' own tiles and after a meeting
+          (2300, 1, 1, 2301, 4), (5, 21, 23, 2211, 8), (2297, 1, 1, 2303, 140), (5, 21, 23, 2209, 132)]
+
+
+@pytest.mark.parametrize("typ", range(4), ids=[TYPE_NAMES[t] for t in range(4)])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda v: "x".join(map(str, v)))
+def test_product_forms(hip, typ, shape):
+    n, oh, ow, kn, kw = shape
+    print("case", TYPE_NAMES[typ], shape, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5 + typ + n + kn + kw)
+    at, wt = act_is_ternary(typ), weight_is_ternary(typ)
+    words = lambda rows, tern: torch.randint(-2**63, 2**63 - 1, (rows * kw * (2 if tern else 1),), generator=g, device="cuda", dtype=torch.int64)
+    m, ku = n * oh * ow, 64 * kw - 9
+    a, b = words(m, at), words(kn, wt)
+    ea, eb = hip.expand_rows(hip.ENGINE_MFMA_F4, a, m, kw, at), hip.expand_rows(hip.ENGINE_MFMA_F4, b, kn, kw, wt)
+    want = hip.mm_engine(hip.ENGINE_VALU, typ, a, b, n, oh, ow, kn, kw, -0.25, ku).reshape(-1)
+    for kept in (False, True):
+        out = torch.full((m * kn + 64,), float("nan"), device="cuda")
+        if kept:
+            hip.mm_expanded(hip.ENGINE_MFMA_F4, typ, ea, eb, n, oh, ow, kn, kw, -0.25, ku, out=out)
+        else:
+            hip.mm_engine(hip.ENGINE_MFMA_F4, typ, a, b, n, oh, ow, kn, kw, -0.25, ku, out=out)
+        assert torch.equal(out[:m * kn].view(torch.int32), want.view(torch.int32)), kept
+        assert bool(torch.isnan(out[m * kn:]).all())
