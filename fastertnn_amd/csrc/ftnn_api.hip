@@ -1132,8 +1132,10 @@ static int select_engine(int type, int64_t M, int KN, int Kw) {
 //   * a launch is nearly all there is: few results and short rows (49 x 24 x 256 BNN NCHW 3.2 us on the vector ALU / 4.1 from rows,
 //     196 x 96 x 1024 TNN NCHW 3.6 / 4.0); binary operands are cheap there, so BNN holds out longest (256 x 64 x 262144 63 / 69);
 //   * a product has a few columns, of which a tile's 32 are mostly empty (10000 x 1 x 4096 BNN 3.8 / 4.8);
-//   * a row is one group of words, which keeps three of a workgroup's four wavefronts idle, and the results are many (10^6 x 1 x
-//     256 TNN 37 / 54, 4000 x 1000 x 256 BTN 7.9 / 9.9, 802816 x 64 x 256 BNN NCHW 49 / 77).
+//   * a row is one group of words and the results are some, but not many (1001 x 700 x 256 NCHW TNN 6.2 / 6.7, 1572 x 700 x 256 BNN NCHW
+//     6.5 / 6.9).  Where they are many the stores are all there is, and rows are ahead again (1250001 x 16 TNN 50 / 46, 645162 x 31 TNN
+//     99 / 28, 312501 x 64 BNN NCHW 25 / 18, 14001 x 250 TNN NCHW 11.0 / 8.2, 7143 x 700 BTN 11.0 / 8.7, 8001 x 250 BTN NCHW 10.3 / 6.8), but for a few
+//     columns (2500001 x 8 TBN 60 / 65).  `many` is where that had shown on every shape measured.
 // With these lines 2 in 100 products of the sweep are more than 5 % slower than on the vector ALU (16 in 100 without them), and the
 // mean over all is 0.6 % from the better of the two (2.0).
 static bool valu_ahead_of_rows(int type, int64_t M, bool nchw, int KN, int Kw) {
@@ -1142,7 +1144,8 @@ static bool valu_ahead_of_rows(int type, int64_t M, bool nchw, int KN, int Kw) {
     if (KN <= 512 && M <= 20000 && results <= 32768 && Kw <= short_rows) return true;
     if (nchw && KN <= 1000 && M <= 30000 && results <= 131072 && Kw <= 16) return true;
     if (M >= 32 && M <= 30000 && M * Kw <= 640000 && ((KN <= 4 && Kw <= 64) || (KN <= 8 && Kw <= 16))) return true;
-    if (Kw > 4) return false;
+    const int64_t many = nchw ? (type == kBNN ? 3250000 : 1500000) : type == kBTN ? 1500000 : 5000000;
+    if (Kw > 4 || (KN >= 16 && results >= many)) return false;
     if (nchw) return KN <= 1000 && (type != kBTN || M < 10000);
     return type == kBTN ? KN > 96 : M >= 100000 && KN <= 64 && KN % 32 != 0;
 }

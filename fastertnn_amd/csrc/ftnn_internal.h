@@ -264,8 +264,11 @@ bool mm_rows_within_limits(int64_t M, int KN, int Kw);
 hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
                           float alpha, float* d_y, hipStream_t st);
 
-// The same for operands in packed4 form (launch_mfma_pack4) with their rows' sums.  False where workgroup tiles through LDS are ahead:
-// nothing has been done then.
+// whether that is ahead of both operands packed by a launch and multiplied then
+bool mm_rows_ahead_of_packing(int64_t M, int OHW, int KN, int Kw);
+
+// The same for operands in packed4 form (launch_mfma_pack4) with their rows' sums.  False where workgroup tiles through LDS (k_mfma_p4) are
+// ahead: nothing has been done then.
 bool launch_mm_packed(int type, const void* d_ac, const void* d_bc, const int* sA, const int* sB, int64_t M, int OHW, int KN, int Kw,
                       int K_unpack, float alpha, float* d_y, hipStream_t st, hipError_t* err);
 

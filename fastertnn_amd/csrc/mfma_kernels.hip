@@ -1207,7 +1207,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && 
     }
 }
 
-// tiles of 256 x 256 below which the 128 x 128 kernel is used (FTNN_MFMA_SMALL_BELOW: tuning aid)
+// tiles of 256 x 256 below which the 128 x 128 tiles of k_mfma and of the record blocks' product are used (FTNN_MFMA_SMALL_BELOW: tuning aid)
 inline int64_t mfma_small_tile_below() {
     static const int64_t v = []() {
         const char* e = getenv("FTNN_MFMA_SMALL_BELOW");
@@ -1217,8 +1217,8 @@ inline int64_t mfma_small_tile_below() {
 }
 
 // Two workgroups of the smaller tiles share a compute unit: where rows are long, one's stores go on beside the other's multiplies,
-// and only the write-back at the end of a launch through the caches is left (stores_past_caches).  Operands kept, us past / through
-// the caches: 30000 x 150 x 4096 (64 words) 23.2 / 19.9, x 16384 55.3 / 55.2, 5905 x 1474 x 27904 121 / 129.
+// and only the write-back at the end of a launch through the caches is left (stores_past_caches).  us past / through the caches, on fp4
+// tiles of 128 x 128: 30000 x 150 x 4096 (64 words) 23.2 / 19.9, x 16384 55.3 / 55.2, 5905 x 1474 x 27904 121 / 129.
 inline bool tile_hides_stores(int WT, int Kw) { return WT < 4 && Kw > 128; }
 
 template <bool SWAP, bool NT, int WTP, int WTQ, int KF, int NS>
@@ -1279,9 +1279,10 @@ hipError_t launch_expand(bool tern, const uint32_t* rows_ptr, int rows, int G, u
     return hipGetLastError();
 }
 
-template <bool SWAP, bool NT, int WT, int NS>
-hipError_t launch_gemm_p4_tile_as(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, const int* sP,
+template <bool SWAP, bool NT>
+hipError_t launch_gemm_p4_as(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, const int* sP,
                                const int* sQ, int off, int form, float alpha, hipStream_t st) {
+    constexpr int WT = 4, NS = 4;
     auto kern = k_mfma_p4<SWAP, NT, WT, NS>;
     constexpr size_t lds_bytes = (size_t)NS * 4 * WT * 1024;
     // hand-counted LDS-direct loads: no scratch (see launch_gemm_tile); the opt-in to more than 64 KiB of LDS is per kernel
@@ -1301,20 +1302,12 @@ hipError_t launch_gemm_p4_tile_as(const uint4* Pc, const uint4* Qc, float* Y, in
     return hipGetLastError();
 }
 
-template <bool SWAP, int WT, int NS>
-hipError_t launch_gemm_p4_tile(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, const int* sP,
-                               const int* sQ, int off, int form, float alpha, hipStream_t st) {
-    return stores_past_caches(SWAP ? OHW : KN, M, KN) || tile_hides_stores(WT, 2 * KP)
-               ? launch_gemm_p4_tile_as<SWAP, true, WT, NS>(Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha, st)
-               : launch_gemm_p4_tile_as<SWAP, false, WT, NS>(Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha, st);
-}
-
 template <bool SWAP>
 hipError_t launch_gemm_p4(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, const int* sP, const int* sQ,
                           int off, int form, float alpha, hipStream_t st) {
-    const int64_t big = (((int64_t)M + 255) / 256) * ((KN + 255) / 256);
-    return big < mfma_small_tile_below() ? launch_gemm_p4_tile<SWAP, 2, 4>(Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha, st)
-                                         : launch_gemm_p4_tile<SWAP, 4, 4>(Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha, st);
+    return stores_past_caches(SWAP ? OHW : KN, M, KN)
+               ? launch_gemm_p4_as<SWAP, true>(Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha, st)
+               : launch_gemm_p4_as<SWAP, false>(Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha, st);
 }
 
 }  // namespace
@@ -1392,12 +1385,8 @@ hipError_t launch_mfma_gemm_packed4(int type, const void* d_ac, const void* d_bc
     const int bias = type == kBNN ? 64 * Kw - K_unpack : 0;   // as launch_mfma_gemm
     const int off = 64 * Kw + bias;                           // the lanes of a row pair, padding included
     const int form = type == kTNN ? 0 : 1;
-    // below 160 tiles of 256 x 256, and for products narrower than half of such a tile, the wavefronts of a workgroup split K, but for short
-    // rows with many results
     hipError_t e;
-    if (((M + 255) / 256 * ((KN + 255) / 256) < mfma_small_tile_below() || KN < 128 || M < 128) &&
-        launch_mm_packed(type, d_ac, d_bc, sA, sB, M, OHW, KN, Kw, K_unpack, alpha, d_y, st, &e))
-        return e;
+    if (launch_mm_packed(type, d_ac, d_bc, sA, sB, M, OHW, KN, Kw, K_unpack, alpha, d_y, st, &e)) return e;
     return OHW > 1 ? launch_gemm_p4<true>(Bc, Ac, d_y, (int)M, KN, OHW, Kw / 2, sB, sA, off, form, alpha, st)
                    : launch_gemm_p4<false>(Ac, Bc, d_y, (int)M, KN, OHW, Kw / 2, sA, sB, off, form, alpha, st);
 }
@@ -1600,18 +1589,18 @@ hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const Co
     return by_mode(std::true_type{}, std::false_type{});   // BTN, BNN
 }
 
-// A whole call from packed rows below 160 tiles of 256 x 256 multiplies the rows as they are (k_rows): packing both operands
+// A whole call from packed rows below 160 tiles of 256 x 256 multiplies the rows as they are (k_rows) and needs no scratch: packing both operands
 // first costs such a product more than the packed4 kernel gains.  Device time of the two, us (rows / packed4 or, before
-// k_rows, fragments): 2048 x 2048 x 16384 (64 tiles) 31.5 / 44, 3072 x 3072 x 24576 (144) 107 / 136; from 256 tiles on packed4
-// is ahead at any K (4096 x 4096 x 32768 218 / 190, x 2048 35 / 32, x 512 27 / 24).  Products narrower than 128 would leave more
-// than half of such a tile empty.
+// k_rows, fragments): 2048 x 2048 x 16384 (64 tiles) 31.5 / 44, 3072 x 3072 x 24576 (144) 107 / 136.  Products narrower than 128 would leave
+// more than half of such a tile empty.  From 160 tiles on scratch is asked for, and the estimates decide (mm_rows_ahead_of_packing: short
+// rows stay as they are; 4096 x 4096 x 32768 218 / 190, x 2048 36 / 42, x 256 16 / 26).
 static bool few_big_tiles(int64_t M, int KN) { return ((M + 255) / 256) * ((KN + 255) / 256) < mfma_small_tile_below(); }
 bool mm_from_rows(int64_t M, int KN, int Kw) {
     return mm_rows_within_limits(M, KN, Kw) && (few_big_tiles(M, KN) || KN < 128 || M < 128);
 }
 
 // What the explicit engine asks its callers for: both operands as fragments below 160 tiles, in packed4 form from there on.
-// A product from the rows touches none of it; AUTO asks for none there.
+// A product from the rows touches none of it; AUTO asks for none below 160 tiles.
 int64_t mfma_f4_mm_scratch_bytes(int64_t M, int KN, int Kw) {
     return few_big_tiles(M, KN) ? mfma_fragment_bytes(true, M, Kw) + mfma_fragment_bytes(true, KN, Kw)
                                 : mfma_packed4_bytes(M, Kw) + mfma_packed4_bytes(KN, Kw);
@@ -1621,7 +1610,8 @@ hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* 
                           int KN, int Kw, int K_unpack, float alpha, float* d_y, void* d_scratch,
                           hipStream_t st) {
     const bool a_tern = (type == kTNN || type == kTBN), b_tern = (type == kTNN || type == kBTN);
-    if (f4 && mm_from_rows(M, KN, Kw)) return launch_mm_rows(type, d_a, d_b, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
+    if (f4 && (mm_from_rows(M, KN, Kw) || mm_rows_ahead_of_packing(M, OHW, KN, Kw)))
+        return launch_mm_rows(type, d_a, d_b, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
     if (f4) {   // the fp4 GEMM takes its operands at two bits per lane
         void* Ac = d_scratch;
         void* Bc = static_cast<char*>(d_scratch) + mfma_packed4_bytes(M, Kw);

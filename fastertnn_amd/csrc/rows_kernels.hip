@@ -2,8 +2,8 @@
 //
 // k_mfma and k_mfma_p4 (mfma_kernels.hip) read operands that a launch of their own has brought into matrix-core form.  For
 // products below a few hundred 256 x 256 tiles that launch and its round trip through memory cost as much as the product
-// itself.  Here a wavefront fetches the bit planes as they lie, 16 bytes of signs and zeros per lane, and makes the
-// E2M1 nibbles in registers beside the multiplies: 10 vector instructions per 32 rows x 64 lanes, so that a wavefront
+// itself, and from there on they still do where rows are short.  Here a wavefront fetches the bit planes as they lie, 16 bytes of
+// signs and zeros per lane, and makes the E2M1 nibbles in registers beside the multiplies: 10 vector instructions per 32 rows x 64 lanes, so that a wavefront
 // tile of 4 x 4 blocks of 32 x 32 spends 6 issue slots per multiply of 8 slots.
 //
 //   * The wavefronts of a workgroup work on ONE output tile and split K: wavefront w takes the groups of four words
@@ -135,12 +135,25 @@ struct RowsOut {
 // Blocks that meet in LDS at a time
 constexpr int meeting_blocks(int nm, int ks) { return nm * ks * 4 > 144 ? nm / 2 : nm; }
 
+// The quads that wavefront ks of a workgroup finishes: block and quad of the block.  KS > 1: in rounds of R blocks, of each the quads
+// ks, ks + KS, ...
+template <int NM, int KS>
+struct QuadOf {
+    static constexpr int R = meeting_blocks(NM, KS), PER_ROUND = KS == 1 ? 4 * NM : R * 4 < KS ? 1 : R * 4 / KS, ROUNDS = KS == 1 ? 1 : NM / R,
+                         N = PER_ROUND * ROUNDS;
+    static_assert(KS == 1 || (KS % 4 == 0 && (R * 4 < KS || R * 4 % KS == 0) && NM % R == 0), "whole quads per wavefront");
+    static __device__ __forceinline__ int block(int i, int ks) {
+        return KS == 1 ? i / 4 : i / PER_ROUND * R + i % PER_ROUND * (KS / 4) + (KS == 4 ? 0 : ks >> 2);
+    }
+    static __device__ __forceinline__ int sub(int i, int ks) { return KS == 1 ? i % 4 : KS == 4 ? ks : ks & 3; }
+};
+
 // Where a product's results go.  Accumulator e of block (a, b): P row 32 (prb0 + a) + 8 (e / 4) + 4 h + e % 4, Q row 32 (qrb0 + b) + lr; four
-// of them are a quad.  result(quad of sums, P row, Q row) is what is stored, for a P row within the operand.
+// of them are a quad.  result(quad of sums, i) is what is stored, for quad i of the wavefront (QuadOf).
 // PReLU in the reference's two forms, "f <= 0 -> f *= alpha" (mm_p2_final_tnn_avx2.c:204-208) and "r >= 0 ? r : alpha * r"
 // (mm_p2_final_tbn_avx2.c:73): results are integers below 2^24, so both are one compare, against 0.5 or 0.
-template <bool WHOLE, bool NT, typename F>
-__device__ __forceinline__ void put_quad(const float4& sum, int p0, int qrb, const RowsOut& ro, int prow, int qrow, int lane, F&& result) {
+template <bool WHOLE, bool NT>
+__device__ __forceinline__ void put_quad(const float4& t, int p0, int qrb, const RowsOut& ro, int prow, int qrow, int lane) {
     const int lr = lane & 31, h = lane >> 5;   // P rows p0 + 4 h .. + 3 (p0 uniform) of Q block qrb
     const size_t stride = ro.p_stride;
     const uint32_t q = (uint32_t)(qrb * 32 + lr), img = fastdiv(q, ro.img);
@@ -152,7 +165,6 @@ __device__ __forceinline__ void put_quad(const float4& sum, int p0, int qrb, con
     };
     const int p = p0 + 4 * h;
     if (WHOLE || (q < (uint32_t)qrow && p < prow)) {
-        const float4 t = result(sum, p, (int)q);
         put(t.x, d + lo);
         if (WHOLE || p + 1 < prow) put(t.y, d + stride + lo);
         if (WHOLE || p + 2 < prow) put(t.z, d + 2 * stride + lo);
@@ -171,14 +183,14 @@ __device__ __forceinline__ void by_wholeness(int prb0, int qrb0, int prow, int q
 template <int WTP, int WTQ, int KS, bool NT, typename F>
 __device__ __forceinline__ void meet_and_store(v16f (&acc)[WTP][WTQ], float4* lds, const RowsOut& ro, int prb0, int qrb0, int prow, int qrow,
                                                int ks, int lane, F&& result) {
-    constexpr int NM = WTP * WTQ, R = meeting_blocks(NM, KS), QUADS = R * 4 < KS ? 1 : R * 4 / KS;
-    static_assert(KS % 4 == 0 && (R * 4 < KS || R * 4 % KS == 0) && NM % R == 0, "whole quads per wavefront");
+    typedef QuadOf<WTP * WTQ, KS> QO;
+    constexpr int R = QO::R, QUADS = QO::PER_ROUND;
 #pragma unroll
-    for (int r0 = 0; r0 < NM; r0 += R) {
+    for (int round = 0; round < QO::ROUNDS; round++) {
         __syncthreads();   // every wavefront is done with its ring, or with the round before
 #pragma unroll
         for (int j = 0; j < R; j++) {
-            const v16f& c = acc[(r0 + j) / WTQ][(r0 + j) % WTQ];
+            const v16f& c = acc[(round * R + j) / WTQ][(round * R + j) % WTQ];
 #pragma unroll
             for (int e4 = 0; e4 < 4; e4++)
                 lds[((ks * R + j) * 4 + e4) * 64 + lane] = make_float4(c[4 * e4], c[4 * e4 + 1], c[4 * e4 + 2], c[4 * e4 + 3]);
@@ -198,12 +210,13 @@ __device__ __forceinline__ void meet_and_store(v16f (&acc)[WTP][WTQ], float4* ld
                 t[i].z += u.z;
                 t[i].w += u.w;
             }
+            t[i] = result(t[i], round * QUADS + i);
         }
         by_wholeness<WTP, WTQ>(prb0, qrb0, prow, qrow, [&](auto whole) {
 #pragma unroll
             for (int i = 0; i < QUADS; i++) {
-                const int blk = r0 + i * (KS / 4) + (KS == 4 ? 0 : ks >> 2), sub = KS == 4 ? ks : ks & 3;   // of quad i KS + ks
-                put_quad<decltype(whole)::value, NT>(t[i], (prb0 + blk / WTQ) * 32 + 8 * sub, qrb0 + blk % WTQ, ro, prow, qrow, lane, result);
+                const int blk = QO::block(round * QUADS + i, ks);
+                put_quad<decltype(whole)::value, NT>(t[i], (prb0 + blk / WTQ) * 32 + 8 * QO::sub(i, ks), qrb0 + blk % WTQ, ro, prow, qrow, lane);
             }
         });
     }
@@ -212,15 +225,17 @@ __device__ __forceinline__ void meet_and_store(v16f (&acc)[WTP][WTQ], float4* ld
 // the same for a wavefront with whole sums
 template <int WTP, int WTQ, bool NT, typename F>
 __device__ __forceinline__ void store_whole_sums(v16f (&acc)[WTP][WTQ], const RowsOut& ro, int prb0, int qrb0, int prow, int qrow, int lane, F&& result) {
+    float4 t[WTP * WTQ * 4];
+#pragma unroll
+    for (int i = 0; i < WTP * WTQ * 4; i++) {
+        const v16f& c = acc[i / 4 / WTQ][i / 4 % WTQ];
+        const int e = 4 * (i % 4);
+        t[i] = result(make_float4(c[e], c[e + 1], c[e + 2], c[e + 3]), i);
+    }
     by_wholeness<WTP, WTQ>(prb0, qrb0, prow, qrow, [&](auto whole) {
 #pragma unroll
-        for (int blk = 0; blk < WTP * WTQ; blk++) {
-            const v16f& c = acc[blk / WTQ][blk % WTQ];
-#pragma unroll
-            for (int e4 = 0; e4 < 4; e4++)
-                put_quad<decltype(whole)::value, NT>(make_float4(c[4 * e4], c[4 * e4 + 1], c[4 * e4 + 2], c[4 * e4 + 3]),
-                                                 (prb0 + blk / WTQ) * 32 + 8 * e4, qrb0 + blk % WTQ, ro, prow, qrow, lane, result);
-        }
+        for (int i = 0; i < WTP * WTQ * 4; i++)
+            put_quad<decltype(whole)::value, NT>(t[i], (prb0 + i / 4 / WTQ) * 32 + 8 * (i % 4), qrb0 + i / 4 % WTQ, ro, prow, qrow, lane);
     });
 }
 
@@ -394,7 +409,7 @@ __global__ __launch_bounds__(64 * (KS == 1 ? 4 : KS)) void k_rows(const char* __
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in the LDS that the partial tiles take now
 
-    auto result = [&](const float4& t, int, int) {
+    auto result = [&](const float4& t, int) {
         auto prelu = [&](float v) {
             const float r = v - ro.bias;
             return r < ro.lim ? r * ro.alpha : r;
@@ -481,10 +496,13 @@ __global__ __launch_bounds__(64 * (KS == 1 ? 4 : KS)) void k_packed(const uint4*
         }
     }
     // dot = 4 sum - sum of the P row - sum of the Q row - lanes (off: with BNN's constant), all of it below 2^24; the sums are there for
-    // whole blocks of rows
-    auto result = [&](const float4& t, int p, int q) {
-        const int4 s = *reinterpret_cast<const int4*>(sP + p);
-        const int o = sQ[q] + off;
+    // whole blocks of rows.  All of them are read before the first store, which they would wait for (loads and stores are counted together and in
+    // order): 123056 x 635 x 3328 225 -> 204 us, 9660 x 10247 x 256 118 -> 98.  Ahead of the operands they gain nothing more.
+    typedef QuadOf<NM, KS> QO;
+    auto result = [&](const float4& t, int i) {
+        const int blk = QO::block(i, ks);
+        const int4 s = *reinterpret_cast<const int4*>(sP + min(prb0 + blk / WTQ, prbmax) * 32 + 8 * QO::sub(i, ks) + 4 * (lane >> 5));
+        const int o = sQ[min(qrb0 + blk % WTQ, qrbmax) * 32 + (lane & 31)] + off;
         auto prelu = [&](float v, int sp) {
             const float r = (float)((int)(v * 4.0f) - sp - o);
             return r < ro.lim ? r * ro.alpha : r;
@@ -545,17 +563,17 @@ struct ProductForm {
     int p, q, ks;
     double a, b, c, d, e;
 };
-constexpr int64_t kOwnTilesFrom = 650000;   // results from which wavefronts have tiles of their own; 3045 x 188 x 512 4.0 split / 4.7, 169 x 4816 x 512 5.5 / 4.4
-template <int NF>
-int form_of(const ProductForm (&forms)[NF], int64_t prow, int64_t qrow, int words) {
+// the least estimate among the first `count` forms
+int form_of(const ProductForm* forms, int count, int64_t prow, int64_t qrow, int words) {
     const int64_t pb = (prow + 31) / 32, qb = (qrow + 31) / 32;
     int best = -1;
-    double least = 1e30;
-    for (int i = 0; i < NF; i++) {
+    double least = 1e300;
+    for (int i = 0; i < count; i++) {
         const ProductForm& f = forms[i];
         const int own = f.ks == 1 ? 2 : 1;   // 2 x 2 tiles per workgroup
         const int64_t tiles = ((pb + f.p * own - 1) / (f.p * own)) * ((qb + f.q * own - 1) / (f.q * own));
-        if (tiles > kMaxRowsTiles || (f.ks == 1 && f.p == 1 && prow * qrow < kOwnTilesFrom) || (f.ks == 8 && tiles > 256)) continue;
+        // (fitted, and measured, on up to 256 tiles only: eight wavefronts on one)
+        if (tiles > kMaxRowsTiles || (f.ks == 8 && tiles > 256)) continue;
         const double n1 = (double)((tiles + 255) / 256 - 1), w = (double)words / f.ks;
         const double t = f.a + f.b * n1 + w * (f.c + f.d * n1) + f.e * 1e-6 * (double)prow * (double)qrow;
         if (t < least) least = t, best = i;
@@ -563,22 +581,26 @@ int form_of(const ProductForm (&forms)[NF], int64_t prow, int64_t qrow, int word
     return best;
 }
 
-// Fits to 430 products below 160 tiles of 256 x 256, 32 x 32 x 256 to 8192 x 8192 x 32768 and all types, every form measured: the choice is 0.6 %
-// from the best form in the mean and takes 0.95 of the time of the squares on four wavefronts alone.  us, before / now: 332 x 8180 x 256
-// BTN 8.2 / 5.3, 534 x 4978 x 768 9.1 / 6.5, 2506 x 1365 x 512 BNN 9.3 / 6.5, 190 x 5514 x 26368 37.5 / 27.3, 1446 x 725 x 20736 TBN 24.8 / 21.3; the other
-// way 1020 x 398 x 27392 13.6 / 15.6, 158 x 2048 x 18688 11.8 / 13.0.
-constexpr ProductForm kRowsForms[] = {{1, 1, 4, 3.39, 0.005, 0.0578, 0.0486, 1.03}, {2, 2, 4, 4.27, 0.32, 0.1143, 0.1157, 0.94},
-                                      {3, 3, 4, 6.18, 3.07, 0.1792, 0.2319, 0.81},  {4, 4, 4, 8.61, 5.10, 0.2513, 0.3557, 0.66},
-                                      {1, 1, 1, 3.45, 0.0, 0.0616, 0.0364, 0.57},   {1, 1, 8, 3.56, 0.10, 0.0927, 0.1047, 1.51}};
+// Fits to 995 products, 32 x 32 x 256 to 8192 x 8192 x 131072 below 160 tiles of 256 x 256 and up to 1.5e8 results above, all types, row-major and
+// NCHW, every form measured; the last one is both operands packed by a launch and then multiplied in their best form (below).  The
+// choice is 0.9 % from the best form in the mean.  us, four wavefronts that split K / now: 332 x 8180 x 256 BTN 8.2 / 5.3, 534 x 4978 x 768
+// 9.1 / 6.5, 2506 x 1365 x 512 BNN 9.3 / 6.5, 190 x 5514 x 26368 37.5 / 27.3, 1446 x 725 x 20736 TBN 24.8 / 21.3.  From 160 tiles on, packed first / now: 3328 x
+// 3328 x 1024 TNN 31 / 16, 6016 x 6016 x 256 56 / 31, 137912 x 157 x 512 68 / 27, 12014 x 1415 x 2816 TBN 68 / 39, 14694 x 2992 x 1792 90 / 60.
+constexpr ProductForm kRowsForms[] = {{1, 1, 4, 3.43, 0.04, 0.0621, 0.0497, 0.72}, {2, 2, 4, 3.88, 0.71, 0.1107, 0.1156, 0.66},
+                                      {3, 3, 4, 5.74, 3.18, 0.1986, 0.2273, 0.81}, {4, 4, 4, 7.79, 3.66, 0.2677, 0.3204, 0.69},
+                                      {1, 1, 1, 3.54, 0.00, 0.0502, 0.0455, 0.47}, {1, 1, 8, 3.75, 0.09, 0.0858, 0.1057, 0.82},
+                                      {2, 2, 1, 4.62, 0.00, 0.1076, 0.1139, 0.56}, {4, 4, 1, 18.69, 10.44, 0.3071, 0.2606, 0.51}};
+constexpr int kRowsFormsOfRows = (int)(sizeof(kRowsForms) / sizeof(kRowsForms[0])) - 1;   // without the last
 
 template <bool TP, bool TQ>
 hipError_t launch_rows_types(const char* P, const char* Q, int64_t prow, int64_t qrow, int Kw, const RowsOut& ro, hipStream_t st) {
-    switch (form_of(kRowsForms, prow, qrow, Kw)) {
+    switch (form_of(kRowsForms, kRowsFormsOfRows, prow, qrow, Kw)) {
         case 0: return launch_rows_tile<TP, TQ, 1, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
         case 1: return launch_rows_tile<TP, TQ, 2, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
         case 2: return launch_rows_tile<TP, TQ, 3, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
         case 4: return launch_rows_tile<TP, TQ, 1, 1>(P, Q, prow, qrow, Kw / 4, ro, st);
         case 5: return launch_rows_tile<TP, TQ, 1, 8>(P, Q, prow, qrow, Kw / 4, ro, st);
+        case 6: return launch_rows_tile<TP, TQ, 2, 1>(P, Q, prow, qrow, Kw / 4, ro, st);
         default: return launch_rows_tile<TP, TQ, 4, 4>(P, Q, prow, qrow, Kw / 4, ro, st);
     }
 }
@@ -618,6 +640,11 @@ bool mm_rows_within_limits(int64_t M, int KN, int Kw) {
     return 64LL * Kw < (1LL << 24) && rows_tiles(M, KN, 128) <= kMaxRowsTiles;
 }
 
+bool mm_rows_ahead_of_packing(int64_t M, int OHW, int KN, int Kw) {
+    if (!mm_rows_within_limits(M, KN, Kw)) return false;
+    return form_of(kRowsForms, kRowsFormsOfRows + 1, OHW > 1 ? KN : M, OHW > 1 ? M : KN, Kw) != kRowsFormsOfRows;
+}
+
 hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
                           float alpha, float* d_y, hipStream_t st) {
     const bool at = type == kTNN || type == kTBN, wt = type == kTNN || type == kBTN;
@@ -643,16 +670,17 @@ hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int6
 }
 
 namespace {
-// Operands kept: the forms above, or none: workgroup tiles of 128 x 128 through LDS (k_mfma_p4, the last estimate) are ahead then.  Fits to the same
-// 430 products; the choice is 0.6 % from the best form in the mean.  k_mfma_p4, which these all ran on before, and now, us: 256 x 256 x 4096
+// Operands kept: the forms above, or workgroup tiles of 256 x 256 through LDS (k_mfma_p4, the last).  Fits to the same products; the
+// choice is 1 % from the best form in the mean.  us, on k_mfma_p4 alone (tiles of 128 x 128 below 160 of 256 x 256) / now: 256 x 256 x 4096
 // 11.5 / 4.3, 36 x 246 x 15616 30.5 / 6.2, 182 x 1444 x 26624 48.6 / 12.3, 1024 x 1024 x 8192 20.3 / 7.2, 2048 x 2048 x 16384 37.0 / 27, 534 x 4978 x 768
-// 9.3 / 6.9.  Tiles of 32 x 32 and 64 x 64 are bound by the L1 (46 bytes per cycle and compute unit), 128 x 128 by the matrix pipe (1040
-// cycles per pair of words for 1024 of multiplies).
-constexpr ProductForm kPackedForms[] = {{1, 1, 4, 3.65, 0.18, 0.0887, 0.0753, 1.27}, {1, 1, 8, 3.92, 0.60, 0.1519, 0.1587, 1.36},
-                                        {1, 2, 4, 3.90, 0.13, 0.1243, 0.1206, 1.00}, {2, 1, 4, 4.00, 0.23, 0.1297, 0.1112, 0.96},
-                                        {2, 2, 4, 4.81, 0.63, 0.1699, 0.1837, 0.72}, {3, 3, 4, 6.66, 3.11, 0.3229, 0.3832, 0.73},
-                                        {4, 4, 4, 9.58, 5.15, 0.5087, 0.5714, 0.62}, {1, 1, 1, 3.86, 0.0, 0.0954, 0.0537, 0.75},
-                                        {2, 2, 1, 6.41, 0.0, 0.2050, 0.1193, 0.57} /* k_mfma_p4 */};
+// 9.3 / 6.9; 3328 x 3328 x 1024 22 / 15, 6016 x 6016 x 1024 58 / 38, 8192 x 8192 x 1536 98 / 68, 20021 x 2017 x 256 BNN 53 / 38, 42190 x 2443 x 256 157 / 96, 8396 x 1216 x
+// 3072 31 / 21.  Tiles of 32 x 32 and 64 x 64 that split K are bound by the L1 (46 bytes per cycle and compute unit), 128 x 128 by the matrix pipe
+// (1040 cycles per pair of words for 1024 of multiplies); short rows with many results by the stores (3.5 - 5.5 TB/s).
+constexpr ProductForm kPackedForms[] = {{1, 1, 4, 3.51, 0.14, 0.0976, 0.0756, 0.75}, {1, 1, 8, 3.95, 0.53, 0.1324, 0.1691, 1.32},
+                                        {1, 2, 4, 4.54, 0.17, 0.1246, 0.1200, 0.57}, {2, 1, 4, 3.79, 0.36, 0.0982, 0.1142, 0.62},
+                                        {2, 2, 4, 4.43, 0.58, 0.1742, 0.1811, 0.69}, {3, 3, 4, 6.36, 3.52, 0.3449, 0.3770, 0.44},
+                                        {4, 4, 4, 8.44, 4.48, 0.5230, 0.5731, 0.28}, {1, 1, 1, 3.67, 0.02, 0.0740, 0.0585, 0.71},
+                                        {2, 2, 1, 4.39, 0.25, 0.1764, 0.1700, 0.62}, {4, 4, 1, 14.28, 7.83, 0.5053, 0.5027, 0.42}};
 
 }  // namespace
 
@@ -677,7 +705,7 @@ bool launch_mm_packed(int type, const void* d_ac, const void* d_bc, const int* s
         *err = e;
         return true;
     };
-    switch (form_of(kPackedForms, prow, qrow, KP)) {
+    switch (form_of(kPackedForms, (int)(sizeof(kPackedForms) / sizeof(kPackedForms[0])), prow, qrow, KP)) {
         case 0: return go(launch_packed_tile<1, 1, 4, 8>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         case 1: return go(launch_packed_tile<1, 1, 8, 8>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         case 2: return go(launch_packed_tile<1, 2, 4, 6>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
@@ -686,6 +714,7 @@ bool launch_mm_packed(int type, const void* d_ac, const void* d_bc, const int* s
         case 5: return go(launch_packed_tile<3, 3, 4, 4>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         case 6: return go(launch_packed_tile<4, 4, 4, 3>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         case 7: return go(launch_packed_tile<1, 1, 1, 6>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
+        case 8: return go(launch_packed_tile<2, 2, 1, 4>(P, Q, prow, qrow, KP, sP, sQ, off, ro, st));
         default: return false;
     }
 }

@@ -16,7 +16,11 @@ SHAPES = [(33, 1, 1, 20000, 4), (20000, 1, 1, 33, 8), (1025, 1, 1, 897, 4), (897
           # eight wavefronts that split K
           (1, 1, 1, 1, 128), (31, 1, 1, 97, 260), (3, 5, 7, 129, 300), (65, 1, 1, 33, 1000), (257, 1, 1, 131, 452),
           # rows that are no whole sectors of results beyond 4 Mi: through the caches, on the wavefronts' own tiles and after a meeting
-          (2300, 1, 1, 2301, 4), (5, 21, 23, 2211, 8), (2297, 1, 1, 2303, 140), (5, 21, 23, 2209, 132)]
+          (2300, 1, 1, 2301, 4), (5, 21, 23, 2211, 8), (2297, 1, 1, 2303, 140), (5, 21, 23, 2209, 132),
+          # 160 tiles of 256 x 256 and more: wavefronts on 2 x 2 blocks of their own, with one block, row or column inside, or none
+          (3105, 1, 1, 3361, 32), (5, 25, 27, 3169, 28), (6177, 1, 1, 1825, 40), (41, 11, 13, 1889, 36), (3137, 1, 1, 3201, 64),
+          # four wavefronts on one tile, and both operands packed first
+          (4129, 1, 1, 2593, 100), (4129, 1, 1, 2625, 260), (3, 37, 41, 2593, 100), (20001, 1, 1, 609, 128)]
 
 
 @pytest.mark.parametrize("typ", range(4), ids=[TYPE_NAMES[t] for t in range(4)])
