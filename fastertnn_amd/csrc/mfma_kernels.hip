@@ -890,7 +890,7 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
 // (mm_p2_final_tnn_avx2.c:204-208), else "r >= 0 ? r : alpha * r" (mm_p2_final_tbn_avx2.c:73).
 // QMODE: 0 = fp32 NCHW result, 1 / 2 = ternary / binary hand-over to the next layer (QuantOut).
 // All three are compile-time so that the per-element epilogue carries no selects for them.
-// TA x TB: blocks of 32 kernels x 32 pixels per wavefront.  2 x 2, or 1 x 1 with S = 4 for layers with few tiles: a
+// TA x TB: blocks of 32 kernels x 32 pixels per wavefront.  2 x 2, or 1 x 1 with S = 4, or S = 8 on a workgroup of eight, for layers with few tiles: a
 // wavefront moves a bounded number of bytes per cycle from a cold L2 whatever its prefetch depth, so a small layer gets faster
 // only with more wavefronts, on more compute units.  Kernel tiles of 32 come in pairs under the hand-over (a pixel's
 // record is written by two workgroups, 8 bytes each; a tile past KN writes padding lanes).
@@ -903,15 +903,15 @@ __global__ __launch_bounds__(256) void k_mfma_s2(const uint4* __restrict__ Pc, c
 // stores too, relative to the tile's first image and kernel: y_span bounds what a tile reaches from there, whatever the size
 // of the result.
 template <bool ABIN, bool FORM0, int QMODE, int TA, int TB, int S, bool BUF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((S == 1 && QMODE != 0) ? 3 : 1, 8))) void k_conv_f4(
+__global__ __launch_bounds__(S == 8 ? 512 : 256) __attribute__((amdgpu_waves_per_eu((S == 1 && QMODE != 0) ? 3 : 1, 8))) void k_conv_f4(
     const uint4* __restrict__ P2, const uint4* __restrict__ Wf, float* __restrict__ Y, int M, int KN, int OHW, int KP /* pairs a weight row is stored at */,
     int bias, float alpha, FastDiv dOHW, ConvGeom cg, PairWalk pw, QuantOut qo, uint32_t p2_bytes, uint32_t wf_bytes, uint32_t y_span, XcdOrder xo, uint32_t launched_x, uint32_t kernel_tiles) {
-    constexpr int WPB = 4;                // wavefronts per workgroup (single-wavefront workgroups for S = 1
+    constexpr int WPB = S == 8 ? 8 : 4;   // wavefronts per workgroup (single-wavefront workgroups for S = 1
                                           // measured slower: neighbours no longer share weight fragments in L1)
     constexpr int NB = 3;                 // register sets of records: NB - 1 pairs of loads in flight; four and six measured slower
     constexpr int NBLK = TA * TB;
     constexpr int PUB = NBLK == 1 ? 1 : 4 - 4 / S;   // blocks a wavefront hands to the others of its tile
-    __shared__ float4 red[S > 1 ? 4 * PUB * 4 * 64 : 1];   // [wavefront][slot][e / 4][lane]
+    __shared__ float4 red[S > 1 ? WPB * PUB * 4 * 64 : 1];   // [wavefront][slot][e / 4][lane]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ks = wave % S, pt = wave / S;   // K share and pixel tile of this wavefront
@@ -1529,7 +1529,7 @@ hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const Co
     }();
     if (tune) split = tune;
     while (split > 1 && pw.NP < split) split /= 2;   // no wavefront without K words of its own, forced or not
-    const int wpb = 4, tpb = wpb / split;   // wavefronts and pixel tiles per workgroup (see the kernel)
+    const int tpb = 4 / split;   // pixel tiles per workgroup (see the kernel)
     // Few 64 x 64 tiles: tiles of 32 x 32, four times the workgroups.  fp32 results of fewer than 120 words up to 300 tiles; but where 190 to
     // 256 tiles give most of the 256 compute units one workgroup each and a row is long (72 words), those are ahead unless the last
     // kernel tile is half empty.  Layer and quantiser in a graph, us, 64 x 64 split four ways / 32 x 32: 216 tiles x 108 words 9.8 / 10.4,
@@ -1537,6 +1537,11 @@ hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const Co
     const bool one_round = cg.K >= 72 && tiles >= 190 && tiles <= 256 && (KN + 31) / 32 % 2 == 0;
     static const int64_t tune_small = getenv("FTNN_CONV_SMALL_BELOW") ? atoi(getenv("FTNN_CONV_SMALL_BELOW")) : -1;
     const bool small = tiles < (tune_small >= 0 ? tune_small : qo.mode == 0 && cg.K < 120 && !one_round ? 300 : 150);
+    // Small tiles that do not fill the compute units and long rows: eight wavefronts split K.  A run of K words is a chain of loads, two pairs in
+    // flight, and the exchange grows by 0.2 us.  Layer and quantiser in a graph, us, on four / eight wavefronts: 24 tiles x 392 words 12.1 / 10.1,
+    // 99 x 525 19.2 / 15.0, 189 x 425 16.8 / 12.9, 158 x 196 9.5 / 8.4, 96 x 75 7.6 / 7.0; the other way 100 x 18 6.0 / 6.2, 976 x 18 7.6 / 9.2,
+    // 305 x 72 8.8 / 9.4.  Of 213 layers the 86 within these lines take 0.75 - 1.0 of the time; hand-overs are of chains whose rows are shorter.
+    const bool deep = small && !tune && qo.mode == 0 && cg.K >= 75 && ((M + 31) / 32) * ((KN + 31) / 32) <= 256;
     dim3 grid((unsigned)(((M + 63) / 64 + tpb - 1) / tpb), (unsigned)((KN + 63) / 64));
     if (small) grid = dim3((unsigned)((M + 31) / 32), (unsigned)(qo.mode != 0 ? 2 * ((KN + 63) / 64) : (KN + 31) / 32));
     if (M > 0x7fffff00LL) return hipErrorInvalidValue;   // pixel indices stay below 2^31
@@ -1562,7 +1567,7 @@ hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const Co
         constexpr bool A = decltype(abin)::value, F = decltype(form0)::value;
         constexpr int Q = decltype(qmode)::value, T = decltype(blocks)::value, SP = decltype(sp)::value;
         auto go = [&](auto kern) -> hipError_t {
-            hipLaunchKernelGGL(kern, launched, dim3(64 * wpb), 0, st, P2, Wf, d_y, (int)M, KN, OHW, KP, bias, alpha, dOHW, cg, pw, qo,
+            hipLaunchKernelGGL(kern, launched, dim3(SP == 8 ? 512 : 256), 0, st, P2, Wf, d_y, (int)M, KN, OHW, KP, bias, alpha, dOHW, cg, pw, qo,
                                clip(p2_bytes), clip(wf_bytes), clip(y_span), xo, launched.x, grid.y);
             return hipGetLastError();
         };
@@ -1572,6 +1577,8 @@ hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const Co
         typedef std::integral_constant<int, 1> one;
         typedef std::integral_constant<int, 2> two;
         typedef std::integral_constant<int, 4> four;
+        if constexpr (decltype(qmode)::value == 0)
+            if (deep) return launch(abin, form0, qmode, one{}, std::integral_constant<int, 8>{});
         if (small) return launch(abin, form0, qmode, one{}, four{});
         if (split == 1) return launch(abin, form0, qmode, two{}, one{});
         if (split == 2) return launch(abin, form0, qmode, two{}, two{});
