@@ -22,6 +22,8 @@
 #include "ftnn_internal.h"
 #include "host_hash.h"
 
+static bool valu_ahead_of_rows(int type, int64_t M, bool nchw, int KN, int Kw);
+
 namespace ftnn {
 
 static thread_local char g_err[512] = "";
@@ -947,26 +949,25 @@ int conv_f4_expanded(int type, const float* d_x, const float* d_thr, const void*
     return e == hipSuccess ? FTNN_OK : hip_fail(e, "fp4 conv launch");
 }
 
-// the vector-ALU layer: quantise to bit planes, then the implicit-im2row GEMM (or, for few channels, the dense
-// re-packing and the plain GEMM)
+// the vector-ALU layer: quantise to bit planes, then the implicit-im2row GEMM (or, for few channels, the plain GEMM of dense rows, on the
+// matrix cores where the caller leaves the engine open and they are ahead)
 int conv_valu(int type, const float* d_x, const float* d_thr, const int64_t* d_qw, int N, int C, int H, int W,
               int KN, int KH, int KW, int H_pad, int W_pad, int H_stride, int W_stride, float prelu_alpha,
-              void* d_scratch, float* d_y, hipStream_t st, const QuantOut& qo, bool weights_prepared) {
+              void* d_scratch, float* d_y, hipStream_t st, const QuantOut& qo, bool weights_prepared, bool any_engine) {
     const int OH = out_dim(H, H_pad, KH, H_stride), OW = out_dim(W, W_pad, KW, W_stride);
     const bool act_ternary = (type == kTNN || type == kTBN);
     const bool w_ternary = (type == kTNN || type == kBTN);
-    hipError_t e = launch_quantize(act_ternary, d_x, d_thr, N, C, H, W, d_scratch, st);
-    if (e != hipSuccess) return hip_fail(e, "quantize launch");
+    hipError_t e;
     int T, Kd;
     if (dense_applies(C, KH, KW, &T, &Kd)) {
-        // few channels: re-pack both operands with several taps per word and run the plain GEMM
+        // few channels: both operands re-packed with several taps per word, and the plain GEMM
         char* base = static_cast<char*>(d_scratch);
         const int64_t p_bytes = (ftnn_pack_scratch_bytes(N, C, H, W, act_ternary) + 255) / 256 * 256;
         const int64_t rows_bytes =
             ((int64_t)N * OH * OW * round4(Kd) * (act_ternary ? 16 : 8) + 255) / 256 * 256;
         int64_t* d_rows = reinterpret_cast<int64_t*>(base + p_bytes);
         const int64_t* d_wd = d_qw;   // prepared weights are the re-packed rows already
-        e = launch_dense_rows(act_ternary, d_scratch, N, C, H, W, H_pad, W_pad, KH, KW, H_stride, W_stride,
+        e = launch_dense_rows(act_ternary, d_x, d_thr, N, C, H, W, H_pad, W_pad, KH, KW, H_stride, W_stride,
                               d_rows, st);
         if (e != hipSuccess) return hip_fail(e, "dense rows launch");
         if (!weights_prepared) {
@@ -975,10 +976,20 @@ int conv_valu(int type, const float* d_x, const float* d_thr, const int64_t* d_q
             if (e != hipSuccess) return hip_fail(e, "dense weights launch");
             d_wd = d_tmp;
         }
-        e = launch_mm(type, d_rows, d_wd, (int64_t)N * OH * OW, OH * OW, KN, round4(Kd), C * KH * KW,
-                      prelu_alpha, d_y, st, qo);
+        // A product of packed rows, on the matrix cores where the caller leaves the engine open and k_rows is ahead: as a layer, us, vector ALU /
+        // k_rows: 64 x 16 x 56 x 56 -> 64, 3 x 3, TNN 42 / 29, 7 x 11 x 86 x 86 -> 136, 7 x 7, BTN 54 / 27, 10 x 16 x 48 x 48 -> 256 BNN 17.4 / 11.9.
+        // Few kernels on one group of words leave its tiles mostly empty (256 x 16 x 16 x 16 -> 8 BTN 10.9 / 12.5).
+        const int64_t M = (int64_t)N * OH * OW;
+        const int Kw = round4(Kd);
+        if (any_engine && qo.mode == 0 && (KN >= 16 || Kw > 4) && mm_rows_within_limits(M, KN, Kw) &&
+            !valu_ahead_of_rows(type, M, OH * OW > 1, KN, Kw))
+            e = launch_mm_rows(type, d_rows, d_wd, M, OH * OW, KN, Kw, C * KH * KW, prelu_alpha, d_y, st);
+        else
+            e = launch_mm(type, d_rows, d_wd, M, OH * OW, KN, Kw, C * KH * KW, prelu_alpha, d_y, st, qo);
         return e == hipSuccess ? FTNN_OK : hip_fail(e, "mm launch");
     }
+    e = launch_quantize(act_ternary, d_x, d_thr, N, C, H, W, d_scratch, st);
+    if (e != hipSuccess) return hip_fail(e, "quantize launch");
     const ConvGeom cg = {H, W, cpack_of(C), OH, OW, KW, cpack_of(C) * KH * KW, H_pad, W_pad, H_stride, W_stride,
                          make_fastdiv((uint32_t)OW), make_fastdiv((uint32_t)cpack_of(C)), make_fastdiv((uint32_t)KW)};
     e = launch_mm_implicit(type, d_scratch, d_qw, cg, N, KN, C * KH * KW, prelu_alpha, d_y, st, qo);
@@ -1286,7 +1297,8 @@ int ftnn_conv_engine(int engine, int type, const float* d_x, const float* d_thr,
     if ((int64_t)N * OH * OW > 0x7fffffffLL) return fail(FTNN_EINVAL, "more than 2^31-1 output rows");
     const bool fits_f4 = (int64_t)N * H * W * cpack_of(C) <= 0x7fffffffLL &&
                          (int64_t)N * OH * OW * conv_f4_weight_words(C, KH, KW) <= 0x7fffffffLL;
-    if (engine == FTNN_ENGINE_AUTO)   // a layer beyond the fp4 kernel's 32-bit pixel indices goes to the vector ALU
+    const bool any_engine = engine == FTNN_ENGINE_AUTO;
+    if (any_engine)   // a layer beyond the fp4 kernel's 32-bit pixel indices goes to the vector ALU
         engine = fits_f4 ? select_conv_engine(type, N, C, H, W, KN, KH, KW, OH, OW) : FTNN_ENGINE_VALU;
     const bool w_ternary = (type == kTNN || type == kBTN);
     if (engine == FTNN_ENGINE_MFMA_F4) {
@@ -1312,7 +1324,7 @@ int ftnn_conv_engine(int engine, int type, const float* d_x, const float* d_thr,
     }
     if (engine != FTNN_ENGINE_VALU) return fail(FTNN_EINVAL, "layer engine %d (vector ALU and fp4 only)", engine);
     return conv_valu(type, d_x, d_thr, d_qw, N, C, H, W, KN, KH, KW, H_pad, W_pad, H_stride, W_stride, prelu_alpha,
-                     d_scratch, d_y, (hipStream_t)stream, QuantOut(), false);
+                     d_scratch, d_y, (hipStream_t)stream, QuantOut(), false, any_engine);
 }
 
 int64_t ftnn_conv_weights_bytes(int type, int C, int KN, int KH, int KW) {
@@ -1363,7 +1375,7 @@ int ftnn_conv_prepared(int type, const float* d_x, const float* d_thr, const voi
                                 W_stride, prelu_alpha, d_scratch, d_y, (hipStream_t)stream, QuantOut());
     }
     return conv_valu(type, d_x, d_thr, static_cast<const int64_t*>(d_prepared), N, C, H, W, KN, KH, KW, H_pad, W_pad,
-                     H_stride, W_stride, prelu_alpha, d_scratch, d_y, (hipStream_t)stream, QuantOut(), true);
+                     H_stride, W_stride, prelu_alpha, d_scratch, d_y, (hipStream_t)stream, QuantOut(), true, true);
 }
 
 int ftnn_conv(int type, const float* d_x, const float* d_thr, const int64_t* d_qw, int N, int C,

@@ -205,9 +205,9 @@ hipError_t launch_quantize_f4(bool ternary, const float* d_x, const float* d_thr
 // quantise only, into Packing-2 rows: fp32 [N][C] -> N rows (activations of a fully connected layer as launch_mm_rows reads them)
 hipError_t launch_quantize_rows(bool ternary, const float* d_x, const float* d_thr, int N, int C, int64_t* d_out, hipStream_t st);
 
-// dense re-packing of both operands for layers with C <= 32 (several taps per 64-lane word)
+// dense re-packing of both operands for layers with C <= 32 (several taps per 64-lane word), the activations from fp32
 bool dense_applies(int C, int KH, int KW, int* T_out, int* Kd_out);
-hipError_t launch_dense_rows(bool ternary, const void* d_p, int N, int C, int H, int W, int H_pad, int W_pad,
+hipError_t launch_dense_rows(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W, int H_pad, int W_pad,
                              int kH, int kW, int H_stride, int W_stride, int64_t* d_out, hipStream_t st);
 hipError_t launch_dense_weights(bool ternary, const int64_t* d_qw, int KN, int C, int kH, int kW,
                                 int64_t* d_out, hipStream_t st);
@@ -301,10 +301,11 @@ int conv_f4_expanded(int type, const float* d_x, const float* d_thr, const void*
                      int W, int KN, int KH, int KW, int H_pad, int W_pad, int H_stride, int W_stride,
                      float prelu_alpha, void* d_p2, float* d_y, hipStream_t st, const QuantOut& qo);
 // the vector-ALU layer; d_scratch as for ftnn_conv
-// (weights_prepared: for a few-channel layer d_qw already holds the re-packed rows of launch_dense_weights)
+// (weights_prepared: for a few-channel layer d_qw already holds the re-packed rows of launch_dense_weights; any_engine: their product
+// may run on the matrix cores)
 int conv_valu(int type, const float* d_x, const float* d_thr, const int64_t* d_qw, int N, int C, int H, int W,
               int KN, int KH, int KW, int H_pad, int W_pad, int H_stride, int W_stride, float prelu_alpha,
-              void* d_scratch, float* d_y, hipStream_t st, const QuantOut& qo, bool weights_prepared);
+              void* d_scratch, float* d_y, hipStream_t st, const QuantOut& qo, bool weights_prepared, bool any_engine);
 // bytes of the fp4 layer's operand region (d_p2 above) for this shape, rounded up to 256: P2, or for a
 // few-channel layer the nibble pixels and dense rows
 int64_t conv_f4_operand_bytes(int N, int C, int H, int W, int KH, int KW, int OH, int OW, int KN, int W_stride);

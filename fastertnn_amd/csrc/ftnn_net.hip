@@ -108,7 +108,7 @@ int enqueue_layer(ftnn_net* net, const NetPart& part, int i, const float*& in, b
                               part.d_p2[(size_t)net->p2_buf[i]], out, st, qo);
     else
         rc = conv_valu(L.type, in, net->d_thr[i], L.d_qw, part.batch, L.C, L.H, L.W, L.KN, L.KH, L.KW, L.pad, L.pad,
-                       L.stride, L.stride, L.prelu_alpha, part.d_scratch, out, st, qo, false);
+                       L.stride, L.stride, L.prelu_alpha, part.d_scratch, out, st, qo, false, true);
     p2_ready = next_f4;
     in = out;
     return rc;

@@ -18,6 +18,9 @@
 // ballot kernels (k_pack_weights, k_pack_gemm_operand): offline work in the
 // reference, HBM-bound here (a wavefront per output word group, several coalesced
 // loads in flight per lane).
+#include <algorithm>
+#include <type_traits>
+
 #include "ftnn_internal.h"
 
 namespace ftnn {
@@ -302,48 +305,69 @@ __global__ __launch_bounds__(256) void k_pack_weights(const float* __restrict__ 
 // bit (t % T) * C + c.  Unused lanes are (sign 0, zero 1) / 0 exactly like the reference's fill, and
 // the existing GEMM kernels run unchanged on Kd = ceil(KH*KW / T) words instead of KH*KW.
 
-// activations: one work-item per (row, dense word); gathers T taps from P (C_pack = 1)
-template <bool TERN>
-__global__ __launch_bounds__(256) void k_dense_rows(const unsigned long long* __restrict__ P, int C, int T,
-                                                    int H, int W, int OH, int OW, int KW, int taps, int Kd,
-                                                    int Kdw, int H_pad, int W_pad, int H_stride,
-                                                    int W_stride, int64_t total,
-                                                    unsigned long long* __restrict__ out) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= total) return;
-    const int64_t r = e / Kdw;
-    const int d = (int)(e - r * Kdw);
-    unsigned long long s = 0ull, z = ~0ull;
-    if (d < Kd) {
-        const int ow = (int)(r % OW);
-        const int64_t t2 = r / OW;
-        const int oh = (int)(t2 % OH);
-        const int64_t n = t2 / OH;
-        const unsigned long long cmask = (1ull << C) - 1ull;
-        for (int j = 0; j < T; j++) {
-            const int tap = d * T + j;
-            if (tap >= taps) break;
-            const int kh = tap / KW, kw = tap - kh * KW;
-            const int ih = oh * H_stride + kh - H_pad, iw = ow * W_stride + kw - W_pad;
-            if (ih >= 0 && ih < H && iw >= 0 && iw < W) {
-                const size_t o = (size_t)n * H * W + (size_t)ih * W + iw;
+// activations, straight from the fp32 input: a workgroup makes four words of 32 rows.  Each half wavefront takes a tap of the 32 pixels at a time,
+// its channels as MC loads in flight (those past C read the last one again), coalesced along the pixels; the tap's lanes meet in LDS, and a
+// thread strings the T taps of one word together.  Bound by latency where layers are small; large ones read each input KH KW / strides
+// times, from the caches.  Device time, us, quantised planes then rows (two launches) / this, 3 x 3, TNN: 11 x 16 x 15 x 16 2.8 + 4.0 / 4.0,
+// 10 x 16 x 48 x 48 3.0 + 4.3 / 5.4, 64 x 16 x 56 x 56 5.8 + 13.4 / 15.6; 5 x 5, 32 x 16 x 64 x 64 4.6 + 14.7 / 18.5.
+// OFF: an element's place, 32 bits where the input is below 4 GiB (the loads then take a scalar base).
+template <bool TERN, int MC, typename OFF>
+__global__ __launch_bounds__(256) void k_dense_rows(const float* __restrict__ x, const float* __restrict__ thr, int C, int T, int H, int W, FastDiv dOHW,
+                                                    FastDiv dOW, FastDiv dKW, int taps, int Kdw, int H_pad, int W_pad, int H_stride, int W_stride,
+                                                    uint32_t M, int groups, int group_step, unsigned long long* __restrict__ out) {
+    extern __shared__ uint32_t masks[];   // [tap of the group][plane][33]
+    const int px = threadIdx.x & 31;
+    const uint32_t r = min(blockIdx.x * 32u + px, M - 1u), n = fastdiv(r, dOHW), pix = r - n * dOHW.d;
+    const int oh = (int)fastdiv(pix, dOW), ow = (int)(pix - (uint32_t)oh * dOW.d);
+    const float t = thr[n];
+    const size_t HW = (size_t)H * W;
+    const OFF image = (OFF)n * (OFF)(C * HW);
+    for (int g = blockIdx.y; g < groups; g += group_step) {
+        const int first = g * 4 * T, count = min(4 * T, taps - first);
+        for (int i = threadIdx.x >> 5; i < count; i += 8) {
+            const uint32_t tap = (uint32_t)(first + i), kh = fastdiv(tap, dKW);
+            const int ih = oh * H_stride + (int)kh - H_pad, iw = ow * W_stride + (int)(tap - kh * dKW.d) - W_pad;
+            const bool inside = (unsigned)ih < (unsigned)H && (unsigned)iw < (unsigned)W;
+            const OFF at = (image + (OFF)(inside ? ih * W + iw : 0)) * (OFF)4;
+            float v[MC];
+#pragma unroll
+            for (int c = 0; c < MC; c++)
+                v[c] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(x + (size_t)min(c, C - 1) * HW) + at);
+            uint32_t neg = 0u, nz = 0u;
+#pragma unroll
+            for (int c = 0; c < MC; c++) {
                 if (TERN) {
-                    const ulonglong2 v = reinterpret_cast<const ulonglong2*>(P)[o];
-                    s |= (v.x & cmask) << (j * C);
-                    z &= ~((~v.y & cmask) << (j * C));
+                    // strict compares, src/tnns/ternarize2row_avx2.c:443-449
+                    neg |= v[c] < -t ? 1u << c : 0u;
+                    nz |= v[c] > t ? 1u << c : 0u;
                 } else {
-                    s |= (P[o] & cmask) << (j * C);
+                    // src/tnns/binarize2row_avx2.c:19-21
+                    neg |= v[c] < t ? 1u << c : 0u;
                 }
             }
+            nz |= neg;
+            const uint32_t live = inside ? 0xffffffffu >> (32 - C) : 0u;
+            masks[i * 66 + px] = neg & live;
+            if (TERN) masks[i * 66 + 33 + px] = nz & live;
         }
-    }
-    if (!TERN && d >= Kd) s = 0ull;
-    if (TERN) {
-        unsigned long long* row = out + (size_t)r * 2 * Kdw;
-        row[p2_pos(d, 0)] = s;
-        row[p2_pos(d, 1)] = z;
-    } else {
-        out[(size_t)r * Kdw + d] = s;
+        __syncthreads();
+        // a word of a pixel and, for ternary lanes, one of its planes per thread
+        const int w = threadIdx.x & 3, p = threadIdx.x >> 2 & 31, plane = threadIdx.x >> 7;
+        const uint32_t row = blockIdx.x * 32u + (uint32_t)p;
+        if (row < M && plane < (TERN ? 2 : 1)) {
+            const uint32_t* m = masks + 33 * plane + p;
+            const int end = min(T, count - w * T);   // taps of this word
+            unsigned long long s = 0ull;
+            for (int j0 = 0; j0 < end; j0 += 8)
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const uint32_t lanes = m[(w * T + min(j0 + j, end - 1)) * 66];
+                    if (j0 + j < end) s |= (unsigned long long)lanes << ((j0 + j) * C);
+                }
+            if (TERN) out[(size_t)row * 2 * Kdw + p2_pos(4 * g + w, plane)] = plane ? ~s : s;
+            else out[(size_t)row * Kdw + 4 * g + w] = s;
+        }
+        __syncthreads();
     }
 }
 
@@ -528,23 +552,38 @@ bool dense_applies(int C, int KH, int KW, int* T_out, int* Kd_out) {
     return round4(taps) >= 2 * round4(Kd);   // at least halves the GEMM work
 }
 
-hipError_t launch_dense_rows(bool ternary, const void* d_p, int N, int C, int H, int W, int H_pad, int W_pad,
+hipError_t launch_dense_rows(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W, int H_pad, int W_pad,
                              int kH, int kW, int H_stride, int W_stride, int64_t* d_out, hipStream_t st) {
     int T, Kd;
     dense_applies(C, kH, kW, &T, &Kd);
     const int OH = out_dim(H, H_pad, kH, H_stride), OW = out_dim(W, W_pad, kW, W_stride);
-    const int Kdw = round4(Kd);
-    const int64_t total = (int64_t)N * OH * OW * Kdw;
-    const unsigned blocks = (unsigned)((total + 255) / 256);
-    const unsigned long long* P = static_cast<const unsigned long long*>(d_p);
+    const int64_t M = (int64_t)N * OH * OW;
+    if (M > 0x7fffffffLL) return hipErrorInvalidValue;
+    // workgroups enough: each makes all the words of its rows, the input then comes through one L2 only (32 x 16 x 64 x 64, 5 x 5, BNN:
+    // 26.5 -> 24.4 us as a layer)
+    const int Kdw = round4(Kd), groups = Kdw / 4, step = M >= 65536 ? 1 : std::min(groups, 65535), taps = kH * kW;
+    const dim3 grid((unsigned)((M + 31) / 32), (unsigned)step);
+    const size_t lds = (size_t)std::min(4 * T, taps) * 66 * 4;   // 67.6 KB for one channel: above 64 KiB
     unsigned long long* out = reinterpret_cast<unsigned long long*>(d_out);
-    if (ternary)
-        hipLaunchKernelGGL((k_dense_rows<true>), dim3(blocks), dim3(256), 0, st, P, C, T, H, W, OH, OW, kW,
-                           kH * kW, Kd, Kdw, H_pad, W_pad, H_stride, W_stride, total, out);
-    else
-        hipLaunchKernelGGL((k_dense_rows<false>), dim3(blocks), dim3(256), 0, st, P, C, T, H, W, OH, OW, kW,
-                           kH * kW, Kd, Kdw, H_pad, W_pad, H_stride, W_stride, total, out);
-    return hipGetLastError();
+    auto go = [&](auto kern) -> hipError_t {
+        if (lds > (64u << 10)) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 256 * 66 * 4);
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, d_x, d_thr, C, T, H, W, make_fastdiv((uint32_t)(OH * OW)), make_fastdiv((uint32_t)OW),
+                           make_fastdiv((uint32_t)kW), taps, Kdw, H_pad, W_pad, H_stride, W_stride, (uint32_t)M, groups, step, out);
+        return hipGetLastError();
+    };
+    auto by_channels = [&](auto tern) -> hipError_t {
+        constexpr bool TERN = decltype(tern)::value;
+        if ((int64_t)N * C * H * W >= (1LL << 30)) return go(k_dense_rows<TERN, 32, size_t>);
+        if (C <= 8) return go(k_dense_rows<TERN, 8, uint32_t>);
+        if (C <= 12) return go(k_dense_rows<TERN, 12, uint32_t>);
+        if (C <= 16) return go(k_dense_rows<TERN, 16, uint32_t>);
+        if (C <= 24) return go(k_dense_rows<TERN, 24, uint32_t>);
+        return go(k_dense_rows<TERN, 32, uint32_t>);
+    };
+    return ternary ? by_channels(std::true_type{}) : by_channels(std::false_type{});
 }
 
 bool dense_f4_applies(int C, int KH, int KW) { return C <= 8 && dense_applies(C, KH, KW, nullptr, nullptr); }

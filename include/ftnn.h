@@ -268,7 +268,8 @@ FTNN_API int ftnn_conv_static(int type, const float *d_x, const float *d_thr, co
  * FTNN_ENGINE_VALU      quantise to bit planes, vector-ALU popcount GEMM with implicit im2row;
  * FTNN_ENGINE_MFMA_F4   quantise to two bits per lane, bring the weights into the same form
  *                       (in d_scratch) and run the fp4 matrix-core layer kernel;
- * FTNN_ENGINE_AUTO      what ftnn_conv does: ftnn_select_conv_engine()'s choice.
+ * FTNN_ENGINE_AUTO      what ftnn_conv does: ftnn_select_conv_engine()'s choice; where that re-packs few channels for the
+ *                       vector ALU, the product of the re-packed rows runs on whichever engine is ahead.
  * ftnn_conv_scratch_bytes() covers every engine.
  */
 FTNN_API int ftnn_select_conv_engine(int type, int N, int C, int H, int W, int KN, int KH, int KW, int H_pad,
