@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "ftnn_internal.h"
+#include "layer_plans.h"
 
 namespace ftnn {
 
@@ -317,7 +318,9 @@ __global__ __launch_bounds__(256) void k_dense_rows(const float* __restrict__ x,
                                                     uint32_t M, int groups, int group_step, unsigned long long* __restrict__ out) {
     extern __shared__ uint32_t masks[];   // [tap of the group][plane][33]
     const int px = threadIdx.x & 31;
-    const uint32_t r = min(blockIdx.x * 32u + px, M - 1u), n = fastdiv(r, dOHW), pix = r - n * dOHW.d;
+    const uint32_t row0 = (blockIdx.z * kDenseBlocksX + blockIdx.x) * 32u;   // below 2^32 (dense_rows_grid)
+    if (row0 >= M) return;                                                   // the whole workgroup
+    const uint32_t r = min(row0 + px, M - 1u), n = fastdiv(r, dOHW), pix = r - n * dOHW.d;
     const int oh = (int)fastdiv(pix, dOW), ow = (int)(pix - (uint32_t)oh * dOW.d);
     const float t = thr[n];
     const size_t HW = (size_t)H * W;
@@ -353,7 +356,7 @@ __global__ __launch_bounds__(256) void k_dense_rows(const float* __restrict__ x,
         __syncthreads();
         // a word of a pixel and, for ternary lanes, one of its planes per thread
         const int w = threadIdx.x & 3, p = threadIdx.x >> 2 & 31, plane = threadIdx.x >> 7;
-        const uint32_t row = blockIdx.x * 32u + (uint32_t)p;
+        const uint32_t row = row0 + (uint32_t)p;
         if (row < M && plane < (TERN ? 2 : 1)) {
             const uint32_t* m = masks + 33 * plane + p;
             const int end = min(T, count - w * T);   // taps of this word
@@ -559,10 +562,9 @@ hipError_t launch_dense_rows(bool ternary, const float* d_x, const float* d_thr,
     const int OH = out_dim(H, H_pad, kH, H_stride), OW = out_dim(W, W_pad, kW, W_stride);
     const int64_t M = (int64_t)N * OH * OW;
     if (M > 0x7fffffffLL) return hipErrorInvalidValue;
-    // workgroups enough: each makes all the words of its rows, the input then comes through one L2 only (32 x 16 x 64 x 64, 5 x 5, BNN:
-    // 26.5 -> 24.4 us as a layer)
-    const int Kdw = round4(Kd), groups = Kdw / 4, step = M >= 65536 ? 1 : std::min(groups, 65535), taps = kH * kW;
-    const dim3 grid((unsigned)((M + 31) / 32), (unsigned)step);
+    const int Kdw = round4(Kd), groups = Kdw / 4, taps = kH * kW;
+    const DenseGrid dg = dense_rows_grid(M, groups);
+    const dim3 grid(dg.x, dg.y, dg.z);
     const size_t lds = (size_t)std::min(4 * T, taps) * 66 * 4;   // 67.6 KB for one channel: above 64 KiB
     unsigned long long* out = reinterpret_cast<unsigned long long*>(d_out);
     auto go = [&](auto kern) -> hipError_t {
@@ -571,7 +573,7 @@ hipError_t launch_dense_rows(bool ternary, const float* d_x, const float* d_thr,
             if (e != hipSuccess) return e;
         }
         hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, d_x, d_thr, C, T, H, W, make_fastdiv((uint32_t)(OH * OW)), make_fastdiv((uint32_t)OW),
-                           make_fastdiv((uint32_t)kW), taps, Kdw, H_pad, W_pad, H_stride, W_stride, (uint32_t)M, groups, step, out);
+                           make_fastdiv((uint32_t)kW), taps, Kdw, H_pad, W_pad, H_stride, W_stride, (uint32_t)M, groups, (int)dg.y, out);
         return hipGetLastError();
     };
     auto by_channels = [&](auto tern) -> hipError_t {

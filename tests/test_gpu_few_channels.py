@@ -66,3 +66,22 @@ def test_input_of_more_than_4_gib(hip):
     got = hip.conv(BNN, x, thr, qw, kn, 3, 3, 1, 1, 0.5).reshape(n, -1)
     want = hip.conv(BNN, x[-3:].contiguous(), thr[-3:].contiguous(), qw, kn, 3, 3, 1, 1, 0.5).reshape(3, -1)
     assert torch.equal(got[-3:], want)
+
+
+@pytest.mark.parametrize("typ,c,kn", [(0, 9, 2), (2, 1, 2), (3, 3, 2), (1, 9, 16)], ids=("tnn9", "btn1", "bnn3", "tbn9"))
+def test_more_than_2_to_29_pixels(hip, typ, c, kn):
+    """more row blocks than a grid's x takes, inputs on both sides of 4 GiB: the first and the last images against batches of their own"""
+    import torch
+    n, h, w = 8193, 256, 256
+    print("case", TYPE_NAMES[typ], n, c, h, w, kn, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn((n, c, h, w), generator=g, device="cuda")
+    wt = weight_is_ternary(typ)
+    qw = hip.pack_weights(torch.randn((kn, c, 3, 3), generator=g, device="cuda"), torch.full((kn,), 0.5 if wt else 0.0, device="cuda"), wt)
+    thr = torch.full((n,), 0.4 if act_is_ternary(typ) else 0.1, device="cuda")
+    got = hip.conv(typ, x, thr, qw, kn, 3, 3, 1, 1, 0.5).reshape(n, -1)
+    for part in (slice(0, 2), slice(n - 2, n)):
+        want = hip.conv(typ, x[part].contiguous(), thr[part].contiguous(), qw, kn, 3, 3, 1, 1, 0.5).reshape(2, -1)
+        assert torch.equal(got[part], want), part
+    del x, got, want
+    torch.cuda.empty_cache()

@@ -1,0 +1,35 @@
+"""The rules by which layers are cut into launches (fastertnn_amd/csrc/layer_plans.h, the code the launchers run): the grid over the dense
+rows of a few-channel layer, up to the most output pixels a call may have.  CPU only."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def _run(tmp_path, program):
+    src, exe = tmp_path / "plans.cpp", tmp_path / "plans"
+    src.write_text('#include <stdio.h>\n#include <stdlib.h>\n#include "layer_plans.h"\nusing namespace ftnn;\n' + program)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fsanitize=undefined", "-fno-sanitize-recover=all", "-I", os.path.join(ROOT, "fastertnn_amd", "csrc"),
+                    str(src), "-o", str(exe)], check=True, timeout=120)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-500:] + r.stderr[-500:]
+    return r.stdout
+
+
+def test_grid_of_dense_rows(tmp_path):
+    """every block of 32 rows once, no dimension beyond a launch's, no row index beyond 32 bits"""
+    out = _run(tmp_path, r"""
+int main() {
+    const long long M[] = {1, 32, 33, 65535, 65536, (1LL << 28) - 31, 1LL << 28, (1LL << 28) + 1, (1LL << 29) - 32, (1LL << 29) - 31, 1LL << 29, 1LL << 30, (1LL << 30) + 1, 0x7fffffffLL};
+    for (long long m : M)
+        for (int groups : {1, 3, 65535, 65536, 1 << 20}) {
+            const DenseGrid g = dense_rows_grid(m, groups);
+            const long long blocks = (m + 31) / 32, last = (long long)(g.z - 1) * kDenseBlocksX + g.x - 1;
+            if (g.x * 256LL >= 1LL << 32 || g.y < 1 || g.y > 65535 || g.z < 1 || g.z > 65535 || (long long)g.y > groups) return printf("%lld: grid\n", m), 1;
+            if (g.x > kDenseBlocksX || (g.z > 1 && g.x != kDenseBlocksX) || last < blocks - 1 || (g.z > 1 && (g.z - 1) * (long long)kDenseBlocksX >= blocks)) return printf("%lld: blocks\n", m), 1;
+            if (last * 32 + 31 >= 1LL << 32) return printf("%lld: rows\n", m), 1;
+        }
+    printf("ok\n");
+}
+""")
+    assert out == "ok\n"
