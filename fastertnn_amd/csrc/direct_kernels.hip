@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "ftnn_internal.h"
+#include "layer_plans.h"
 
 namespace ftnn {
 
@@ -399,6 +400,10 @@ bool launch_direct_f4(int type, const float* d_x, const float* d_thr, const void
                             getenv("FTNN_CONV_SMALL_BELOW") || getenv("FTNN_CONV_TILES_FROM");
     DirectPlan p = {};
     if (off || !direct_plan(type, d_x, cg, C, N, KN, &p)) return false;
+    // One launch reads the input while it stores the result; a result that lies over its input (or the thresholds) needs the input
+    // quantised before the first store.
+    const int64_t y_bytes = 4LL * N * KN * cg.OH * cg.OW;
+    if (ranges_meet(d_y, y_bytes, d_x, 4LL * N * C * cg.H * cg.W) || ranges_meet(d_y, y_bytes, d_thr, 4LL * N)) return false;
     DirectArgs& a = p.a;
     a.x = d_x, a.thr = d_thr, a.Wf = static_cast<const uint4*>(d_wf), a.Y = d_y;
     // BNN: the channel lanes past C are +1 in both operands; padding words are skipped

@@ -8,6 +8,11 @@
 
 namespace ftnn {
 
+inline bool ranges_meet(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + (uintptr_t)b_bytes && y < x + (uintptr_t)a_bytes;
+}
+
 // The grid of k_dense_rows: blocks of 32 rows along x and, past 2^23 of them, z (a grid dimension holds fewer than 2^32 threads), groups
 // of four words along y.  Workgroups enough: each makes all the words of its rows, the input then comes through one L2 only (32 x 16 x 64 x 64,
 // 5 x 5, BNN: 26.5 -> 24.4 us as a layer).

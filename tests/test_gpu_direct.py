@@ -100,3 +100,29 @@ def test_under_capture(hip, oracle):
         want = hip.conv(TNN, x, thr, qw, 70, 3, 3, 1, 1, 0.5, engine=hip.ENGINE_VALU)
         torch.cuda.synchronize()
         assert torch.equal(out, want), rep
+
+
+@pytest.mark.parametrize("typ", range(4), ids=[TYPE_NAMES[t] for t in range(4)])
+@pytest.mark.parametrize("layer", [(8, 128, 28, 28, 128, 3, 3, 1, 1), (4, 64, 16, 16, 64, 1, 1, 0, 1), (8, 512, 1, 1, 512, 1, 1, 0, 1), (8, 40, 1, 1, 300, 1, 1, 0, 1)],
+                         ids=lambda v: "x".join(map(str, v)))
+def test_result_over_its_input(hip, typ, layer):
+    """the result in the place of the input, over a part of it at either end, and over the thresholds: as in a place of its own"""
+    n, c, h, w, kn, kh, kw, pad, stride = layer
+    print("case", TYPE_NAMES[typ], layer, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(9 + typ)
+    wt = weight_is_ternary(typ)
+    values = torch.randn((n, c, h, w), generator=g, device="cuda")
+    thr0 = torch.linspace(0.2, 0.8, n, device="cuda") if act_is_ternary(typ) else torch.linspace(-0.3, 0.3, n, device="cuda")
+    qw = hip.pack_weights(torch.randn((kn, c, kh, kw), generator=g, device="cuda"), torch.full((kn,), 0.5 if wt else 0.0, device="cuda"), wt)
+    prep = hip.prepare_conv_weights(typ, qw, c, kn, kh, kw)
+    want = hip.conv_prepared(typ, values, thr0, prep, kn, kh, kw, pad, stride, 0.5)
+    nx, ny = values.numel(), want.numel()
+    lead = max(nx, ny)
+    for at in (0, nx // 2, -(ny // 2), nx - 1, 1 - ny, None):   # the result's place, from the input's; None: over the thresholds
+        buf = torch.zeros(nx + 2 * lead + n, device="cuda")
+        x, thr = buf[lead:lead + nx].view(values.shape), buf[-n:]
+        x.copy_(values), thr.copy_(thr0)
+        y0 = lead + at if at is not None else buf.numel() - ny
+        out = buf[y0:y0 + ny].view(want.shape)
+        hip.conv_prepared(typ, x, thr, prep, kn, kh, kw, pad, stride, 0.5, out=out)
+        assert torch.equal(out, want), at

@@ -1,5 +1,6 @@
 """The rules by which layers are cut into launches (fastertnn_amd/csrc/layer_plans.h, the code the launchers run): the grid over the dense
-rows of a few-channel layer, up to the most output pixels a call may have.  CPU only."""
+rows of a few-channel layer, up to the most output pixels a call may have, and the comparison of a result's place with its input's.
+CPU only."""
 import os
 import subprocess
 
@@ -29,6 +30,20 @@ int main() {
             if (g.x > kDenseBlocksX || (g.z > 1 && g.x != kDenseBlocksX) || last < blocks - 1 || (g.z > 1 && (g.z - 1) * (long long)kDenseBlocksX >= blocks)) return printf("%lld: blocks\n", m), 1;
             if (last * 32 + 31 >= 1LL << 32) return printf("%lld: rows\n", m), 1;
         }
+    printf("ok\n");
+}
+""")
+    assert out == "ok\n"
+
+
+def test_ranges_that_meet(tmp_path):
+    out = _run(tmp_path, r"""
+int main() {
+    const char* p = (const char*)0x7f0000001000ull;
+    struct { long a, an, b, bn; bool meet; } c[] = {{0, 64, 64, 64, 0}, {64, 64, 0, 64, 0}, {0, 64, 63, 1, 1}, {63, 1, 0, 64, 1}, {0, 64, 0, 64, 1}, {16, 4, 0, 64, 1},
+                                                    {0, 64, 16, 4, 1}, {0, 1L << 40, (1L << 40) - 4, 4, 1}, {0, 1L << 40, 1L << 40, 4, 0}};
+    for (auto& v : c)
+        if (ranges_meet(p + v.a, v.an, p + v.b, v.bn) != v.meet) return printf("%ld %ld\n", v.a, v.b), 1;
     printf("ok\n");
 }
 """)
