@@ -43,3 +43,29 @@ def test_product_forms(hip, typ, shape):
             hip.mm_engine(hip.ENGINE_MFMA_F4, typ, a, b, n, oh, ow, kn, kw, -0.25, ku, out=out)
         assert torch.equal(out[:m * kn].view(torch.int32), want.view(torch.int32)), kept
         assert bool(torch.isnan(out[m * kn:]).all())
+
+
+@pytest.mark.parametrize("typ", range(4), ids=[TYPE_NAMES[t] for t in range(4)])
+@pytest.mark.parametrize("shape", [(3328, 1, 1, 3328, 16), (4, 29, 29, 3200, 16)], ids=lambda v: "x".join(map(str, v)))
+def test_result_over_an_operand(hip, typ, shape):
+    """products of 160 tiles of 256 x 256 and more of short rows, with scratch, the result from an operand's first and last word on: as in a place of its own"""
+    n, oh, ow, kn, kw = shape
+    print("case", TYPE_NAMES[typ], shape, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(8 + typ)
+    at, wt = act_is_ternary(typ), weight_is_ternary(typ)
+    words = lambda rows, tern: torch.randint(-2**63, 2**63 - 1, (rows * kw * (2 if tern else 1),), generator=g, device="cuda", dtype=torch.int64)
+    m = n * oh * ow
+    a, b = words(m, at), words(kn, wt)
+    scratch = torch.empty(hip.mm_scratch_bytes(hip.ENGINE_AUTO, typ, n, oh, ow, kn, kw), dtype=torch.uint8, device="cuda")
+    want = hip.mm_engine(hip.ENGINE_VALU, typ, a, b, n, oh, ow, kn, kw, 0.5, 64 * kw - 9)
+    for engine in (hip.ENGINE_AUTO, hip.ENGINE_MFMA_F4):
+        for which in (0, 1):
+            for at_end in (False, True):
+                own, other = (a, b) if which == 0 else (b, a)
+                buf = torch.empty(own.numel() + (m * kn + 1) // 2, dtype=torch.int64, device="cuda")
+                held = buf[:own.numel()]
+                held.copy_(own)
+                start = 2 * (own.numel() - 1) if at_end else 0
+                out = buf.view(torch.float32)[start:start + m * kn].view(n, kn, oh, ow)
+                hip.mm_engine(engine, typ, *((held, other) if which == 0 else (other, held)), n, oh, ow, kn, kw, 0.5, 64 * kw - 9, out=out, scratch=scratch)
+                assert torch.equal(out, want), (engine, which, at_end)
