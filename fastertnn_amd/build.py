@@ -1,6 +1,8 @@
 """Build libftnn_hip.so in-tree with hipcc for gfx950 (cross-compiles without a GPU), and the Python module over it."""
 import importlib.machinery
 import os
+import shlex
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -48,20 +50,42 @@ BINDING = os.path.join(HERE, "_call" + importlib.machinery.EXTENSION_SUFFIXES[0]
 
 
 def binding_command():
-    """the compiler call that makes _call from csrc/py_call.cpp (host code only)"""
-    import torch
+    """the compiler call that makes _call from csrc/py_call.cpp (host code only), or what it needs that is not there"""
+    try:
+        import torch
+    except ImportError as e:
+        return None, str(e)
     root = os.path.dirname(torch.__file__)
     rocm = os.path.dirname(os.path.dirname(HIPCC))
-    inc = [sysconfig.get_paths()["include"], os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
-           os.path.join(rocm, "include")]
-    return ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-             "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI] + ["-isystem" + d for d in inc] +
-            [os.path.join(CSRC, "py_call.cpp"), "-o", BINDING, "-L" + HERE, "-lftnn_hip", "-Wl,-rpath,$ORIGIN", "-L" + os.path.join(root, "lib"),
-             "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"])
+    cxx = shlex.split(os.environ.get("CXX", "g++"))
+    include = sysconfig.get_paths()["include"]
+    for what in (os.path.join(include, "Python.h"), os.path.join(root, "include", "c10", "hip", "HIPStream.h"), os.path.join(root, "lib", "libc10_hip.so")):
+        if not os.path.exists(what):
+            return None, "no " + what
+    if not shutil.which(cxx[0]):
+        return None, "no compiler " + cxx[0]
+    inc = [include, os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"), os.path.join(rocm, "include")]
+    return cxx + ["-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                  "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, '-DFTNN_TORCH="%s"' % torch.__version__] + ["-isystem" + d for d in inc] + [
+        os.path.join(CSRC, "py_call.cpp"), "-o", BINDING, "-L" + HERE, "-lftnn_hip", "-Wl,-rpath,$ORIGIN", "-L" + os.path.join(root, "lib"),
+        "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"], ""
+
+
+def build_binding():
+    """Compile the Python module; returns its path, or None where torch, Python's headers or a host compiler are missing (lib.py then
+    makes every call through ctypes).  The library itself needs none of them."""
+    cmd, missing = binding_command()
+    if os.path.exists(BINDING):
+        os.remove(BINDING)   # none is better than one of another library
+    if cmd is None:
+        print("%s is not built: %s" % (os.path.basename(BINDING), missing), file=sys.stderr)
+        return None
+    subprocess.run(cmd, check=True)
+    return BINDING
 
 
 def build_library(verbose=False):
-    """Compile every HIP source and link the shared library, then the Python module; returns the library's path."""
+    """Compile every HIP source and link the shared library, then the Python module where that can be; returns the library's path."""
     objs = []
     procs = []
     for src in SOURCES:
@@ -88,7 +112,7 @@ def build_library(verbose=False):
             print(out)
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", LIB]
     subprocess.run(cmd, check=True)
-    subprocess.run(binding_command(), check=True)
+    build_binding()
     return LIB
 
 

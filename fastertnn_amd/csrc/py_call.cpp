@@ -167,4 +167,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_call", "ftnn device calls without
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__call(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__call(void) {
+    PyObject* const m = PyModule_Create(&module);
+    // the torch whose tensors it reads: another one's may lie otherwise in memory
+    if (m && PyModule_AddStringConstant(m, "torch_version", FTNN_TORCH) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

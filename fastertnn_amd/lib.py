@@ -9,6 +9,7 @@ last array over it, as a C caller would free it.
 """
 import ctypes as C
 import os
+import warnings
 
 import numpy as np
 
@@ -122,7 +123,7 @@ def pack_scratch_bytes(n, c, h, w, ternary):
 # the first device call (importing it inside every wrapper costs 0.3 us), and the stream is asked for as the bare handle
 # (0.1 us; the Stream object of torch.cuda.current_stream() costs 2.7).  The calls that a program makes once per layer or
 # product go through `_call` (csrc/py_call.cpp), which takes plain arguments and answers None to anything else; what follows
-# in their wrappers is then the way through ctypes.
+# in their wrappers is then the way through ctypes, the only one where there is no such module for this torch.
 torch = None
 _call = None
 
@@ -137,8 +138,21 @@ def _native():
     global _call
     _torch()
     if _call is None:
-        from . import _call   # links against torch, which has to be loaded first
+        try:
+            from . import _call   # links against torch, which has to be loaded first
+            if _call.torch_version != torch.__version__:
+                raise ImportError("built for torch %s" % _call.torch_version)
+        except ImportError as e:
+            warnings.warn("fastertnn_amd._call cannot be used (%s): every call goes through ctypes, 2 us of host time slower" % e, RuntimeWarning)
+            _call = _ThroughCtypes()
     return _call
+
+
+class _ThroughCtypes:
+    """in the place of the module: leaves every call to what follows in its wrapper"""
+
+    def __getattr__(self, name):
+        return lambda *args: None
 
 
 def _stream():
