@@ -968,7 +968,7 @@ int conv_valu(int type, const float* d_x, const float* d_thr, const int64_t* d_q
         int64_t* d_rows = reinterpret_cast<int64_t*>(base + p_bytes);
         const int64_t* d_wd = d_qw;   // prepared weights are the re-packed rows already
         e = launch_dense_rows(act_ternary, d_x, d_thr, N, C, H, W, H_pad, W_pad, KH, KW, H_stride, W_stride,
-                              d_rows, st);
+                              d_scratch, d_rows, st);
         if (e != hipSuccess) return hip_fail(e, "dense rows launch");
         if (!weights_prepared) {
             int64_t* d_tmp = reinterpret_cast<int64_t*>(base + p_bytes + rows_bytes);

@@ -208,7 +208,7 @@ hipError_t launch_quantize_rows(bool ternary, const float* d_x, const float* d_t
 // dense re-packing of both operands for layers with C <= 32 (several taps per 64-lane word), the activations from fp32
 bool dense_applies(int C, int KH, int KW, int* T_out, int* Kd_out);
 hipError_t launch_dense_rows(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W, int H_pad, int W_pad,
-                             int kH, int kW, int H_stride, int W_stride, int64_t* d_out, hipStream_t st);
+                             int kH, int kW, int H_stride, int W_stride, void* d_p /* room for launch_quantize's planes */, int64_t* d_out, hipStream_t st);
 hipError_t launch_dense_weights(bool ternary, const int64_t* d_qw, int KN, int C, int kH, int kW,
                                 int64_t* d_out, hipStream_t st);
 

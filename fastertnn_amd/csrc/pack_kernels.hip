@@ -309,10 +309,10 @@ __global__ __launch_bounds__(256) void k_pack_weights(const float* __restrict__ 
 // activations, straight from the fp32 input: a workgroup makes four words of 32 rows.  Each half wavefront takes a tap of the 32 pixels at a time,
 // its channels as MC loads in flight (those past C read the last one again), coalesced along the pixels; the tap's lanes meet in LDS, and a
 // thread strings the T taps of one word together.  Bound by latency where layers are small; large ones read each input KH KW / strides
-// times, from the caches.  Device time, us, quantised planes then rows (two launches) / this, 3 x 3, TNN: 11 x 16 x 15 x 16 2.8 + 4.0 / 4.0,
+// times, from the caches (dense_rows_from_input).  Device time, us, quantised planes then rows (two launches) / this, 3 x 3, TNN: 11 x 16 x 15 x 16 2.8 + 4.0 / 4.0,
 // 10 x 16 x 48 x 48 3.0 + 4.3 / 5.4, 64 x 16 x 56 x 56 5.8 + 13.4 / 15.6; 5 x 5, 32 x 16 x 64 x 64 4.6 + 14.7 / 18.5.
-// OFF: an element's place, 32 bits where the input is below 4 GiB (the loads then take a scalar base).
-template <bool TERN, int MC, typename OFF>
+// The input is below 4 GiB: an element's place takes 32 bits, and the loads a scalar base.
+template <bool TERN, int MC>
 __global__ __launch_bounds__(256) void k_dense_rows(const float* __restrict__ x, const float* __restrict__ thr, int C, int T, int H, int W, FastDiv dOHW,
                                                     FastDiv dOW, FastDiv dKW, int taps, int Kdw, int H_pad, int W_pad, int H_stride, int W_stride,
                                                     uint32_t M, int groups, int group_step, unsigned long long* __restrict__ out) {
@@ -324,14 +324,14 @@ __global__ __launch_bounds__(256) void k_dense_rows(const float* __restrict__ x,
     const int oh = (int)fastdiv(pix, dOW), ow = (int)(pix - (uint32_t)oh * dOW.d);
     const float t = thr[n];
     const size_t HW = (size_t)H * W;
-    const OFF image = (OFF)n * (OFF)(C * HW);
+    const uint32_t image = n * (uint32_t)(C * HW);
     for (int g = blockIdx.y; g < groups; g += group_step) {
         const int first = g * 4 * T, count = min(4 * T, taps - first);
         for (int i = threadIdx.x >> 5; i < count; i += 8) {
             const uint32_t tap = (uint32_t)(first + i), kh = fastdiv(tap, dKW);
             const int ih = oh * H_stride + (int)kh - H_pad, iw = ow * W_stride + (int)(tap - kh * dKW.d) - W_pad;
             const bool inside = (unsigned)ih < (unsigned)H && (unsigned)iw < (unsigned)W;
-            const OFF at = (image + (OFF)(inside ? ih * W + iw : 0)) * (OFF)4;
+            const uint32_t at = (image + (uint32_t)(inside ? ih * W + iw : 0)) * 4u;
             float v[MC];
 #pragma unroll
             for (int c = 0; c < MC; c++)
@@ -371,6 +371,49 @@ __global__ __launch_bounds__(256) void k_dense_rows(const float* __restrict__ x,
             else out[(size_t)row * Kdw + 4 * g + w] = s;
         }
         __syncthreads();
+    }
+}
+
+// The same rows from the input's bit planes (launch_quantize's, C_pack = 1), a dense word of a row per thread: a tap is one load of 8 or 16
+// bytes instead of C of 4.
+template <bool TERN>
+__global__ __launch_bounds__(256) void k_dense_rows_planes(const unsigned long long* __restrict__ P, int C, int T, int H, int W, int OH, int OW, int KW,
+                                                           int taps, int Kd, int Kdw, int H_pad, int W_pad, int H_stride, int W_stride, int64_t total,
+                                                           unsigned long long* __restrict__ out) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= total) return;
+    const int64_t r = e / Kdw;
+    const int d = (int)(e - r * Kdw);
+    unsigned long long s = 0ull, z = ~0ull;
+    if (d < Kd) {
+        const int ow = (int)(r % OW);
+        const int64_t t2 = r / OW;
+        const int oh = (int)(t2 % OH);
+        const int64_t n = t2 / OH;
+        const unsigned long long cmask = (1ull << C) - 1ull;
+        for (int j = 0; j < T; j++) {
+            const int tap = d * T + j;
+            if (tap >= taps) break;
+            const int kh = tap / KW, kw = tap - kh * KW;
+            const int ih = oh * H_stride + kh - H_pad, iw = ow * W_stride + kw - W_pad;
+            if (ih >= 0 && ih < H && iw >= 0 && iw < W) {
+                const size_t o = (size_t)n * H * W + (size_t)ih * W + iw;
+                if (TERN) {
+                    const ulonglong2 v = reinterpret_cast<const ulonglong2*>(P)[o];
+                    s |= (v.x & cmask) << (j * C);
+                    z &= ~((~v.y & cmask) << (j * C));
+                } else {
+                    s |= (P[o] & cmask) << (j * C);
+                }
+            }
+        }
+    }
+    if (TERN) {
+        unsigned long long* row = out + (size_t)r * 2 * Kdw;
+        row[p2_pos(d, 0)] = s;
+        row[p2_pos(d, 1)] = z;
+    } else {
+        out[(size_t)r * Kdw + d] = s;
     }
 }
 
@@ -556,13 +599,24 @@ bool dense_applies(int C, int KH, int KW, int* T_out, int* Kd_out) {
 }
 
 hipError_t launch_dense_rows(bool ternary, const float* d_x, const float* d_thr, int N, int C, int H, int W, int H_pad, int W_pad,
-                             int kH, int kW, int H_stride, int W_stride, int64_t* d_out, hipStream_t st) {
+                             int kH, int kW, int H_stride, int W_stride, void* d_p, int64_t* d_out, hipStream_t st) {
     int T, Kd;
     dense_applies(C, kH, kW, &T, &Kd);
     const int OH = out_dim(H, H_pad, kH, H_stride), OW = out_dim(W, W_pad, kW, W_stride);
     const int64_t M = (int64_t)N * OH * OW;
     if (M > 0x7fffffffLL) return hipErrorInvalidValue;
     const int Kdw = round4(Kd), groups = Kdw / 4, taps = kH * kW;
+    if (!dense_rows_from_input(ternary, (int64_t)N * H * W, C, M, taps, W_stride)) {
+        if (M * Kdw > 0xffffff00LL) return hipErrorInvalidValue;   // threads of a grid dimension
+        const hipError_t e = launch_quantize(ternary, d_x, d_thr, N, C, H, W, d_p, st);
+        if (e != hipSuccess) return e;
+        auto planes = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)((M * Kdw + 255) / 256)), dim3(256), 0, st, static_cast<const unsigned long long*>(d_p), C, T, H, W, OH, OW, kW,
+                               taps, Kd, Kdw, H_pad, W_pad, H_stride, W_stride, M * Kdw, reinterpret_cast<unsigned long long*>(d_out));
+            return hipGetLastError();
+        };
+        return ternary ? planes(k_dense_rows_planes<true>) : planes(k_dense_rows_planes<false>);
+    }
     const DenseGrid dg = dense_rows_grid(M, groups);
     const dim3 grid(dg.x, dg.y, dg.z);
     const size_t lds = (size_t)std::min(4 * T, taps) * 66 * 4;   // 67.6 KB for one channel: above 64 KiB
@@ -578,12 +632,13 @@ hipError_t launch_dense_rows(bool ternary, const float* d_x, const float* d_thr,
     };
     auto by_channels = [&](auto tern) -> hipError_t {
         constexpr bool TERN = decltype(tern)::value;
-        if ((int64_t)N * C * H * W >= (1LL << 30)) return go(k_dense_rows<TERN, 32, size_t>);
-        if (C <= 8) return go(k_dense_rows<TERN, 8, uint32_t>);
-        if (C <= 12) return go(k_dense_rows<TERN, 12, uint32_t>);
-        if (C <= 16) return go(k_dense_rows<TERN, 16, uint32_t>);
-        if (C <= 24) return go(k_dense_rows<TERN, 24, uint32_t>);
-        return go(k_dense_rows<TERN, 32, uint32_t>);
+        switch (dense_loads(C)) {
+            case 8: return go(k_dense_rows<TERN, 8>);
+            case 12: return go(k_dense_rows<TERN, 12>);
+            case 16: return go(k_dense_rows<TERN, 16>);
+            case 24: return go(k_dense_rows<TERN, 24>);
+            default: return go(k_dense_rows<TERN, 32>);
+        }
     };
     return ternary ? by_channels(std::true_type{}) : by_channels(std::false_type{});
 }

@@ -17,6 +17,10 @@ LAYERS = [(1, 9, 5, 7, 3, 3, 3, 1, 1), (4, 12, 13, 13, 58, 1, 5, 0, 1), (3, 16, 
 # the explicit vector-ALU engine takes fewer channels too; one channel fills four words with 256 taps
 FEW = [(2, 1, 40, 50, 9, 17, 16, 8, 1), (2, 3, 20, 20, 33, 7, 7, 3, 2), (1, 8, 9, 9, 20, 3, 3, 1, 1), (1, 1, 30, 30, 4, 5, 5, 0, 1)]
 
+# from the input's bit planes (dense_rows_from_input says so of each, tests/test_layer_plans.py): pixels by the hundred thousand or windows that share most of their taps
+PLANES = [(26, 17, 63, 63, 8, 11, 11, 0, 2), (5, 19, 41, 47, 10, 13, 13, 0, 1), (9, 24, 60, 61, 20, 9, 9, 4, 2), (13, 32, 90, 91, 33, 4, 4, 2, 2), (3, 9, 99, 120, 17, 17, 17, 8, 3)]
+FEW_PLANES = [(4, 3, 120, 121, 9, 11, 11, 5, 2), (1, 1, 300, 300, 4, 17, 17, 0, 2)]
+
 
 def _check(hip, oracle, typ, layer, engines):
     import torch
@@ -85,3 +89,9 @@ def test_more_than_2_to_29_pixels(hip, typ, c, kn):
         assert torch.equal(got[part], want), part
     del x, got, want
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("typ", ALL_TYPES, ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("layer", PLANES + FEW_PLANES, ids=lambda v: "x".join(map(str, v)))
+def test_from_bit_planes(hip, oracle, typ, layer):
+    _check(hip, oracle, typ, layer, (None, hip.ENGINE_AUTO, hip.ENGINE_VALU) if layer in PLANES else (hip.ENGINE_VALU,))

@@ -1,5 +1,5 @@
 """The rules by which layers are cut into launches (fastertnn_amd/csrc/layer_plans.h, the code the launchers run): the grid over the dense
-rows of a few-channel layer, up to the most output pixels a call may have, and the comparison of a result's place with its input's.
+rows of a few-channel layer, up to the most output pixels a call may have, which form makes them, and the comparison of a result's place with its input's.
 CPU only."""
 import os
 import subprocess
@@ -44,6 +44,28 @@ int main() {
                                                     {0, 64, 16, 4, 1}, {0, 1L << 40, (1L << 40) - 4, 4, 1}, {0, 1L << 40, 1L << 40, 4, 0}};
     for (auto& v : c)
         if (ranges_meet(p + v.a, v.an, p + v.b, v.bn) != v.meet) return printf("%ld %ld\n", v.a, v.b), 1;
+    printf("ok\n");
+}
+""")
+    assert out == "ok\n"
+
+
+def test_form_of_dense_rows(tmp_path):
+    """sides of the line that were measured more than a tenth apart, and inputs that 32-bit offsets do not reach"""
+    from tests.test_gpu_few_channels import FEW_PLANES, PLANES
+    planes = ""
+    for n, c, h, w, kn, kh, kw, pad, stride in PLANES + FEW_PLANES:
+        oh, ow = (h + 2 * pad - kh) // stride + 1, (w + 2 * pad - kw) // stride + 1
+        planes += "{0, %d, %d, %d, %d, %d, %d, 0}, {1, %d, %d, %d, %d, %d, %d, 0}, " % (2 * (n, c, h * w, oh * ow, kh * kw, stride))
+    out = _run(tmp_path, r"""
+int main() {
+    struct { bool tern; long n; int c, hw, oh, taps, stride; bool input; } v[] = {
+        {0, 22, 9, 209 * 209, 207 * 207, 9, 1, 1}, {1, 52, 11, 45 * 45, 53 * 45, 9, 1, 1}, {1, 11, 16, 15 * 16, 15 * 16, 9, 1, 1}, {1, 64, 16, 56 * 56, 56 * 56, 9, 1, 1},
+        {0, 61, 19, 186 * 186, 89 * 89, 81, 2, 0}, {1, 26, 17, 70 * 70, 30 * 30, 121, 2, 0}, {0, 60, 14, 223 * 18, 207 * 2, 289, 1, 0}, {1, 42, 12, 206 * 206, 196 * 196, 121, 1, 0},
+        {0, 26, 17, 63 * 63, 27 * 27, 121, 2, 0}, {1, 36, 16, 211 * 48, 211 * 48, 25, 1, 0},
+        {1, 16383, 16, 64 * 64, 1, 9, 64, 1}, {1, 16384, 16, 64 * 64, 1, 9, 64, 0}, """ + planes + r"""};
+    for (auto& l : v)
+        if (dense_rows_from_input(l.tern, l.n * l.hw, l.c, l.n * l.oh, l.taps, l.stride) != l.input) return printf("%ld x %d, %d taps\n", l.n, l.c, l.taps), 1;
     printf("ok\n");
 }
 """)
