@@ -21,6 +21,7 @@
 #include "../../include/ftnn.h"
 #include "ftnn_internal.h"
 #include "host_hash.h"
+#include "layer_plans.h"
 
 static bool valu_ahead_of_rows(int type, int64_t M, bool nchw, int KN, int Kw);
 
@@ -978,10 +979,9 @@ int conv_valu(int type, const float* d_x, const float* d_thr, const int64_t* d_q
         }
         // A product of packed rows, on the matrix cores where the caller leaves the engine open and k_rows is ahead: as a layer, us, vector ALU /
         // k_rows: 64 x 16 x 56 x 56 -> 64, 3 x 3, TNN 42 / 29, 7 x 11 x 86 x 86 -> 136, 7 x 7, BTN 54 / 27, 10 x 16 x 48 x 48 -> 256 BNN 17.4 / 11.9.
-        // Few kernels on one group of words leave its tiles mostly empty (256 x 16 x 16 x 16 -> 8 BTN 10.9 / 12.5).
         const int64_t M = (int64_t)N * OH * OW;
         const int Kw = round4(Kd);
-        if (any_engine && qo.mode == 0 && (KN >= 16 || Kw > 4) && mm_rows_within_limits(M, KN, Kw) &&
+        if (any_engine && qo.mode == 0 && !few_kernels(M, KN, Kw) && mm_rows_within_limits(M, KN, Kw) &&
             !valu_ahead_of_rows(type, M, OH * OW > 1, KN, Kw))
             e = launch_mm_rows(type, d_rows, d_wd, M, OH * OW, KN, Kw, C * KH * KW, prelu_alpha, d_y, st);
         else

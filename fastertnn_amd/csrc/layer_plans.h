@@ -46,4 +46,10 @@ inline bool dense_rows_from_input(bool ternary, int64_t pixels /* of the input *
     return read * dense_loads(C) * (W_stride > 1 ? 0.473 : 0.223) < 0.9 + 15.5 * in + read * (ternary ? 1.49 : 1.94);
 }
 
+// Few kernels leave the tiles of k_rows mostly empty, so that such a layer's dense rows stay on the vector ALU: up to 15 on one group of words
+// (256 x 16 x 16 x 16 -> 8 BTN 10.9 us on the vector ALU / 12.5), up to eight on some more (7 x 14 x 94 x 94 -> 8, 5 x 5, TBN 17.4 / 19.9; 57024 pixels -> 3,
+// 28 words, TBN 32.6 / 37.6), but 212064 -> 3, 32 words, BTN 118 / 70 and 10000 -> 10, 60 words, TNN 24.6 / 19.3.  Of 400 layers of 1 to 24 kernels 4 are 6 to
+// 9 % slower than on the vector ALU (15 by the first line alone).
+inline bool few_kernels(int64_t M, int KN, int Kw) { return (KN < 16 && Kw == 4) || (KN <= 8 && Kw <= 44 && M <= 100000); }
+
 }  // namespace ftnn

@@ -70,3 +70,17 @@ int main() {
 }
 """)
     assert out == "ok\n"
+
+
+def test_few_kernels(tmp_path):
+    """layers of few kernels that measured slower off the vector ALU, and neighbours that measured faster"""
+    out = _run(tmp_path, r"""
+int main() {
+    struct { long m; int kn, kw; bool valu; } v[] = {{65536, 8, 4, 1}, {61852, 8, 8, 1}, {57024, 3, 28, 1}, {89787, 1, 20, 1}, {28611, 6, 36, 1}, {56295, 1, 44, 1},
+                                                    {212064, 3, 32, 0}, {119070, 3, 44, 0}, {13482, 6, 60, 0}, {10000, 10, 60, 0}, {153164, 12, 12, 0}, {65536, 16, 4, 0}};
+    for (auto& l : v)
+        if (few_kernels(l.m, l.kn, l.kw) != l.valu) return printf("%ld %d %d\n", l.m, l.kn, l.kw), 1;
+    printf("ok\n");
+}
+""")
+    assert out == "ok\n"
