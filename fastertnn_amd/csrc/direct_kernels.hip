@@ -21,10 +21,7 @@
 // 8 x 128 x 28 x 28 -> 128, 3 x 3 6.6 / 6.2; 1 x 64 x 16 x 16 -> 256, 3 x 3 5.1 / 4.1; 3 x 64 x 39 x 39 -> 256, 1 x 1 6.3 / 5.1; 8 x 512 -> 1000
 // fully connected 4.9 / 4.2; 1 x 7660 -> 413 6.2 / 4.8: 0.87 in the mean of 110 layers.  Queued from Python 9.7 / 7.2 with 3.5 us of
 // arguments each.
-#include <algorithm>
-
 #include "ftnn_internal.h"
-#include "layer_plans.h"
 
 namespace ftnn {
 
@@ -34,10 +31,8 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
-constexpr int kLgW = 3, kWaves = 1 << kLgW, kThreads = 64 * kWaves;   // (four wavefronts: slower from two pieces of input on)
+constexpr int kLgW = kDirectLgWaves, kThreads = 64 << kLgW;
 constexpr int G = 4;   // pairs of K words in flight
-constexpr int kLdsBytes = 64 << 10;
-constexpr uint32_t kNowhere = 0x80000000u;   // an offset that, with a few planes added to it, lies beyond every image taken here
 
 struct DirectArgs {
     const float* x;
@@ -50,7 +45,7 @@ struct DirectArgs {
     int rstep, cstep;         // input rows / columns between neighbouring region pixels
     int lrow, lcol;           // region rows / columns between neighbouring output pixels
     int H_stride, W_stride, H_pad, W_pad, KW;
-    int lgTW, tiles_x, lgS;
+    int lgTW, lgS;
     int OHt, OWt;             // rows and columns of outputs that a tile's region serves
     int vec4;
     FastDiv dRP, dRW, dTX, dTI, dCP, dKW;
@@ -196,7 +191,7 @@ __global__ __launch_bounds__(kThreads) void k_direct_f4(DirectArgs a) {
             const uint32_t pl = q >> 2, j = q & 3u;   // dword j of the record: channels c0 + 8 q + i
             f.c0 = (int)(pl * 64u + 32u * (j & 1u) + 4u * (j >> 1));
             f.at = (pl * (uint32_t)a.RP + px) * 4u + j;
-            const uint32_t o = f.inside ? (uint32_t)f.c0 * plane + (uint32_t)(ih * a.W + iw) * 4u : kNowhere;
+            const uint32_t o = f.inside ? (uint32_t)f.c0 * plane + (uint32_t)(ih * a.W + iw) * 4u : kDirectNowhere;
 #pragma unroll
             for (int e = 0; e < 16; e++)
                 f.v[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)(o + (uint32_t)(8 * (e >> 2) + (e & 3)) * plane), 0, 0));
@@ -313,82 +308,20 @@ __global__ __launch_bounds__(kThreads) void k_direct_f4(DirectArgs a) {
     }
 }
 
-// Which layers run here, and how.  A workgroup's time grows with the pieces of input it fetches (512 dwords of records of 16 values at a
-// time; 2048 quads for a fully connected one), and a second workgroup per compute unit costs as much as the first.  Lines from 230
-// layers, both forms in a graph, us (two launches / here): 21 x 128 x 9 x 21 -> 256, 3 x 3 6.4 / 6.9 (300 workgroups), 20 x 128 x 20 x 20 ->
-// 128, 3 x 3 6.8 / 8.5 (300); two pieces of input with a window 19 x 256 x 10 x 10 -> 128, 3 x 3 stride 2 5.7 / 5.9, without one
-// 14 x 512 x 12 x 12 -> 64 5.4 / 4.8; all eight wavefronts on kernels of their own and nearly a whole piece 2 x 128 x 53 x 53 -> 256, 3 x 3
-// 7.7 / 8.2, half a piece 24 x 64 x 14 x 14 -> 256, 3 x 3 7.0 / 6.2; fully connected 9 x 2081 -> 3584 (4752 quads) 5.1 / 5.8,
-// 15 x 812 -> 6673 (3120) 5.0 / 5.3, 8 x 1337 -> 1121 (2688) 5.1 / 4.8.
-struct DirectPlan {
-    DirectArgs a;
-    bool fc;
-    unsigned wgs;
-    int64_t lds_bytes;
-};
-bool direct_plan(int type, const float* d_x, const ConvGeom& cg, int C, int N, int KN, DirectPlan* out) {
-    const int KB = (KN + 31) / 32, KH = cg.K / (cg.CP * cg.KW);
-    const int64_t M = (int64_t)N * cg.OH * cg.OW;
-    const bool fc = out->fc = cg.H == 1 && cg.W == 1 && KH == 1 && cg.KW == 1 && cg.H_pad == 0 && cg.W_pad == 0;
-    const int most = fc ? 400 : 256;   // workgroups
-    if ((M + 31) / 32 * ((KB + kWaves - 1) / kWaves) > most) return false;
-    if (((int64_t)cg.CP * 64 + 64) * cg.H * cg.W * 4 > kNowhere) return false;   // offsets within an image
-    DirectArgs& a = out->a;
-    a.N = N, a.C = C, a.CP = cg.CP, a.H = cg.H, a.W = cg.W, a.KN = KN, a.OH = cg.OH, a.OW = cg.OW;
+// the kernel's arguments for a plan, but for the pointers and the type's constants
+DirectArgs direct_args(const DirectPlan& p, const ConvGeom& cg, int C, int N, int KN) {
+    DirectArgs a = {};
+    a.N = N, a.C = C, a.CP = cg.CP, a.H = p.H, a.W = p.W, a.KN = KN, a.OH = p.OH, a.OW = p.OW;
     a.K = cg.K, a.NP = (cg.K + 1) / 2, a.KP = round4(cg.K) / 2;
     a.H_stride = cg.H_stride, a.W_stride = cg.W_stride, a.H_pad = cg.H_pad, a.W_pad = cg.W_pad, a.KW = cg.KW;
     a.dCP = cg.dCP, a.dKW = cg.dKW;
-    int64_t tiles, U;   // U: pieces of work in fetching a tile's input
-    if (fc) {
-        a.RP = a.RW = 32;
-        a.dRP = make_fastdiv((uint32_t)cg.CP * 16u);
-        a.vec4 = C % 4 == 0 && reinterpret_cast<uintptr_t>(d_x) % 16 == 0;
-        tiles = (N + 31) / 32;
-        U = (int64_t)std::min(32, N) * cg.CP * 16;
-        if (U > 3072) return false;
-        // binary weights take half the bytes as rows: 4 x 2312 -> 9837 (5.8 MB of records) 6.1 / 6.0, 3 x 2750 -> 12499 (8.6) 6.0 / 5.4 with the
-        // weights within the Infinity Cache, which larger ones need not be
-        if ((type == kTBN || type == kBNN) && (int64_t)KN * cg.CP * 16 > (8 << 20)) return false;
-    } else {
-        if (KH == 1 && cg.KW == 1 && cg.H_pad == 0 && cg.W_pad == 0 && cg.H_stride == 1 && cg.W_stride == 1) {
-            a.W = a.OW = cg.H * cg.W;
-            a.H = a.OH = 1;
-        }
-        a.rstep = KH == 1 ? a.H_stride : 1, a.cstep = cg.KW == 1 ? a.W_stride : 1;
-        a.lrow = KH == 1 ? 1 : a.H_stride, a.lcol = cg.KW == 1 ? 1 : a.W_stride;
-        int64_t best = INT64_MAX, RPbest = 0;
-        for (int lg = 5; lg >= 2; lg--) {
-            const int TW = 1 << lg, TH = 32 >> lg;
-            const int OWt = std::min(TW, a.OW), OHt = std::min(TH, a.OH);
-            const int64_t RW = (int64_t)(OWt - 1) * a.lcol + cg.KW, RH = (int64_t)(OHt - 1) * a.lrow + KH;
-            if (RW > 4096 || RH > 4096) continue;
-            const int64_t tx = (a.OW + TW - 1) / TW, ty = (a.OH + TH - 1) / TH;
-            const int64_t cost = tx * ty * (RW * RH + 16);
-            if (cost < best) {
-                best = cost, RPbest = RW * RH;
-                a.lgTW = lg, a.OWt = OWt, a.OHt = OHt, a.RW = (int)RW, a.tiles_x = (int)tx;
-                a.dTX = make_fastdiv((uint32_t)tx), a.dTI = make_fastdiv((uint32_t)(tx * ty));
-            }
-        }
-        U = RPbest * cg.CP * 4;
-        if (best == INT64_MAX || U > (cg.K == cg.CP && a.cstep == 1 && a.rstep == 1 ? 1024 : 512)) return false;
-        a.RP = (int)RPbest;
-        a.dRP = make_fastdiv((uint32_t)a.RP), a.dRW = make_fastdiv((uint32_t)a.RW);
-        tiles = (int64_t)N * a.dTI.d;
-    }
-    // K split: eight ways on long rows, and on the shortest, where a workgroup's time goes with the blocks it stores; else four; less where that
-    // takes more than 256 workgroups.  us at 8 / 4 / 2 / 1: 10 x 128 x 8 x 8 -> 64, 5 x 5 4.4 / 4.9 / 5.6 / 7.3, 5 x 64 x 2 x 5 -> 512, 1 x 1 4.0 / 4.0 / 4.2 / 4.5,
-    // 10 x 256 x 9 x 9 -> 256, 1 x 1 4.7 / 4.6 / 4.7 / 5.1.
-    int lgS = a.NP >= 16 || (a.NP <= 2 && tiles * KB <= 192) ? kLgW : 2;
-    auto groups_at = [&](int lg) { return (KB + (kWaves >> lg) - 1) >> (kLgW - lg); };
-    while (lgS > 0 && tiles * groups_at(lgS) > 256) lgS--;
-    if (tiles * groups_at(lgS) > most || (!fc && lgS == 0 && U > 384 && cg.K > cg.CP)) return false;
-    a.lgS = lgS;
-    out->wgs = (unsigned)(tiles * groups_at(lgS));
-    out->lds_bytes = std::max<int64_t>((int64_t)a.CP * a.RP * 16 + 16 + 8LL * a.NP, kThreads * 64);
-    if (out->lds_bytes > kLdsBytes) return false;
-    a.xo = make_xcd_order((uint64_t)tiles, (uint32_t)groups_at(lgS), false);
-    return true;
+    a.RW = p.RW, a.RP = p.RP;
+    a.rstep = p.rstep, a.cstep = p.cstep, a.lrow = p.lrow, a.lcol = p.lcol;
+    a.lgTW = p.lgTW, a.OWt = p.OWt, a.OHt = p.OHt, a.lgS = p.lgS;
+    a.dRP = make_fastdiv(p.fc ? (uint32_t)cg.CP * 16u : (uint32_t)p.RP);
+    a.dRW = make_fastdiv((uint32_t)p.RW), a.dTX = make_fastdiv(p.tiles_x), a.dTI = make_fastdiv(p.image_tiles);
+    a.xo = make_xcd_order((uint64_t)p.tiles, (uint32_t)p.groups, false);
+    return a;
 }
 
 }  // namespace
@@ -398,13 +331,14 @@ bool launch_direct_f4(int type, const float* d_x, const float* d_thr, const void
     // tuning aid, and off where another one forces a form of the layer kernels
     static const bool off = getenv("FTNN_NO_DIRECT_LAYERS") || getenv("FTNN_CONV_SPLIT") || getenv("FTNN_CONV_NO_BUFFER_LOADS") ||
                             getenv("FTNN_CONV_SMALL_BELOW") || getenv("FTNN_CONV_TILES_FROM");
-    DirectPlan p = {};
-    if (off || !direct_plan(type, d_x, cg, C, N, KN, &p)) return false;
+    DirectPlan p;
+    if (off || !direct_plan(type, cg, C, N, KN, &p)) return false;
     // One launch reads the input while it stores the result; a result that lies over its input (or the thresholds) needs the input
     // quantised before the first store.
     const int64_t y_bytes = 4LL * N * KN * cg.OH * cg.OW;
     if (ranges_meet(d_y, y_bytes, d_x, 4LL * N * C * cg.H * cg.W) || ranges_meet(d_y, y_bytes, d_thr, 4LL * N)) return false;
-    DirectArgs& a = p.a;
+    DirectArgs a = direct_args(p, cg, C, N, KN);
+    a.vec4 = C % 4 == 0 && reinterpret_cast<uintptr_t>(d_x) % 16 == 0;
     a.x = d_x, a.thr = d_thr, a.Wf = static_cast<const uint4*>(d_wf), a.Y = d_y;
     // BNN: the channel lanes past C are +1 in both operands; padding words are skipped
     a.bias = type == kBNN ? (float)(64 * cg.K - K_unpack) : 0.0f;
@@ -412,7 +346,7 @@ bool launch_direct_f4(int type, const float* d_x, const float* d_thr, const void
     a.lim = type == kTNN ? 0.5f : 0.0f;
     a.alpha = alpha;
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(p.wgs), dim3(kThreads), (size_t)p.lds_bytes, st, a);
+        hipLaunchKernelGGL(kern, dim3((unsigned)(p.tiles * p.groups)), dim3(kThreads), (size_t)p.lds_bytes, st, a);
         *err = hipGetLastError();
         return true;
     };

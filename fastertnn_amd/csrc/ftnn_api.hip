@@ -21,7 +21,6 @@
 #include "../../include/ftnn.h"
 #include "ftnn_internal.h"
 #include "host_hash.h"
-#include "layer_plans.h"
 
 static bool valu_ahead_of_rows(int type, int64_t M, bool nchw, int KN, int Kw);
 

@@ -3,15 +3,13 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "layer_plans.h"
 #include "pair_walk.h"
 
 namespace ftnn {
 
-constexpr int kTNN = 0, kTBN = 1, kBTN = 2, kBNN = 3;
-
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-inline int cpack_of(int C) { return (int)(((int64_t)C + 63) / 64); }
 inline int round4(int k) { return 4 * ((k + 3) / 4); }
 inline int out_dim(int in, int pad, int k, int stride) { return (in + 2 * pad - k) / stride + 1; }
 

@@ -8,6 +8,10 @@
 
 namespace ftnn {
 
+constexpr int kTNN = 0, kTBN = 1, kBTN = 2, kBNN = 3;
+
+inline int cpack_of(int C) { return (int)(((int64_t)C + 63) / 64); }
+
 inline bool ranges_meet(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
     const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
     return x < y + (uintptr_t)b_bytes && y < x + (uintptr_t)a_bytes;
@@ -51,5 +55,92 @@ inline bool dense_rows_from_input(bool ternary, int64_t pixels /* of the input *
 // 28 words, TBN 32.6 / 37.6), but 212064 -> 3, 32 words, BTN 118 / 70 and 10000 -> 10, 60 words, TNN 24.6 / 19.3.  Of 400 layers of 1 to 24 kernels 4 are 6 to
 // 9 % slower than on the vector ALU (15 by the first line alone).
 inline bool few_kernels(int64_t M, int KN, int Kw) { return (KN < 16 && Kw == 4) || (KN <= 8 && Kw <= 44 && M <= 100000); }
+
+// A small layer in one launch (k_direct_f4): eight wavefronts per workgroup, on a tile of 32 pixels or images.
+constexpr int kDirectLgWaves = 3;   // (four wavefronts: slower from two pieces of input on)
+constexpr uint32_t kDirectNowhere = 0x80000000u;   // an offset that, with a few planes added to it, lies beyond every image taken here
+struct DirectPlan {
+    bool fc;
+    int H, W, OH, OW;         // as the kernel sees the image: one row for 1 x 1 windows without a stride
+    int lgTW, OHt, OWt;       // a tile is 2^lgTW pixels wide; rows and columns of outputs that its region of the input serves
+    int RW, RP;               // the region: pixels of a row, in all
+    int rstep, cstep, lrow, lcol;
+    uint32_t tiles_x, image_tiles;
+    int lgS, groups;          // 2^lgS wavefronts split K; workgroups per tile
+    int64_t tiles, pieces, lds_bytes;
+};
+// Which layers run here, and how.  A workgroup's time grows with the pieces of input it fetches (512 dwords of records of 16 values at a
+// time; 2048 quads for a fully connected one), and a second workgroup per compute unit costs as much as the first.  Lines from 230
+// layers, both forms in a graph, us (two launches / here): 21 x 128 x 9 x 21 -> 256, 3 x 3 6.4 / 6.9 (300 workgroups), 20 x 128 x 20 x 20 ->
+// 128, 3 x 3 6.8 / 8.5 (300); two pieces of input with a window 19 x 256 x 10 x 10 -> 128, 3 x 3 stride 2 5.7 / 5.9, without one
+// 14 x 512 x 12 x 12 -> 64 5.4 / 4.8; all eight wavefronts on kernels of their own and nearly a whole piece 2 x 128 x 53 x 53 -> 256, 3 x 3
+// 7.7 / 8.2, half a piece 24 x 64 x 14 x 14 -> 256, 3 x 3 7.0 / 6.2; fully connected 9 x 2081 -> 3584 (4752 quads) 5.1 / 5.8,
+// 15 x 812 -> 6673 (3120) 5.0 / 5.3, 8 x 1337 -> 1121 (2688) 5.1 / 4.8.
+inline bool direct_plan(int type, const ConvGeom& cg, int C, int N, int KN, DirectPlan* out) {
+    constexpr int kWaves = 1 << kDirectLgWaves;
+    DirectPlan& a = *out;
+    a = DirectPlan();
+    const int KB = (KN + 31) / 32, KH = cg.K / (cg.CP * cg.KW), NP = (cg.K + 1) / 2;
+    const int64_t M = (int64_t)N * cg.OH * cg.OW;
+    const bool fc = a.fc = cg.H == 1 && cg.W == 1 && KH == 1 && cg.KW == 1 && cg.H_pad == 0 && cg.W_pad == 0;
+    const int most = fc ? 400 : 256;   // workgroups
+    if ((M + 31) / 32 * ((KB + kWaves - 1) / kWaves) > most) return false;
+    if (((int64_t)cg.CP * 64 + 64) * cg.H * cg.W * 4 > kDirectNowhere) return false;   // offsets within an image
+    a.H = cg.H, a.W = cg.W, a.OH = cg.OH, a.OW = cg.OW;
+    a.tiles_x = a.image_tiles = 1;
+    int64_t U;   // pieces of work in fetching a tile's input
+    if (fc) {
+        a.RP = a.RW = 32;
+        a.tiles = (N + 31) / 32;
+        U = (int64_t)std::min(32, N) * cg.CP * 16;
+        if (U > 3072) return false;
+        // binary weights take half the bytes as rows: 4 x 2312 -> 9837 (5.8 MB of records) 6.1 / 6.0, 3 x 2750 -> 12499 (8.6) 6.0 / 5.4 with the
+        // weights within the Infinity Cache, which larger ones need not be
+        if ((type == kTBN || type == kBNN) && (int64_t)KN * cg.CP * 16 > (8 << 20)) return false;
+    } else {
+        if (KH == 1 && cg.KW == 1 && cg.H_pad == 0 && cg.W_pad == 0 && cg.H_stride == 1 && cg.W_stride == 1) {
+            a.W = a.OW = cg.H * cg.W;
+            a.H = a.OH = 1;
+        }
+        a.rstep = KH == 1 ? cg.H_stride : 1, a.cstep = cg.KW == 1 ? cg.W_stride : 1;
+        a.lrow = KH == 1 ? 1 : cg.H_stride, a.lcol = cg.KW == 1 ? 1 : cg.W_stride;
+        int64_t best = INT64_MAX, RPbest = 0;
+        for (int lg = 5; lg >= 2; lg--) {
+            const int TW = 1 << lg, TH = 32 >> lg;
+            const int OWt = std::min(TW, a.OW), OHt = std::min(TH, a.OH);
+            const int64_t RW = (int64_t)(OWt - 1) * a.lcol + cg.KW, RH = (int64_t)(OHt - 1) * a.lrow + KH;
+            if (RW > 4096 || RH > 4096) continue;
+            const int64_t tx = (a.OW + TW - 1) / TW, ty = (a.OH + TH - 1) / TH;
+            const int64_t cost = tx * ty * (RW * RH + 16);
+            if (cost < best) {
+                best = cost, RPbest = RW * RH;
+                a.lgTW = lg, a.OWt = OWt, a.OHt = OHt, a.RW = (int)RW;
+                a.tiles_x = (uint32_t)tx, a.image_tiles = (uint32_t)(tx * ty);
+            }
+        }
+        U = RPbest * cg.CP * 4;
+        if (best == INT64_MAX || U > (cg.K == cg.CP && a.cstep == 1 && a.rstep == 1 ? 1024 : 512)) return false;
+        a.RP = (int)RPbest;
+        a.tiles = (int64_t)N * a.image_tiles;
+    }
+    a.pieces = U;
+    // K split: eight ways on long rows, and on the shortest, where a workgroup's time goes with the blocks it stores; else four; less where that
+    // takes more than 256 workgroups.  us at 8 / 4 / 2 / 1: 10 x 128 x 8 x 8 -> 64, 5 x 5 4.4 / 4.9 / 5.6 / 7.3, 5 x 64 x 2 x 5 -> 512, 1 x 1 4.0 / 4.0 / 4.2 / 4.5,
+    // 10 x 256 x 9 x 9 -> 256, 1 x 1 4.7 / 4.6 / 4.7 / 5.1.
+    a.lgS = NP >= 16 || (NP <= 2 && a.tiles * KB <= 192) ? kDirectLgWaves : 2;
+    auto groups_at = [&](int lg) { return (KB + (kWaves >> lg) - 1) >> (kDirectLgWaves - lg); };
+    while (a.lgS > 0 && a.tiles * groups_at(a.lgS) > 256) a.lgS--;
+    a.groups = groups_at(a.lgS);
+    if (a.tiles * a.groups > most || (!fc && a.lgS == 0 && U > 384 && cg.K > cg.CP)) return false;
+    // Fewer than four wavefronts on a K: a wavefront's run of pairs becomes what a workgroup takes longest for, a workgroup of many for one tile
+    // sooner than the only one, and tiles of a pixel or two are all store.  Of 1000 layers those that this leaves are 0.83 of the two launches' time in the
+    // mean, two of them slower by more than 3 % (5); without it 86, up to 1.86.  us, two launches / here: 26 x 224 x 3 x 6 -> 1429, 3 x 5 stride 2 (runs
+    // of 30) 6.8 / 12.0, 17 x 95 x 5 x 5 -> 1045, 3 x 3 (9, two workgroups per tile) 6.5 / 7.5, 26 x 40 x 3 x 3 -> 1810, 3 x 3 to one pixel 5.8 / 7.2,
+    // but 8 x 128 x 28 x 28 -> 128, 3 x 3 (5, the only one) 6.6 / 6.2.
+    const int run = (NP + (1 << a.lgS) - 1) >> a.lgS;
+    if (!fc && a.lgS <= 1 && (run > (a.groups == 1 ? 9 : 4) || 20 * M <= 3 * 32 * a.tiles)) return false;
+    a.lds_bytes = std::max<int64_t>((int64_t)cg.CP * a.RP * 16 + 16 + 8LL * NP, (64 << kDirectLgWaves) * 64);
+    return a.lds_bytes <= (64 << 10);
+}
 
 }  // namespace ftnn

@@ -26,7 +26,6 @@
 #include <type_traits>
 
 #include "ftnn_internal.h"
-#include "layer_plans.h"
 
 namespace ftnn {
 

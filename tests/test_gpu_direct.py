@@ -22,6 +22,13 @@ LINES = [(b, 64, 16, 16, 64, 3, 3, 1, 1) for b in (16, 17, 31, 32, 33, 65)] + [(
         [(4, c, 8, 8, 64, 1, 1, 0, 1) for c in (512, 513)] + [(1, 128, 53, 53, k, 3, 3, 1, 1) for k in (64, 256)]
 FC_LINES = [(3, c, 77) for c in (4096, 4097, 4160)] + [(17, 700, 12800), (17, 700, 12801), (1, 2752, 12190), (1, 2752, 12194)]
 
+# every split of K (2^lgS wavefronts on one) with one workgroup per tile and several, windows and none; tests/test_layer_plans.py holds each to its split
+SPLITS = {(2, 200, 4, 7, 31, 3, 3, 0, 1): (3, 1), (2, 200, 4, 7, 70, 3, 3, 0, 1): (3, 3), (2, 130, 6, 31, 20, 3, 1, 1, 1): (2, 1), (3, 100, 12, 13, 100, 3, 3, 1, 1): (2, 2),
+          (8, 128, 28, 28, 100, 3, 3, 1, 1): (1, 1), (60, 40, 8, 8, 250, 3, 3, 0, 1): (1, 2), (24, 64, 14, 13, 250, 3, 3, 1, 1): (0, 1), (20, 60, 12, 12, 500, 1, 1, 0, 1): (0, 2),
+          (20, 130, 9, 9, 270, 1, 1, 0, 1): (1, 3)}
+# left to two launches: a single pixel per tile, runs of 10 pairs of K words and more, or of five where a tile has several workgroups
+BEYOND = [(26, 40, 3, 3, 1810, 3, 3, 0, 1), (26, 224, 3, 6, 1429, 3, 5, 0, 2), (17, 95, 5, 5, 1045, 3, 3, 1, 1), (4, 79, 12, 12, 864, 3, 3, 1, 1), (24, 47, 6, 6, 600, 5, 5, 2, 1)]
+
 
 def _run(hip, typ, layer, alpha, thr=None, x=None, aligned=True):
     n, c, h, w, kn, kh, kw, pad, stride = layer
@@ -50,7 +57,7 @@ def _run(hip, typ, layer, alpha, thr=None, x=None, aligned=True):
 
 
 @pytest.mark.parametrize("typ", range(4), ids=[TYPE_NAMES[t] for t in range(4)])
-@pytest.mark.parametrize("layer", LAYERS + LINES, ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("layer", LAYERS + LINES + list(SPLITS) + BEYOND, ids=lambda v: "x".join(map(str, v)))
 def test_layers(hip, typ, layer):
     print("case", TYPE_NAMES[typ], layer, flush=True)
     _run(hip, typ, layer, -0.25)

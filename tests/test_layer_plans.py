@@ -84,3 +84,55 @@ int main() {
 }
 """)
     assert out == "ok\n"
+
+
+def _plans(tmp_path, layers):
+    """of each layer and type: whether it runs in one launch, lgS, workgroups per tile"""
+    geoms = []
+    for n, c, h, w, kn, kh, kw, pad, stride in layers:
+        oh, ow = (h + 2 * pad - kh) // stride + 1, (w + 2 * pad - kw) // stride + 1
+        geoms.append("{%d, %d, %d, %d, %d, %d, %d, %d, %d, %d, %d}" % (n, c, h, w, kn, kh, kw, pad, stride, oh, ow))
+    out = _run(tmp_path, r"""
+int main() {
+    const int layers[][11] = {""" + ", ".join(geoms) + r"""};
+    for (auto& l : layers) {
+        const int cp = cpack_of(l[1]);
+        const ConvGeom cg = {l[2], l[3], cp, l[9], l[10], l[6], cp * l[5] * l[6], l[7], l[7], l[8], l[8], make_fastdiv((uint32_t)l[10]), make_fastdiv((uint32_t)cp), make_fastdiv((uint32_t)l[6])};
+        for (int type = 0; type < 4; type++) {
+            DirectPlan p;
+            const bool runs = direct_plan(type, cg, l[1], l[0], l[4], &p);
+            if (runs && (p.lds_bytes > 65536 || p.tiles * p.groups > 400 || (p.groups << (3 - p.lgS)) * 32 < l[4])) exit(1);
+            printf("%d %d %d\n", runs, p.lgS, p.groups);
+        }
+    }
+}
+""").split()
+    v = [(out[i] == "1", int(out[i + 1]), int(out[i + 2])) for i in range(0, len(out), 3)]
+    return [v[i:i + 4] for i in range(0, len(v), 4)]
+
+
+def test_which_layers_run_in_one_launch(tmp_path):
+    """the shapes of tests/test_gpu_direct.py run where that file has them run"""
+    from tests.test_gpu_direct import BEYOND, FC, FC_LINES, LAYERS, LINES, SPLITS
+    two = {(2, 129, 3, 40, 40, 3, 3, 0, 3), (1, 64, 17, 17, 31, 7, 7, 3, 1)} | set(LINES[4:6] + LINES[7:10] + LINES[11:12] + LINES[13:]) | set(BEYOND)
+    layers = LAYERS + LINES + list(SPLITS) + BEYOND
+    for layer, plan in zip(layers, _plans(tmp_path, layers)):
+        assert [p[0] for p in plan] == [layer not in two] * 4, layer
+        if layer in SPLITS:
+            assert plan[0][1:] == SPLITS[layer], (layer, plan)
+    # fully connected: pieces of input, then records of binary weights beyond 8 MiB
+    fc = FC + FC_LINES
+    plans = _plans(tmp_path, [(n, c, 1, 1, kn, 1, 1, 0, 1) for n, c, kn in fc])
+    for layer, plan in zip(fc, plans):
+        runs = [True] * 4 if layer not in FC_LINES[1:3] else [False] * 4
+        if layer == FC_LINES[-1]:
+            runs = [True, False, True, False]
+        assert [p[0] for p in plan] == runs, layer
+
+
+def test_layers_that_measured_slower_in_one_launch(tmp_path):
+    slow = [(36, 44, 2, 2, 942, 5, 5, 2, 1), (38, 245, 6, 6, 636, 3, 3, 0, 2), (23, 178, 5, 5, 1432, 5, 5, 0, 1), (29, 44, 3, 3, 1295, 7, 7, 3, 2), (14, 110, 5, 5, 1169, 3, 3, 1, 1),
+            (22, 160, 2, 2, 1109, 5, 5, 2, 1), (29, 36, 3, 3, 1638, 3, 3, 0, 2), (3, 79, 28, 28, 227, 5, 2, 2, 1), (2, 69, 23, 23, 388, 5, 2, 2, 1)]
+    faster = [(8, 128, 28, 28, 128, 3, 3, 1, 1), (24, 64, 14, 14, 256, 3, 3, 1, 1), (1, 64, 16, 16, 256, 3, 3, 1, 1), (3, 64, 39, 39, 256, 1, 1, 0, 1)]
+    assert [p[0][0] for p in _plans(tmp_path, slow)] == [False] * len(slow)
+    assert [p[0][0] for p in _plans(tmp_path, faster)] == [True] * len(faster)
