@@ -5,6 +5,7 @@
 
 #include "layer_plans.h"
 #include "pair_walk.h"
+#include "product_forms.h"
 
 namespace ftnn {
 
@@ -257,13 +258,9 @@ hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* 
                           hipStream_t st);
 
 // ---- rows_kernels.hip: the fp4 matrix-core product of packed rows as they are, one launch, no scratch ----
-// fp32 sums of +-1 products stay exact, and the grid holds the product
-bool mm_rows_within_limits(int64_t M, int KN, int Kw);
+// (where mm_rows_within_limits: fp32 sums of +-1 products stay exact, and the grid holds the product)
 hipError_t launch_mm_rows(int type, const int64_t* d_a, const int64_t* d_b, int64_t M, int OHW, int KN, int Kw, int K_unpack,
                           float alpha, float* d_y, hipStream_t st);
-
-// whether that is ahead of both operands packed by a launch and multiplied then
-bool mm_rows_ahead_of_packing(int64_t M, int OHW, int KN, int Kw);
 
 // The same for operands in packed4 form (launch_mfma_pack4) with their rows' sums.  False where workgroup tiles through LDS (k_mfma_p4) are
 // ahead: nothing has been done then.
