@@ -56,6 +56,42 @@ inline bool dense_rows_from_input(bool ternary, int64_t pixels /* of the input *
 // 9 % slower than on the vector ALU (15 by the first line alone).
 inline bool few_kernels(int64_t M, int KN, int Kw) { return (KN < 16 && Kw == 4) || (KN <= 8 && Kw <= 44 && M <= 100000); }
 
+// How k_conv_f4 cuts a layer of M pixels, KN kernels and rows of K words.
+//
+// K split: enough wavefronts to occupy the chip's 1024 SIMDs, but no exchange where the tiles alone do that (a tile = 64
+// kernels x 64 pixels).  Where a wavefront's run of K is long, a second round of a few tiles costs more than the exchange.
+// Lines of the fp32 results: fits to 920 layers (every split and the small tile measured; the mean layer is 0.5 % from its
+// best); e.g. us on splits 1 / 2 / 4 / small tiles: 944 tiles x 135 words 36 / 29 / 30 / 37, 724 x 36 23 / 17 / 17 / 19, 320 x 200
+// 37 / 25 / 22 / 25, 216 x 18 10.2 / 8.9 / 8.0 / 7.7, 1568 x 144 54 / 57 / 57 / 70.  Hand-overs, which keep wavefronts shorter at the
+// end, have the lines of a sweep of their own (90 chains: 0.5 % from their best).
+//
+// Few 64 x 64 tiles: tiles of 32 x 32, four times the workgroups.  fp32 results of fewer than 120 words up to 300 tiles; but where 190 to
+// 256 tiles give most of the 256 compute units one workgroup each and a row is long (72 words), those are ahead unless the last
+// kernel tile is half empty.  Layer and quantiser in a graph, us, 64 x 64 split four ways / 32 x 32: 216 tiles x 108 words 9.8 / 10.4,
+// 240 x 99 11.2 / 11.7, 208 x 117 12.5 / 13.5 (20 such layers 3 % ahead in the mean); 160 x 99 10.8 / 10.2, 280 x 90 11.3 / 10.9, 196 x 36 7.3 / 7.2.
+//
+// Small tiles that do not fill the compute units and long rows: eight wavefronts split K.  A run of K words is a chain of loads, two pairs in
+// flight, and the exchange grows by 0.2 us.  Layer and quantiser in a graph, us, on four / eight wavefronts: 24 tiles x 392 words 12.1 / 10.1,
+// 99 x 525 19.2 / 15.0, 189 x 425 16.8 / 12.9, 158 x 196 9.5 / 8.4, 96 x 75 7.6 / 7.0; the other way 100 x 18 6.0 / 6.2, 976 x 18 7.6 / 9.2,
+// 305 x 72 8.8 / 9.4.  Of 213 layers the 86 within these lines take 0.75 - 1.0 of the time; hand-overs are of chains whose rows are shorter.
+struct LayerCut {
+    bool small, deep;   // tiles of 32 x 32; K split over eight wavefronts (of small tiles)
+    int split;          // over 1, 2 or 4 of a workgroup's wavefronts
+};
+// force_split: 0, or the split to take; small_below: -1, or the count of 64 x 64 tiles below which tiles are small (tuning aids)
+inline LayerCut layer_cut(int64_t M, int KN, int K, bool hand_over, int force_split, int64_t small_below) {
+    LayerCut c;
+    const int64_t tiles = ((M + 63) / 64) * ((KN + 63) / 64);
+    const bool long_run = !hand_over && K >= 40;
+    const int64_t from1 = hand_over ? 600 : long_run ? 1500 : 1024, from2 = hand_over ? 450 : long_run ? 800 : 520;
+    c.split = force_split ? force_split : tiles >= from1 ? 1 : tiles >= from2 ? 2 : 4;
+    while (c.split > 1 && (K + 1) / 2 < c.split) c.split /= 2;   // no wavefront without K words of its own, forced or not
+    const bool one_round = K >= 72 && tiles >= 190 && tiles <= 256 && (KN + 31) / 32 % 2 == 0;
+    c.small = tiles < (small_below >= 0 ? small_below : !hand_over && K < 120 && !one_round ? 300 : 150);
+    c.deep = c.small && !force_split && !hand_over && K >= 75 && ((M + 31) / 32) * ((KN + 31) / 32) <= 256;
+    return c;
+}
+
 // A small layer in one launch (k_direct_f4): eight wavefronts per workgroup, on a tile of 32 pixels or images.
 constexpr int kDirectLgWaves = 3;   // (four wavefronts: slower from two pieces of input on)
 constexpr uint32_t kDirectNowhere = 0x80000000u;   // an offset that, with a few planes added to it, lies beyond every image taken here
@@ -69,7 +105,7 @@ struct DirectPlan {
     int lgS, groups;          // 2^lgS wavefronts split K; workgroups per tile
     int64_t tiles, pieces, lds_bytes;
 };
-// Which layers run here, and how.  A workgroup's time grows with the pieces of input it fetches (512 dwords of records of 16 values at a
+// Which layers run there, and how.  A workgroup's time grows with the pieces of input it fetches (512 dwords of records of 16 values at a
 // time; 2048 quads for a fully connected one), and a second workgroup per compute unit costs as much as the first.  Lines from 230
 // layers, both forms in a graph, us (two launches / here): 21 x 128 x 9 x 21 -> 256, 3 x 3 6.4 / 6.9 (300 workgroups), 20 x 128 x 20 x 20 ->
 // 128, 3 x 3 6.8 / 8.5 (300); two pieces of input with a window 19 x 256 x 10 x 10 -> 128, 3 x 3 stride 2 5.7 / 5.9, without one

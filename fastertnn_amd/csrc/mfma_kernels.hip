@@ -1512,36 +1512,15 @@ hipError_t launch_conv_f4(int type, const void* d_p2, const void* d_wf, const Co
     const PairWalk pw = make_pair_walk(cg);
     // BNN: the channel lanes past C are +1 in both operands (see launch_mfma_gemm); padding words are skipped
     const int bias = type == kBNN ? 64 * cg.K - K_unpack : 0;
-    // K split: enough wavefronts to occupy the chip's 1024 SIMDs, but no exchange where the tiles alone do that (a tile = 64
-    // kernels x 64 pixels).  Where a wavefront's run of K is long, a second round of a few tiles costs more than the exchange.
-    // Lines of the fp32 results: fits to 920 layers (every split and the small tile measured; the mean layer is 0.5 % from its
-    // best); e.g. us on splits 1 / 2 / 4 / small tiles: 944 tiles x 135 words 36 / 29 / 30 / 37, 724 x 36 23 / 17 / 17 / 19, 320 x 200
-    // 37 / 25 / 22 / 25, 216 x 18 10.2 / 8.9 / 8.0 / 7.7, 1568 x 144 54 / 57 / 57 / 70.  Hand-overs, which keep wavefronts shorter at the
-    // end, have the lines of a sweep of their own (90 chains: 0.5 % from their best).
-    const int64_t tiles = ((M + 63) / 64) * ((KN + 63) / 64);
-    const bool long_run = qo.mode == 0 && cg.K >= 40;
-    const int64_t from1 = qo.mode != 0 ? 600 : long_run ? 1500 : 1024, from2 = qo.mode != 0 ? 450 : long_run ? 800 : 520;
-    int split = tiles >= from1 ? 1 : (tiles >= from2 ? 2 : 4);
     static const int tune = []() {   // tuning aid: force the K split (1, 2 or 4; anything else is ignored)
         const char* e = getenv("FTNN_CONV_SPLIT");
         const int v = e ? atoi(e) : 0;
         return (v == 1 || v == 2 || v == 4) ? v : 0;
     }();
-    if (tune) split = tune;
-    while (split > 1 && pw.NP < split) split /= 2;   // no wavefront without K words of its own, forced or not
-    const int tpb = 4 / split;   // pixel tiles per workgroup (see the kernel)
-    // Few 64 x 64 tiles: tiles of 32 x 32, four times the workgroups.  fp32 results of fewer than 120 words up to 300 tiles; but where 190 to
-    // 256 tiles give most of the 256 compute units one workgroup each and a row is long (72 words), those are ahead unless the last
-    // kernel tile is half empty.  Layer and quantiser in a graph, us, 64 x 64 split four ways / 32 x 32: 216 tiles x 108 words 9.8 / 10.4,
-    // 240 x 99 11.2 / 11.7, 208 x 117 12.5 / 13.5 (20 such layers 3 % ahead in the mean); 160 x 99 10.8 / 10.2, 280 x 90 11.3 / 10.9, 196 x 36 7.3 / 7.2.
-    const bool one_round = cg.K >= 72 && tiles >= 190 && tiles <= 256 && (KN + 31) / 32 % 2 == 0;
     static const int64_t tune_small = getenv("FTNN_CONV_SMALL_BELOW") ? atoi(getenv("FTNN_CONV_SMALL_BELOW")) : -1;
-    const bool small = tiles < (tune_small >= 0 ? tune_small : qo.mode == 0 && cg.K < 120 && !one_round ? 300 : 150);
-    // Small tiles that do not fill the compute units and long rows: eight wavefronts split K.  A run of K words is a chain of loads, two pairs in
-    // flight, and the exchange grows by 0.2 us.  Layer and quantiser in a graph, us, on four / eight wavefronts: 24 tiles x 392 words 12.1 / 10.1,
-    // 99 x 525 19.2 / 15.0, 189 x 425 16.8 / 12.9, 158 x 196 9.5 / 8.4, 96 x 75 7.6 / 7.0; the other way 100 x 18 6.0 / 6.2, 976 x 18 7.6 / 9.2,
-    // 305 x 72 8.8 / 9.4.  Of 213 layers the 86 within these lines take 0.75 - 1.0 of the time; hand-overs are of chains whose rows are shorter.
-    const bool deep = small && !tune && qo.mode == 0 && cg.K >= 75 && ((M + 31) / 32) * ((KN + 31) / 32) <= 256;
+    const LayerCut cut = layer_cut(M, KN, cg.K, qo.mode != 0, tune, tune_small);
+    const int split = cut.split, tpb = 4 / split;   // pixel tiles per workgroup (see the kernel)
+    const bool small = cut.small, deep = cut.deep;
     dim3 grid((unsigned)(((M + 63) / 64 + tpb - 1) / tpb), (unsigned)((KN + 63) / 64));
     if (small) grid = dim3((unsigned)((M + 31) / 32), (unsigned)(qo.mode != 0 ? 2 * ((KN + 63) / 64) : (KN + 31) / 32));
     if (M > 0x7fffff00LL) return hipErrorInvalidValue;   // pixel indices stay below 2^31

@@ -106,9 +106,9 @@ def test_row_major_gemm_all_types(hip, oracle, typ, mnk):
 @pytest.mark.parametrize("typ", ALL_TYPES, ids=lambda t: TYPE_NAMES[t])
 @pytest.mark.parametrize("shape", [(3333, 1, 1, 3100, 4), (5, 29, 29, 2700, 12)], ids=["row_major", "nchw"])
 def test_matrix_core_engines_with_256x256_tiles(hip, oracle, typ, shape):
-    """the tile kernels work on 256 x 256 tiles from 160 of those on; below, the int8 engine takes smaller tiles and the fp4 engine
-    multiplies the packed rows: the cases above are all of the first kind, these are of the second (ragged in both
-    directions, row-major and NCHW stores)"""
+    """from 160 tiles of 256 x 256 on the int8 engine works on such tiles; below, on smaller ones: the cases above are all of the first
+    kind, these are of the second (ragged in both directions, row-major and NCHW stores).  The fp4 engine multiplies the packed rows of
+    both; its 256 x 256 tiles take long rows (test_every_form in tests/test_gpu_product_forms.py)"""
     n, oh, ow, kn, kw = shape
     m = n * oh * ow
     assert ((m + 255) // 256) * ((kn + 255) // 256) >= 160
@@ -148,8 +148,8 @@ def test_matrix_core_engines_with_128x128_tiles(hip, oracle, typ, shape):
 
 @pytest.mark.parametrize("typ", ALL_TYPES, ids=lambda t: TYPE_NAMES[t])
 def test_weights_kept_in_engine_form_serve_every_batch(hip, oracle, typ):
-    """ftnn_expand_rows once for the weights, then ftnn_mm_expanded for activations of several sizes: few rows (128 x 128
-    tiles), many rows (256 x 256 tiles), a conv-shaped result; the engine form of an operand must not depend on the
+    """ftnn_expand_rows once for the weights, then ftnn_mm_expanded for activations of several sizes: few rows, many rows
+    (256 x 256 tiles on the int8 engine), a conv-shaped result; the engine form of an operand must not depend on the
     other operand or on the tiling that a call picks.  Both matrix-core engines, ragged everywhere, K tail."""
     kn, kw = 2700, 8
     ku = 64 * kw - 5

@@ -1,5 +1,5 @@
-"""Products of operands kept in the fp4 engine's form whose wavefronts split K (k_packed in fastertnn_amd/csrc/rows_kernels.hip): every
-tile at ragged edges, rows shorter than a workgroup has wavefronts, K shares of every remainder, row-major and NCHW results, all
+"""Products of operands kept in the fp4 engine's form (k_packed in fastertnn_amd/csrc/rows_kernels.hip; every form of it is reached by
+tests/test_gpu_product_forms.py): tiles at ragged edges, rows shorter than a workgroup has wavefronts, K shares of every remainder, row-major and NCHW results, all
 types, bit for bit against the vector-ALU engine, with nothing written past the result."""
 import pytest
 import torch
@@ -12,9 +12,9 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(1, 1, 1, 1, 4), (33, 1, 1, 65, 4), (31, 1, 1, 32, 8), (130, 1, 1, 500, 36), (64, 1, 1, 33, 20), (2, 3, 5, 40, 12), (3, 7, 11, 129, 28),
           # ... and on eight, short and long shares
           (1, 1, 1, 1, 172), (36, 1, 1, 246, 244), (33, 1, 1, 90, 300), (1, 5, 9, 70, 204),
-          # 32 x 64, 64 x 32 (and the other way around where the result is NCHW)
+          # many results of short rows: tiles of 32 x 32 of the wavefronts' own; (2102, ..., 24) 64 x 32 on four wavefronts
           (645, 1, 1, 1549, 4), (3, 17, 31, 1005, 4), (2102, 1, 1, 467, 24), (1, 30, 49, 650, 24),
-          # 64 x 64, 96 x 96, 128 x 128, then k_mfma_p4
+          # 64 x 64, 96 x 96, 128 x 128, then the wavefronts' own tiles again
           (551, 1, 1, 935, 160), (1, 20, 46, 560, 164), (1149, 1, 1, 1841, 136), (1, 43, 43, 1140, 140), (1698, 1, 1, 1874, 204), (1, 43, 44, 1700, 208),
           (1330, 1, 1, 2330, 4), (2, 32, 33, 1500, 4),
           # more than 160 tiles of 256 x 256, narrow

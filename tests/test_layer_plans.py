@@ -1,6 +1,6 @@
 """The rules by which layers are cut into launches (fastertnn_amd/csrc/layer_plans.h, the code the launchers run): the grid over the dense
-rows of a few-channel layer, up to the most output pixels a call may have, which form makes them, and the comparison of a result's place with its input's.
-CPU only."""
+rows of a few-channel layer, up to the most output pixels a call may have, which form makes them and where few kernels leave the matrix cores, the
+comparison of a result's place with its input's, which layers run in one launch, and how the layer kernel cuts the others.  CPU only."""
 import os
 import subprocess
 
@@ -136,3 +136,36 @@ def test_layers_that_measured_slower_in_one_launch(tmp_path):
     faster = [(8, 128, 28, 28, 128, 3, 3, 1, 1), (24, 64, 14, 14, 256, 3, 3, 1, 1), (1, 64, 16, 16, 256, 3, 3, 1, 1), (3, 64, 39, 39, 256, 1, 1, 0, 1)]
     assert [p[0][0] for p in _plans(tmp_path, slow)] == [False] * len(slow)
     assert [p[0][0] for p in _plans(tmp_path, faster)] == [True] * len(faster)
+
+
+def test_cut_of_layers(tmp_path):
+    """the shapes of tests/test_gpu_deep_layers.py stand on the sides of the lines that they are there for: eight wavefronts on one tile from
+    75 words on and up to 256 tiles of 32 x 32, never with a split forced or a hand-over"""
+    from tests.test_gpu_deep_layers import LAYERS
+    deep = [layer not in (LAYERS[0], LAYERS[7], LAYERS[-1]) for layer in LAYERS]
+    assert not any(p[0] for plan in _plans(tmp_path, LAYERS) for p in plan)   # none in one launch
+    rows = []
+    for n, c, h, w, kn, kh, kw, pad, stride in LAYERS:
+        oh, ow = (h + 2 * pad - kh) // stride + 1, (w + 2 * pad - kw) // stride + 1
+        rows.append((n * oh * ow, kn, -(-c // 64) * kh * kw))
+    out = _run(tmp_path, r"""
+int main() {
+    const long v[][3] = {""" + ", ".join("{%d, %d, %d}" % r for r in rows) + r"""};
+    for (auto& l : v) {
+        const LayerCut c = layer_cut(l[0], l[1], l[2], false, 0, -1);
+        if (layer_cut(l[0], l[1], l[2], true, 0, -1).deep || layer_cut(l[0], l[1], l[2], false, 4, -1).deep || (c.deep && !c.small)) return 1;
+        printf("%d ", c.deep);
+    }
+    // every split keeps a pair of words for each wavefront; results with few tiles take small ones
+    for (long tiles : {1, 149, 150, 299, 300, 449, 450, 519, 520, 599, 600, 799, 800, 1023, 1024, 1499, 1500})
+        for (int K : {1, 2, 3, 4, 5, 8, 39, 40, 119, 120})
+            for (bool hand_over : {false, true}) {
+                const LayerCut c = layer_cut(64 * tiles, 64, K, hand_over, 0, -1);
+                const long from1 = hand_over ? 600 : K >= 40 ? 1500 : 1024, from2 = hand_over ? 450 : K >= 40 ? 800 : 520;
+                const int want = tiles >= from1 ? 1 : tiles >= from2 ? 2 : 4;
+                if ((K + 1) / 2 < c.split || c.split > want || ((K + 1) / 2 >= want && c.split != want)) return 2;
+                if (c.small != (tiles < (hand_over || K >= 120 ? 150 : 300))) return 3;
+            }
+}
+""")
+    assert [v == "1" for v in out.split()] == deep, list(zip(LAYERS, rows, out.split()))

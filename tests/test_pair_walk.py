@@ -49,7 +49,7 @@ void layer(int CP, int H, int W, int KH, int KW, int pad, int64_t images) {
         for (int64_t img : {(int64_t)0, images - 1})
             for (int h = 0; h < 2; h++) {
                 share<UNIT, true>(pw, cg, img, at[0], at[1], 0, pw.NP, h);
-                for (int S : {2, 4})
+                for (int S : {2, 4, 8})
                     for (int ks = 0; ks < S; ks++)
                         share<UNIT, false>(pw, cg, img, at[0], at[1], (int)((uint32_t)(pw.NP * ks) / S), (int)((uint32_t)(pw.NP * (ks + 1)) / S), h);
             }

@@ -1,5 +1,5 @@
-"""Which form of a matrix-core product runs (fastertnn_amd/csrc/product_forms.h, the code the launchers run): the choice between estimates that say
-the same.  CPU only."""
+"""Which form of a matrix-core product runs (fastertnn_amd/csrc/product_forms.h, the code the launchers run): the forms that the
+shapes of the GPU tests are there for, and the choice between estimates that say the same.  CPU only."""
 import os
 import subprocess
 
@@ -42,3 +42,21 @@ def test_a_tie_keeps_the_smaller_tile(choose):
     clear = {(896, 1, 1, 873, 20): 4, (240, 1, 1, 5957, 24): 4, (332, 1, 1, 8180, 4): 4, (2506, 1, 1, 1365, 8): 4, (3328, 1, 1, 3328, 16): 6, (1024, 1, 1, 1024, 128): 1, (1999, 1, 1, 1733, 228): 3, (1, 1, 1, 7660, 120): 5}
     for shapes in (ties, clear):
         assert {s: c[1] for s, c in zip(shapes, choose(shapes))} == shapes
+
+
+def test_shapes_of_the_gpu_test_run_the_forms_they_are_there_for(choose):
+    from tests.test_gpu_product_forms import FORMS
+    reached = {"rows": {}, "kept": {}}
+    for (n, oh, ow, kn, kw), want, got in zip(FORMS, FORMS.values(), choose(list(FORMS))):
+        m, row = n * oh * ow, oh * ow if oh * ow > 1 else kn
+        small = -(-m // 256) * -(-kn // 256) < 160 or kn < 128 or m < 128   # from packed rows without an estimate (mm_from_rows)
+        assert (got[1] if small or got[0] else 7, got[2]) == want, (n, oh, ow, kn, kw)
+        past = row % 16 == 0 or m * kn <= 4 << 20   # stores_past_caches
+        for side, form in zip(("rows", "kept"), want):
+            reached[side].setdefault(form, set()).update((past, "nchw" if oh * ow > 1 else "row-major"))
+    # forms on up to 256 tiles of 32 x 32 have no large results, nor does any choice of 32 x 32 on four wavefronts
+    small_only = {"rows": (0, 5), "kept": (0, 1)}
+    for side, count in (("rows", 8), ("kept", 10)):
+        for form in range(count):
+            want = {True, "nchw", "row-major"} | (set() if form in small_only[side] else {False})
+            assert reached[side][form] == want, (side, form)
