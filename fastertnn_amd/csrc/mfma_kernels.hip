@@ -521,19 +521,23 @@ __device__ __forceinline__ void store_tile_offset(const Acc<true>::type (&acc)[W
     }
 }
 
-// The fp4 GEMM on packed4 operands.  Same tiling as k_mfma<true, ...> (2 x 2 wavefronts, WT x WT blocks of 32 x 32 each,
-// steps of two K words, ring of kNS stages filled by LDS-direct loads that the kernel counts by hand), with one 1 KiB block
+// The fp4 GEMM on packed4 operands.  Same tiling as k_mfma<true, ...> (2 x 2 wavefronts, 4 x 4 blocks of 32 x 32 each,
+// steps of two K words, ring of four stages filled by LDS-direct loads that the kernel counts by hand), with one 1 KiB block
 // per row block and step.  A step: the first K word's 16 multiplies run while the second one's operands are unpacked;
 // then the barrier; the second K word's multiplies run beside the loads of stage s + kNS and the LDS reads of stage
 // s + 1, one read per slot of two multiplies (a 16-byte LDS read holds the wavefront's issue for 16 cycles), each block
 // unpacked LAG slots after its read -- the last LAG blocks in the first slots of the next step.
-template <bool SWAP, bool NT, int WT, int kNS>
+struct TileP4 {
+    static constexpr int WT = 4, NS = 4;
+    static constexpr size_t lds_bytes = (size_t)NS * 4 * WT * 1024;
+};
+template <bool SWAP, bool NT>
 __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, const uint4* __restrict__ Qc, float* __restrict__ Y,
                                                  int M, int KN, int OHW, int KP, const int* __restrict__ sP,
                                                  const int* __restrict__ sQ, int off, int form, float alpha) {
     extern __shared__ uint4 lds[];   // kNS stages of kFR KiB
     typedef typename Acc<true>::type acc_t;
-    constexpr int RB = 2 * WT, kFR = 2 * RB, kFW = kFR / 4, NL = 2 * WT;   // kFW = WT blocks staged per wavefront and step
+    constexpr int WT = TileP4::WT, kNS = TileP4::NS, RB = 2 * WT, kFR = 2 * RB, kFW = kFR / 4, NL = 2 * WT;   // kFW = WT blocks staged per wavefront and step
     static_assert(NL % kFW == 0 && (NL / 2) % 2 == 0, "loads and reads spread evenly over the slots");
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -604,7 +608,7 @@ __global__ __launch_bounds__(256) void k_mfma_p4(const uint4* __restrict__ Pc, c
     // slots between the LDS read of a block and its unpacking: far enough for the read to have landed, near enough for
     // every block to be unpacked by the slot that multiplies it first (block b: slot 0 for P block 0, (b - 1) / (WT / 2)
     // for Q block b - 1, 2 (b - WT) for P block b - WT)
-    constexpr int LAG = WT >= 4 ? 4 : 3;
+    constexpr int LAG = 4;
     static_assert(LAG <= NL - 1 && LAG <= NL - WT + (WT - 1) / (WT / 2) && LAG <= WT + 1, "a block is unpacked before its first multiply");
     auto step_body = [&](int s, auto full_tag) {
         constexpr bool FULL = decltype(full_tag)::value;   // FULL: s + kNS < nstep
@@ -1282,23 +1286,21 @@ hipError_t launch_expand(bool tern, const uint32_t* rows_ptr, int rows, int G, u
 template <bool SWAP, bool NT>
 hipError_t launch_gemm_p4_as(const uint4* Pc, const uint4* Qc, float* Y, int M, int KN, int OHW, int KP, const int* sP,
                                const int* sQ, int off, int form, float alpha, hipStream_t st) {
-    constexpr int WT = 4, NS = 4;
-    auto kern = k_mfma_p4<SWAP, NT, WT, NS>;
-    constexpr size_t lds_bytes = (size_t)NS * 4 * WT * 1024;
+    auto kern = k_mfma_p4<SWAP, NT>;
     // hand-counted LDS-direct loads: no scratch (see launch_gemm_tile); the opt-in to more than 64 KiB of LDS is per kernel
     static const hipError_t configured = []() {
-        const void* k = reinterpret_cast<const void*>(&k_mfma_p4<SWAP, NT, WT, NS>);
+        const void* k = reinterpret_cast<const void*>(&k_mfma_p4<SWAP, NT>);
         hipFuncAttributes attr;
         hipError_t e = hipFuncGetAttributes(&attr, k);
         if (e == hipSuccess && attr.localSizeBytes != 0) e = hipErrorLaunchFailure;
         if (e != hipSuccess) return e;
-        return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)((size_t)NS * 4 * WT * 1024));
+        return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)TileP4::lds_bytes);
     }();
     if (configured != hipSuccess) return configured;
-    const int prow = SWAP ? KN : M, qrow = SWAP ? M : KN, edge = 64 * WT;
+    const int prow = SWAP ? KN : M, qrow = SWAP ? M : KN, edge = 64 * TileP4::WT;
     dim3 grid((prow + edge - 1) / edge, (qrow + edge - 1) / edge);
     if (grid.y > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, st, Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha);
+    hipLaunchKernelGGL(kern, grid, dim3(256), TileP4::lds_bytes, st, Pc, Qc, Y, M, KN, OHW, KP, sP, sQ, off, form, alpha);
     return hipGetLastError();
 }
 
