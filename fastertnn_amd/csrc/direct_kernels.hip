@@ -18,9 +18,9 @@
 // What bounds it: the chain launch -> arguments -> input -> LDS -> multiplies -> LDS -> result, 2.5 to 3 us beside the launch, and
 // the L1, which delivers the pieces of the input's rows a cache line at a time.  Every tile reads its halo and every workgroup
 // all channels, so this is for small layers only (direct_plan).  Device time in a graph, us, quantiser + layer kernel / here:
-// 8 x 128 x 28 x 28 -> 128, 3 x 3 6.6 / 6.2; 1 x 64 x 16 x 16 -> 256, 3 x 3 5.1 / 4.1; 3 x 64 x 39 x 39 -> 256, 1 x 1 6.3 / 5.1; 8 x 512 -> 1000
-// fully connected 4.9 / 4.2; 1 x 7660 -> 413 6.2 / 4.8: 0.87 in the mean of 110 layers.  Queued from Python 9.7 / 7.2 with 3.5 us of
-// arguments each.
+// 8 x 128 x 28 x 28 -> 128, 3 x 3 6.5 / 6.2; 1 x 64 x 16 x 16 -> 256, 3 x 3 5.1 / 4.4; 3 x 64 x 39 x 39 -> 256, 1 x 1 6.5 / 5.3; 8 x 512 -> 1000
+// fully connected 4.9 / 4.3; 1 x 7660 -> 413 6.1 / 4.9: 0.84 in the mean of 800 layers with a window.  Queued from Python, where a launch is also 2.2 us of the
+// host's, the same five 7.6 / 6.1, 7.6 / 4.3, 7.6 / 5.1, 7.8 / 4.2, 7.7 / 4.8.
 #include "ftnn_internal.h"
 
 namespace ftnn {

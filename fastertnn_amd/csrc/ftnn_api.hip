@@ -1145,9 +1145,11 @@ static int select_engine(int type, int64_t M, int KN, int Kw) {
 //   * a row is one group of words and the results are some, but not many (1001 x 700 x 256 NCHW TNN 6.2 / 6.7, 1572 x 700 x 256 BNN NCHW
 //     6.5 / 6.9).  Where they are many the stores are all there is, and rows are ahead again (1250001 x 16 TNN 50 / 46, 645162 x 31 TNN
 //     99 / 28, 312501 x 64 BNN NCHW 25 / 18, 14001 x 250 TNN NCHW 11.0 / 8.2, 7143 x 700 BTN 11.0 / 8.7, 8001 x 250 BTN NCHW 10.3 / 6.8), but for a few
-//     columns (2500001 x 8 TBN 60 / 65).  `many` is where that had shown on every shape measured.
-// With these lines 2 in 100 products of the sweep are more than 5 % slower than on the vector ALU (16 in 100 without them), and the
-// mean over all is 0.6 % from the better of the two (2.0).
+//     columns (2500001 x 8 TBN 60 / 65).  `many` is where that had shown on every shape measured, and far on for row-major
+//     products of 16 to 64 columns from 100000 rows on: 45 of those below it took 1.1 to 3.7 times as long as from rows (121879 x 30 BNN
+//     22 / 6.0, 110966 x 42 TNN 28 / 9.1).
+// With these lines 3 in 100 of 600 other products are more than 5 % slower than on the vector ALU (16 in 100 without them), and the
+// mean is 1.1 % from the better of the two (2.1).
 static bool valu_ahead_of_rows(int type, int64_t M, bool nchw, int KN, int Kw) {
     const int64_t results = M * KN;
     const int short_rows = type == kTNN ? 16 : type != kBNN ? 64 : M <= 256 && KN < 128 ? 4096 : 256;

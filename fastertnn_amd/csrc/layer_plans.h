@@ -169,8 +169,8 @@ inline bool direct_plan(int type, const ConvGeom& cg, int C, int N, int KN, Dire
     a.groups = groups_at(a.lgS);
     if (a.tiles * a.groups > most || (!fc && a.lgS == 0 && U > 384 && cg.K > cg.CP)) return false;
     // Fewer than four wavefronts on a K: a wavefront's run of pairs becomes what a workgroup takes longest for, a workgroup of many for one tile
-    // sooner than the only one, and tiles of a pixel or two are all store.  Of 1000 layers those that this leaves are 0.83 of the two launches' time in the
-    // mean, two of them slower by more than 3 % (5); without it 86, up to 1.86.  us, two launches / here: 26 x 224 x 3 x 6 -> 1429, 3 x 5 stride 2 (runs
+    // sooner than the only one, and tiles of a pixel or two are all store.  Of 1000 layers this leaves 801, which take 0.84 of the two launches' time in
+    // the mean, two of them up to 5 % more; without it 86 took more than 3 % more, up to 1.86 times as long.  us, two launches / here: 26 x 224 x 3 x 6 -> 1429, 3 x 5 stride 2 (runs
     // of 30) 6.8 / 12.0, 17 x 95 x 5 x 5 -> 1045, 3 x 3 (9, two workgroups per tile) 6.5 / 7.5, 26 x 40 x 3 x 3 -> 1810, 3 x 3 to one pixel 5.8 / 7.2,
     // but 8 x 128 x 28 x 28 -> 128, 3 x 3 (5, the only one) 6.6 / 6.2.
     const int run = (NP + (1 << a.lgS) - 1) >> a.lgS;

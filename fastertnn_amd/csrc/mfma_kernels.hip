@@ -1598,10 +1598,12 @@ hipError_t launch_mm_mfma(bool f4, int type, const int64_t* d_a, const int64_t* 
                           int KN, int Kw, int K_unpack, float alpha, float* d_y, void* d_scratch,
                           hipStream_t st) {
     const bool a_tern = (type == kTNN || type == kTBN), b_tern = (type == kTNN || type == kBTN);
-    // A product that packs its operands first may have its result over them, whatever the estimates say.
-    const int64_t y_bytes = 4 * M * KN;
-    const bool over = ranges_meet(d_y, y_bytes, d_a, M * Kw * (a_tern ? 16 : 8)) || ranges_meet(d_y, y_bytes, d_b, (int64_t)KN * Kw * (b_tern ? 16 : 8));
-    if (f4 && (mm_from_rows(M, KN, Kw) || (!over && mm_rows_ahead_of_packing(M, OHW, KN, Kw))))
+    // a product that packs its operands first may have its result over them, whatever the estimates say (asked within mm_rows_within_limits only)
+    auto over = [&]() {
+        const int64_t y_bytes = 4 * M * KN;
+        return ranges_meet(d_y, y_bytes, d_a, M * Kw * (a_tern ? 16 : 8)) || ranges_meet(d_y, y_bytes, d_b, (int64_t)KN * Kw * (b_tern ? 16 : 8));
+    };
+    if (f4 && (mm_from_rows(M, KN, Kw) || (mm_rows_ahead_of_packing(M, OHW, KN, Kw) && !over())))
         return launch_mm_rows(type, d_a, d_b, M, OHW, KN, Kw, K_unpack, alpha, d_y, st);
     if (f4) {   // the fp4 GEMM takes its operands at two bits per lane
         void* Ac = d_scratch;

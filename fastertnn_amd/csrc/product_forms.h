@@ -53,7 +53,7 @@ constexpr double kRowsTie = 0.99;
 inline int rows_form(int64_t prow, int64_t qrow, int Kw) { return form_of(kRowsForms, kRowsFormsOfRows, kRowsTie, prow, qrow, Kw); }
 
 inline bool mm_rows_within_limits(int64_t M, int KN, int Kw) {
-    return 64LL * Kw < (1LL << 24) && rows_tiles(M, KN, 128) <= kMaxRowsTiles;
+    return 64LL * Kw < (1LL << 24) && M <= 0x7fffffffLL && rows_tiles(M, KN, 128) <= kMaxRowsTiles;   // (more rows are more tiles, or overflow)
 }
 // whether the product of the rows as they are is ahead of both operands packed by a launch and multiplied then
 inline bool mm_rows_ahead_of_packing(int64_t M, int64_t OHW, int KN, int Kw) {

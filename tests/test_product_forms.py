@@ -22,7 +22,8 @@ int main() {
     int kn, kw;
     while (scanf("%lld %lld %lld %d %d", &n, &oh, &ow, &kn, &kw) == 5) {
         const long long M = n * oh * ow, OHW = oh * ow, p = OHW > 1 ? kn : M, q = OHW > 1 ? M : kn;
-        printf("%d %d %d\n", mm_rows_ahead_of_packing(M, OHW, kn, kw), rows_form(p, q, kw), packed_form(p, q, kw / 2));
+        if (M > 0x7fffffffLL) printf("%d 0 0\n", mm_rows_within_limits(M, kn, kw));   // (no such product is launched)
+        else printf("%d %d %d\n", mm_rows_ahead_of_packing(M, OHW, kn, kw), rows_form(p, q, kw), packed_form(p, q, kw / 2));
     }
 }
 """)
@@ -60,3 +61,10 @@ def test_shapes_of_the_gpu_test_run_the_forms_they_are_there_for(choose):
         for form in range(count):
             want = {True, "nchw", "row-major"} | (set() if form in small_only[side] else {False})
             assert reached[side][form] == want, (side, form)
+
+
+def test_limits_of_sizes_that_no_call_launches(choose):
+    """rows up to the largest that a size query may name: refused without an overflow (the program above is built to end there)"""
+    last = 0x7fffffff
+    assert choose([(last, last, 1, last, 4), (last, last, 1, 1, 4), (1 << 31, 1, 1, 1, 4), (last, 1, 1, 1, 4)])[:3] == [(0, 0, 0)] * 3
+    assert choose([(last, 1, 1, last, 4)])[0][0] == 0 and choose([(16777208 * 128, 1, 1, 1, 4)])[0][0] == 1
