@@ -95,3 +95,31 @@ def test_more_than_2_to_29_pixels(hip, typ, c, kn):
 @pytest.mark.parametrize("layer", PLANES + FEW_PLANES, ids=lambda v: "x".join(map(str, v)))
 def test_from_bit_planes(hip, oracle, typ, layer):
     _check(hip, oracle, typ, layer, (None, hip.ENGINE_AUTO, hip.ENGINE_VALU) if layer in PLANES else (hip.ENGINE_VALU,))
+
+
+@pytest.mark.parametrize("layer", [LAYERS[2], PLANES[0], FEW[0]], ids=("input", "planes", "one channel"))
+def test_under_capture(hip, layer):
+    """replays between eager work, each on another input"""
+    import torch
+    n, c, h, w, kn, kh, kw, pad, stride = layer
+    print("case", layer, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x = torch.randn((n, c, h, w), generator=g, device="cuda")
+    thr = torch.full((n,), 0.4, device="cuda")
+    qw = hip.pack_weights(torch.randn((kn, c, kh, kw), generator=g, device="cuda"), torch.full((kn,), 0.5, device="cuda"), True)
+    oh, ow = hip.out_dim(h, pad, kh, stride), hip.out_dim(w, pad, kw, stride)
+    out = torch.empty((n, kn, oh, ow), device="cuda")
+    scratch = torch.empty(hip.conv_scratch_bytes(0, n, c, h, w, kn, kh, kw, pad, stride), dtype=torch.uint8, device="cuda")
+    once = lambda y: hip.conv(0, x, thr, qw, kn, kh, kw, pad, stride, 0.5, scratch=scratch, out=y, engine=hip.ENGINE_VALU)
+    once(out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        once(out)
+    for rep in range(4):
+        x.normal_()
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = once(torch.empty_like(out))
+        assert torch.equal(out, want), rep
